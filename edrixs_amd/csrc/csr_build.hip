@@ -9,18 +9,20 @@
 // order and equal columns are summed left to right in term order, exact zeros
 // retained.  Values are val * sign * ham_sign.
 //
-// Device mapping: one 64-lane wavefront per row.  Lanes evaluate 64 terms at a
-// time; survivors are compacted with a ballot into an LDS list that stays in
-// term order; the list is bitonic-sorted on the key (column << 32 | term << 1 |
-// sign), which orders by column and, within a column, by term; a head lane per
-// column then sums its run sequentially, which is exactly the reference's
-// accumulation order.  A count pass sizes the rows, an exclusive scan (int64)
-// builds row pointers, a fill pass writes columns and values.
+// A count pass sizes the rows, an exclusive scan (int64) builds row pointers, a
+// fill pass writes columns and values.  Two kernels do the passes:
+//   * k_plan_count / k_plan_fill (termplan.hip), for complete bases: 64 rows per
+//     workgroup over the terms grouped by column;
+//   * k_build, for incomplete bases (columns found by search), more than 4096
+//     terms, or rows longer than the plan kernels' LDS lists (255 entries, about 185
+//     with words of more than 32 bits): one 64-lane wavefront per row.  Lanes
+//     evaluate 64 terms at a time; survivors are compacted with a ballot into an
+//     LDS list that stays in term order; the list is bitonic-sorted on the key
+//     (column << 32 | term << 1 | sign), which orders by column and, within a
+//     column, by term; a head lane per column then sums its run sequentially,
+//     which is exactly the reference's accumulation order.
 
 namespace {
-
-enum { ROW_PLAIN = 0, ROW_COREHOLE = 1, ROW_FULLCORE = 2 };
-enum { COL_PLAIN = 0, COL_COREHOLE = 1, COL_VALONLY = 2 };
 
 struct BuildParams {
     int64_t M;             // rows
@@ -312,7 +314,9 @@ __global__ void k_to_c64(int64_t n, const double2 *in, float2 *out) {
 // ------------------------------------------------------------ host driver
 
 struct TermTable {
-    uint32_t *d_ops = nullptr;
+    std::vector<uint32_t> ops;       // packed 0-based operator positions, one byte each
+    std::vector<double2> vals;
+    uint32_t *d_ops = nullptr;       // device copies, made by upload_terms
     double2 *d_vals = nullptr;
     int nhop = 0, T = 0;
     ~TermTable() {
@@ -321,15 +325,17 @@ struct TermTable {
     }
 };
 
-int upload_terms(const edx_tensor2 *hop, int64_t nhop, const edx_tensor4 *coul, int64_t ncoul,
-                 TermTable &tt) {
+int parse_terms(const edx_tensor2 *hop, int64_t nhop, const edx_tensor4 *coul, int64_t ncoul,
+                TermTable &tt) {
     EDX_CHECK(nhop >= 0 && ncoul >= 0 && nhop + ncoul < (1 << 29), EDX_ERR_ARG,
               "term counts out of range");
     EDX_CHECK(nhop == 0 || hop, EDX_ERR_ARG, "null hopping terms");
     EDX_CHECK(ncoul == 0 || coul, EDX_ERR_ARG, "null Coulomb terms");
     const int64_t T = nhop + ncoul;
-    std::vector<uint32_t> ops(T ? T : 1);
-    std::vector<double2> vals(T ? T : 1);
+    std::vector<uint32_t> &ops = tt.ops;
+    std::vector<double2> &vals = tt.vals;
+    ops.resize(T ? T : 1);
+    vals.resize(T ? T : 1);
     auto pos = [](int32_t i, int64_t t) -> int {
         return (i >= 1 && i <= 63) ? (i - 1) : -1;
     };
@@ -350,12 +356,18 @@ int upload_terms(const edx_tensor2 *hop, int64_t nhop, const edx_tensor4 *coul, 
     }
     tt.nhop = (int)nhop;
     tt.T = (int)T;
-    tt.d_ops = (uint32_t *)edx::dmalloc(ops.size() * sizeof(uint32_t), "term ops");
-    tt.d_vals = (double2 *)edx::dmalloc(vals.size() * sizeof(double2), "term values");
+    return EDX_OK;
+}
+
+int upload_terms(TermTable &tt) {
+    if (tt.d_ops) return EDX_OK;
+    tt.d_ops = (uint32_t *)edx::dmalloc(tt.ops.size() * sizeof(uint32_t), "term ops");
+    tt.d_vals = (double2 *)edx::dmalloc(tt.vals.size() * sizeof(double2), "term values");
     EDX_CHECK(tt.d_ops && tt.d_vals, EDX_ERR_NOMEM, "%s", edx_last_error());
-    EDX_HIP(edx::copy_sync(tt.d_ops, ops.data(), ops.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-    EDX_HIP(edx::copy_sync(tt.d_vals, vals.data(), vals.size() * sizeof(double2),
-                      hipMemcpyHostToDevice));
+    EDX_HIP(edx::copy_sync(tt.d_ops, tt.ops.data(), tt.ops.size() * sizeof(uint32_t),
+                           hipMemcpyHostToDevice));
+    EDX_HIP(edx::copy_sync(tt.d_vals, tt.vals.data(), tt.vals.size() * sizeof(double2),
+                           hipMemcpyHostToDevice));
     return EDX_OK;
 }
 
@@ -380,8 +392,94 @@ int launch_cap(const BuildParams &p, int cap) {
     }
 }
 
+// A build under way: row pointers (first the counts), the flag word of the
+// counting kernels (overflow, longest row), then columns and values.
+struct BuildOut {
+    int64_t *rowptr = nullptr;
+    int *flag = nullptr;
+    int32_t *cols = nullptr;
+    double2 *vals = nullptr;
+    int64_t nnz = 0;
+    ~BuildOut() {
+        edx::dfree(rowptr);
+        edx::dfree(flag);
+        edx::dfree(cols);
+        edx::dfree(vals);
+    }
+};
+
+// Row pointers from the counts, then room for the entries; flag: the flag
+// word's value if the caller wants it with the same wait.
+int build_alloc(BuildOut &o, int64_t M, int *flag) {
+    EDX_TRY(exclusive_scan(o.rowptr, M + 1));
+    if (flag)
+        EDX_HIP(hipMemcpyAsync(flag, o.flag, sizeof(int), hipMemcpyDeviceToHost, edx::stream()));
+    EDX_HIP(edx::copy_sync(&o.nnz, o.rowptr + M, sizeof(int64_t), hipMemcpyDeviceToHost));
+    o.cols = (int32_t *)edx::dmalloc((o.nnz ? o.nnz : 1) * sizeof(int32_t), "CSR columns");
+    o.vals = (double2 *)edx::dmalloc((o.nnz ? o.nnz : 1) * sizeof(double2), "CSR values");
+    return o.cols && o.vals ? EDX_OK : EDX_ERR_NOMEM;
+}
+
+// The plan kernels' build; *done stays false where a row is too long for them.
+template <int RK, int CK, class W>
+int build_by_plan(const BuildParams &p, const PlanSpaces &sp, const TermTable &tt, BuildOut &o,
+                  bool *done) {
+    PlanStore<W> plan;
+    EDX_TRY(plan_make<W>(sp, tt.ops.data(), tt.vals.data(), tt.nhop, tt.T, p.omega_on != 0,
+                         p.omega, p.negate != 0, false, plan));
+    EDX_HIP(hipMemsetAsync(o.rowptr + p.M, 0, sizeof(int64_t), edx::stream()));
+    EDX_HIP(hipMemsetAsync(o.flag, 0, sizeof(int), edx::stream()));
+    EDX_TRY((plan_count<RK, W>(plan.p, o.rowptr, o.flag)));
+    int maxrow = 0;
+    EDX_TRY(build_alloc(o, p.M, &maxrow));
+    if (maxrow > plan_max_row<W>(plan.p)) {
+        edx::dfree(o.cols);
+        edx::dfree(o.vals);
+        o.cols = nullptr;
+        o.vals = nullptr;
+        return EDX_OK;
+    }
+    *done = true;
+    EDX_TRY((plan_fill<RK, CK, W>(plan.p, maxrow, o.rowptr, o.cols, o.vals)));
+    EDX_HIP(hipStreamSynchronize(edx::stream()));
+    return EDX_OK;
+}
+
+// The term-by-term build.
 template <int RK, int CK>
-int build_csr(BuildParams p, int64_t ncols, int precision, edx_csr **out) {
+int build_by_term(BuildParams p, TermTable &tt, BuildOut &o) {
+    EDX_TRY(upload_terms(tt));
+    p.ops = tt.d_ops;
+    p.tv = tt.d_vals;
+    p.counts = o.rowptr;
+    p.overflow = o.flag;
+    // the omega diagonal counts as one more term
+    int maxc = p.T + (p.omega_on ? 1 : 0);
+    int cap = maxc <= 256 ? 256 : (maxc <= 1024 ? 1024 : 4096);
+    for (;;) {
+        EDX_HIP(hipMemsetAsync(o.rowptr + p.M, 0, sizeof(int64_t), edx::stream()));
+        EDX_HIP(hipMemsetAsync(o.flag, 0, sizeof(int), edx::stream()));
+        EDX_TRY((launch_cap<RK, CK, false>(p, cap)));
+        int h = 0;
+        EDX_HIP(edx::copy_sync(&h, o.flag, sizeof(int), hipMemcpyDeviceToHost));
+        if (!h) break;
+        if (cap == 4096)
+            return edx::set_error(EDX_ERR_CAPACITY,
+                                  "a row produced more than 4096 surviving terms; not supported");
+        cap = (cap == 256) ? 1024 : 4096;
+    }
+    EDX_TRY(build_alloc(o, p.M, nullptr));
+    p.rowptr = o.rowptr;
+    p.cols = o.cols;
+    p.vals = o.vals;
+    EDX_TRY((launch_cap<RK, CK, true>(p, cap)));
+    EDX_HIP(hipStreamSynchronize(edx::stream()));
+    return EDX_OK;
+}
+
+template <int RK, int CK>
+int build_csr(BuildParams p, const edx_basis *left, const edx_basis *right, TermTable &tt,
+              int64_t ncols, int precision, edx_csr **out) {
     EDX_CHECK(out, EDX_ERR_ARG, "null output");
     EDX_CHECK(ncols < ((int64_t)1 << 31) && p.M < ((int64_t)1 << 31), EDX_ERR_ARG,
               "dimension %lld x %lld exceeds the int32 column index range", (long long)p.M,
@@ -389,74 +487,28 @@ int build_csr(BuildParams p, int64_t ncols, int precision, edx_csr **out) {
     EDX_CHECK(precision == EDX_C128 || precision == EDX_C64, EDX_ERR_ARG, "bad precision %d",
               precision);
     EDX_TRY(edx::ensure_binomials());
-    int64_t *rowptr = (int64_t *)edx::dmalloc((p.M + 1) * sizeof(int64_t), "row pointers");
-    int *overflow = (int *)edx::dmalloc(sizeof(int), "overflow flag");
-    if (!rowptr || !overflow) {
-        edx::dfree(rowptr);
-        edx::dfree(overflow);
-        return EDX_ERR_NOMEM;
+    BuildOut o;
+    o.rowptr = (int64_t *)edx::dmalloc((p.M + 1) * sizeof(int64_t), "row pointers");
+    o.flag = (int *)edx::dmalloc(sizeof(int), "build flag");
+    if (!o.rowptr || !o.flag) return EDX_ERR_NOMEM;
+    const PlanSpaces sp{RK, CK, p.nv, p.nc, left, right};
+    bool done = false;
+    if (p.M > 0 && plan_usable(sp, tt.ops.data(), tt.nhop, tt.T)) {
+        if (plan_bits(sp) <= 32) EDX_TRY((build_by_plan<RK, CK, uint32_t>(p, sp, tt, o, &done)));
+        else EDX_TRY((build_by_plan<RK, CK, uint64_t>(p, sp, tt, o, &done)));
     }
-    p.counts = rowptr;
-    p.overflow = overflow;
-    // the omega diagonal counts as one more term
-    int maxc = p.T + (p.omega_on ? 1 : 0);
-    int cap = maxc <= 256 ? 256 : (maxc <= 1024 ? 1024 : 4096);
-    int rc = EDX_OK;
-    for (;;) {
-        EDX_HIP(hipMemsetAsync(rowptr + p.M, 0, sizeof(int64_t), edx::stream()));
-        EDX_HIP(hipMemsetAsync(overflow, 0, sizeof(int), edx::stream()));
-        if ((rc = launch_cap<RK, CK, false>(p, cap))) break;
-        int h = 0;
-        EDX_HIP(edx::copy_sync(&h, overflow, sizeof(int), hipMemcpyDeviceToHost));
-        if (!h) break;
-        if (cap == 4096) {
-            rc = edx::set_error(EDX_ERR_CAPACITY,
-                                "a row produced more than 4096 surviving terms; not supported");
-            break;
-        }
-        cap = (cap == 256) ? 1024 : 4096;
-    }
-    if (!rc) rc = exclusive_scan(rowptr, p.M + 1);
-    int64_t nnz = 0;
-    if (!rc) {
-        hipError_t e = edx::copy_sync(&nnz, rowptr + p.M, sizeof(int64_t), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = edx::hip_fail(e, "edx::copy_sync(nnz)", __FILE__, __LINE__);
-    }
-    int32_t *cols = nullptr;
-    double2 *vals = nullptr;
-    if (!rc) {
-        cols = (int32_t *)edx::dmalloc((nnz ? nnz : 1) * sizeof(int32_t), "CSR columns");
-        vals = (double2 *)edx::dmalloc((nnz ? nnz : 1) * sizeof(double2), "CSR values");
-        if (!cols || !vals) rc = EDX_ERR_NOMEM;
-    }
-    if (!rc) {
-        p.rowptr = rowptr;
-        p.cols = cols;
-        p.vals = vals;
-        rc = launch_cap<RK, CK, true>(p, cap);
-    }
-    if (!rc) {
-        hipError_t e = hipStreamSynchronize(edx::stream());
-        if (e != hipSuccess) rc = edx::hip_fail(e, "build", __FILE__, __LINE__);
-    }
-    edx::dfree(overflow);
-    if (rc) {
-        edx::dfree(rowptr);
-        edx::dfree(cols);
-        edx::dfree(vals);
-        return rc;
-    }
+    if (!done) EDX_TRY((build_by_term<RK, CK>(p, tt, o)));
     edx_csr *a = new edx_csr{};
     a->corehole_layout = p.inter;
     if (RK == ROW_COREHOLE && CK == COL_COREHOLE && p.inter) a->nc_slots = p.nc;
     a->m = p.M;
     a->n = ncols;
-    a->nnz = nnz;
-    a->d_rowptr = rowptr;
-    a->d_cols = cols;
-    a->d_vals = vals;
+    a->nnz = o.nnz;
+    a->d_rowptr = std::exchange(o.rowptr, nullptr);
+    a->d_cols = std::exchange(o.cols, nullptr);
+    a->d_vals = std::exchange(o.vals, nullptr);
     if (precision == EDX_C64) {
-        rc = edx_csr_add_c64(a);
+        const int rc = edx_csr_add_c64(a);
         if (rc) {
             edx_csr_free(a);
             return rc;
@@ -468,8 +520,6 @@ int build_csr(BuildParams p, int64_t ncols, int precision, edx_csr **out) {
 
 BuildParams base_params(const TermTable &tt) {
     BuildParams p{};
-    p.ops = tt.d_ops;
-    p.tv = tt.d_vals;
     p.nhop = tt.nhop;
     p.T = tt.T;
     return p;
@@ -497,7 +547,7 @@ int edx_build_ham_i(const edx_basis *fock, const edx_tensor2 *hop, int64_t nhopp
     EDX_CHECK(fock, EDX_ERR_ARG, "null basis");
     EDX_TRY(check_ham_sign(ham_sign));
     TermTable tt;
-    EDX_TRY(upload_terms(hop, nhopp, coul, ncoul, tt));
+    EDX_TRY(parse_terms(hop, nhopp, coul, ncoul, tt));
     BuildParams p = base_params(tt);
     p.M = fock->n;
     p.left = fock->d_words;
@@ -506,7 +556,7 @@ int edx_build_ham_i(const edx_basis *fock, const edx_tensor2 *hop, int64_t nhopp
     p.omega_on = ham_sign < 0;
     p.omega = make_double2(omega_re, omega_im);
     p.negate = ham_sign < 0;
-    return build_csr<ROW_PLAIN, COL_PLAIN>(p, fock->n, precision, out);
+    return build_csr<ROW_PLAIN, COL_PLAIN>(p, fock, fock, tt, fock->n, precision, out);
 }
 
 int edx_build_ham_n(const edx_basis *fock_n, int num_val_orbs, int num_core_orbs,
@@ -517,7 +567,7 @@ int edx_build_ham_n(const edx_basis *fock_n, int num_val_orbs, int num_core_orbs
     EDX_TRY(check_ham_sign(ham_sign));
     EDX_TRY(check_core(num_val_orbs, num_core_orbs));
     TermTable tt;
-    EDX_TRY(upload_terms(hop, nhopp, coul, ncoul, tt));
+    EDX_TRY(parse_terms(hop, nhopp, coul, ncoul, tt));
     BuildParams p = base_params(tt);
     p.M = fock_n->n * num_core_orbs;
     p.left = fock_n->d_words;
@@ -529,7 +579,7 @@ int edx_build_ham_n(const edx_basis *fock_n, int num_val_orbs, int num_core_orbs
     p.omega_on = ham_sign < 0;
     p.omega = make_double2(omega_re, omega_im);
     p.negate = ham_sign < 0;
-    return build_csr<ROW_COREHOLE, COL_COREHOLE>(p, p.M, precision, out);
+    return build_csr<ROW_COREHOLE, COL_COREHOLE>(p, fock_n, fock_n, tt, p.M, precision, out);
 }
 
 int edx_build_transop_i(const edx_basis *fock_n, const edx_basis *fock_i, int num_val_orbs,
@@ -538,7 +588,7 @@ int edx_build_transop_i(const edx_basis *fock_n, const edx_basis *fock_i, int nu
     EDX_CHECK(fock_n && fock_i, EDX_ERR_ARG, "null basis");
     EDX_TRY(check_core(num_val_orbs, num_core_orbs));
     TermTable tt;
-    EDX_TRY(upload_terms(trans, ntran, nullptr, 0, tt));
+    EDX_TRY(parse_terms(trans, ntran, nullptr, 0, tt));
     BuildParams p = base_params(tt);
     p.M = fock_n->n * num_core_orbs;
     p.left = fock_n->d_words;
@@ -547,7 +597,7 @@ int edx_build_transop_i(const edx_basis *fock_n, const edx_basis *fock_i, int nu
     p.nv = num_val_orbs;
     p.nc = num_core_orbs;
     p.inter = edx::corehole_layout() == EDX_COREHOLE_INTERLEAVED;
-    return build_csr<ROW_COREHOLE, COL_VALONLY>(p, fock_i->n, precision, out);
+    return build_csr<ROW_COREHOLE, COL_VALONLY>(p, fock_n, fock_i, tt, fock_i->n, precision, out);
 }
 
 int edx_build_transop_f(const edx_basis *fock_f, const edx_basis *fock_n, int num_val_orbs,
@@ -556,7 +606,7 @@ int edx_build_transop_f(const edx_basis *fock_f, const edx_basis *fock_n, int nu
     EDX_CHECK(fock_f && fock_n, EDX_ERR_ARG, "null basis");
     EDX_TRY(check_core(num_val_orbs, num_core_orbs));
     TermTable tt;
-    EDX_TRY(upload_terms(trans, ntran, nullptr, 0, tt));
+    EDX_TRY(parse_terms(trans, ntran, nullptr, 0, tt));
     BuildParams p = base_params(tt);
     p.M = fock_f->n;
     p.left = fock_f->d_words;
@@ -565,7 +615,7 @@ int edx_build_transop_f(const edx_basis *fock_f, const edx_basis *fock_n, int nu
     p.nv = num_val_orbs;
     p.nc = num_core_orbs;
     p.inter = edx::corehole_layout() == EDX_COREHOLE_INTERLEAVED;
-    return build_csr<ROW_FULLCORE, COL_COREHOLE>(p, fock_n->n * num_core_orbs, precision, out);
+    return build_csr<ROW_FULLCORE, COL_COREHOLE>(p, fock_f, fock_n, tt, fock_n->n * num_core_orbs, precision, out);
 }
 
 int edx_csr_info(const edx_csr *a, int64_t *m, int64_t *n, int64_t *nnz, int *precision) {

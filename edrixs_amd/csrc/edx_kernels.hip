@@ -18,6 +18,7 @@
 #include "device.h"
 
 #include "basis.hip"
+#include "termplan.hip"
 #include "csr_build.hip"
 #include "spmv.hip"
 #include "blas.hip"

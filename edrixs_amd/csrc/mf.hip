@@ -194,12 +194,15 @@ int mf_make(const edx_tensor2 *hop, int64_t nhopp, const edx_tensor4 *coul, int6
     EDX_TRY(check_ham_sign(ham_sign));
     EDX_TRY(edx::ensure_binomials());
     edx_mfop *o = new edx_mfop;
-    int rc = upload_terms(hop, nhopp, coul, ncoul, o->tt);
+    int rc = parse_terms(hop, nhopp, coul, ncoul, o->tt);
+    if (!rc) rc = upload_terms(o->tt);
     if (rc) {
         delete o;
         return rc;
     }
     o->p = base_params(o->tt);
+    o->p.ops = o->tt.d_ops;
+    o->p.tv = o->tt.d_vals;
     const int T = o->tt.T;
     o->d_masks = (MfMask *)edx::dmalloc((size_t)(T ? T : 1) * sizeof(MfMask), "term masks");
     if (!o->d_masks) {

@@ -1,0 +1,547 @@
+// Term plans: the terms of an operator grouped by the column they lead to
+// (part of edx_kernels.hip).  Used by the CSR builds and the matrix-free apply.
+//
+// Every term is a string of annihilations and creations applied to a row's
+// word w (the order of src/ham.f90: ind1 [, ind2] out, then the others in).
+// Whether it survives, where it leads and its fermion sign are closed forms of
+// w (Jordan-Wigner strings of fixed positions):
+//     survives   (w & M) == V      every operator's orbital is filled / empty
+//     column     w ^ F             F = the orbitals the string flips
+//     sign       (-1)^(popc(w & S) + c)
+// where S is the XOR of the "orbitals below" masks of the operators and c the
+// constant part of the flips made on the way.  Terms with the same F reach the
+// same column from any row, so a row has at most one entry per distinct F: the
+// terms (a thousand for an impurity with a core shell) collapse into groups (a
+// hundred or two), most of them of two to six terms.  Only the column-deciding
+// part of F counts for operators whose columns ignore the core word
+// (src/ham.f90:806-808).
+//
+// For a complete basis on both sides a term either keeps the particle numbers
+// the column space asks for or never reaches it, whatever the row, so columns
+// need no membership test.  Incomplete bases keep the term-by-term build.
+
+namespace {
+
+enum { ROW_PLAIN = 0, ROW_COREHOLE = 1, ROW_FULLCORE = 2 };
+enum { COL_PLAIN = 0, COL_COREHOLE = 1, COL_VALONLY = 2 };
+
+// the words of a plan: 32 bits where valence and core orbitals fit, else 64
+template <class W> struct PlanTest {   // four survival tests; bit: the group's in its chunk
+    W m[4], v[4];
+    uint32_t bit, pad;
+};
+template <class W> struct PlanTerm {
+    W m, v, s;
+    uint32_t neg;     // c, and the operator's overall sign
+};
+template <class W> struct PlanGroup {
+    W flip;
+    int32_t tbeg, tend;   // its terms, in term order
+    int32_t pad;
+};
+
+constexpr int PLAN_ROWS = 64;        // rows per workgroup: lane = row
+constexpr int PLAN_WAVES = 4;        // waves share the groups (chunks) of the same rows
+constexpr int PLAN_CHUNK = 32;       // groups per chunk (bits of a survival mask)
+constexpr int PLAN_MAX_TERMS = 4096; // the term-by-term build's limit per row
+constexpr int PLAN_BIG = 24;         // a group of more terms (the diagonal) is summed per row
+
+// A plan on the device, with what its kernels need to know of the spaces.
+template <class W> struct Plan {
+    const PlanTest<W> *tests;
+    const int32_t *chunks;           // nchunk + 1 offsets into tests
+    const PlanTerm<W> *terms;
+    const double2 *vals;             // value of each term, the sign not applied
+    const PlanGroup<W> *groups;
+    int nchunk, gpc;                 // chunks (a multiple of PLAN_WAVES), groups per chunk
+    int big;                         // group summed lane = row, or -1
+    int diag;                        // group of the diagonal when omega is added, or -1
+    double2 omega;
+    int64_t M;                       // rows
+    const int64_t *left;             // valence words of the row space
+    int64_t nleft;
+    int nv, nc, nbits, nocc;         // nbits, nocc: the column basis
+    int64_t nright;                  // its size
+    int inter;                       // core-hole index valence * nc + slot
+};
+
+template <class W> __device__ __forceinline__ int plan_popc(W x) {
+    if constexpr (sizeof(W) == 4) return __popc(x);
+    else return __popcll(x);
+}
+
+template <int RK, class W>
+__device__ __forceinline__ W plan_row_word(const Plan<W> &p, int64_t row) {
+    const uint32_t r = (uint32_t)row;          // dimensions are below 2^31
+    if (RK == ROW_PLAIN) return (W)p.left[r];
+    const W full = (W)((W(1) << p.nc) - 1);
+    if (RK == ROW_FULLCORE) return (W)((full << p.nv) | (W)p.left[r]);
+    const uint32_t nl = (uint32_t)p.nleft, nc = (uint32_t)p.nc;
+    const uint32_t v = p.inter ? r / nc : r % nl, k = p.inter ? r - v * nc : r / nl;
+    return (W)(((full ^ (W(1) << (p.nc - 1 - k))) << p.nv) | (W)p.left[v]);   // src/ham.f90:419-421
+}
+
+// Order key of a column: ascending keys are ascending columns.
+template <int CK, class W>
+__device__ __forceinline__ W plan_key(const Plan<W> &p, W w) {
+    if (CK == COL_PLAIN) return w;
+    const W val = w & (W)((W(1) << p.nv) - 1);
+    if (CK == COL_VALONLY) return val;
+    return p.inter ? (W)((val << p.nc) | (w >> p.nv)) : w;
+}
+
+// Column of a word; s_bin[p * nocc + k] = C(p, k + 1) staged in LDS.
+template <int CK, class W>
+__device__ __forceinline__ int32_t plan_col(const Plan<W> &p, W w, const int32_t *s_bin) {
+    W val = CK == COL_PLAIN ? w : w & (W)((W(1) << p.nv) - 1);
+    int32_t l = 0;
+    const int32_t *b = s_bin;
+    while (val) {
+        const int q = (sizeof(W) == 4 ? __ffs((unsigned)val) : __ffsll((unsigned long long)val)) - 1;
+        l += b[q * p.nocc];
+        ++b;
+        val &= val - 1;
+    }
+    if (CK != COL_COREHOLE) return l;
+    const W holes = (W)(((W(1) << p.nc) - 1) ^ (w >> p.nv));
+    const int k = p.nc - 1 - ((sizeof(W) == 4 ? __ffs((unsigned)holes)
+                                              : __ffsll((unsigned long long)holes)) - 1);
+    return p.inter ? l * p.nc + k : (int32_t)(k * p.nright) + l;
+}
+
+template <class W>
+__device__ __forceinline__ void plan_stage_binomials(const Plan<W> &p, int32_t *s_bin) {
+    for (int i = threadIdx.x; i < p.nbits * p.nocc; i += blockDim.x) {
+        const int64_t b = binom_dev(i / p.nocc, i % p.nocc + 1);
+        s_bin[i] = b < (int64_t(1) << 31) ? (int32_t)b : 0;   // larger ones are in no rank
+    }
+}
+
+// Which groups of chunk c have a surviving term on word w.  Chunk, test and
+// group numbers are uniform over the wave, so the tests come by scalar loads
+// and each costs two vector instructions for 64 rows.
+template <class W>
+__device__ __forceinline__ uint32_t plan_mask(const Plan<W> &p, int c, W w) {
+    const int ib = p.chunks[c], ie = p.chunks[c + 1];
+    uint32_t mask = 0;
+#pragma unroll 2
+    for (int i = ib; i < ie; ++i) {
+        const PlanTest<W> &t = p.tests[i];
+        const bool ok = ((w & t.m[0]) == t.v[0]) | ((w & t.m[1]) == t.v[1]) |
+                        ((w & t.m[2]) == t.v[2]) | ((w & t.m[3]) == t.v[3]);
+        mask |= ok ? t.bit : 0u;
+    }
+    return mask;
+}
+
+template <class W>
+__device__ __forceinline__ void plan_add_term(const PlanTerm<W> &t, double2 v, W w, double2 &acc) {
+    if ((w & t.m) == t.v) {
+        if ((plan_popc<W>(w & t.s) ^ t.neg) & 1) v = make_double2(-v.x, -v.y);
+        acc.x += v.x;
+        acc.y += v.y;
+    }
+}
+
+// Sum of a group's surviving terms in term order.  -0.0 + v is v bit for bit,
+// so the sum is the reference's, which starts from the first survivor.
+template <class W>
+__device__ __forceinline__ double2 plan_sum(const Plan<W> &p, int tb, int te, W w) {
+    double2 acc = make_double2(-0.0, -0.0);
+#pragma unroll 2
+    for (int t = tb; t < te; ++t) plan_add_term<W>(p.terms[t], p.vals[t], w, acc);
+    return acc;
+}
+
+__device__ __forceinline__ int plan_wave() {
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+// Entries per row: the number of groups with a survivor.  maxrow gets the
+// longest row.
+template <int RK, class W>
+__global__ __launch_bounds__(256) void k_plan_count(Plan<W> p, int64_t *counts, int *maxrow) {
+    __shared__ int s_cnt[PLAN_WAVES][PLAN_ROWS];
+    const int lane = threadIdx.x & 63, wave = plan_wave();
+    const int64_t r = (int64_t)blockIdx.x * PLAN_ROWS + lane;
+    const W w = r < p.M ? plan_row_word<RK, W>(p, r) : W(0);
+    int n = 0;
+    for (int c = wave; c < p.nchunk; c += PLAN_WAVES) n += __popc(plan_mask<W>(p, c, w));
+    s_cnt[wave][lane] = n;
+    __syncthreads();
+    if (wave == 0) {
+        n = 0;
+        if (r < p.M) {
+            for (int q = 0; q < PLAN_WAVES; ++q) n += s_cnt[q][lane];
+            if (counts) counts[r] = n;
+        }
+        for (int off = 32; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off, 64));
+        // a stale read only costs an atomic that changes nothing
+        if (lane == 0 && n > *(volatile int *)maxrow) atomicMax(maxrow, n);
+    }
+}
+
+// Lists the row's surviving groups: entry e of row `lane` at list[e * 64 +
+// lane] by emit(e, group), groups in plan order; returns the row's count.
+// Every thread of the workgroup calls it (barriers inside).
+template <class W, class Emit>
+__device__ __forceinline__ int plan_expand(const Plan<W> &p, W w, bool on, int (*s_cnt)[PLAN_ROWS],
+                                           Emit emit) {
+    const int lane = threadIdx.x & 63, wave = plan_wave();
+    int n = 0;
+    for (int c0 = 0; c0 < p.nchunk; c0 += PLAN_WAVES) {
+        const int c = c0 + wave;
+        uint32_t mask = on ? plan_mask<W>(p, c, w) : 0u;
+        __syncthreads();
+        s_cnt[wave][lane] = __popc(mask);
+        __syncthreads();
+        int e = n;
+        for (int q = 0; q < PLAN_WAVES; ++q) {
+            const int k = s_cnt[q][lane];
+            if (q < wave) e += k;
+            n += k;
+        }
+        while (mask) {
+            emit(e++, c * p.gpc + __ffs((int)mask) - 1);
+            mask &= mask - 1;
+        }
+    }
+    return n;
+}
+
+// Fills the rows' columns and values.  A workgroup of four waves owns 64
+// consecutive rows.  (1) lane = row: each wave finds the surviving groups of
+// its chunks and lists (column key, group) per row in LDS; one wave sums the
+// diagonal group, whose hundreds of density terms are the same for every lane.
+// (2) lane = row: an entry's place in its row is the number of smaller keys.
+// (3) lane = entry, in output order: sums its group's few terms, ranks its
+// column and stores, so a wave writes 64 consecutive columns and values.
+// 512 * cap bytes of LDS and 4 KB decide the workgroups per CU (cap = the longest
+// row, about 40: six); the time goes to the integer instructions of (1) and (3),
+// the 20 bytes per entry are written behind them.  Measured, count and fill:
+// H_i norb 24 (2.7M rows, 44M entries) 0.11 + 1.09 ms (0.9 TB/s written), by the
+// term-by-term kernel 16.1 + 21.4 ms; H_n norb 21 N 9 (2.1M rows, 50M entries)
+// 0.19 + 1.76 ms, before 27.9 + 36.9 ms.
+template <int RK, int CK, class W>
+__global__ __launch_bounds__(256) void k_plan_fill(Plan<W> p, int cap,
+                                                   const int64_t *__restrict__ rowptr,
+                                                   int32_t *__restrict__ cols,
+                                                   double2 *__restrict__ vals) {
+    extern __shared__ char s_mem[];
+    W *s_key = reinterpret_cast<W *>(s_mem);                                  // [cap][64]
+    int32_t *s_bin = reinterpret_cast<int32_t *>(s_key + cap * PLAN_ROWS);   // nbits * nocc
+    uint16_t *s_grp = reinterpret_cast<uint16_t *>(s_bin + p.nbits * p.nocc);   // [cap][64]
+    uint16_t *s_flat = s_grp + cap * PLAN_ROWS;                               // [cap * 64]
+    __shared__ W s_w[PLAN_ROWS];
+    __shared__ double2 s_big[PLAN_ROWS];
+    __shared__ int s_cnt[PLAN_WAVES][PLAN_ROWS];
+    const int lane = threadIdx.x & 63, wave = plan_wave();
+    const int64_t r0 = (int64_t)blockIdx.x * PLAN_ROWS, r = r0 + lane;
+    const bool on = r < p.M;
+    const W w = on ? plan_row_word<RK, W>(p, r) : W(0);
+    if (wave == 0) s_w[lane] = w;
+    plan_stage_binomials<W>(p, s_bin);
+    if (p.big >= 0 && wave == PLAN_WAVES - 1) {
+        const PlanGroup<W> g = p.groups[p.big];
+        s_big[lane] = plan_sum<W>(p, g.tbeg, g.tend, w);
+    }
+    const int n = plan_expand<W>(p, w, on, s_cnt, [&](int e, int g) {
+        if (e < cap) {
+            s_key[e * PLAN_ROWS + lane] = plan_key<CK, W>(p, w ^ p.groups[g].flip);
+            s_grp[e * PLAN_ROWS + lane] = (uint16_t)g;
+        }
+    });
+    __syncthreads();
+    const int64_t base = rowptr[r0];
+    const int off = on ? (int)(rowptr[r] - base) : 0;
+    for (int i0 = wave; i0 < n; i0 += 4 * PLAN_WAVES) {
+        W key[4];
+        int below[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * PLAN_WAVES;
+            key[u] = i < n ? s_key[i * PLAN_ROWS + lane] : W(0);
+            below[u] = 0;
+        }
+        for (int j = 0; j < n; ++j) {
+            const W kj = s_key[j * PLAN_ROWS + lane];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) below[u] += kj < key[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * PLAN_WAVES;
+            if (i < n) s_flat[off + below[u]] = (uint16_t)(lane | (i << 6));
+        }
+    }
+    __syncthreads();
+    const int64_t rend = r0 + PLAN_ROWS < p.M ? r0 + PLAN_ROWS : p.M;
+    const int total = (int)(rowptr[rend] - base);
+    for (int e = threadIdx.x; e < total; e += 256) {
+        const int f = s_flat[e], row = f & 63;
+        const int gi = s_grp[(f >> 6) * PLAN_ROWS + row];
+        const W rw = s_w[row];
+        const PlanGroup<W> g = p.groups[gi];
+        double2 acc = gi == p.big ? s_big[row] : plan_sum<W>(p, g.tbeg, g.tend, rw);
+        if (gi == p.diag) acc = make_double2(acc.x + p.omega.x, acc.y + p.omega.y);
+        cols[base + e] = plan_col<CK, W>(p, rw ^ g.flip, s_bin);
+        vals[base + e] = acc;
+    }
+}
+
+// ------------------------------------------------------------------ host side
+
+struct PlanSpaces {
+    int rk, ck;
+    int nv, nc;
+    const edx_basis *left, *right;
+};
+
+// A term as the device needs it, in 64-bit words; false if it never reaches
+// the column space.
+struct HostTerm {
+    uint64_t m = 0, v = 0, f = 0, s = 0, group = 0;
+    uint32_t neg = 0;
+};
+
+bool plan_term(const PlanSpaces &sp, uint32_t op, bool hop, bool negate, HostTerm &t) {
+    const int pos[4] = {(int)(op & 63), (int)(op >> 8 & 63), (int)(op >> 16 & 63), (int)(op >> 24 & 63)};
+    const int nops = hop ? 2 : 4;
+    const int top = sp.ck == COL_PLAIN && sp.rk == ROW_PLAIN ? sp.right->nbits : sp.nv + sp.nc;
+    int dval = 0, dcore = 0;
+    for (int q = 0; q < nops; ++q) {
+        const uint64_t bit = 1ull << pos[q], below = bit - 1;
+        const bool filled = q < nops / 2;   // taken out first, then put in
+        const bool now = (t.m & bit) ? ((t.v ^ t.f) & bit) != 0 : filled;
+        if (now != filled) return false;    // a second operator of the same kind on one orbital
+        if (!(t.m & bit)) {
+            t.m |= bit;
+            if (filled) t.v |= bit;
+        }
+        t.neg ^= (uint32_t)__builtin_popcountll(t.f & below) & 1u;
+        t.s ^= below;
+        t.f ^= bit;
+        if (sp.rk == ROW_PLAIN || pos[q] < sp.nv) dval += filled ? -1 : 1;
+        else dcore += filled ? -1 : 1;
+    }
+    if (negate) t.neg ^= 1u;
+    if (top < 64 && (t.f >> top) != 0) return false;
+    if (top < 64 && (t.v >> top) != 0) return false;   // needs an orbital no row has
+    if (sp.left->nocc + dval != sp.right->nocc) return false;
+    t.group = t.f;
+    if (sp.ck == COL_VALONLY) t.group = t.f & ((1ull << sp.nv) - 1);
+    if (sp.ck == COL_COREHOLE &&
+        (sp.rk == ROW_COREHOLE ? sp.nc - 1 : sp.nc) + dcore != sp.nc - 1)
+        return false;
+    return true;
+}
+
+// A plan's device storage (one buffer) and description.
+template <class W> struct PlanStore {
+    Plan<W> p{};
+    void *d_buf = nullptr;
+    ~PlanStore() { edx::dfree(d_buf); }
+    PlanStore() = default;
+    PlanStore(const PlanStore &) = delete;
+    PlanStore &operator=(const PlanStore &) = delete;
+};
+
+// Groups the terms.  merge: terms that differ in their value only become one
+// (the matrix-free apply, whose sums need not keep the term order).
+template <class W>
+int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int nhop, int T,
+              bool omega_on, double2 omega, bool negate, bool merge, PlanStore<W> &out) {
+    struct Group {
+        uint64_t key;
+        std::vector<int> terms;
+    };
+    std::vector<HostTerm> ht;
+    std::vector<double2> hv;
+    std::vector<Group> groups;
+    ht.reserve(T);
+    hv.reserve(T);
+    int hsize = 64;
+    while (hsize < 4 * (T + 1)) hsize *= 2;
+    std::vector<int> table(hsize, -1);
+    auto group_of = [&](uint64_t key) {
+        uint64_t h = key * 0x9e3779b97f4a7c15ull;
+        for (int i = (int)(h >> 40) & (hsize - 1);; i = (i + 1) & (hsize - 1)) {
+            if (table[i] < 0) {
+                table[i] = (int)groups.size();
+                groups.push_back(Group{key, {}});
+            }
+            if (groups[table[i]].key == key) return table[i];
+        }
+    };
+    if (omega_on) group_of(0);   // the diagonal, present in every row
+    for (int t = 0; t < T; ++t) {
+        HostTerm h;
+        if (!plan_term(sp, ops[t], t < nhop, negate, h)) continue;
+        Group &g = groups[group_of(h.group)];
+        if (merge) {
+            bool found = false;
+            for (int q : g.terms)
+                if (ht[q].m == h.m && ht[q].v == h.v && ht[q].s == h.s) {
+                    const double sg = ht[q].neg == h.neg ? 1.0 : -1.0;
+                    hv[q].x += sg * tv[t].x;
+                    hv[q].y += sg * tv[t].y;
+                    found = true;
+                    break;
+                }
+            if (found) continue;
+        }
+        g.terms.push_back((int)ht.size());
+        ht.push_back(h);
+        hv.push_back(tv[t]);
+    }
+    const int G = (int)groups.size();
+    int nchunk = (G + PLAN_CHUNK - 1) / PLAN_CHUNK;
+    nchunk = std::max((nchunk + PLAN_WAVES - 1) / PLAN_WAVES, 1) * PLAN_WAVES;
+    const int gpc = std::max((G + nchunk - 1) / nchunk, 1);
+    std::vector<PlanTest<W>> tests;
+    std::vector<int32_t> chunks(nchunk + 1, 0);
+    std::vector<PlanTerm<W>> terms;
+    std::vector<double2> vals;
+    std::vector<PlanGroup<W>> dg(std::max(G, 1));
+    int big = -1, nbig = PLAN_BIG;
+    std::vector<std::pair<uint64_t, uint64_t>> kept;
+    for (int c = 0; c < nchunk; ++c) {
+        chunks[c] = (int32_t)tests.size();
+        for (int g = c * gpc; g < std::min((c + 1) * gpc, G); ++g) {
+            const Group &gr = groups[g];
+            PlanGroup<W> &d = dg[g];
+            d.flip = 0;
+            d.tbeg = (int32_t)terms.size();
+            for (int q : gr.terms) {
+                terms.push_back(PlanTerm<W>{(W)ht[q].m, (W)ht[q].v, (W)ht[q].s, ht[q].neg});
+                vals.push_back(hv[q]);
+                d.flip = (W)ht[q].f;
+            }
+            if (sp.ck == COL_VALONLY) d.flip = (W)gr.key;
+            d.tend = (int32_t)terms.size();
+            if (d.tend - d.tbeg > nbig) {
+                nbig = d.tend - d.tbeg;
+                big = g;
+            }
+            // survival tests, weakest first: one implied by a weaker one adds nothing
+            kept.clear();
+            if (omega_on && g == 0) {
+                kept.emplace_back(0, 0);
+            } else {
+                for (int bits = 1; bits <= 4; ++bits)
+                    for (int q : gr.terms) {
+                        if (__builtin_popcountll(ht[q].m) != bits) continue;
+                        bool implied = false;
+                        for (auto &k : kept)
+                            if ((ht[q].m & k.first) == k.first && (ht[q].v & k.first) == k.second) {
+                                implied = true;
+                                break;
+                            }
+                        if (!implied) kept.emplace_back(ht[q].m, ht[q].v);
+                    }
+            }
+            for (size_t i = 0; i < kept.size(); i += 4) {
+                PlanTest<W> q{};
+                q.bit = 1u << (g - c * gpc);
+                for (int u = 0; u < 4; ++u) {
+                    const auto &k = kept[std::min(i + u, kept.size() - 1)];
+                    q.m[u] = (W)k.first;
+                    q.v[u] = (W)k.second;
+                }
+                tests.push_back(q);
+            }
+        }
+    }
+    chunks[nchunk] = (int32_t)tests.size();
+    auto up = [](size_t b) { return (b + 63) / 64 * 64; };
+    // two spare records: the scalar loads of the unrolled loop stay inside
+    const size_t b_tests = up((tests.size() + 2) * sizeof(PlanTest<W>));
+    const size_t b_chunks = up(chunks.size() * sizeof(int32_t));
+    const size_t b_terms = up((terms.size() + 2) * sizeof(PlanTerm<W>));
+    const size_t b_vals = up((vals.size() + 2) * sizeof(double2));
+    const size_t b_groups = up(dg.size() * sizeof(PlanGroup<W>));
+    std::vector<char> buf(b_tests + b_chunks + b_terms + b_vals + b_groups, 0);
+    char *h = buf.data();
+    const size_t o_chunks = b_tests, o_terms = o_chunks + b_chunks, o_vals = o_terms + b_terms,
+                 o_groups = o_vals + b_vals;
+    if (!tests.empty()) memcpy(h, tests.data(), tests.size() * sizeof(PlanTest<W>));
+    memcpy(h + o_chunks, chunks.data(), chunks.size() * sizeof(int32_t));
+    if (!terms.empty()) {
+        memcpy(h + o_terms, terms.data(), terms.size() * sizeof(PlanTerm<W>));
+        memcpy(h + o_vals, vals.data(), vals.size() * sizeof(double2));
+    }
+    memcpy(h + o_groups, dg.data(), dg.size() * sizeof(PlanGroup<W>));
+    out.d_buf = edx::dmalloc(buf.size(), "term plan");
+    if (!out.d_buf) return EDX_ERR_NOMEM;
+    EDX_HIP(edx::copy_sync(out.d_buf, h, buf.size(), hipMemcpyHostToDevice));
+    char *d = (char *)out.d_buf;
+    Plan<W> &p = out.p;
+    p.tests = (const PlanTest<W> *)d;
+    p.chunks = (const int32_t *)(d + o_chunks);
+    p.terms = (const PlanTerm<W> *)(d + o_terms);
+    p.vals = (const double2 *)(d + o_vals);
+    p.groups = (const PlanGroup<W> *)(d + o_groups);
+    p.nchunk = nchunk;
+    p.gpc = gpc;
+    p.big = big;
+    p.diag = omega_on ? 0 : -1;
+    p.omega = omega;
+    p.left = sp.left->d_words;
+    p.nleft = sp.left->n;
+    p.M = sp.rk == ROW_COREHOLE ? sp.left->n * sp.nc : sp.left->n;
+    p.nv = sp.nv;
+    p.nc = sp.nc;
+    p.nbits = sp.right->nbits;
+    p.nocc = sp.right->nocc;
+    p.nright = sp.right->n;
+    p.inter = edx::corehole_layout() == EDX_COREHOLE_INTERLEAVED;
+    return EDX_OK;
+}
+
+// Whether the spaces have closed-form columns: complete bases of one valence
+// width, and no orbital outside the words where columns ignore the core word.
+bool plan_usable(const PlanSpaces &sp, const uint32_t *ops, int nhop, int T) {
+    if (!sp.left->complete || !sp.right->complete || T > PLAN_MAX_TERMS) return false;
+    if (sp.left->nbits != sp.right->nbits) return false;
+    if (sp.rk != ROW_PLAIN && sp.left->nbits != sp.nv) return false;
+    if (sp.ck == COL_VALONLY)
+        for (int t = 0; t < T; ++t)
+            for (int q = 0; q < (t < nhop ? 2 : 4); ++q)
+                if ((int)(ops[t] >> (8 * q) & 63) >= sp.nv + sp.nc) return false;
+    return true;
+}
+
+int plan_bits(const PlanSpaces &sp) {
+    return sp.rk == ROW_PLAIN && sp.ck == COL_PLAIN ? sp.right->nbits : sp.nv + sp.nc;
+}
+
+constexpr int PLAN_LDS = 144 << 10;   // of 160 KB, with room for the static arrays
+
+// Longest row the fill's lists can hold.
+template <class W> int plan_max_row(const Plan<W> &p) {
+    const int per = PLAN_ROWS * (int)(sizeof(W) + 4);
+    return std::min((PLAN_LDS - p.nbits * p.nocc * 4) / per, 255);
+}
+
+template <int RK, class W>
+int plan_count(const Plan<W> &p, int64_t *counts, int *d_maxrow) {
+    hipLaunchKernelGGL((k_plan_count<RK, W>), dim3((unsigned)((p.M + PLAN_ROWS - 1) / PLAN_ROWS)),
+                       dim3(256), 0, edx::stream(), p, counts, d_maxrow);
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
+}
+
+template <int RK, int CK, class W>
+int plan_fill(const Plan<W> &p, int maxrow, const int64_t *rowptr, int32_t *cols, double2 *vals) {
+    const int cap = std::max((maxrow + 3) / 4 * 4, 4);
+    const size_t lds = (size_t)cap * PLAN_ROWS * (sizeof(W) + 4) + (size_t)p.nbits * p.nocc * 4;
+    if (lds > (64 << 10))
+        EDX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_plan_fill<RK, CK, W>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_plan_fill<RK, CK, W>), dim3((unsigned)((p.M + PLAN_ROWS - 1) / PLAN_ROWS)),
+                       dim3(256), lds, edx::stream(), p, cap, rowptr, cols, vals);
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
+}
+
+}  // namespace

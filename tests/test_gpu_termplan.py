@@ -1,0 +1,130 @@
+"""CSR builds over the term plan at the edges of its range, against the oracle
+(values equal, not close): workgroup remainders, 32- and 64-bit words, both core-hole layouts,
+columns that ignore the core word, and the calls that keep the term-by-term
+build (incomplete bases, rows longer than the plan's lists, many terms)."""
+import numpy as np
+import pytest
+
+from edrixs_amd import siam
+from oracle import oracle as o
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def core():
+    from edrixs_amd import core as c
+    return c
+
+
+def _same(A, R, perm_rows=None, perm_cols=None):
+    """Row pointers, columns and values of A equal the oracle's (rows and
+    columns permuted by perm: new index i holds old index perm[i])."""
+    rp, cols, vals = A.download()
+    ref_rp, ref_c, ref_v = (np.asarray(x) for x in (R.rowptr, R.cols, R.vals))
+    if perm_rows is not None or perm_cols is not None:
+        pr = np.arange(len(ref_rp) - 1) if perm_rows is None else perm_rows
+        inv = None
+        if perm_cols is not None:
+            inv = np.empty(len(perm_cols), dtype=np.int64)
+            inv[perm_cols] = np.arange(len(perm_cols))
+        oc, ov, orp = [], [], [0]
+        for r in pr:
+            c, v = ref_c[ref_rp[r]:ref_rp[r + 1]], ref_v[ref_rp[r]:ref_rp[r + 1]]
+            if inv is not None:
+                c = inv[c]
+                k = np.argsort(c, kind="stable")
+                c, v = c[k], v[k]
+            oc.append(c)
+            ov.append(v)
+            orp.append(orp[-1] + len(c))
+        ref_rp, ref_c, ref_v = np.array(orp), np.concatenate(oc), np.concatenate(ov)
+    assert np.array_equal(rp, ref_rp)
+    assert np.array_equal(cols, ref_c)
+    assert np.array_equal(vals, ref_v)
+
+
+def _terms(n, seed, nnz_u, density=0.5):
+    rng = np.random.default_rng(seed)
+    return (siam.emat_terms(H.random_hermitian_emat(n, rng, density=density)),
+            siam.umat_terms(H.random_hermitian_umat(n, rng, nnz=nnz_u)))
+
+
+@pytest.mark.parametrize("nbits,nocc", [(1, 0), (1, 1), (5, 5), (6, 1), (8, 4), (12, 6), (31, 2),
+                                        (32, 2), (33, 2), (40, 1), (62, 1)])
+def test_plain_builds_at_word_and_workgroup_edges(core, nbits, nocc):
+    ht, ut = _terms(min(nbits, 14), nbits, 60)
+    if nbits > 14:       # spread the orbitals over the whole word
+        step = (nbits - 1) // 13
+        for f in ("ind1", "ind2"):
+            ht[f] = 1 + (ht[f] - 1) * step
+        for f in ("ind1", "ind2", "ind3", "ind4"):
+            ut[f] = 1 + (ut[f] - 1) * step
+    fock = H.fock_words(nbits, nocc)
+    b = core.Basis.combinations(nbits, nocc)
+    for omega, sign in ((0j, 1.0), (-0.75 + 0.25j, -1.0)):
+        _same(core.build_ham_i(b, ht, ut, omega=omega, ham_sign=sign),
+              o.build_ham_i(fock, ht, ut, omega=omega, ham_sign=sign))
+
+
+@pytest.mark.parametrize("nv,nc,nocc", [(7, 6, 3), (10, 2, 5), (26, 6, 2), (28, 6, 1)])
+def test_corehole_operators_in_both_layouts(core, nv, nc, nocc):
+    """H_n, absorption and emission operators of random terms over valence and
+    core orbitals, core-core ones among them (absorption columns ignore the
+    core word, so such terms meet in one column)."""
+    ntot = nv + nc
+    rng = np.random.default_rng(nv)
+    ht, ut = _terms(ntot, 5, 200, density=0.4)
+    tr = siam.emat_terms(rng.normal(size=(ntot, ntot)) * (rng.random((ntot, ntot)) < 0.3))
+    fi, fn = H.fock_words(nv, nocc), H.fock_words(nv, nocc + 1)
+    bi, bn = core.Basis.combinations(nv, nocc), core.Basis.combinations(nv, nocc + 1)
+    perm = core.corehole_permutation(len(fn), nc)
+    for lay, p in (("reference", None), ("interleaved", perm)):
+        for omega, sign in ((0j, 1.0), (1.5 + 0.5j, -1.0)):
+            A = core.build_ham_n(bn, nv, nc, ht, ut, omega=omega, ham_sign=sign, layout=lay)
+            _same(A, o.build_ham_n(fn, nv, nc, ht, ut, omega=omega, ham_sign=sign), p, p)
+        _same(core.build_transop_i(bn, bi, nv, nc, tr, layout=lay),
+              o.build_transop_i(fn, fi, nv, nc, tr), p, None)
+        _same(core.build_transop_f(bi, bn, nv, nc, tr, layout=lay),
+              o.build_transop_f(fi, fn, nv, nc, tr), None, p)
+
+
+def test_terms_outside_the_words_and_impossible_terms(core):
+    """Orbitals no row has, an orbital taken out or put in twice, spectators, and
+    duplicates that cancel to an explicit zero."""
+    fock = H.fock_words(6, 3)
+    b = core.Basis.combinations(6, 3)
+    hop = [[1, 9, 1.0, 0.0], [9, 9, 2.0, 0.0], [2, 2, -0.0, 0.0], [1, 2, 0.5, 1.0],
+           [1, 2, -0.5, -1.0], [40, 1, 3.0, 0.0]]
+    coul = [[1, 1, 2, 3, 1.0, 0.0], [1, 2, 4, 4, 1.0, 0.0], [1, 2, 2, 1, 0.25, 0.0],
+            [1, 2, 1, 2, 0.25, -0.0], [3, 1, 1, 5, 0.75, 0.1], [1, 3, 5, 1, 0.75, 0.1],
+            [2, 33, 33, 2, 1.0, 0.0]]
+    for sign in (1.0, -1.0):
+        _same(core.build_ham_i(b, hop, coul, omega=0.5j, ham_sign=sign),
+              o.build_ham_i(fock, hop, coul, omega=0.5j, ham_sign=sign))
+    _same(core.build_ham_i(b, None, None), o.build_ham_i(fock, None, None))
+
+
+@pytest.mark.parametrize("case", ["incomplete", "long_rows", "many_terms"])
+def test_builds_that_keep_the_term_by_term_kernel(core, case):
+    if case == "long_rows":       # more than 255 entries in a row
+        n, N = 16, 8
+        ht, ut = _terms(n, 3, 2000, density=1.0)
+        assert len(ht) + len(ut) <= 4096
+    elif case == "many_terms":    # more than 4096 terms, fewer than 4096 survivors
+        n, N = 10, 2
+        ht, ut = _terms(n, 4, 4200, density=1.0)
+        ut = np.concatenate([ut, ut])
+    else:
+        n, N = 9, 4
+        ht, ut = _terms(n, 5, 80)
+    fock = H.fock_words(n, N)
+    if case == "incomplete":
+        fock = fock[1::2].copy()
+    R = o.build_ham_i(fock, ht, ut)
+    if case == "long_rows":
+        assert np.diff(R.rowptr).max() > 255
+    if case == "many_terms":
+        assert len(ht) + len(ut) > 4096
+    _same(core.build_ham_i(core.Basis.from_words(fock, n), ht, ut), R)
