@@ -1,18 +1,20 @@
 // Matrix-free Hamiltonian apply (part of edx_kernels.hip).
 //
 // For spaces too large to keep as CSR (the core-hole space at norb=26, N=13:
-// 57,946,200 rows), y = c0 H x + c1 z is computed on the fly.  A 64-lane wave
-// owns a row: its lanes test the terms in parallel and apply the same operator
-// steps as the CSR build (op_ann / op_cre: occupancy test and fermion sign;
-// row_word / col_of: the core-hole layout of src/ham.f90:419-446 and the
-// combinatorial rank), so every surviving term lands on the column and with
-// the sign the CSR build gives it; the lanes accumulate val * sign * x[col]
-// over the surviving terms and the wave reduces.  The omega diagonal of ham_sign = -1 is added last as
-// in src/ham.f90:156-176.  Only the summation order of duplicate terms
-// differs from a CSR product, so results agree to rounding.
+// 57,946,200 rows), y = c0 H x + c1 z is computed on the fly: every term is
+// tested, signed and ranked as the CSR build does (the core-hole layout of
+// src/ham.f90:419-446), so it lands on the column and with the sign the build
+// gives it.  The omega diagonal of ham_sign = -1 is added last as in
+// src/ham.f90:156-176.  Only the summation order differs from a CSR product,
+// so results agree to rounding.
 //
 // No matrix is read: per row the traffic is the gathers of x and the epilogue
-// vectors, and the work is the term tests (integer ALU).
+// vectors, and the work is the term tests (integer ALU).  Two kernels:
+//   * k_plan_apply, for complete bases: 64 rows per workgroup over the terms
+//     grouped by column (termplan.hip), those of equal action merged;
+//   * k_mf, for incomplete bases, more than 4096 terms or rows of more than 255
+//     entries: one 64-lane wave per row, its lanes testing the terms in
+//     parallel and accumulating val * sign * x[col] over the survivors.
 
 namespace {
 
@@ -144,6 +146,63 @@ __global__ __launch_bounds__(64) void k_mf(BuildParams p, const MfMask *__restri
     if (e.dvec && lane == 0) e.partials[blockIdx.x] = dot;
 }
 
+// The product over a term plan.  A workgroup of four waves owns 64 rows.  Lane
+// = row throughout: the waves find the surviving groups of their chunks and
+// list them per row in LDS; the diagonal group, whose density terms are the
+// same for every lane, is summed by one wave from scalar loads; then wave q
+// takes entries q, q + 4, ... of each row (sum of the group's terms, column
+// rank, x gather) and the four partial rows are added in wave order, so the
+// result does not depend on timing.  Bound by integer and LDS instructions (a
+// thousand terms tested, 24 columns ranked per row; the vectors take 0.03 ms):
+// H_n norb 20, 1.0M rows, 0.56 ms a product, by k_mf 4.38 ms.
+template <int RK, int CK, class W>
+__global__ __launch_bounds__(256) void k_plan_apply(Plan<W> p, int cap, const double2 *__restrict__ x,
+                                                    SpmvEpi e) {
+    if (e.run && *e.run == 0) return;
+    extern __shared__ int32_t s_bin[];                                          // nbits * nocc
+    uint16_t *s_grp = reinterpret_cast<uint16_t *>(s_bin + p.nbits * p.nocc);   // [cap][64]
+    __shared__ int s_cnt[PLAN_WAVES][PLAN_ROWS];
+    __shared__ double2 s_acc[PLAN_WAVES][PLAN_ROWS];
+    __shared__ double2 s_big[PLAN_ROWS];
+    const int lane = threadIdx.x & 63, wave = plan_wave();
+    const int64_t r = (int64_t)blockIdx.x * PLAN_ROWS + lane;
+    const bool on = r < p.M;
+    const W w = on ? plan_row_word<RK, W>(p, r) : W(0);
+    plan_stage_binomials<W>(p, s_bin);
+    const int n = plan_expand<W>(p, w, on, s_cnt, [&](int i, int g) {
+        if (i < cap) s_grp[i * PLAN_ROWS + lane] = (uint16_t)g;
+    });
+    if (p.big >= 0 && wave == PLAN_WAVES - 1) {
+        const PlanGroup<W> g = p.groups[p.big];
+        s_big[lane] = plan_sum<W>(p, g.tbeg, g.tend, w);
+    }
+    __syncthreads();
+    double2 acc = make_double2(0.0, 0.0);
+    for (int i = wave; i < n; i += PLAN_WAVES) {
+        const int gi = s_grp[i * PLAN_ROWS + lane];
+        const PlanGroup<W> g = p.groups[gi];
+        const double2 xv = x[plan_col<CK, W>(p, w ^ g.flip, s_bin)];
+        double2 v = gi == p.big ? s_big[lane] : plan_sum<W>(p, g.tbeg, g.tend, w);
+        if (gi == p.diag) v = cadd(v, p.omega);
+        acc = cadd(acc, cmul(v, xv));
+    }
+    s_acc[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+    double2 dot = make_double2(0, 0);
+    if (on) {
+        for (int q = 1; q < PLAN_WAVES; ++q) acc = cadd(acc, s_acc[q][lane]);
+        double2 out = e.c0 ? cmul(*e.c0, acc) : acc;
+        if (e.z) out = cadd(out, e.c1 ? cmul(*e.c1, e.z[r]) : e.z[r]);
+        e.y[r] = out;
+        if (e.dvec) dot = cconjmul(e.dvec[r], out);
+    }
+    if (e.dvec) {
+        dot = wave_sum64(dot);
+        if (lane == 0) e.partials[blockIdx.x] = dot;
+    }
+}
+
 }  // namespace
 
 struct edx_mfop {
@@ -151,12 +210,17 @@ struct edx_mfop {
     TermTable tt;
     MfMask *d_masks = nullptr;
     int corehole = 0;   // row/column layout: core-hole space (H_n) or plain (H_i)
+    PlanStore<uint32_t> plan32;   // the one in use has terms grouped for k_plan_apply
+    PlanStore<uint64_t> plan64;
+    int plan = 0;       // its word bits, or 0: k_mf
+    int maxrow = 0;     // longest row of the plan
     ~edx_mfop() { edx::dfree(d_masks); }
 };
 
 namespace {
 
 int mf_blocks(const edx_mfop *op) {
+    if (op->plan) return (int)std::max<int64_t>((op->p.M + PLAN_ROWS - 1) / PLAN_ROWS, 1);
     int64_t b = op->p.M;
     const int64_t cap = (int64_t)edx::num_cus() * 256;
     if (b > cap) b = cap;
@@ -165,11 +229,53 @@ int mf_blocks(const edx_mfop *op) {
 
 int64_t mf_partials_len(const edx_mfop *op) { return mf_blocks(op) + FOLD_N + 64; }
 
+template <int RK, int CK, class W>
+void mf_launch_plan(const edx_mfop *op, const Plan<W> &p, int nb, const double2 *x,
+                    const SpmvEpi &e) {
+    const int cap = std::max(op->maxrow, 1);
+    const size_t lds = (size_t)p.nbits * p.nocc * 4 + (size_t)cap * PLAN_ROWS * 2;
+    hipLaunchKernelGGL((k_plan_apply<RK, CK, W>), dim3(nb), dim3(256), lds, edx::stream(), p, cap,
+                       x, e);
+}
+
+// Groups the operator's terms where the basis allows; the longest row sizes
+// the kernel's lists.
+template <int RK, int CK, class W>
+int mf_plan(edx_mfop *op, const PlanSpaces &sp, PlanStore<W> &store) {
+    EDX_TRY(plan_make<W>(sp, op->tt.ops.data(), op->tt.vals.data(), op->tt.nhop, op->tt.T,
+                         op->p.omega_on != 0, op->p.omega, op->p.negate != 0, true, store));
+    store.p.inter = 0;
+    DevBuf flag;
+    EDX_TRY(flag.alloc(sizeof(int), "longest row"));
+    EDX_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), edx::stream()));
+    EDX_TRY((plan_count<RK, W>(store.p, nullptr, flag.as<int>())));
+    EDX_HIP(edx::copy_sync(&op->maxrow, flag.p, sizeof(int), hipMemcpyDeviceToHost));
+    if (op->maxrow <= 255) op->plan = 8 * (int)sizeof(W);
+    return EDX_OK;
+}
+
+template <int RK, int CK> int mf_try_plan(edx_mfop *op, const edx_basis *fock) {
+    const PlanSpaces sp{RK, CK, op->p.nv, op->p.nc, fock, fock};
+    if (op->p.M == 0 || !plan_usable(sp, op->tt.ops.data(), op->tt.nhop, op->tt.T) ||
+        op->p.M >= ((int64_t)1 << 31))
+        return EDX_OK;
+    return plan_bits(sp) <= 32 ? mf_plan<RK, CK, uint32_t>(op, sp, op->plan32)
+                               : mf_plan<RK, CK, uint64_t>(op, sp, op->plan64);
+}
+
 int mf_launch(const edx_mfop *op, const double2 *x, const SpmvEpi &e, int *nblocks_out) {
     const int nb = mf_blocks(op);
     if (nblocks_out) *nblocks_out = nb;
     if (op->p.M == 0) return EDX_OK;
-    if (op->corehole)
+    if (op->plan == 32 && op->corehole)
+        mf_launch_plan<ROW_COREHOLE, COL_COREHOLE>(op, op->plan32.p, nb, x, e);
+    else if (op->plan == 32)
+        mf_launch_plan<ROW_PLAIN, COL_PLAIN>(op, op->plan32.p, nb, x, e);
+    else if (op->plan == 64 && op->corehole)
+        mf_launch_plan<ROW_COREHOLE, COL_COREHOLE>(op, op->plan64.p, nb, x, e);
+    else if (op->plan == 64)
+        mf_launch_plan<ROW_PLAIN, COL_PLAIN>(op, op->plan64.p, nb, x, e);
+    else if (op->corehole)
         hipLaunchKernelGGL((k_mf<ROW_COREHOLE, COL_COREHOLE>), dim3(nb), dim3(64), 0,
                            edx::stream(), op->p, op->d_masks, x, e);
     else
@@ -239,6 +345,11 @@ int edx_mf_ham_i(const edx_basis *fock, const edx_tensor2 *hop, int64_t nhopp,
     o->p.nleft = fock->n;
     o->p.right = view_of(fock);
     o->corehole = 0;
+    const int rc = mf_try_plan<ROW_PLAIN, COL_PLAIN>(o, fock);
+    if (rc) {
+        delete o;
+        return rc;
+    }
     *out = o;
     return EDX_OK;
 }
@@ -257,6 +368,11 @@ int edx_mf_ham_n(const edx_basis *fock_n, int num_val_orbs, int num_core_orbs,
     o->p.nv = num_val_orbs;
     o->p.nc = num_core_orbs;
     o->corehole = 1;
+    const int rc = mf_try_plan<ROW_COREHOLE, COL_COREHOLE>(o, fock_n);
+    if (rc) {
+        delete o;
+        return rc;
+    }
     *out = o;
     return EDX_OK;
 }

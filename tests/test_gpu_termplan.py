@@ -128,3 +128,42 @@ def test_builds_that_keep_the_term_by_term_kernel(core, case):
     if case == "many_terms":
         assert len(ht) + len(ut) > 4096
     _same(core.build_ham_i(core.Basis.from_words(fock, n), ht, ut), R)
+
+
+@pytest.mark.parametrize("space,nv,nocc", [("i", 6, 1), ("i", 8, 4), ("i", 33, 2), ("i", 16, 8),
+                                           ("n", 7, 3), ("n", 28, 1)])
+def test_matrix_free_apply_at_word_and_workgroup_edges(core, space, nv, nocc):
+    """y += H x from the term plan against the oracle's product.  Both add the
+    same products in another order (the plan also adds equal terms' values
+    first): each row of n entries of T terms in all differs by at most
+    (n + T) eps times the sum of |value| |x|, bounded here through the longest
+    row and the largest term."""
+    import torch
+    nc = 6 if space == "n" else 0
+    rng = np.random.default_rng(nv)
+    ht, ut = _terms(min(nv + nc, 16), 7, 250)
+    if nv + nc > 16:
+        step = (nv + nc - 1) // 15
+        for t, fs in ((ht, ("ind1", "ind2")), (ut, ("ind1", "ind2", "ind3", "ind4"))):
+            for f in fs:
+                t[f] = 1 + (t[f] - 1) * step
+    fock = H.fock_words(nv, nocc)
+    b = core.Basis.combinations(nv, nocc)
+    for omega, sign in ((0j, 1.0), (0.5 - 0.25j, -1.0)):
+        if space == "i":
+            op = core.mf_ham_i(b, ht, ut, omega=omega, ham_sign=sign)
+            R = o.build_ham_i(fock, ht, ut, omega=omega, ham_sign=sign)
+        else:
+            op = core.mf_ham_n(b, nv, nc, ht, ut, omega=omega, ham_sign=sign)
+            R = o.build_ham_n(fock, nv, nc, ht, ut, omega=omega, ham_sign=sign)
+        x = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
+        y0 = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
+        dev = [torch.from_numpy(v).cuda() for v in (x, y0)]
+        y = op.apply(*dev).cpu().numpy()
+        ref = o.matvec(R, x, y0)
+        T = len(ht) + len(ut) + 1
+        big = max(np.abs(ht["re"] + 1j * ht["im"]).max(), np.abs(ut["re"] + 1j * ut["im"]).max(),
+                  abs(omega), 1.0)
+        assert np.abs(y - ref).max() <= 2 * T * 2.3e-16 * T * big * np.abs(x).max()
+        again = op.apply(dev[0], torch.from_numpy(y0).cuda()).cpu().numpy()
+        assert np.array_equal(y, again)
