@@ -1,0 +1,43 @@
+"""The division-free continued fraction against the nested one in extended
+precision, at the edges of its blocks, stages and range."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("neff", [1, 2, 7, 8, 9, 511, 512, 513, 521, 2500])
+@pytest.mark.parametrize("nw,scale", [(1, 1.0), (65, 1.0), (130, 1e-12), (64, 1e12), (64, 1e20),
+                                      (64, 1e-20)])
+def test_fraction_matches_extended_precision(neff, nw, scale):
+    """Rounding is that of coefficients off by a few eps: with T perturbed by dT,
+    the fraction norm <1|(z - T)^-1|1> changes by at most norm |dT| / gamma^2,
+    |dT| <= c eps (|z - a| + 2 b) with c = 8 for the operations of a step.
+    Scales 1e20 and 1e-20 leave the recurrence's range."""
+    from edrixs_amd import core
+    rng = np.random.default_rng(neff + nw)
+    a, b = rng.normal(20.0, 6.0, neff) * scale, np.abs(rng.normal(8.0, 2.0, neff)) * scale
+    om, g = np.linspace(-30.0, 50.0, nw) * scale, np.full(nw, 0.4 * scale)
+    norm, e, weight = 0.7, 3.0 * scale, 0.6
+    start = rng.normal(size=nw) / scale
+    got = core.cf_spectrum(a, b, norm, e, om, g, weight=weight, out=start.copy())
+    al, bl = a.astype(np.longdouble), b.astype(np.longdouble)
+    z = (om.astype(np.longdouble) + e) + 1j * g.astype(np.longdouble)
+    t = np.zeros(nw, dtype=np.clongdouble)
+    for j in range(neff - 1, 0, -1):
+        t = bl[j - 1] ** 2 / (z - al[j] - t)
+    ref = start - np.imag(1 / (z - al[0] - t)) * norm * weight / np.pi
+    eps = np.finfo(float).eps
+    width = np.abs(z[:, None] - al[None, :]).max() + 2 * bl.max()
+    tol = weight * norm / np.pi * 8 * eps * width / g[0] ** 2 + 4 * eps * np.abs(ref).max()
+    assert np.abs(got - ref).max() <= tol
+
+
+def test_breakdown_and_zero_couplings():
+    """A zero coupling ends the fraction there; the coefficients behind it do not matter."""
+    from edrixs_amd import core
+    om = np.linspace(-5.0, 5.0, 70)
+    a, b = np.array([1.0, -2.0, 0.5, 9.0, 4.0]), np.array([0.8, 0.0, 3.0, 2.0, 1.0])
+    s = core.cf_spectrum(a, b, 1.0, 0.0, om, 0.3)
+    t = core.cf_spectrum(a[:2], b[:2], 1.0, 0.0, om, 0.3)
+    np.testing.assert_allclose(s, t, rtol=1e-14)
