@@ -42,6 +42,7 @@ struct BEpi {
     const double2 *c2;     // per RHS [K] or nullptr (no x term)
     const double2 *dvec;   // interleaved or nullptr
     double2 *partials;     // [nblocks * K]
+    StepTail tail;         // scalar work after the product
 };
 
 __device__ __forceinline__ double2 epilogue(const BEpi &e, int k, int64_t o, double2 hx,
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(256) void k_spmm_rlp(int64_t m, int K, const int64_
 }
 
 // Row-split schedule: G lanes per row, KT right-hand sides per pass (blockIdx.y).
-template <int G, int KT, class VP, class XT, class ACC, bool SPLIT>
+template <int G, int KT, class VP, class XT, class ACC, bool SPLIT, bool TAIL>
 __global__ __launch_bounds__(256) void k_spmm_il(int64_t m, int K, const int64_t *__restrict__ rowptr,
                                                  const int32_t *__restrict__ cols, VP vals,
                                                  const double2 *__restrict__ diag,
@@ -276,8 +277,10 @@ __global__ __launch_bounds__(256) void k_spmm_il(int64_t m, int K, const int64_t
 #pragma unroll
         for (int q = 0; q < KT; ++q) {
             double2 s = block_sum_256(dot[q]);
-            if (threadIdx.x == 0 && k0 + q < K) e.partials[(int64_t)blockIdx.x * K + k0 + q] = s;
+            if (threadIdx.x == 0 && k0 + q < K)
+                part_put<TAIL>(e.partials + (int64_t)blockIdx.x * K + k0 + q, s);
         }
+        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -288,7 +291,7 @@ __global__ __launch_bounds__(256) void k_spmm_il(int64_t m, int K, const int64_t
 // one XCD (blockIdx.x % 8) sweep one contiguous eighth of the rows, so rows
 // that gather the same X lines share that XCD's L2; otherwise consecutive
 // 16-row groups go to consecutive workgroups, i.e. to all eight XCDs.
-template <int NPL, class VP, class XT, class ACC, bool SPLIT>
+template <int NPL, class VP, class XT, class ACC, bool SPLIT, bool TAIL>
 __global__ __launch_bounds__(256) void k_spmm_rl(int64_t m, int K, const int64_t *__restrict__ rowptr,
                                                  const int32_t *__restrict__ cols, VP vals,
                                                  const double2 *__restrict__ diag,
@@ -373,8 +376,9 @@ __global__ __launch_bounds__(256) void k_spmm_rl(int64_t m, int K, const int64_t
             if (k >= K) continue;
             double2 s = make_double2(0, 0);
             for (int g = 0; g < 16; ++g) s = cadd(s, red[(g * NPL + q) * 16 + ll]);
-            e.partials[(int64_t)blockIdx.x * K + k] = s;
+            part_put<TAIL>(e.partials + (int64_t)blockIdx.x * K + k, s);
         }
+        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -384,7 +388,7 @@ int bspmm_blocks(int64_t m) {
     int64_t cap = (int64_t)edx::num_cus() * 8;
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
-    return (int)blocks;
+    return (int)((blocks + 7) / 8 * 8);   // the XCD-contiguous schedules need a multiple of 8
 }
 
 int pick_lanes(const edx_csr *a) {
@@ -411,6 +415,13 @@ int elem_grid_x(int64_t n) {
     return (int)g;
 }
 
+// Workgroups per 16 right-hand sides of a step's vector update: see
+// step_vec_blocks.
+int step_elem_grid_x(int64_t n) {
+    const int g = elem_grid_x(n);
+    return n <= (1 << 17) ? std::min(g, edx::num_cus()) : g;
+}
+
 struct ELaunch {
     dim3 grid, block;
 };
@@ -429,7 +440,9 @@ ELaunch elaunch(int64_t n, int K) {
     const int64_t rstart = (int64_t)blockIdx.x * ESLOTS + slot;
 
 // per-(block, k) sum over the 64 slots in slot order -> partials[blockIdx.x*K + k]
-__device__ __forceinline__ void elem_reduce(double2 acc, int K, double2 *partials) {
+template <bool TAIL = false>
+__device__ __forceinline__ void elem_reduce(double2 acc, int K, double2 *partials,
+                                            const StepTail &tail = StepTail{}) {
     __shared__ double2 red[ESLOTS * 16];
     const int kte = blockDim.x / ESLOTS;
     const int kk = threadIdx.x % kte, slot = threadIdx.x / kte;
@@ -439,8 +452,9 @@ __device__ __forceinline__ void elem_reduce(double2 acc, int K, double2 *partial
     if (slot == 0 && k < K) {
         double2 s = make_double2(0, 0);
         for (int q = 0; q < ESLOTS; ++q) s = cadd(s, red[q * kte + kk]);
-        partials[(int64_t)blockIdx.x * K + k] = s;
+        part_put<TAIL>(partials + (int64_t)blockIdx.x * K + k, s);
     }
+    step_tail<TAIL>(tail, partials);
 }
 
 // partials of sum_r conj(a) b per RHS
@@ -526,25 +540,6 @@ __global__ void k_bdiv_sqrt_norm(int64_t n, int K, double2 *v, const double *nor
 
 // ------------------------------------------------------- batched Krylov
 
-// The recurrence keeps its vectors unnormalized: the stored u_i is the
-// residual w_i of the previous step, with v_i = u_i / s_i and s_i = beta_i
-// (s_1 = 1 after the start vector is normalized).  The product of a step is
-// y = (1/s_i) H u_i - (beta_i / s_{i-1}) u_{i-1} = H v_i - beta_i v_{i-1}, its
-// dot <u_i|y> / s_i = alpha_i, and the residual y - (alpha_i / s_i) u_i is the
-// next stored vector: no pass divides a vector by beta.
-struct BKrylov {
-    double *alpha;     // [maxn * K], alpha[(i-1)*K + k]
-    double *beta;      // [(maxn+1) * K]
-    double *norm;      // [K]
-    int *neff;         // [K]
-    int *run;          // [(maxn+1) * K]
-    double2 *c1;       // [K]  -beta_i / s_{i-1}: coefficient of u_{i-1} in the product
-    double2 *sums;     // [K]
-    double2 *c0;       // [K]  1 / s_i: scale of H u_i in the product
-    double *acoef;     // [K]  alpha_i / s_i: coefficient of u_i in the residual
-    double *scur;      // [K]  s_i
-};
-
 // doubles of the per-RHS tail of the scalar block (norm .. scur) per RHS
 constexpr int BK_TAIL = 1 + 2 + 2 + 2 + 1 + 1;
 
@@ -559,20 +554,10 @@ __global__ void k_bk_init(BKrylov s, int K, const double2 *sums) {
     s.run[k] = sums[k].x > 0.0 ? 1 : 0;
 }
 
-__global__ void k_bk_alpha(BKrylov s, int K, int i, const double2 *sums) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
-    if (!s.run[(i - 1) * K + k]) return;
-    const double inv = s.c0[k].x;
-    const double a = sums[k].x * inv;
-    s.alpha[(int64_t)(i - 1) * K + k] = a;
-    s.acoef[k] = a * inv;
-    s.neff[k] = i;
-}
-
 // y -= alpha_k x ; partial |y|^2
+template <bool TAIL>
 __global__ void k_baxpy_norm(int64_t n, int K, double2 *y, const double2 *x, const double *alpha_i,
-                             double2 *partials) {
+                             double2 *partials, StepTail tail) {
     ELEM_SETUP
     double2 s = make_double2(0, 0);
     if (kv) {
@@ -584,22 +569,7 @@ __global__ void k_baxpy_norm(int64_t n, int K, double2 *y, const double2 *x, con
             s.x += v.x * v.x + v.y * v.y;
         }
     }
-    elem_reduce(s, K, partials);
-}
-
-__global__ void k_bk_beta(BKrylov s, int K, int i, const double2 *sums) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
-    if (!s.run[(i - 1) * K + k]) {
-        s.run[i * K + k] = 0;
-        return;
-    }
-    const double b = sqrt(sums[k].x);
-    s.beta[(int64_t)i * K + k] = b;
-    s.c1[k] = make_double2(-b / s.scur[k], -0.0);
-    s.scur[k] = b;
-    s.c0[k] = make_double2(b > 0.0 ? 1.0 / b : 0.0, 0.0);
-    s.run[i * K + k] = fabs(b) < 1e-10 ? 0 : 1;   // src/lanczos.f90:290-293
+    elem_reduce<TAIL>(s, K, partials, tail);
 }
 
 // ------------------------------------------------------- batched MINRES
@@ -882,6 +852,7 @@ struct BSched {
     int p;
 };
 int fac_spmm_launch(const edx_csr *a, int K, const double2 *X, const BEpi &e, int bpc);
+int fac_spmm_blocks(const edx_csr *a, int bpc);
 double fac_bytes_k(const edx_csr *a, int K, bool z, bool dvec);
 inline bool fac_spmm_ok(const edx_csr *a, int precision, int K) {
     return precision == EDX_C128I && a->d_fr_rowptr && a->nc_slots == 6 && K >= 2 && K <= 4;
@@ -909,11 +880,22 @@ void forced_bsched(int K, BSched *sched) {
 }
 
 // Workgroups (and dot partials per right-hand side) of a schedule's launch.
-// The pipelined schedule needs a multiple of 8 and at most bspmm_blocks(m),
-// the partials every caller provides.
+// The pipelined and factored schedules need a multiple of 8 and at most
+// bspmm_blocks(m), the partials every caller provides; a matrix with fewer rows
+// than their grid would take gets a smaller one.
 int bsched_blocks(const edx_csr *a, BSched sched) {
-    if (sched.rl >= 2) return (edx::num_cus() * sched.p + 7) / 8 * 8;
+    if (sched.rl == 3) return fac_spmm_blocks(a, sched.p);
+    if (sched.rl >= 2)
+        return std::min((edx::num_cus() * sched.p + 7) / 8 * 8,
+                        (int)std::min<int64_t>((a->m + 127) / 128 * 8, 1 << 20));
     return bspmm_blocks(a->m);
+}
+
+// Passes (blockIdx.y) of a schedule's launch.
+int bsched_passes(int K, BSched sched) {
+    if (sched.rl == 3) return 1;
+    if (sched.rl == 1) return (K + 16 * sched.p - 1) / (16 * sched.p);
+    return sched.rl ? (K + 15) / 16 : (K + BKT - 1) / BKT;
 }
 
 int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, const float2 *X32,
@@ -966,24 +948,30 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
         const int npl = sched.p;
         dim3 grid((unsigned)nb, (unsigned)((K + 16 * npl - 1) / (16 * npl)));
         const int xmap = nb % 8 == 0 && xcd_map_enabled();
-#define EDX_RL(NP)                                                                                 \
-    case NP:                                                                                       \
+#define EDX_RLT(NP, TL)                                                                            \
         if (precision == EDX_C128)                                                                 \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const double2 *, double2, double, false>), grid,      \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const double2 *, double2, double, false, TL>), grid,      \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const double2 *)a->d_vals, nullptr, X64, X64, e, xmap);           \
         else if (precision == EDX_C64)                                                             \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, float2, float, false>), grid,         \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, float2, float, false, TL>), grid,         \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const float2 *)a->d_vals32, nullptr, X32, X64, e, xmap);          \
         else if (precision == EDX_C128I)                                                           \
-            hipLaunchKernelGGL((k_spmm_rl<NP, IdxPtr, double2, double, true>), grid, dim3(256), 0,  \
+            hipLaunchKernelGGL((k_spmm_rl<NP, IdxPtr, double2, double, true, TL>), grid, dim3(256), 0,  \
                                stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,                  \
                                IdxPtr{a->d_off_idx, a->d_vtab}, a->d_diag, X64, X64, e, xmap);     \
         else                                                                                       \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, double2, double, true>), grid,        \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, double2, double, true, TL>), grid,        \
                                dim3(256), 0, stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,    \
-                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e, xmap);    \
+                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e, xmap);
+#define EDX_RL(NP)                                                                                 \
+    case NP:                                                                                       \
+        if (e.tail.count) {                                                                        \
+            EDX_RLT(NP, true)                                                                      \
+        } else {                                                                                   \
+            EDX_RLT(NP, false)                                                                     \
+        }                                                                                          \
         break;
         switch (npl) {
             EDX_RL(1)
@@ -992,28 +980,35 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
             EDX_RL(8)
             default: return set_error(EDX_ERR_ARG, "bad RHS tile %d", 16 * npl);
         }
+#undef EDX_RLT
 #undef EDX_RL
     } else {
         const int G = sched.p;
         dim3 grid((unsigned)nb, (unsigned)((K + BKT - 1) / BKT));
-#define EDX_BSPMM(GG)                                                                              \
-    case GG:                                                                                       \
+#define EDX_BSPMMT(GG, TL)                                                                         \
         if (precision == EDX_C128)                                                                 \
-            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const double2 *, double2, double, false>), grid, \
+            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const double2 *, double2, double, false, TL>), grid, \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const double2 *)a->d_vals, nullptr, X64, X64, e);                 \
         else if (precision == EDX_C64)                                                             \
-            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const float2 *, float2, float, false>), grid,    \
+            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const float2 *, float2, float, false, TL>), grid,    \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const float2 *)a->d_vals32, nullptr, X32, X64, e);                \
         else if (precision == EDX_C128I)                                                           \
-            hipLaunchKernelGGL((k_spmm_il<GG, BKT, IdxPtr, double2, double, true>), grid,           \
+            hipLaunchKernelGGL((k_spmm_il<GG, BKT, IdxPtr, double2, double, true, TL>), grid,           \
                                dim3(256), 0, stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,    \
                                IdxPtr{a->d_off_idx, a->d_vtab}, a->d_diag, X64, X64, e);           \
         else                                                                                       \
-            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const float2 *, double2, double, true>), grid,   \
+            hipLaunchKernelGGL((k_spmm_il<GG, BKT, const float2 *, double2, double, true, TL>), grid,   \
                                dim3(256), 0, stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,    \
-                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e);          \
+                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e);
+#define EDX_BSPMM(GG)                                                                              \
+    case GG:                                                                                       \
+        if (e.tail.count) {                                                                        \
+            EDX_BSPMMT(GG, true)                                                                   \
+        } else {                                                                                   \
+            EDX_BSPMMT(GG, false)                                                                  \
+        }                                                                                          \
         break;
         switch (G) {
             EDX_BSPMM(4)
@@ -1022,6 +1017,7 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
             EDX_BSPMM(32)
             default: return set_error(EDX_ERR_ARG, "unsupported lanes %d", G);
         }
+#undef EDX_BSPMMT
 #undef EDX_BSPMM
     }
     EDX_LAUNCH_CHECK();
@@ -1040,9 +1036,11 @@ BSched bspmm_rule(const edx_csr *a, int K) {
 
 // Y = epilogue(H X) for K interleaved RHS.  For C64, X32 holds the complex64
 // copy of X (interleaved); X64 is always the complex128 X (split diagonal and
-// shift terms read it).
+// shift terms read it).  With e_in.tail set, the launch ends with the step's
+// scalar work where it is narrow enough, and *nblocks_out is 0 then.
 int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const float2 *X32,
-          const BEpi &e, int *nblocks_out) {
+          const BEpi &e_in, int *nblocks_out) {
+    BEpi e = e_in;
     if (K == 1 && a->m >= TUNE_MIN_ROWS && !e.c2) {
         // one right-hand side of a large matrix: the tuned single-vector kernel
         // (its vector then fits the last-level cache, which an interleaved
@@ -1054,6 +1052,7 @@ int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const floa
         se.c1 = e.c1;
         se.dvec = e.dvec;
         se.partials = e.partials;
+        se.tail = e.tail;
         return spmv_launch(a, precision, precision == EDX_C64 ? (const void *)X32 : (const void *)X64,
                            se, 0, nblocks_out);
     }
@@ -1067,7 +1066,10 @@ int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const floa
                          "form, the indexed precision and 2 <= K <= 4");
     if (sched.rl == 4 && !packed_spmm_ok(a, precision))
         return set_error(EDX_ERR_ARG, "multi-RHS schedule 4 needs the packed indexed form");
-    if (nblocks_out) *nblocks_out = bsched_blocks(a, sched);
+    if (sched.rl == 2 || sched.rl == 4 ||
+        !tail_fits(bsched_blocks(a, sched), bsched_passes(K, sched), K))
+        e.tail.count = nullptr;
+    if (nblocks_out) *nblocks_out = e.tail.count ? 0 : bsched_blocks(a, sched);
     // the packed words read 4 bytes of index per nonzero instead of 6
     const double bytes = sched.rl == 3 ? fac_bytes_k(a, K, e.z != nullptr, e.dvec != nullptr)
                          : spmv_bytes_k(a, precision, K, e.z != nullptr, e.dvec != nullptr) -
@@ -1329,6 +1331,30 @@ struct Dbuf {
 
 }  // namespace
 
+namespace {
+
+// Launch of the update that ends a step of K interleaved recurrences, on nbx
+// workgroups per 16 of them; then beta's part of the step where the launch had
+// no tail.
+int baxpy_norm_step(int64_t n, int K, double2 *y, const double2 *x, const double *a,
+                    double2 *partials, StepTail t, int nbx) {
+    const ELaunch el = elaunch(n, K);
+    const dim3 grid(nbx, el.grid.y);
+    t.op = TAIL_BETA;
+    if (tail_fits(nbx, el.grid.y, K)) {
+        hipLaunchKernelGGL(k_baxpy_norm<true>, grid, el.block, 0, edx::stream(), n, K, y, x, a,
+                           partials, t);
+        EDX_LAUNCH_CHECK();
+        return EDX_OK;
+    }
+    hipLaunchKernelGGL(k_baxpy_norm<false>, grid, el.block, 0, edx::stream(), n, K, y, x, a, partials,
+                       t);
+    EDX_LAUNCH_CHECK();
+    return step_finish_launch(t, partials, nbx);
+}
+
+}  // namespace
+
 // A batched Krylov recurrence that can be advanced in pieces: the vectors, the
 // run flags and the (alpha, beta) history stay on the device between calls.
 // The scalar arrays grow geometrically (device-to-device copy) when a call
@@ -1342,7 +1368,7 @@ struct edx_krylov_batch {
     int cap = 0;         // steps the scalar arrays hold
     bool live = true;    // some RHS has not broken down
     int curr = 0, prev = 1;
-    Dbuf vb, x32, part, sc, flags;
+    Dbuf vb, x32, part, sc, flags, count;
     BKrylov st{};
 };
 
@@ -1401,6 +1427,8 @@ int kb_start(edx_krylov_batch *q, const double2 *V0cm, int cap) {
     EDX_TRY(q->part.alloc(std::max<size_t>((size_t)std::max(nbs, nbe) * K + 64,
                                            (size_t)edx::spmv_partials_len(q->h)) * sizeof(double2),
                           "partials"));
+    EDX_TRY(q->count.alloc(TAIL_BYTES, "arrival counters"));
+    EDX_HIP(hipMemsetAsync(q->count.p, 0, TAIL_BYTES, s));
     EDX_TRY(kb_layout(q, cap, nullptr, nullptr, 0));
     const BKrylov &st = q->st;
     double2 *v0 = q->vb.as<double2>();
@@ -1429,14 +1457,17 @@ int kb_advance(edx_krylov_batch *q, int nsteps) {
     }
     const int64_t n = q->n;
     const int K = q->K;
-    const int kb = (K + 63) / 64;
     hipStream_t s = edx::stream();
     const BKrylov &st = q->st;
     double2 *v[2] = {q->vb.as<double2>(), q->vb.as<double2>() + (size_t)n * K};
-    const int nbe = elem_grid_x(n);
+    const int nbe = step_elem_grid_x(n);
     const int nbv = vec_blocks(n);
     // the same condition routes the product to the single-vector SpMV (bspmm)
     const bool single = K == 1 && q->h->m >= TUNE_MIN_ROWS;
+    double2 *part = q->part.as<double2>();
+    StepTail t{};
+    t.K = K;
+    t.st = st;
     const int end = q->done + nsteps;
     int checked = q->done;
     for (int i = q->done + 1; i <= end; ++i) {
@@ -1448,24 +1479,19 @@ int kb_advance(edx_krylov_batch *q, int nsteps) {
         e.c0 = st.c0;
         e.c1 = st.c1;
         e.dvec = v[curr];
-        e.partials = q->part.as<double2>();
+        e.partials = part;
+        t.count = q->count.as<unsigned>();
+        t.op = TAIL_ALPHA;
+        t.i = i;
+        e.tail = t;
         int nb = 0;
         EDX_TRY(edx::bspmm(q->h, q->precision, K, v[curr], q->x32.as<float2>(), e, &nb));
-        hipLaunchKernelGGL(k_breduce, dim3(K), dim3(256), 0, s, q->part.as<double2>(), nb, K, st.sums);
-        hipLaunchKernelGGL(k_bk_alpha, dim3(kb), dim3(64), 0, s, st, K, i, st.sums);
+        EDX_TRY(step_finish_launch(t, part, nb));
         // u_{i+1} = y - (alpha_i/s_i) u_i, kept unnormalized (s_{i+1} = beta_{i+1})
-        if (single) {   // one vector of a large matrix: the plain vector kernels
-            hipLaunchKernelGGL(k_axpy_norm, dim3(nbv), dim3(VB), 0, s, n, v[prev], v[curr],
-                               st.acoef, q->part.as<double2>(), nullptr);
-            hipLaunchKernelGGL(k_breduce, dim3(1), dim3(256), 0, s, q->part.as<double2>(), nbv, 1,
-                               st.sums);
-        } else {
-            ELAUNCH(k_baxpy_norm, n, K, n, K, v[prev], v[curr], st.acoef, q->part.as<double2>());
-            hipLaunchKernelGGL(k_breduce, dim3(K), dim3(256), 0, s, q->part.as<double2>(), nbe, K,
-                               st.sums);
-        }
-        hipLaunchKernelGGL(k_bk_beta, dim3(kb), dim3(64), 0, s, st, K, i, st.sums);
-        EDX_LAUNCH_CHECK();
+        if (single)   // one vector of a large matrix: the plain vector kernel
+            EDX_TRY(axpy_norm_step(n, v[prev], v[curr], st.acoef, part, nullptr, t, nbv));
+        else
+            EDX_TRY(baxpy_norm_step(n, K, v[prev], v[curr], st.acoef, part, t, nbe));
         std::swap(q->curr, q->prev);
         q->done = i;
         if (i - checked >= 32 || i == end) {

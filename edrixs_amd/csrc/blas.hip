@@ -18,6 +18,13 @@ int vec_blocks(int64_t n) {
     return (int)g;
 }
 
+// Workgroups of a step's vector update: a vector of up to 2^17 rows takes few
+// enough for the update to end with the step's scalar work.
+int step_vec_blocks(int64_t n) {
+    const int g = vec_blocks(n);
+    return n <= (1 << 17) ? std::min(g, edx::num_cus()) : g;
+}
+
 // sum of partials[0, nb) by one block; returns the total in thread 0
 __device__ double2 reduce_partials(const double2 *partials, int nb) {
     __shared__ double sx[VB], sy[VB];
@@ -64,9 +71,10 @@ __global__ __launch_bounds__(VB) void k_div_real(int64_t n, double2 *y, const do
 }
 
 // y = y - a * x (a real, device) and partials of |y|^2
+template <bool TAIL>
 __global__ __launch_bounds__(VB) void k_axpy_norm(int64_t n, double2 *y, const double2 *x,
                                                   const double *a, double2 *partials,
-                                                  const int *run) {
+                                                  const int *run, StepTail tail) {
     if (run && *run == 0) return;
     const double al = *a;
     double2 s = make_double2(0, 0);
@@ -76,7 +84,24 @@ __global__ __launch_bounds__(VB) void k_axpy_norm(int64_t n, double2 *y, const d
         s.x += v.x * v.x + v.y * v.y;
     }
     s = block_sum_256(s);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+    if (threadIdx.x == 0) part_put<TAIL>(partials + blockIdx.x, s);
+    step_tail<TAIL>(tail, partials);
+}
+
+// Launch of the update that ends a step, on nb workgroups; then beta's part of
+// the step where the launch had no tail.
+int axpy_norm_step(int64_t n, double2 *y, const double2 *x, const double *a, double2 *partials,
+                   const int *run, StepTail t, int nb) {
+    hipStream_t s = edx::stream();
+    t.op = TAIL_BETA;
+    if (tail_fits(nb, 1, 1)) {
+        hipLaunchKernelGGL(k_axpy_norm<true>, dim3(nb), dim3(VB), 0, s, n, y, x, a, partials, run, t);
+        EDX_LAUNCH_CHECK();
+        return EDX_OK;
+    }
+    hipLaunchKernelGGL(k_axpy_norm<false>, dim3(nb), dim3(VB), 0, s, n, y, x, a, partials, run, t);
+    EDX_LAUNCH_CHECK();
+    return step_finish_launch(t, partials, nb);
 }
 
 // ------------------------------------------------ Krylov (build_krylov_mp)
@@ -108,32 +133,10 @@ __global__ __launch_bounds__(VB) void k_krylov_norm(const double2 *partials, int
     }
 }
 
-// alpha_i = Re <v_i | w>   (src/lanczos.f90:277-281)
-__global__ __launch_bounds__(VB) void k_krylov_alpha(const double2 *partials, int nb,
-                                                     KrylovDev *st, double *alpha, int i,
-                                                     const int *run) {
-    if (!run[i - 1]) return;
-    double2 s = reduce_partials(partials, nb);
-    if (threadIdx.x == 0) {
-        alpha[i - 1] = s.x;
-        st->neff = i;
-    }
-}
-
-// beta_i = sqrt(<w|w>); stop when beta_i < 1e-10 (src/lanczos.f90:285-293)
-__global__ __launch_bounds__(VB) void k_krylov_beta(const double2 *partials, int nb,
-                                                    KrylovDev *st, double *beta, int i, int *run) {
-    if (!run[i - 1]) {
-        if (threadIdx.x == 0) run[i] = 0;
-        return;
-    }
-    double2 s = reduce_partials(partials, nb);
-    if (threadIdx.x == 0) {
-        const double b = sqrt(s.x);
-        beta[i] = b;
-        st->coef[1] = make_double2(-b, -0.0);
-        run[i] = fabs(b) < 1e-10 ? 0 : 1;
-    }
+// The state of one recurrence as the step tails see it: a batch of one.
+inline BKrylov krylov_state(KrylovDev *st, double *alpha, double *beta, int *run) {
+    return BKrylov{alpha,        beta,         &st->norm,  &st->neff, run,
+                   &st->coef[1], &st->sum,     &st->coef[0], &st->acoef, &st->scur};
 }
 
 // -------------------------------------------------------- MINRES (linsys)

@@ -20,6 +20,7 @@
 #include "basis.hip"
 #include "termplan.hip"
 #include "csr_build.hip"
+#include "steptail.hip"
 #include "spmv.hip"
 #include "blas.hip"
 #include "krylov.hip"

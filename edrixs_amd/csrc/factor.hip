@@ -369,7 +369,7 @@ __global__ __launch_bounds__(256, WPE) void k_spmv_fac(FacArgs f, const double2 
 // R entry K contiguous values.  A capped grid (a multiple of 8 workgroups)
 // walks XCD-contiguous eighths of the valence rows, 4 (64 / NC) valence rows
 // per workgroup per pass; dot partials per workgroup and right-hand side.
-template <int NC, int K>
+template <int NC, int K, bool TAIL>
 __global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__restrict__ X, BEpi e) {
     extern __shared__ double2 s_tab[];
     __shared__ double2 red[4][K];
@@ -487,9 +487,10 @@ __global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__re
         __syncthreads();
         if (threadIdx.x < K) {
             const int k = threadIdx.x;
-            e.partials[(int64_t)blockIdx.x * K + k] =
-                cadd(cadd(red[0][k], red[1][k]), cadd(red[2][k], red[3][k]));
+            part_put<TAIL>(e.partials + (int64_t)blockIdx.x * K + k,
+                           cadd(cadd(red[0][k], red[1][k]), cadd(red[2][k], red[3][k])));
         }
+        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -549,19 +550,37 @@ int fac_launch(const edx_csr *a, const double2 *x, const SpmvEpi &e_in, int *nbl
     return EDX_OK;
 }
 
+// Workgroups of the multi-RHS factored product at bpc per CU: no more than
+// there are rows for.
+int fac_spmm_blocks(const edx_csr *a, int bpc) {
+    const int64_t mv = a->m / a->nc_slots, rows = fac_rows_per_block(a->nc_slots);
+    const int64_t nb = std::min<int64_t>((int64_t)num_cus() * bpc, (mv + rows - 1) / rows);
+    return (int)((std::max<int64_t>(nb, 1) + 7) / 8 * 8);
+}
+
 // Launch of the multi-RHS factored product with bpc workgroups per CU
 // (K = 2, 3 or 4; the caller has checked the form exists).
 int fac_spmm_launch(const edx_csr *a, int K, const double2 *X, const BEpi &e, int bpc) {
-    const int nb = (num_cus() * bpc + 7) / 8 * 8;
+    const int nb = fac_spmm_blocks(a, bpc);
     const FacArgs f = fac_args(a);
     const size_t lds = fac_lds_bytes(a);
     if (a->m == 0) return EDX_OK;
+#define EDX_FAC_CASE(KK)                                                                          \
+    case KK:                                                                                      \
+        if (e.tail.count)                                                                         \
+            hipLaunchKernelGGL((k_spmm_fac<6, KK, true>), dim3(nb), dim3(256), lds, stream(), f, X, \
+                               e);                                                                \
+        else                                                                                      \
+            hipLaunchKernelGGL((k_spmm_fac<6, KK, false>), dim3(nb), dim3(256), lds, stream(), f, X, \
+                               e);                                                                \
+        break;
     switch (K) {
-        case 2: hipLaunchKernelGGL((k_spmm_fac<6, 2>), dim3(nb), dim3(256), lds, stream(), f, X, e); break;
-        case 3: hipLaunchKernelGGL((k_spmm_fac<6, 3>), dim3(nb), dim3(256), lds, stream(), f, X, e); break;
-        case 4: hipLaunchKernelGGL((k_spmm_fac<6, 4>), dim3(nb), dim3(256), lds, stream(), f, X, e); break;
+        EDX_FAC_CASE(2)
+        EDX_FAC_CASE(3)
+        EDX_FAC_CASE(4)
         default: return set_error(EDX_ERR_ARG, "factored multi-RHS product for K = %d not built", K);
     }
+#undef EDX_FAC_CASE
     EDX_LAUNCH_CHECK();
     return EDX_OK;
 }

@@ -61,17 +61,20 @@ struct KrylovScratch {
     double2 *v;        // 2 n
     double2 *part;     // max(partials_len, vec_blocks(n))
     KrylovDev *S;
-    double *ab;        // 2 maxn + 2
+    double *ab;        // 2 maxn + 2, right behind S (read back with it)
     int *run;          // maxn + 2
+    unsigned *count;   // arrival counters of the step tails
 };
+
+constexpr size_t KRYLOV_HEAD = (sizeof(KrylovDev) + 15) / 16 * 16;
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 size_t krylov_scratch_bytes(int64_t n, int64_t partials_len, int maxn) {
     const int64_t np = std::max<int64_t>(partials_len, vec_blocks(n));
     return align256(2 * (size_t)n * sizeof(double2)) + align256((size_t)np * sizeof(double2)) +
-           align256(sizeof(KrylovDev)) + align256((2 * (size_t)maxn + 2) * sizeof(double)) +
-           align256(((size_t)maxn + 2) * sizeof(int));
+           align256(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double)) +
+           align256(((size_t)maxn + 2) * sizeof(int)) + align256(TAIL_BYTES);
 }
 
 KrylovScratch krylov_scratch_carve(char *base, int64_t n, int64_t partials_len, int maxn) {
@@ -82,10 +85,11 @@ KrylovScratch krylov_scratch_carve(char *base, int64_t n, int64_t partials_len, 
     k.part = (double2 *)base;
     base += align256((size_t)np * sizeof(double2));
     k.S = (KrylovDev *)base;
-    base += align256(sizeof(KrylovDev));
-    k.ab = (double *)base;
-    base += align256((2 * (size_t)maxn + 2) * sizeof(double));
+    k.ab = (double *)(base + KRYLOV_HEAD);
+    base += align256(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double));
     k.run = (int *)base;
+    base += align256(((size_t)maxn + 2) * sizeof(int));
+    k.count = (unsigned *)base;
     return k;
 }
 
@@ -98,20 +102,23 @@ __global__ void k_zero_words(int64_t nwords, uint64_t *p) {
 }
 
 // build_krylov_mp (src/lanczos.f90:210-303) over any product
-// prod(x, epilogue, &nblocks) that writes y = c0 A x + c1 z with dot partials;
+// prod(x, epilogue, &nblocks) that writes y = c0 A x + c1 z with dot partials
+// (nblocks of them left to sum, 0 if it ran the epilogue's tail);
 // the run's device memory comes in k (see KrylovScratch).
 template <class Prod>
 int krylov_loop_in(int64_t n, Prod prod, const KrylovScratch &k, const double2 *v0, int maxn,
                    int *neff, double *alpha, double *beta, double *norm) {
-    int nbv = vec_blocks(n);
+    int nbv = step_vec_blocks(n);
     double2 *v[2] = {k.v, k.v + n};
     double *d_alpha = k.ab, *d_beta = k.ab + maxn + 1;
     int *run = k.run;
     KrylovDev *S = k.S;
     hipStream_t s = edx::stream();
-    // clear the vectors, the history and the run flags (fill kernels, no memset nodes)
-    const int64_t nz[3] = {4 * n, 2 * (int64_t)maxn + 2, ((int64_t)maxn + 2 + 1) / 2};
-    uint64_t *pz[3] = {(uint64_t *)k.v, (uint64_t *)k.ab, (uint64_t *)k.run};
+    // clear the second vector, the history, the run flags and the counters
+    // (fill kernels, no memset nodes)
+    const int64_t nz[3] = {2 * n, 2 * (int64_t)maxn + 2,
+                           (int64_t)(align256(((size_t)maxn + 2) * sizeof(int)) + TAIL_BYTES) / 8};
+    uint64_t *pz[3] = {(uint64_t *)v[1], (uint64_t *)k.ab, (uint64_t *)k.run};
     for (int q = 0; q < 3; ++q)
         hipLaunchKernelGGL(k_zero_words, dim3(vec_blocks(nz[q])), dim3(VB), 0, s, nz[q], pz[q]);
     EDX_HIP(hipMemcpyAsync(v[0], v0, n * sizeof(double2), hipMemcpyDeviceToDevice, s));
@@ -122,10 +129,16 @@ int krylov_loop_in(int64_t n, Prod prod, const KrylovScratch &k, const double2 *
     hipLaunchKernelGGL(k_krylov_norm, dim3(1), dim3(VB), 0, s, part_p, nbv, S);
     hipLaunchKernelGGL(k_div_real, dim3(nbv), dim3(VB), 0, s, n, v[0], &S->sqrt_norm, nullptr);
     EDX_LAUNCH_CHECK();
+    StepTail t{};
+    t.K = 1;
+    t.st = krylov_state(S, d_alpha, d_beta, run);
     int curr = 0, prev = 1;
     int checked = 0;
     for (int i = 1; i <= maxn; ++i) {
-        // prev = -beta_{i-1} prev + H curr ; partial <curr|prev>
+        // y = (1/s_i) H u_i - (beta_i/s_{i-1}) u_{i-1}; alpha_i from <u_i|y>
+        t.count = k.count;
+        t.op = TAIL_ALPHA;
+        t.i = i;
         SpmvEpi e{};
         e.y = v[prev];
         e.z = v[prev];
@@ -134,16 +147,12 @@ int krylov_loop_in(int64_t n, Prod prod, const KrylovScratch &k, const double2 *
         e.dvec = v[curr];
         e.partials = part_p;
         e.run = run + (i - 1);
+        e.tail = t;
         int nb = 0;
         EDX_TRY(prod((const double2 *)v[curr], e, &nb, run + (i - 1)));
-        hipLaunchKernelGGL(k_krylov_alpha, dim3(1), dim3(VB), 0, s, part_p, nb, S,
-                           d_alpha, i, run);
-        hipLaunchKernelGGL(k_axpy_norm, dim3(nbv), dim3(VB), 0, s, n, v[prev], v[curr],
-                           d_alpha + (i - 1), part_p, run + (i - 1));
-        hipLaunchKernelGGL(k_krylov_beta, dim3(1), dim3(VB), 0, s, part_p, nbv, S,
-                           d_beta, i, run);
-        hipLaunchKernelGGL(k_div_real, dim3(nbv), dim3(VB), 0, s, n, v[prev], d_beta + i, run + i);
-        EDX_LAUNCH_CHECK();
+        EDX_TRY(step_finish_launch(t, part_p, nb));
+        // u_{i+1} = y - (alpha_i/s_i) u_i; beta_{i+1} from its norm
+        EDX_TRY(axpy_norm_step(n, v[prev], v[curr], &S->acoef, part_p, run + (i - 1), t, nbv));
         std::swap(curr, prev);
         if (i - checked >= 32 && i < maxn) {   // stop launching once the recurrence broke down
             int r = 1;
@@ -152,11 +161,14 @@ int krylov_loop_in(int64_t n, Prod prod, const KrylovScratch &k, const double2 *
             if (!r) break;
         }
     }
+    // the state and alpha_1 .. alpha_maxn, (beta_0,) beta_1 .. beta_maxn behind it
+    std::vector<char> h(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double));
+    EDX_HIP(edx::copy_sync(h.data(), S, h.size(), hipMemcpyDeviceToHost));
     KrylovDev hs;
-    EDX_HIP(edx::copy_sync(&hs, S, sizeof(KrylovDev), hipMemcpyDeviceToHost));
-    EDX_HIP(edx::copy_sync(alpha, d_alpha, maxn * sizeof(double), hipMemcpyDeviceToHost));
-    // beta_1 .. beta_maxn
-    EDX_HIP(edx::copy_sync(beta, d_beta + 1, maxn * sizeof(double), hipMemcpyDeviceToHost));
+    memcpy(&hs, h.data(), sizeof(hs));
+    const char *hab = h.data() + KRYLOV_HEAD;
+    memcpy(alpha, hab, maxn * sizeof(double));
+    memcpy(beta, hab + ((size_t)maxn + 2) * sizeof(double), maxn * sizeof(double));
     *neff = hs.neff;
     *norm = hs.norm;
     return EDX_OK;

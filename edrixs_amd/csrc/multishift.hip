@@ -33,81 +33,6 @@ namespace {
 
 constexpr int MS_MAXK = 256;   // shifts per call (one block holds their scalars)
 
-struct MsShift {
-    double2 sigma;
-    double2 eta;       // pivot eta_i of the current step
-    double2 inv_eta;   // 1 / eta_i
-    double2 zeta;      // zeta_i
-    double res;        // residual estimate of the last finished iterate (absolute)
-    int active;        // still iterating
-    int iters;         // iterate the stored projection belongs to
-};
-
-struct MsCtl {
-    double tol_abs;
-    int nactive;
-};
-
-__device__ __forceinline__ double2 crecip(double2 a) {
-    const double d = a.x * a.x + a.y * a.y;
-    return make_double2(a.x / d, -a.y / d);
-}
-
-__device__ __forceinline__ double cabs2(double2 a) { return sqrt(a.x * a.x + a.y * a.y); }
-
-// Step i (1-based) of the shift recurrences, after alpha_i is known.  A shift
-// whose iterate i-1 already meets the tolerance is frozen there.  Block r
-// serves right-hand side r of R: alpha_i, beta_{i-1} and the run flag of step
-// i-1 at [(i - 1) R + r], its K shifts at sh[r K ..], its control at ctl[r].
-__global__ __launch_bounds__(256) void k_ms_scalars(int i, const double *alpha, const double *beta,
-                                                    int R, const double *sqrt_norm, MsShift *sh,
-                                                    int K, MsCtl *ctl, const int *run) {
-    const int rr = blockIdx.x;
-    const int64_t o = (int64_t)(i - 1) * R + rr;
-    if (!run[o]) return;
-    sh += (int64_t)rr * K;
-    ctl += rr;
-    __shared__ int cnt[256];
-    int c = 0;
-    const double tol = ctl->tol_abs;
-    const double nb = sqrt_norm[rr];
-    for (int k = threadIdx.x; k < K; k += 256) {
-        MsShift s = sh[k];
-        const double a = alpha[o];
-        if (i == 1) {
-            s.eta = make_double2(s.sigma.x - a, s.sigma.y);
-            s.zeta = make_double2(nb, 0.0);
-            s.active = 1;
-            s.iters = 0;
-            s.res = nb;
-        } else if (s.active) {
-            const double bp = beta[o];
-            const double2 ratio = cmul(s.zeta, s.inv_eta);   // zeta_{i-1} / eta_{i-1}
-            s.res = bp * cabs2(ratio);
-            if (s.res <= tol) {
-                s.active = 0;
-            } else {
-                s.zeta = cscale(ratio, bp);
-                const double2 t = cscale(s.inv_eta, bp * bp);
-                s.eta = make_double2(s.sigma.x - a - t.x, s.sigma.y - t.y);
-            }
-        }
-        if (s.active) {
-            s.inv_eta = crecip(s.eta);
-            s.iters = i;
-            ++c;
-        }
-        sh[k] = s;
-    }
-    cnt[threadIdx.x] = c;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) cnt[threadIdx.x] += cnt[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) ctl->nactive = cnt[0];
-}
-
 // A projection operator: a CSR with complex128 values, and where it has one
 // (csr_add_packed_all) its packed words (column | value number << 24) with
 // the table of distinct values, read instead of the columns and values.
@@ -340,40 +265,6 @@ __global__ __launch_bounds__(256) void k_ms_update(int64_t mP, MsP P,
     }
 }
 
-// The Lanczos vectors are kept unnormalized: u_i with v_i = u_i / s_i and
-// s_i = beta_i (s_1 = 1).  alpha_i = <u_i | y> / s_i for the product
-// y = (1/s_i) H u_i - (beta_i / s_{i-1}) u_{i-1}, and u_{i+1} = y - (alpha_i / s_i) u_i.
-__global__ __launch_bounds__(VB) void k_ms_alpha(const double2 *partials, int nb, KrylovDev *st,
-                                                 double *alpha, int i, const int *run) {
-    if (!run[i - 1]) return;
-    double2 s = reduce_partials(partials, nb);
-    if (threadIdx.x == 0) {
-        const double inv = st->coef[0].x;
-        const double a = s.x * inv;
-        alpha[i - 1] = a;
-        st->acoef = a * inv;
-        st->neff = i;
-    }
-}
-
-// beta_i as in build_krylov_mp; the recurrence also stops once no shift is active
-__global__ __launch_bounds__(VB) void k_ms_beta(const double2 *partials, int nb, KrylovDev *st,
-                                                double *beta, int i, int *run, const MsCtl *ctl) {
-    if (!run[i - 1]) {
-        if (threadIdx.x == 0) run[i] = 0;
-        return;
-    }
-    double2 s = reduce_partials(partials, nb);
-    if (threadIdx.x == 0) {
-        const double b = sqrt(s.x);
-        beta[i] = b;
-        st->coef[1] = make_double2(-b / st->scur, -0.0);
-        st->scur = b;
-        st->coef[0] = make_double2(b > 0.0 ? 1.0 / b : 0.0, 0.0);
-        run[i] = (fabs(b) < 1e-10 || ctl->nactive == 0) ? 0 : 1;
-    }
-}
-
 // shifts still active when the recurrence ends keep iterate neff (block r:
 // right-hand side r of R, beta_m at beta[m R + r])
 __global__ void k_ms_finish(const int *neff, const double *beta, int R, MsShift *sh, int K) {
@@ -440,7 +331,7 @@ int shifted_fom_run(const edx_csr *h, int precision, const double2 *b, int K, co
         const int64_t mp = proj[p] ? proj[p]->m : n;
         if (mp && K) EDX_HIP(hipMemsetAsync(out[p], 0, (size_t)mp * K * sizeof(double2), s));
     }
-    DevBuf vb, x32, part, st, ab, runf, shb, ctlb, qb, wb, slb;
+    DevBuf vb, x32, part, st, ab, runf, shb, ctlb, qb, wb, slb, cntb;
     EDX_TRY(vb.alloc(2 * (size_t)n * sizeof(double2), "fom lanczos vectors"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc((size_t)n * sizeof(float2), "fom x32"));
     const int nbv = vec_blocks(n);
@@ -451,6 +342,8 @@ int shifted_fom_run(const edx_csr *h, int precision, const double2 *b, int K, co
     EDX_TRY(runf.alloc(((size_t)maxit + 2) * sizeof(int), "run flags"));
     EDX_TRY(shb.alloc((size_t)K * sizeof(MsShift), "shift state"));
     EDX_TRY(ctlb.alloc(sizeof(MsCtl), "shift control"));
+    EDX_TRY(cntb.alloc(TAIL_BYTES, "arrival counters"));
+    EDX_HIP(hipMemsetAsync(cntb.p, 0, TAIL_BYTES, s));
     size_t qtot = 0;
     std::vector<size_t> qoff(nproj);
     for (int p = 0; p < nproj; ++p) {
@@ -507,9 +400,20 @@ int shifted_fom_run(const edx_csr *h, int precision, const double2 *b, int K, co
     hipLaunchKernelGGL(k_div_real, dim3(nbv), dim3(VB), 0, s, n, v[0], &S->sqrt_norm, nullptr);
     EDX_LAUNCH_CHECK();
 
+    StepTail t{};
+    t.K = 1;
+    t.st = krylov_state(S, d_alpha, d_beta, run);
+    t.nshift = K;
+    t.sh = sh;
+    t.ctl = ctl;
+    t.sqn = &S->sqrt_norm;
     int curr = 0, prev = 1, checked = 0, last = 0;
     for (int i = 1; i <= maxit; ++i) {
+        t.count = cntb.as<unsigned>();
+        t.op = TAIL_ALPHA;
+        t.i = i;
         SpmvEpi e{};
+        e.tail = t;
         e.y = v[prev];
         e.z = v[prev];
         e.c0 = &S->coef[0];
@@ -519,10 +423,7 @@ int shifted_fom_run(const edx_csr *h, int precision, const double2 *b, int K, co
         e.run = run + (i - 1);
         int nb = 0;
         EDX_TRY(apply(h, precision, v[curr], x32.as<float2>(), e, &nb, run + (i - 1)));
-        hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(VB), 0, s, part.as<double2>(), nb, S,
-                           d_alpha, i, run);
-        hipLaunchKernelGGL(k_ms_scalars, dim3(1), dim3(256), 0, s, i, d_alpha, d_beta, 1,
-                           &S->sqrt_norm, sh, K, ctl, run);
+        EDX_TRY(step_finish_launch(t, part.as<double2>(), nb));
         const int j = (i - 1) % win;   // the step's place in its window
         for (int p = 0; p < nproj; ++p) {
             const edx_csr *P = proj[p];
@@ -540,11 +441,8 @@ int shifted_fom_run(const edx_csr *h, int precision, const double2 *b, int K, co
                                          out[p], run + (i - 1), ctl, 1));
         }
         last = i;
-        hipLaunchKernelGGL(k_axpy_norm, dim3(nbv), dim3(VB), 0, s, n, v[prev], v[curr],
-                           &S->acoef, part.as<double2>(), run + (i - 1));
-        hipLaunchKernelGGL(k_ms_beta, dim3(1), dim3(VB), 0, s, part.as<double2>(), nbv, S, d_beta,
-                           i, run, ctl);
-        EDX_LAUNCH_CHECK();
+        EDX_TRY(axpy_norm_step(n, v[prev], v[curr], &S->acoef, part.as<double2>(), run + (i - 1), t,
+                               nbv));
         std::swap(curr, prev);
         if (i - checked >= 16 && i < maxit) {
             int r = 1;
@@ -588,11 +486,6 @@ __global__ void k_msb_init(int R, int K, const double *norm, double *sqrt_norm, 
     ctl[r] = MsCtl{tol * nb, K};
 }
 
-__global__ void k_msb_stop(int i, int R, int *run, const MsCtl *ctl) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < R && ctl[r].nactive == 0) run[(int64_t)i * R + r] = 0;
-}
-
 int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 *Bcm, int K,
                           const double *sigma, const edx_csr *const *proj, double2 *const *out,
                           double tol, int maxit, int *iters, double *final_res) {
@@ -603,7 +496,7 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
         if (mp) EDX_HIP(hipMemsetAsync(out[r], 0, (size_t)mp * K * sizeof(double2), s));
     }
     const size_t nr = (size_t)n * R;
-    Dbuf vb, x32, part, sc, flags, shb, ctlb, qb, wb, slb, nrm;
+    Dbuf vb, x32, part, sc, flags, shb, ctlb, qb, wb, slb, nrm, cntb;
     EDX_TRY(vb.alloc(2 * nr * sizeof(double2), "batched fom lanczos vectors"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(nr * sizeof(float2), "batched fom x32"));
     const int nbs = bspmm_blocks(n), nbe = elem_grid_x(n);
@@ -617,6 +510,8 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
     EDX_TRY(shb.alloc((size_t)R * K * sizeof(MsShift), "shift states"));
     EDX_TRY(ctlb.alloc((size_t)R * sizeof(MsCtl), "shift controls"));
     EDX_TRY(nrm.alloc((size_t)R * sizeof(double), "rhs norms"));
+    EDX_TRY(cntb.alloc(TAIL_BYTES, "arrival counters"));
+    EDX_HIP(hipMemsetAsync(cntb.p, 0, TAIL_BYTES, s));
     std::vector<size_t> qoff(R), woff(R);
     size_t qtot = 0, wtot = 0;
     const int win = ms_window(K);
@@ -667,8 +562,18 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
     ELAUNCH(k_bdiv_sqrt_norm, n, R, n, R, v[0], st.norm);
     EDX_LAUNCH_CHECK();
 
+    StepTail t{};
+    t.K = R;
+    t.st = st;
+    t.nshift = K;
+    t.sh = sh;
+    t.ctl = ctl;
+    t.sqn = sqn;
     int curr = 0, prev = 1, checked = 0, last = 0;
     for (int i = 1; i <= maxit; ++i) {
+        t.count = cntb.as<unsigned>();
+        t.op = TAIL_ALPHA;
+        t.i = i;
         if (precision == EDX_C64) ELAUNCH(k_il_to_c64, n, R, n, R, v[curr], x32.as<float2>());
         BEpi e{};   // y = (1/s_i) H u_i - (beta_i/s_{i-1}) u_{i-1}; partial <u_i|y>
         e.y = v[prev];
@@ -677,12 +582,10 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
         e.c1 = st.c1;
         e.dvec = v[curr];
         e.partials = part.as<double2>();
+        e.tail = t;
         int nb = 0;
         EDX_TRY(edx::bspmm(h, precision, R, v[curr], x32.as<float2>(), e, &nb));
-        hipLaunchKernelGGL(k_breduce, dim3(R), dim3(256), 0, s, part.as<double2>(), nb, R, st.sums);
-        hipLaunchKernelGGL(k_bk_alpha, dim3(kb), dim3(64), 0, s, st, R, i, st.sums);
-        hipLaunchKernelGGL(k_ms_scalars, dim3(R), dim3(256), 0, s, i, st.alpha, st.beta, R, sqn, sh,
-                           K, ctl, st.run);
+        EDX_TRY(step_finish_launch(t, part.as<double2>(), nb));
         const int j = (i - 1) % win;
         for (int r0 = 0; r0 < R; r0 += MS_PGROUP) {
             MsProjSet ps{};
@@ -716,11 +619,7 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
             }
         last = i;
         // u_{i+1} = y - (alpha_i/s_i) u_i, kept unnormalized (s_{i+1} = beta_{i+1})
-        ELAUNCH(k_baxpy_norm, n, R, n, R, v[prev], v[curr], st.acoef, part.as<double2>());
-        hipLaunchKernelGGL(k_breduce, dim3(R), dim3(256), 0, s, part.as<double2>(), nbe, R, st.sums);
-        hipLaunchKernelGGL(k_bk_beta, dim3(kb), dim3(64), 0, s, st, R, i, st.sums);
-        hipLaunchKernelGGL(k_msb_stop, dim3(kb), dim3(64), 0, s, i, R, st.run, ctl);
-        EDX_LAUNCH_CHECK();
+        EDX_TRY(baxpy_norm_step(n, R, v[prev], v[curr], st.acoef, part.as<double2>(), t, nbe));
         std::swap(curr, prev);
         if (i - checked >= 16 && i < maxit) {
             std::vector<int> rf(R);

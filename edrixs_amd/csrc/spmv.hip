@@ -76,6 +76,7 @@ struct SpmvEpi {
     const int *run;         // nullptr or flag: skip the launch when *run == 0
     int xmap;               // gridDim.x % 8 == 0: XCD-contiguous block order (set by the launcher)
     int lds_tab;            // indexed form: table entries staged in LDS (0: read from global)
+    StepTail tail;          // scalar work after the product (single-vector: K = 1)
 };
 
 // largest value table of the indexed form that the kernels stage in LDS
@@ -114,7 +115,7 @@ __device__ __forceinline__ double2 block_sum_256(double2 v) {
 // SPLIT: the split form (complex64 off-diagonal values in the CSR arrays, the
 // exact FP64 diagonal in diag, complex128 x, FP64 accumulation); the leader
 // adds diag[r] * x[r] to the off-diagonal sum.
-template <int G, class VP, class XT, class ACC, bool SPLIT>
+template <int G, class VP, class XT, class ACC, bool SPLIT, bool TAIL>
 __global__ __launch_bounds__(256) void k_spmv(int64_t m, const int64_t *__restrict__ rowptr,
                                               const int32_t *__restrict__ cols, VP vals,
                                               const XT *__restrict__ x,
@@ -170,7 +171,8 @@ __global__ __launch_bounds__(256) void k_spmv(int64_t m, const int64_t *__restri
     }
     if (e.dvec) {
         double2 s = block_sum_256(dot);
-        if (threadIdx.x == 0) e.partials[blockIdx.x] = s;
+        if (threadIdx.x == 0) part_put<TAIL>(e.partials + blockIdx.x, s);
+        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -642,6 +644,25 @@ bool xcd_map_enabled() {
     return on;
 }
 
+// After a launch of nb workgroups with dot partials: 0 left to sum if the launch
+// ran its tail, else at most FOLD_N.
+int finish_partials(const SpmvEpi &e, int nb, int *nblocks_out) {
+    if (nblocks_out) *nblocks_out = nb;
+    if (!e.dvec) return EDX_OK;
+    if (e.tail.count) {
+        if (nblocks_out) *nblocks_out = 0;
+    } else if (nb > FOLD_N) {
+        hipLaunchKernelGGL(k_fold_partials, dim3(FOLD_N), dim3(256), 0, stream(), e.partials, nb,
+                           e.run);
+        hipLaunchKernelGGL(k_move_folded, dim3(1), dim3(FOLD_N), 0, stream(), e.partials, nb, e.run);
+        EDX_LAUNCH_CHECK();
+        if (nblocks_out) *nblocks_out = FOLD_N;
+    }
+    return EDX_OK;
+}
+
+// With e_in.tail set, the launch ends with the step's scalar work where it is
+// narrow enough, and *nblocks_out is 0 then.
 int spmv_launch(const edx_csr *a, int precision, const void *x, const SpmvEpi &e_in, int lanes,
                 int *nblocks_out) {
     if (precision == EDX_C64D && !a->d_diag)
@@ -658,28 +679,22 @@ int spmv_launch(const edx_csr *a, int precision, const void *x, const SpmvEpi &e
     if (G == FAC_CODE) {
         if (!schedule_available(a, precision, G))
             return set_error(EDX_ERR_ARG, "SpMV schedule %d needs the slot-factored form", G);
-        int nb = 0;
+        int nb = fac_blocks(a);
+        SpmvEpi e = e_in;
+        e.tail.count = nullptr;
         hipEvent_t pe = prof_start(precision, EDX_KERNEL_SPMV_FAC,
-                                   fac_bytes(a, e_in.z != nullptr, e_in.dvec != nullptr), 0.0, 1,
-                                   csr_alg_bytes(a, 1, e_in.z != nullptr));
-        EDX_TRY(fac_launch(a, (const double2 *)x, e_in, &nb));
+                                   fac_bytes(a, e.z != nullptr, e.dvec != nullptr), 0.0, 1,
+                                   csr_alg_bytes(a, 1, e.z != nullptr));
+        EDX_TRY(fac_launch(a, (const double2 *)x, e, &nb));
         prof_stop(pe);
-        if (nblocks_out) *nblocks_out = nb;
-        if (e_in.dvec && nb > FOLD_N) {
-            hipLaunchKernelGGL(k_fold_partials, dim3(FOLD_N), dim3(256), 0, stream(), e_in.partials,
-                               nb, e_in.run);
-            hipLaunchKernelGGL(k_move_folded, dim3(1), dim3(FOLD_N), 0, stream(), e_in.partials, nb,
-                               e_in.run);
-            EDX_LAUNCH_CHECK();
-            if (nblocks_out) *nblocks_out = FOLD_N;
-        }
-        return EDX_OK;
+        return finish_partials(e, nb, nblocks_out);
     }
     const bool pipe = is_pipe_code(G);
     int nb = pipe ? pipe_blocks(G % 10) : spmv_blocks(a, G);
     if (nblocks_out) *nblocks_out = nb;
     if (a->m == 0) return EDX_OK;
     SpmvEpi e = e_in;
+    if (pipe || !tail_fits(nb, 1, 1)) e.tail.count = nullptr;
     e.xmap = nb % 8 == 0 && xcd_map_enabled();
     e.lds_tab = precision == EDX_C128I && pipe && a->nvtab <= LDS_TAB_MAX && lds_tab_enabled()
                     ? (int)a->nvtab
@@ -733,34 +748,32 @@ int spmv_launch(const edx_csr *a, int precision, const void *x, const SpmvEpi &e
 #undef EDX_PIPE_CASE
         EDX_LAUNCH_CHECK();
         prof_stop(pe);
-        if (e.dvec && nb > FOLD_N) {
-            hipLaunchKernelGGL(k_fold_partials, dim3(FOLD_N), dim3(256), 0, stream(), e.partials,
-                               nb, e.run);
-            hipLaunchKernelGGL(k_move_folded, dim3(1), dim3(FOLD_N), 0, stream(), e.partials, nb,
-                               e.run);
-            EDX_LAUNCH_CHECK();
-            if (nblocks_out) *nblocks_out = FOLD_N;
-        }
-        return EDX_OK;
+        return finish_partials(e, nb, nblocks_out);
     }
-#define EDX_SPMV_CASE(GG)                                                                     \
-    case GG:                                                                                  \
-        if (precision == EDX_C128)                                                            \
-            hipLaunchKernelGGL((k_spmv<GG, const double2 *, double2, double, false>), dim3(nb),   \
-                               dim3(256), 0, stream(), a->m, a->d_rowptr, a->d_cols,           \
-                               (const double2 *)a->d_vals, (const double2 *)x, nullptr, e);    \
-        else if (precision == EDX_C64D)                                                       \
-            hipLaunchKernelGGL((k_spmv<GG, const float2 *, double2, double, true>), dim3(nb),     \
-                               dim3(256), 0, stream(), a->m, a->d_off_rowptr, a->d_off_cols,   \
-                               (const float2 *)a->d_off_vals32, (const double2 *)x, a->d_diag, e); \
-        else if (precision == EDX_C128I)                                                      \
-            hipLaunchKernelGGL((k_spmv<GG, IdxPtr, double2, double, true>), dim3(nb), dim3(256),  \
-                               0, stream(), a->m, a->d_off_rowptr, a->d_off_cols,              \
-                               IdxPtr{a->d_off_idx, a->d_vtab}, (const double2 *)x, a->d_diag, e); \
-        else                                                                                  \
-            hipLaunchKernelGGL((k_spmv<GG, const float2 *, float2, float, false>), dim3(nb),      \
-                               dim3(256), 0, stream(), a->m, a->d_rowptr, a->d_cols,           \
-                               (const float2 *)a->d_vals32, (const float2 *)x, nullptr, e);    \
+#define EDX_SPMV_TYPES(GG, TL)                                                                    \
+    if (precision == EDX_C128)                                                                    \
+        hipLaunchKernelGGL((k_spmv<GG, const double2 *, double2, double, false, TL>), dim3(nb),    \
+                           dim3(256), 0, stream(), a->m, a->d_rowptr, a->d_cols,                   \
+                           (const double2 *)a->d_vals, (const double2 *)x, nullptr, e);            \
+    else if (precision == EDX_C64D)                                                               \
+        hipLaunchKernelGGL((k_spmv<GG, const float2 *, double2, double, true, TL>), dim3(nb),      \
+                           dim3(256), 0, stream(), a->m, a->d_off_rowptr, a->d_off_cols,           \
+                           (const float2 *)a->d_off_vals32, (const double2 *)x, a->d_diag, e);     \
+    else if (precision == EDX_C128I)                                                              \
+        hipLaunchKernelGGL((k_spmv<GG, IdxPtr, double2, double, true, TL>), dim3(nb), dim3(256),   \
+                           0, stream(), a->m, a->d_off_rowptr, a->d_off_cols,                      \
+                           IdxPtr{a->d_off_idx, a->d_vtab}, (const double2 *)x, a->d_diag, e);     \
+    else                                                                                          \
+        hipLaunchKernelGGL((k_spmv<GG, const float2 *, float2, float, false, TL>), dim3(nb),       \
+                           dim3(256), 0, stream(), a->m, a->d_rowptr, a->d_cols,                   \
+                           (const float2 *)a->d_vals32, (const float2 *)x, nullptr, e)
+#define EDX_SPMV_CASE(GG)                                                                         \
+    case GG:                                                                                      \
+        if (e.tail.count) {                                                                       \
+            EDX_SPMV_TYPES(GG, true);                                                             \
+        } else {                                                                                  \
+            EDX_SPMV_TYPES(GG, false);                                                            \
+        }                                                                                         \
         break;
     switch (G) {
         EDX_SPMV_CASE(4)
@@ -770,17 +783,11 @@ int spmv_launch(const edx_csr *a, int precision, const void *x, const SpmvEpi &e
         EDX_SPMV_CASE(64)
         default: return set_error(EDX_ERR_ARG, "unsupported lanes per row %d", G);
     }
+#undef EDX_SPMV_TYPES
 #undef EDX_SPMV_CASE
     EDX_LAUNCH_CHECK();
     prof_stop(pe);
-    if (e.dvec && nb > FOLD_N) {
-        hipLaunchKernelGGL(k_fold_partials, dim3(FOLD_N), dim3(256), 0, stream(), e.partials, nb,
-                           e.run);
-        hipLaunchKernelGGL(k_move_folded, dim3(1), dim3(FOLD_N), 0, stream(), e.partials, nb, e.run);
-        EDX_LAUNCH_CHECK();
-        if (nblocks_out) *nblocks_out = FOLD_N;
-    }
-    return EDX_OK;
+    return finish_partials(e, nb, nblocks_out);
 }
 
 int to_c64(int64_t n, const double2 *in, float2 *out, const int *run) {
