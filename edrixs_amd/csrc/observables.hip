@@ -63,7 +63,8 @@ constexpr int CF_MAX_EXP = 50;   // largest coefficient in 2^-50 .. 2^50
 __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ alpha,
                                            const double *__restrict__ beta, double norm, double e_gs,
                                            double weight, int nw, const double *__restrict__ omega,
-                                           const double *__restrict__ gamma, double *spec) {
+                                           const double *__restrict__ gamma, const double *spec,
+                                           double *out) {
     __shared__ double s_a[CF_STAGE], s_b2[CF_STAGE];
     const int w = blockIdx.x * 64 + threadIdx.x;
     const bool on = w < nw;
@@ -99,13 +100,13 @@ __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ 
     }
     if (!on) return;
     const double2 t = cdiv(q, d);
-    spec[w] += -1.0 / 3.14159265358979323846 * t.y * norm * weight;
+    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * t.y * norm * weight;
 }
 
 // The nested fraction, for coefficients of any size.
 __global__ void k_cf_nested(int neff, const double *alpha, const double *beta, double norm,
                             double e_gs, double weight, int nw, const double *omega,
-                            const double *gamma, double *spec) {
+                            const double *gamma, const double *spec, double *out) {
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= nw) return;
     const double2 z = make_double2(omega[w] + e_gs, gamma[w]);
@@ -115,7 +116,7 @@ __global__ void k_cf_nested(int neff, const double *alpha, const double *beta, d
         t = cdiv(make_double2(b2, 0.0), csub(make_double2(z.x - alpha[j], z.y), t));
     }
     t = cdiv(make_double2(1.0, 0.0), csub(make_double2(z.x - alpha[0], z.y), t));
-    spec[w] += -1.0 / 3.14159265358979323846 * t.y * norm * weight;
+    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * t.y * norm * weight;
 }
 
 // Whether the division-free recurrence stays in range: the largest of the
@@ -211,34 +212,47 @@ int edx_cf_spectrum(int neff, const double *alpha, const double *beta, double no
     EDX_CHECK(neff >= 1 && nw >= 0 && alpha && beta && (nw == 0 || (omega && gamma && spec)),
               EDX_ERR_ARG, "bad argument");
     if (nw == 0) return EDX_OK;
-    // one transfer each way: the inputs side by side in page-locked memory
-    // where they fit, else in ordinary memory
-    DevBuf buf;
-    const size_t count = 2 * (size_t)neff + 3 * (size_t)nw, bytes = sizeof(double) * count;
-    EDX_TRY(buf.alloc(bytes, "cf buffers"));
+    // The inputs lie side by side in page-locked memory where they fit, and the
+    // kernel writes its result there.  Where the workgroups together read at most
+    // CF_DIRECT bytes of coefficients it reads the inputs there too: one launch
+    // and one wait (a transfer each way costs another 10 us; 300 poles on 2000
+    // points read 150 KB, 3 us over the bus).  Larger inputs are copied first.
+    constexpr size_t CF_DIRECT = 256 << 10;
+    const int nb = (nw + 63) / 64;
+    const size_t count = 2 * (size_t)neff + 4 * (size_t)nw, bytes = sizeof(double) * count;
     std::vector<double> pageable;
     double *host = (double *)g_stage.get(bytes);
-    if (!host) {
+    const bool pinned = host != nullptr;
+    const bool direct = pinned && (size_t)nb * neff * 16 <= CF_DIRECT;
+    if (!pinned) {
         pageable.resize(count);
         host = pageable.data();
     }
+    const size_t o_om = 2 * (size_t)neff, o_sp = o_om + 2 * (size_t)nw, o_out = o_sp + nw;
     memcpy(host, alpha, neff * sizeof(double));
     memcpy(host + neff, beta, neff * sizeof(double));
-    memcpy(host + 2 * (size_t)neff, omega, nw * sizeof(double));
-    memcpy(host + 2 * (size_t)neff + nw, gamma, nw * sizeof(double));
-    memcpy(host + 2 * (size_t)neff + 2 * (size_t)nw, spec, nw * sizeof(double));
-    double *da = buf.as<double>(), *db = da + neff, *dom = db + neff, *dg = dom + nw, *ds = dg + nw;
+    memcpy(host + o_om, omega, nw * sizeof(double));
+    memcpy(host + o_om + nw, gamma, nw * sizeof(double));
+    memcpy(host + o_sp, spec, nw * sizeof(double));
+    DevBuf buf;
+    double *d = host;
     hipStream_t s = edx::stream();
-    EDX_HIP(hipMemcpyAsync(da, host, bytes, hipMemcpyHostToDevice, s));
+    if (!direct) {
+        EDX_TRY(buf.alloc(bytes, "cf buffers"));
+        d = buf.as<double>();
+        EDX_HIP(hipMemcpyAsync(d, host, o_out * sizeof(double), hipMemcpyHostToDevice, s));
+    }
+    double *out = pinned ? host + o_out : d + o_out;
     if (cf_in_range(neff, alpha, beta, e_gs, nw, omega, gamma))
-        hipLaunchKernelGGL(k_cf, dim3((nw + 63) / 64), dim3(64), 0, s, neff, da, db, norm, e_gs, weight,
-                           nw, dom, dg, ds);
+        hipLaunchKernelGGL(k_cf, dim3(nb), dim3(64), 0, s, neff, d, d + neff, norm, e_gs, weight, nw,
+                           d + o_om, d + o_om + nw, d + o_sp, out);
     else
-        hipLaunchKernelGGL(k_cf_nested, dim3((nw + 63) / 64), dim3(64), 0, s, neff, da, db, norm, e_gs,
-                           weight, nw, dom, dg, ds);
+        hipLaunchKernelGGL(k_cf_nested, dim3(nb), dim3(64), 0, s, neff, d, d + neff, norm, e_gs, weight,
+                           nw, d + o_om, d + o_om + nw, d + o_sp, out);
     EDX_LAUNCH_CHECK();
-    EDX_HIP(edx::copy_sync(host, ds, nw * sizeof(double), hipMemcpyDeviceToHost));
-    memcpy(spec, host, nw * sizeof(double));
+    if (pinned) EDX_HIP(hipStreamSynchronize(s));
+    else EDX_HIP(edx::copy_sync(host + o_out, out, nw * sizeof(double), hipMemcpyDeviceToHost));
+    memcpy(spec, host + o_out, nw * sizeof(double));
     return EDX_OK;
 }
 
