@@ -285,13 +285,143 @@ __global__ __launch_bounds__(VB) void k_gemv_ct(int64_t n, const double2 *V, int
     }
 }
 
-// h[c] = sum_b partials[c * nbx + b]
-__global__ void k_reduce_cols(const double2 *partials, int nbx, int k, double2 *h) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= k) return;
-    double2 s = make_double2(0, 0);
-    for (int b = 0; b < nbx; ++b) s = cadd(s, partials[(int64_t)c * nbx + b]);
-    h[c] = s;
+// h[c] = sum_b partials[c * nbx + b], a workgroup per column; with alpha, the last
+// column is v_j and *alpha = dot + its component
+__global__ __launch_bounds__(VB) void k_reduce_cols(const double2 *partials, int nbx, double2 *h,
+                                                    const double2 *dot, double *alpha) {
+    const double2 s = reduce_partials(partials + (int64_t)blockIdx.x * nbx, nbx);
+    if (threadIdx.x != 0) return;
+    h[blockIdx.x] = s;
+    if (alpha && blockIdx.x == gridDim.x - 1) *alpha = dot->x + s.x;
+}
+
+// ---- one step of fully reorthogonalized Lanczos
+//
+// w = H v_j - alpha v_j - beta v_{j-1}, made orthogonal to the k basis columns V
+// by two classical Gram-Schmidt passes, in three passes over V instead of four
+// (a pass reads 16 n k bytes and little else):
+//   k_cgs_tile<FIRST>  the three-term part and c = V^H w;
+//   k_cgs_tile         w -= V c and c' = V^H w, both from one copy of V in LDS;
+//   k_cgs_last         w -= V c' and |w|^2.
+// The scalars stay on the device, so the host waits once per cycle.  A step over
+// 705,432 rows and 3 to 22 columns (trlan, three states): 370 us with two
+// separate passes of two kernels, one-thread column sums (26 us each) and three
+// waits.  k_cgs_tile reads 22 columns in 35 us (7 TB/s: the basis stays in the
+// last-level cache), lane-per-row kernels with 8 or 12 sums each 52 and 64 us.
+
+constexpr int CGS_ROWS = 64;            // rows per tile
+constexpr int CGS_LD = CGS_ROWS + 1;    // lanes over columns then hit different banks
+constexpr int CGS_MAXK = 64;            // columns whose next tile fits in registers
+
+// FIRST: w = t - dot v - b vprev, v and vprev columns k-1 and k-2 (tri).  Else w -=
+// V h.  Then partials[c * gridDim.x + bx] of V^H w.  A workgroup walks tiles of 64
+// rows: its waves put the columns (lane = row) into LDS, adding up V h on the way,
+// then lanes are columns and the waves (and KP-lane groups, k <= KP) share the
+// rows.  The next tile's columns are loaded into registers before the current
+// tile is worked on.
+template <int KP, bool FIRST>
+__global__ __launch_bounds__(VB) void k_cgs_tile(int64_t n, const double2 *V, int64_t ld, int k,
+                                                 const double2 *h, const double2 *t, int tri,
+                                                 const double *bprev, double2 *w, double2 *partials) {
+    extern __shared__ double2 s_V[];            // [k][CGS_LD]
+    __shared__ double2 s_p[4][CGS_ROWS], s_w[CGS_ROWS], s_h[KP];
+    constexpr int G = 64 / KP;                  // row groups per wave
+    constexpr int NL = KP / 4;                  // columns a wave loads
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane % KP, sub = lane / KP;
+    const double a = FIRST ? h->x : 0.0, b = FIRST && tri ? *bprev : 0.0;   // FIRST: h is the dot
+    if (!FIRST)
+        for (int c = threadIdx.x; c < k; c += VB) s_h[c] = h[c];
+    __syncthreads();
+    double2 acc = make_double2(0, 0);
+    double2 v[NL], wr = make_double2(0, 0);
+    const double2 *win = FIRST ? t : w;
+    auto load = [&](int64_t r0) {
+        const int64_t r = r0 + lane;
+        const bool on = r < n;
+        wr = on ? win[r] : make_double2(0, 0);
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            v[i] = on && wave + 4 * i < k ? V[(int64_t)(wave + 4 * i) * ld + r] : make_double2(0, 0);
+    };
+    const int64_t stride = (int64_t)gridDim.x * CGS_ROWS;
+    int64_t r0 = (int64_t)blockIdx.x * CGS_ROWS;
+    load(r0);
+    for (; r0 < n; r0 += stride) {
+        double2 p = make_double2(0, 0);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int c = wave + 4 * i;
+            if (c < k) {
+                s_V[c * CGS_LD + lane] = v[i];
+                if (!FIRST) p = cadd(p, cmul(v[i], s_h[c]));
+            }
+        }
+        if (!FIRST) s_p[wave][lane] = p;
+        double2 x = wr;
+        load(r0 + stride);
+        __syncthreads();
+        if (wave == 0) {
+            if (FIRST) {
+                x = csub(x, cscale(s_V[(k - 1) * CGS_LD + lane], a));
+                if (tri) x = csub(x, cscale(s_V[(k - 2) * CGS_LD + lane], b));
+            } else {
+                x = csub(x, cadd(cadd(s_p[0][lane], s_p[1][lane]), cadd(s_p[2][lane], s_p[3][lane])));
+            }
+            s_w[lane] = x;
+            if (r0 + lane < n) w[r0 + lane] = x;
+        }
+        __syncthreads();
+        if (col < k)
+            for (int i = sub; i < CGS_ROWS / 4; i += G) {
+                const int row = wave * (CGS_ROWS / 4) + i;
+                acc = cadd(acc, cconjmul(s_V[col * CGS_LD + row], s_w[row]));
+            }
+        __syncthreads();
+    }
+    // the row groups' sums, in order (4 G <= 32 of a column's 65 places)
+    if (col < k) s_V[(wave * G + sub) * k + col] = acc;
+    __syncthreads();
+    for (int c = threadIdx.x; c < k; c += VB) {
+        double2 q = s_V[c];
+        for (int i = 1; i < 4 * G; ++i) q = cadd(q, s_V[i * k + c]);
+        partials[(int64_t)c * gridDim.x + blockIdx.x] = q;
+    }
+}
+
+template <int KP, bool FIRST>
+int cgs_tile_launch(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double2 *h,
+                    const double2 *t, int tri, const double *bprev, double2 *w, double2 *partials) {
+    const size_t lds = (size_t)k * CGS_LD * sizeof(double2);
+    if (lds > (56 << 10))
+        EDX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_cgs_tile<KP, FIRST>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_cgs_tile<KP, FIRST>), dim3(nb), dim3(VB), lds, edx::stream(), n, V, ld, k, h, t,
+                       tri, bprev, w, partials);
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
+}
+
+// k <= CGS_MAXK columns
+template <bool FIRST>
+int cgs_tile(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double2 *h, const double2 *t,
+             int tri, const double *bprev, double2 *w, double2 *partials) {
+    if (k <= 8) return cgs_tile_launch<8, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
+    if (k <= 16) return cgs_tile_launch<16, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
+    if (k <= 32) return cgs_tile_launch<32, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
+    return cgs_tile_launch<64, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
+}
+
+// w = t - dot vj - bprev vprev (more columns than a tile takes)
+__global__ __launch_bounds__(VB) void k_cgs_three(int64_t n, const double2 *t, const double2 *vj,
+                                                  const double2 *dot, const double2 *vprev,
+                                                  const double *bprev, double2 *w) {
+    const double a = dot->x, b = vprev ? *bprev : 0.0;
+    for (int64_t r = blockIdx.x * (int64_t)VB + threadIdx.x; r < n; r += (int64_t)gridDim.x * VB) {
+        double2 x = csub(t[r], cscale(vj[r], a));
+        if (vprev) x = csub(x, cscale(vprev[r], b));
+        w[r] = x;
+    }
 }
 
 // w[r] -= sum_c V[r, c] h[c]
@@ -307,16 +437,87 @@ __global__ __launch_bounds__(VB) void k_gemv_n_sub(int64_t n, const double2 *V, 
     }
 }
 
-// X[:, j] = sum_c V[:, c] S[c + j*k]  (S real, column-major k x nvec)
+// w -= V h and partials of |w|^2
+__global__ __launch_bounds__(VB) void k_cgs_last(int64_t n, const double2 *V, int64_t ld, int k,
+                                                 const double2 *h, double2 *w, double2 *partials) {
+    __shared__ double2 hs[1024];
+    for (int c = threadIdx.x; c < k && c < 1024; c += VB) hs[c] = h[c];
+    __syncthreads();
+    double2 nrm = make_double2(0, 0);
+    for (int64_t r = blockIdx.x * (int64_t)VB + threadIdx.x; r < n; r += (int64_t)gridDim.x * VB) {
+        double2 s = make_double2(0, 0);
+        for (int c = 0; c < k; ++c) s = cadd(s, cmul(V[(int64_t)c * ld + r], c < 1024 ? hs[c] : h[c]));
+        const double2 x = csub(w[r], s);
+        w[r] = x;
+        nrm.x += x.x * x.x + x.y * x.y;
+    }
+    nrm = block_sum_256(nrm);
+    if (threadIdx.x == 0) partials[blockIdx.x] = nrm;
+}
+
+__global__ __launch_bounds__(VB) void k_cgs_beta(const double2 *partials, int nb, double *beta) {
+    const double2 s = reduce_partials(partials, nb);
+    if (threadIdx.x == 0) *beta = sqrt(fabs(s.x));
+}
+
+// the next basis column w / beta; zero where the space is exhausted
+__global__ void k_cgs_next(int64_t n, const double2 *w, const double *beta, double2 *out) {
+    const double b = *beta;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+        out[i] = b < 1e-10 ? make_double2(0, 0) : make_double2(w[i].x / b, w[i].y / b);
+}
+
+// X[:, j] = sum_c V[:, c] S[c + j*k]  (S real, column-major k x nvec).  KC > 0: a
+// row of V (k <= KC columns) in registers, read once for all nvec vectors (12 from
+// 22 columns of 705,432 rows: 400 us reading it for each vector).
+template <int KC>
 __global__ __launch_bounds__(VB) void k_combine(int64_t n, const double2 *V, int64_t ld, int k,
                                                 const double *S, int nvec, double2 *X, int64_t ldx) {
     for (int64_t r = blockIdx.x * (int64_t)VB + threadIdx.x; r < n; r += (int64_t)gridDim.x * VB) {
-        for (int j = 0; j < nvec; ++j) {
-            double2 s = make_double2(0, 0);
-            for (int c = 0; c < k; ++c) s = cadd(s, cscale(V[(int64_t)c * ld + r], S[(int64_t)j * k + c]));
-            X[(int64_t)j * ldx + r] = s;
+        if constexpr (KC > 0) {
+            double2 v[KC];
+#pragma unroll
+            for (int c = 0; c < KC; ++c) v[c] = c < k ? V[(int64_t)c * ld + r] : make_double2(0, 0);
+            for (int j = 0; j < nvec; ++j) {
+                double2 s = make_double2(0, 0);
+#pragma unroll
+                for (int c = 0; c < KC; ++c)
+                    if (c < k) s = cadd(s, cscale(v[c], S[(int64_t)j * k + c]));
+                X[(int64_t)j * ldx + r] = s;
+            }
+        } else {
+            for (int j = 0; j < nvec; ++j) {
+                double2 s = make_double2(0, 0);
+                for (int c = 0; c < k; ++c)
+                    s = cadd(s, cscale(V[(int64_t)c * ld + r], S[(int64_t)j * k + c]));
+                X[(int64_t)j * ldx + r] = s;
+            }
         }
     }
+}
+
+int combine_launch(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double *S, int nvec,
+                   double2 *X, int64_t ldx) {
+    hipStream_t s = edx::stream();
+    if (k <= 16)
+        hipLaunchKernelGGL(k_combine<16>, dim3(nb), dim3(VB), 0, s, n, V, ld, k, S, nvec, X, ldx);
+    else if (k <= 24)
+        hipLaunchKernelGGL(k_combine<24>, dim3(nb), dim3(VB), 0, s, n, V, ld, k, S, nvec, X, ldx);
+    else if (k <= 32)
+        hipLaunchKernelGGL(k_combine<32>, dim3(nb), dim3(VB), 0, s, n, V, ld, k, S, nvec, X, ldx);
+    else
+        hipLaunchKernelGGL(k_combine<0>, dim3(nb), dim3(VB), 0, s, n, V, ld, k, S, nvec, X, ldx);
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
+}
+
+// x += *c y
+__global__ __launch_bounds__(VB) void k_axpy_coef(int64_t n, double2 *x, const double2 *y,
+                                                  const double *c) {
+    const double a = *c;
+    for (int64_t i = blockIdx.x * (int64_t)VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
+        x[i] = cadd(x[i], cscale(y[i], a));
 }
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {

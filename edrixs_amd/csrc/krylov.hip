@@ -101,6 +101,78 @@ __global__ void k_zero_words(int64_t nwords, uint64_t *p) {
         p[i] = 0;
 }
 
+// A recurrence of krylov_loop_in under way: v[0] holds its normalized start
+// vector when it begins.
+struct KrylovRun {
+    int64_t n;
+    KrylovScratch k;
+    int maxn, nbv;
+    double2 *v[2];
+    int curr = 0, prev = 1;
+    StepTail t{};
+    KrylovRun(int64_t n_, const KrylovScratch &k_, int maxn_)
+        : n(n_), k(k_), maxn(maxn_), nbv(step_vec_blocks(n_)), v{k_.v, k_.v + n_} {
+        t.K = 1;
+        t.st = krylov_state(k.S, k.ab, k.ab + maxn + 1, k.run);
+    }
+    // clears the second vector, the history, the run flags and the counters
+    // (fill kernels, no memset nodes), then norm = <v0|v0> and v_1 = v0 / sqrt(norm)
+    // (src/lanczos.f90:256-262) for the start vector v0 in v[0]
+    int begin() {
+        hipStream_t s = edx::stream();
+        const int64_t nz[3] = {2 * n, 2 * (int64_t)maxn + 2,
+                               (int64_t)(align256(((size_t)maxn + 2) * sizeof(int)) + TAIL_BYTES) / 8};
+        uint64_t *pz[3] = {(uint64_t *)v[1], (uint64_t *)k.ab, (uint64_t *)k.run};
+        for (int q = 0; q < 3; ++q)
+            hipLaunchKernelGGL(k_zero_words, dim3(vec_blocks(nz[q])), dim3(VB), 0, s, nz[q], pz[q]);
+        hipLaunchKernelGGL(k_krylov_init, dim3(1), dim3(1), 0, s, k.S, k.run);
+        hipLaunchKernelGGL(k_dot, dim3(nbv), dim3(VB), 0, s, n, v[0], v[0], k.part, nullptr);
+        hipLaunchKernelGGL(k_krylov_norm, dim3(1), dim3(VB), 0, s, k.part, nbv, k.S);
+        hipLaunchKernelGGL(k_div_real, dim3(nbv), dim3(VB), 0, s, n, v[0], &k.S->sqrt_norm, nullptr);
+        EDX_LAUNCH_CHECK();
+        curr = 0;
+        prev = 1;
+        return EDX_OK;
+    }
+    // step i (1-based): y = (1/s_i) H u_i - (beta_i/s_{i-1}) u_{i-1}, alpha_i from
+    // <u_i|y>; u_{i+1} = y - (alpha_i/s_i) u_i, beta_{i+1} from its norm
+    template <class Prod> int step(Prod &prod, int i) {
+        t.count = k.count;
+        t.op = TAIL_ALPHA;
+        t.i = i;
+        SpmvEpi e{};
+        e.y = v[prev];
+        e.z = v[prev];
+        e.c0 = &k.S->coef[0];
+        e.c1 = &k.S->coef[1];
+        e.dvec = v[curr];
+        e.partials = k.part;
+        e.run = k.run + (i - 1);
+        e.tail = t;
+        int nb = 0;
+        EDX_TRY(prod((const double2 *)v[curr], e, &nb, k.run + (i - 1)));
+        EDX_TRY(step_finish_launch(t, k.part, nb));
+        EDX_TRY(axpy_norm_step(n, v[prev], v[curr], &k.S->acoef, k.part, k.run + (i - 1), t, nbv));
+        std::swap(curr, prev);
+        return EDX_OK;
+    }
+    // waits, and reads alpha_1 .. alpha_count, beta_1 .. beta_count (those of the
+    // steps taken so far, neff of them before a breakdown) and <v0|v0>
+    int read(int count, double *alpha, double *beta, int *neff, double *norm) const {
+        // the state, alpha_1 .. alpha_maxn, (beta_0,) beta_1 .. beta_maxn lie together
+        std::vector<char> h(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double));
+        EDX_HIP(edx::copy_sync(h.data(), k.S, h.size(), hipMemcpyDeviceToHost));
+        KrylovDev hs;
+        memcpy(&hs, h.data(), sizeof(hs));
+        const char *hab = h.data() + KRYLOV_HEAD;
+        memcpy(alpha, hab, count * sizeof(double));
+        memcpy(beta, hab + ((size_t)maxn + 2) * sizeof(double), count * sizeof(double));
+        *neff = hs.neff;
+        *norm = hs.norm;
+        return EDX_OK;
+    }
+};
+
 // build_krylov_mp (src/lanczos.f90:210-303) over any product
 // prod(x, epilogue, &nblocks) that writes y = c0 A x + c1 z with dot partials
 // (nblocks of them left to sum, 0 if it ran the epilogue's tail);
@@ -108,70 +180,20 @@ __global__ void k_zero_words(int64_t nwords, uint64_t *p) {
 template <class Prod>
 int krylov_loop_in(int64_t n, Prod prod, const KrylovScratch &k, const double2 *v0, int maxn,
                    int *neff, double *alpha, double *beta, double *norm) {
-    int nbv = step_vec_blocks(n);
-    double2 *v[2] = {k.v, k.v + n};
-    double *d_alpha = k.ab, *d_beta = k.ab + maxn + 1;
-    int *run = k.run;
-    KrylovDev *S = k.S;
-    hipStream_t s = edx::stream();
-    // clear the second vector, the history, the run flags and the counters
-    // (fill kernels, no memset nodes)
-    const int64_t nz[3] = {2 * n, 2 * (int64_t)maxn + 2,
-                           (int64_t)(align256(((size_t)maxn + 2) * sizeof(int)) + TAIL_BYTES) / 8};
-    uint64_t *pz[3] = {(uint64_t *)v[1], (uint64_t *)k.ab, (uint64_t *)k.run};
-    for (int q = 0; q < 3; ++q)
-        hipLaunchKernelGGL(k_zero_words, dim3(vec_blocks(nz[q])), dim3(VB), 0, s, nz[q], pz[q]);
-    EDX_HIP(hipMemcpyAsync(v[0], v0, n * sizeof(double2), hipMemcpyDeviceToDevice, s));
-    double2 *part_p = k.part;
-    hipLaunchKernelGGL(k_krylov_init, dim3(1), dim3(1), 0, s, S, run);
-    // norm = <v0|v0>; v1 = v0 / sqrt(norm)   (src/lanczos.f90:256-262)
-    hipLaunchKernelGGL(k_dot, dim3(nbv), dim3(VB), 0, s, n, v[0], v[0], part_p, nullptr);
-    hipLaunchKernelGGL(k_krylov_norm, dim3(1), dim3(VB), 0, s, part_p, nbv, S);
-    hipLaunchKernelGGL(k_div_real, dim3(nbv), dim3(VB), 0, s, n, v[0], &S->sqrt_norm, nullptr);
-    EDX_LAUNCH_CHECK();
-    StepTail t{};
-    t.K = 1;
-    t.st = krylov_state(S, d_alpha, d_beta, run);
-    int curr = 0, prev = 1;
+    KrylovRun r(n, k, maxn);
+    EDX_HIP(hipMemcpyAsync(r.v[0], v0, n * sizeof(double2), hipMemcpyDeviceToDevice, edx::stream()));
+    EDX_TRY(r.begin());
     int checked = 0;
     for (int i = 1; i <= maxn; ++i) {
-        // y = (1/s_i) H u_i - (beta_i/s_{i-1}) u_{i-1}; alpha_i from <u_i|y>
-        t.count = k.count;
-        t.op = TAIL_ALPHA;
-        t.i = i;
-        SpmvEpi e{};
-        e.y = v[prev];
-        e.z = v[prev];
-        e.c0 = &S->coef[0];
-        e.c1 = &S->coef[1];
-        e.dvec = v[curr];
-        e.partials = part_p;
-        e.run = run + (i - 1);
-        e.tail = t;
-        int nb = 0;
-        EDX_TRY(prod((const double2 *)v[curr], e, &nb, run + (i - 1)));
-        EDX_TRY(step_finish_launch(t, part_p, nb));
-        // u_{i+1} = y - (alpha_i/s_i) u_i; beta_{i+1} from its norm
-        EDX_TRY(axpy_norm_step(n, v[prev], v[curr], &S->acoef, part_p, run + (i - 1), t, nbv));
-        std::swap(curr, prev);
+        EDX_TRY(r.step(prod, i));
         if (i - checked >= 32 && i < maxn) {   // stop launching once the recurrence broke down
-            int r = 1;
-            EDX_HIP(edx::copy_sync(&r, run + i, sizeof(int), hipMemcpyDeviceToHost));
+            int on = 1;
+            EDX_HIP(edx::copy_sync(&on, k.run + i, sizeof(int), hipMemcpyDeviceToHost));
             checked = i;
-            if (!r) break;
+            if (!on) break;
         }
     }
-    // the state and alpha_1 .. alpha_maxn, (beta_0,) beta_1 .. beta_maxn behind it
-    std::vector<char> h(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double));
-    EDX_HIP(edx::copy_sync(h.data(), S, h.size(), hipMemcpyDeviceToHost));
-    KrylovDev hs;
-    memcpy(&hs, h.data(), sizeof(hs));
-    const char *hab = h.data() + KRYLOV_HEAD;
-    memcpy(alpha, hab, maxn * sizeof(double));
-    memcpy(beta, hab + ((size_t)maxn + 2) * sizeof(double), maxn * sizeof(double));
-    *neff = hs.neff;
-    *norm = hs.norm;
-    return EDX_OK;
+    return r.read(maxn, alpha, beta, neff, norm);
 }
 
 // krylov_loop_in with its device memory allocated for the run.
@@ -268,6 +290,7 @@ int minres_run(const edx_csr *a, int precision, const double2 *b, double2 *x, do
 // ------------------------------------------------------------- Lanczos
 
 constexpr int GEMV_NBX = 256;   // row workgroups per column group of the projections
+constexpr int CGS_NBX = 512;    // workgroups of k_cgs_tile
 
 struct Lanczos {
     const edx_csr *h;
@@ -281,6 +304,35 @@ struct Lanczos {
     double2 *part;
     double2 *hvec;
     int nbv;
+    // of the reorthogonalized steps (lanczos_step)
+    double2 *t = nullptr;       // H v
+    double2 *spart = nullptr;   // the product's dot partials
+    double2 *dot = nullptr;
+    double *al = nullptr;       // alpha_j, beta_j of the run's steps, cap_cols each
+    double *be = nullptr;
+};
+
+// Device memory of reorthogonalized steps over cap_cols basis columns.
+struct LanczosBufs {
+    DevBuf w, t, part, hv, spart, sc;
+    int alloc(const edx_csr *h, int64_t n, int cap_cols, int nbv) {
+        EDX_TRY(w.alloc(n * sizeof(double2), "lanczos w"));
+        EDX_TRY(t.alloc(n * sizeof(double2), "lanczos H v"));
+        EDX_TRY(part.alloc(((size_t)cap_cols * CGS_NBX + nbv + 64) * sizeof(double2), "partials"));
+        EDX_TRY(hv.alloc((size_t)cap_cols * sizeof(double2), "coefficients"));
+        EDX_TRY(spart.alloc((size_t)edx::spmv_partials_len(h) * sizeof(double2), "product partials"));
+        return sc.alloc(sizeof(double2) + (size_t)cap_cols * 2 * sizeof(double), "lanczos scalars");
+    }
+    void set(Lanczos &L) const {
+        L.w = w.as<double2>();
+        L.t = t.as<double2>();
+        L.part = part.as<double2>();
+        L.hvec = hv.as<double2>();
+        L.spart = spart.as<double2>();
+        L.dot = sc.as<double2>();
+        L.al = (double *)(L.dot + 1);
+        L.be = L.al + L.cap_cols;
+    }
 };
 
 int host_dot(Lanczos &L, const double2 *a, const double2 *b, double2 *out) {
@@ -300,8 +352,8 @@ int orthogonalize(Lanczos &L, int k, double2 *w, std::vector<double2> *hk) {
     const int nbx = std::min(L.nbv, GEMV_NBX);
     dim3 grid(nbx, (k + 7) / 8);
     hipLaunchKernelGGL(k_gemv_ct, grid, dim3(VB), 0, edx::stream(), L.n, L.basis, L.ld, k, w, L.part);
-    hipLaunchKernelGGL(k_reduce_cols, dim3((k + 255) / 256), dim3(256), 0, edx::stream(), L.part,
-                       nbx, k, L.hvec);
+    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, edx::stream(), L.part, nbx, L.hvec,
+                       nullptr, nullptr);
     hipLaunchKernelGGL(k_gemv_n_sub, dim3(L.nbv), dim3(VB), 0, edx::stream(), L.n, L.basis, L.ld, k,
                        L.hvec, w);
     EDX_LAUNCH_CHECK();
@@ -312,32 +364,56 @@ int orthogonalize(Lanczos &L, int k, double2 *w, std::vector<double2> *hk) {
     return EDX_OK;
 }
 
-// One Lanczos run started from basis column `first` (already normalised and
-// orthogonal to the locked columns [0, first)).  Returns Ritz pairs of the run.
-// One Lanczos step from basis column first+j: w = H v_j - alpha v_j - beta v_{j-1},
-// two classical Gram-Schmidt passes against columns [0, first+j], alpha
-// corrected by the v_j component; appends alpha_j and beta_{j+1} = |w|.
-int lanczos_one(Lanczos &L, int first, int j, std::vector<double> &al, std::vector<double> &be) {
+// One Lanczos step from basis column first+j: L.w = H v_j - alpha v_j - beta
+// v_{j-1} (the last with tri; beta_{j-1} is L.be[j-1]), two classical Gram-Schmidt
+// passes against columns [0, first+j], alpha corrected by the v_j component;
+// leaves alpha_j and beta_{j+1} = |w| in L.al[j], L.be[j], with no wait.
+int lanczos_step(Lanczos &L, int first, int j, bool tri) {
     hipStream_t s = edx::stream();
-    double2 *vj = L.basis + (int64_t)(first + j) * L.ld;
+    const int64_t n = L.n;
+    const int k = first + j + 1, nbx = std::min(L.nbv, GEMV_NBX);
+    const double2 *vj = L.basis + (int64_t)(first + j) * L.ld;
     SpmvEpi e{};
-    e.y = L.w;
-    EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, nullptr, nullptr));
-    double2 a;
-    EDX_TRY(host_dot(L, vj, L.w, &a));
-    double alpha = a.x;
-    const double2 *vprev = j > 0 ? L.basis + (int64_t)(first + j - 1) * L.ld : nullptr;
-    hipLaunchKernelGGL(k_axpby_sub, dim3(L.nbv), dim3(VB), 0, s, L.n, L.w, vj, alpha, vprev,
-                       j > 0 ? be[j - 1] : 0.0);
+    e.y = L.t;
+    e.dvec = vj;
+    e.partials = L.spart;
+    int nb = 0;
+    EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, &nb, nullptr));
+    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(VB), 0, s, L.spart, nb, L.dot, nullptr);
+    const double2 *vprev = tri ? vj - L.ld : nullptr;
+    const double *bprev = tri ? L.be + j - 1 : nullptr;
+    const bool tile = k <= CGS_MAXK;
+    int nbc = tile ? (int)std::min<int64_t>((n + CGS_ROWS - 1) / CGS_ROWS, CGS_NBX) : nbx;
+    if (tile) {
+        EDX_TRY(cgs_tile<true>(nbc, n, L.basis, L.ld, k, L.dot, L.t, tri, bprev, L.w, L.part));
+    } else {   // the two passes as four kernels
+        hipLaunchKernelGGL(k_cgs_three, dim3(L.nbv), dim3(VB), 0, s, n, L.t, vj, L.dot, vprev, bprev, L.w);
+        hipLaunchKernelGGL(k_gemv_ct, dim3(nbx, (k + 7) / 8), dim3(VB), 0, s, n, L.basis, L.ld, k, L.w,
+                           L.part);
+    }
+    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbc, L.hvec, L.dot, L.al + j);
+    if (tile) {
+        EDX_TRY(cgs_tile<false>(nbc, n, L.basis, L.ld, k, L.hvec, nullptr, 0, nullptr, L.w, L.part));
+    } else {
+        hipLaunchKernelGGL(k_gemv_n_sub, dim3(L.nbv), dim3(VB), 0, s, n, L.basis, L.ld, k, L.hvec, L.w);
+        hipLaunchKernelGGL(k_gemv_ct, dim3(nbx, (k + 7) / 8), dim3(VB), 0, s, n, L.basis, L.ld, k, L.w,
+                           L.part);
+    }
+    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbc, L.hvec, nullptr, nullptr);
+    hipLaunchKernelGGL(k_cgs_last, dim3(L.nbv), dim3(VB), 0, s, n, L.basis, L.ld, k, L.hvec, L.w, L.part);
+    hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(VB), 0, s, L.part, L.nbv, L.be + j);
     EDX_LAUNCH_CHECK();
-    std::vector<double2> h1;
-    EDX_TRY(orthogonalize(L, first + j + 1, L.w, &h1));
-    EDX_TRY(orthogonalize(L, first + j + 1, L.w, nullptr));
-    alpha += h1[first + j].x;
-    double2 nb2;
-    EDX_TRY(host_dot(L, L.w, L.w, &nb2));
-    al.push_back(alpha);
-    be.push_back(sqrt(fabs(nb2.x)));
+    return EDX_OK;
+}
+
+// The same with alpha_j and beta_{j+1} appended to the host's lists.
+int lanczos_one(Lanczos &L, int first, int j, std::vector<double> &al, std::vector<double> &be) {
+    EDX_TRY(lanczos_step(L, first, j, j > 0));
+    double ab[2];
+    EDX_HIP(hipMemcpyAsync(ab, L.al + j, sizeof(double), hipMemcpyDeviceToHost, edx::stream()));
+    EDX_HIP(edx::copy_sync(ab + 1, L.be + j, sizeof(double), hipMemcpyDeviceToHost));
+    al.push_back(ab[0]);
+    be.push_back(ab[1]);
     return EDX_OK;
 }
 
@@ -360,6 +436,8 @@ int lanczos_steps(Lanczos &L, int first, int maxn, std::vector<double> &al,
     return EDX_OK;
 }
 
+// One Lanczos run started from basis column `first` (already normalised and
+// orthogonal to the locked columns [0, first)).  Returns Ritz pairs of the run.
 int lanczos_run(Lanczos &L, int first, int nev, int maxiter, double tol, std::vector<double> &ritz,
                 std::vector<double> &S, int &m_out, int &iters) {
     std::vector<double> al, be;   // be[j] couples v_j and v_{j+1}
@@ -420,39 +498,27 @@ int trl_run(Lanczos &L, int first, int nev, int m, int max_cycles, double tol,
         int me = m;   // columns of this cycle (fewer on an invariant subspace)
         double beta = 0.0;
         for (int j = k; j < m; ++j) {
-            double2 *vj = L.basis + (int64_t)(first + j) * L.ld;
-            SpmvEpi e{};
-            e.y = L.w;
-            EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, nullptr, nullptr));
-            double2 a;
-            EDX_TRY(host_dot(L, vj, L.w, &a));
-            double alpha = a.x;
             // three-term part inside a tridiagonal stretch; after a restart the
             // arrow couplings go with the Gram-Schmidt passes
-            const bool tri = j > k;
-            const double2 *vprev = tri ? L.basis + (int64_t)(first + j - 1) * L.ld : nullptr;
-            hipLaunchKernelGGL(k_axpby_sub, dim3(L.nbv), dim3(VB), 0, s, n, L.w, vj, alpha, vprev,
-                               tri ? T[(size_t)(j - 1) * m + j] : 0.0);
-            EDX_LAUNCH_CHECK();
-            std::vector<double2> h1;
-            EDX_TRY(orthogonalize(L, first + j + 1, L.w, &h1));
-            EDX_TRY(orthogonalize(L, first + j + 1, L.w, nullptr));
-            alpha += h1[first + j].x;
-            double2 nb2;
-            EDX_TRY(host_dot(L, L.w, L.w, &nb2));
-            beta = sqrt(fabs(nb2.x));
-            ++iters;
-            T[(size_t)j * m + j] = alpha;
-            if (beta < 1e-10) {
-                me = j + 1;
-                break;
-            }
+            EDX_TRY(lanczos_step(L, first, j, j > k));
             if (j + 1 < m) {
-                T[(size_t)j * m + j + 1] = T[(size_t)(j + 1) * m + j] = beta;
-                hipLaunchKernelGGL(k_copy_div, dim3(L.nbv), dim3(VB), 0, s, n, L.w, beta,
+                hipLaunchKernelGGL(k_cgs_next, dim3(L.nbv), dim3(VB), 0, s, n, L.w, L.be + j,
                                    L.basis + (int64_t)(first + j + 1) * L.ld);
                 EDX_LAUNCH_CHECK();
             }
+        }
+        std::vector<double> al(m - k), be(m - k);
+        EDX_HIP(hipMemcpyAsync(al.data(), L.al + k, (m - k) * sizeof(double), hipMemcpyDeviceToHost, s));
+        EDX_HIP(edx::copy_sync(be.data(), L.be + k, (m - k) * sizeof(double), hipMemcpyDeviceToHost));
+        for (int j = k; j < m; ++j) {
+            ++iters;
+            beta = be[j - k];
+            T[(size_t)j * m + j] = al[j - k];
+            if (beta < 1e-10) {   // an invariant subspace: the steps after it do not count
+                me = j + 1;
+                break;
+            }
+            if (j + 1 < m) T[(size_t)j * m + j + 1] = T[(size_t)(j + 1) * m + j] = beta;
         }
         // Ritz pairs of the me x me projected matrix
         std::vector<cd> A((size_t)me * me), Z((size_t)me * me);
@@ -476,14 +542,12 @@ int trl_run(Lanczos &L, int first, int nev, int m, int max_cycles, double tol,
         EDX_HIP(edx::copy_sync(dS, S.data(), S.size() * sizeof(double), hipMemcpyHostToDevice));
         const double2 *V = L.basis + (int64_t)first * L.ld;
         if (done) {
-            hipLaunchKernelGGL(k_combine, dim3(L.nbv), dim3(VB), 0, s, n, V, L.ld, me, dS, keep, X, n);
-            EDX_LAUNCH_CHECK();
+            EDX_TRY(combine_launch(L.nbv, n, V, L.ld, me, dS, keep, X, n));
             EDX_HIP(hipStreamSynchronize(s));
             take = keep;
             return EDX_OK;
         }
-        hipLaunchKernelGGL(k_combine, dim3(L.nbv), dim3(VB), 0, s, n, V, L.ld, me, dS, keep, tmp, n);
-        EDX_LAUNCH_CHECK();
+        EDX_TRY(combine_launch(L.nbv, n, V, L.ld, me, dS, keep, tmp, n));
         EDX_HIP(hipMemcpyAsync(L.basis + (int64_t)first * L.ld, tmp, (size_t)n * keep * sizeof(double2),
                                hipMemcpyDeviceToDevice, s));
         hipLaunchKernelGGL(k_copy_div, dim3(L.nbv), dim3(VB), 0, s, n, L.w, beta,
@@ -557,18 +621,18 @@ int lanczos_impl(const edx_csr *h, int precision, int nev, int maxiter, double t
     if (!ncv && maxiter > n) maxiter = (int)n;
     const int max_rounds = deflate ? 2 * nev + 2 : 1;
     const int cap_cols = nev + (ncv ? m_trl : maxiter) + 2;
-    DevBuf basis, x32, w, part, hv, tmpS, evec_all, trl_tmp;
+    DevBuf basis, x32, tmpS, evec_all, trl_tmp;
+    LanczosBufs lb;
     EDX_TRY(basis.alloc((size_t)n * cap_cols * sizeof(double2), "lanczos basis"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(n * sizeof(float2), "lanczos x32"));
-    EDX_TRY(w.alloc(n * sizeof(double2), "lanczos w"));
     const int nbv = vec_blocks(n);
-    EDX_TRY(part.alloc(((size_t)cap_cols * GEMV_NBX + nbv + 64) * sizeof(double2), "partials"));
-    EDX_TRY(hv.alloc((size_t)cap_cols * sizeof(double2), "coefficients"));
+    EDX_TRY(lb.alloc(h, n, cap_cols, nbv));
     EDX_TRY(tmpS.alloc((size_t)cap_cols * cap_cols * sizeof(double), "ritz vectors"));
     EDX_TRY(evec_all.alloc((size_t)n * nev * sizeof(double2), "eigenvectors"));
     if (ncv) EDX_TRY(trl_tmp.alloc((size_t)n * m_trl * sizeof(double2), "thick-restart vectors"));
-    Lanczos L{h, precision, n, basis.as<double2>(), n, cap_cols, x32.as<float2>(), w.as<double2>(),
-              part.as<double2>(), hv.as<double2>(), nbv};
+    Lanczos L{h, precision, n, basis.as<double2>(), n, cap_cols, x32.as<float2>(), nullptr, nullptr,
+              nullptr, nbv};
+    lb.set(L);
     hipStream_t s = edx::stream();
     std::vector<double> locked_vals;   // eigenvalues of locked columns [0, nlock)
     int nlock = 0, iters = 0, nconv = 0;
@@ -602,9 +666,8 @@ int lanczos_impl(const edx_csr *h, int precision, int nev, int maxiter, double t
             for (int j = 0; j < take; ++j)
                 for (int c = 0; c < m; ++c) Sk[(size_t)j * m + c] = S[(size_t)j * m + c];
             EDX_HIP(edx::copy_sync(tmpS.p, Sk.data(), Sk.size() * sizeof(double), hipMemcpyHostToDevice));
-            hipLaunchKernelGGL(k_combine, dim3(nbv), dim3(VB), 0, s, n, L.basis + (int64_t)nlock * n,
-                               n, m, tmpS.as<double>(), take, evec_all.as<double2>(), n);
-            EDX_LAUNCH_CHECK();
+            EDX_TRY(combine_launch(nbv, n, L.basis + (int64_t)nlock * n, n, m, tmpS.as<double>(), take,
+                                   evec_all.as<double2>(), n));
         }
         // merge: locked (already lowest of previous rounds) with this run's Ritz values
         std::vector<std::pair<double, int>> cand;   // (value, source: <0 locked k, >=0 new j)
@@ -653,8 +716,9 @@ int lanczos_impl(const edx_csr *h, int precision, int nev, int maxiter, double t
 // every 10 steps (and at the last) tests the nev lowest Ritz pairs of the
 // tridiagonal matrix by their residual estimates |beta_m y_{m,k}| < tol;
 // pass 2 runs the same recurrence again from the same start and accumulates
-// x_k = sum_j y_{j,k} v_j.  Three vectors of n plus nvec outputs; one copy of
-// each level (the Krylov space of one vector holds one).
+// x_k = sum_j y_{j,k} v_j.  Two vectors of n plus nvec outputs; one copy of
+// each level (the Krylov space of one vector holds one).  The scalars stay on the
+// device between the tests.
 int lanczos_rerun_impl(const edx_csr *h, int precision, int nev, int maxiter, double tol,
                        uint64_t seed, int nvec, double *evals, void *d_evecs, int *niter_out) {
     EDX_TRY(check_square(h, precision));
@@ -666,71 +730,42 @@ int lanczos_rerun_impl(const edx_csr *h, int precision, int nev, int maxiter, do
     if (nvec > nev) nvec = nev;
     if (maxiter > n) maxiter = (int)n;
     const int nbv = vec_blocks(n);
-    DevBuf vb, x32, part;
-    EDX_TRY(vb.alloc((size_t)n * 3 * sizeof(double2), "lanczos vectors"));
+    const int64_t plen = edx::spmv_partials_len(h);
+    DevBuf buf, x32, coef;
+    EDX_TRY(buf.alloc(krylov_scratch_bytes(n, plen, maxiter), "lanczos scratch"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(n * sizeof(float2), "lanczos x32"));
-    EDX_TRY(part.alloc(((size_t)nbv + 64) * sizeof(double2), "partials"));
-    Lanczos L{h, precision, n, nullptr, n, 0, x32.as<float2>(), nullptr, part.as<double2>(), nullptr,
-              nbv};
+    KrylovRun r(n, krylov_scratch_carve(buf.as<char>(), n, plen, maxiter), maxiter);
     hipStream_t s = edx::stream();
-    double2 *buf[3] = {vb.as<double2>(), vb.as<double2>() + n, vb.as<double2>() + 2 * n};
     double2 *X = (double2 *)d_evecs;
+    auto prod = [&](const double2 *x, const SpmvEpi &e, int *nb, const int *run) {
+        return apply(h, precision, x, x32.as<float2>(), e, nb, run);
+    };
     // v_1: the seeded start vector, normalised
-    auto start = [&](double2 *v) -> int {
-        hipLaunchKernelGGL(k_random_real, dim3(nbv), dim3(VB), 0, s, n, seed, v);
+    auto start = [&]() -> int {
+        hipLaunchKernelGGL(k_random_real, dim3(nbv), dim3(VB), 0, s, n, seed, r.v[0]);
         EDX_LAUNCH_CHECK();
-        double2 nn;
-        EDX_TRY(host_dot(L, v, v, &nn));
-        EDX_CHECK(nn.x > 0, EDX_ERR_NUMERIC, "zero start vector");
-        hipLaunchKernelGGL(k_scale_real, dim3(nbv), dim3(VB), 0, s, n, v, 1.0 / sqrt(nn.x));
-        EDX_LAUNCH_CHECK();
-        return EDX_OK;
+        return r.begin();
     };
-    // w = H v_j - alpha_j v_j - beta_{j-1} v_{j-1}; alpha from the device when
-    // known < 0, else given
-    auto step = [&](double2 *vprev, double2 *vj, double2 *w, double bprev, double &alpha,
-                    bool measure) -> int {
-        SpmvEpi e{};
-        e.y = w;
-        EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, nullptr, nullptr));
-        if (measure) {
-            double2 a;
-            EDX_TRY(host_dot(L, vj, w, &a));
-            alpha = a.x;
-        }
-        hipLaunchKernelGGL(k_axpby_sub, dim3(nbv), dim3(VB), 0, s, n, w, vj, alpha, vprev, bprev);
-        EDX_LAUNCH_CHECK();
-        return EDX_OK;
-    };
-    std::vector<double> al, be, ritz;
+    std::vector<double> al(maxiter), be(maxiter), ritz;
     int m = 0;
-    {   // pass 1
-        EDX_TRY(start(buf[1]));
-        double2 *v[3] = {buf[0], buf[1], buf[2]};   // v[0] = v_{j-1}, v[1] = v_j, v[2] = w
-        for (int j = 0; j < maxiter; ++j) {
-            double alpha = 0.0;
-            EDX_TRY(step(j > 0 ? v[0] : nullptr, v[1], v[2], j > 0 ? be[j - 1] : 0.0, alpha, true));
-            double2 nb2;
-            EDX_TRY(host_dot(L, v[2], v[2], &nb2));
-            const double beta = sqrt(fabs(nb2.x));
-            al.push_back(alpha);
-            be.push_back(beta);
-            m = j + 1;
-            const bool last = beta < 1e-10 || m == maxiter;
-            if (last || (m >= nev && m % 10 == 0)) {
-                std::vector<double> wv(m), zl(m);
-                EDX_CHECK(edx::tridiag_ql(m, al.data(), be.data(), wv.data(), nullptr, zl.data()) == 0,
-                          EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
-                int nconv = 0;
-                for (int k = 0; k < std::min(nev, m); ++k)
-                    if (fabs(beta * zl[k]) < tol) ++nconv;
-                if (nconv >= std::min(nev, m) || last) break;
-            }
-            // v_{j+1} = w / beta over v_{j-1}, which the next step no longer needs
-            hipLaunchKernelGGL(k_copy_div, dim3(nbv), dim3(VB), 0, s, n, v[2], beta, v[0]);
-            EDX_LAUNCH_CHECK();
-            std::swap(v[0], v[1]);
-        }
+    EDX_TRY(start());
+    for (int done = 0;;) {   // pass 1, from one test to the next
+        int next = (done / 10 + 1) * 10;
+        while (next < nev) next += 10;
+        next = std::min(next, maxiter);
+        for (int i = done + 1; i <= next; ++i) EDX_TRY(r.step(prod, i));
+        double norm = 0.0;
+        EDX_TRY(r.read(next, al.data(), be.data(), &m, &norm));
+        EDX_CHECK(norm > 0, EDX_ERR_NUMERIC, "zero start vector");
+        done = next;
+        const double beta = be[m - 1];
+        std::vector<double> wv(m), zl(m);
+        EDX_CHECK(edx::tridiag_ql(m, al.data(), be.data(), wv.data(), nullptr, zl.data()) == 0,
+                  EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
+        int nconv = 0;
+        for (int k = 0; k < std::min(nev, m); ++k)
+            if (fabs(beta * zl[k]) < tol) ++nconv;
+        if (nconv >= std::min(nev, m) || m < next || beta < 1e-10 || m == maxiter) break;
     }
     ritz.assign(m, 0.0);
     std::vector<double> S((size_t)m * m);   // row k: eigenvector k of the tridiagonal matrix
@@ -738,22 +773,27 @@ int lanczos_rerun_impl(const edx_csr *h, int precision, int nev, int maxiter, do
               EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
     for (int k = 0; k < nev; ++k) evals[k] = k < m ? ritz[k] : 0.0;
     if (nvec > 0) {   // pass 2
+        const int nk = std::min(nvec, m);
+        std::vector<double> c((size_t)nk * m);   // x_k += y_{j,k} v_j, v_j = u_j / beta_{j-1}
+        for (int k = 0; k < nk; ++k)
+            for (int j = 0; j < m; ++j)
+                c[(size_t)k * m + j] = S[(size_t)k * m + j] / (j ? be[j - 1] : 1.0);
+        EDX_TRY(coef.alloc(c.size() * sizeof(double), "ritz coefficients"));
+        EDX_HIP(edx::copy_sync(coef.p, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice));
         EDX_HIP(hipMemsetAsync(X, 0, (size_t)n * nvec * sizeof(double2), s));
-        EDX_TRY(start(buf[1]));
-        double2 *v[3] = {buf[0], buf[1], buf[2]};   // v[0] = v_{j-1}, v[1] = v_j, v[2] = w
+        EDX_TRY(start());
         for (int j = 0; j < m; ++j) {
-            for (int k = 0; k < nvec && k < m; ++k)   // x_k += y_{j,k} v_j
-                hipLaunchKernelGGL(k_axpby_sub, dim3(nbv), dim3(VB), 0, s, n, X + (int64_t)k * n, v[1],
-                                   -S[(size_t)k * m + j], nullptr, 0.0);
+            for (int k = 0; k < nk; ++k)
+                hipLaunchKernelGGL(k_axpy_coef, dim3(nbv), dim3(VB), 0, s, n, X + (int64_t)k * n,
+                                   r.v[r.curr], coef.as<double>() + (size_t)k * m + j);
             EDX_LAUNCH_CHECK();
-            if (j + 1 == m) break;
-            double alpha = al[j];
-            EDX_TRY(step(j > 0 ? v[0] : nullptr, v[1], v[2], j > 0 ? be[j - 1] : 0.0, alpha, false));
-            hipLaunchKernelGGL(k_copy_div, dim3(nbv), dim3(VB), 0, s, n, v[2], be[j], v[0]);
-            EDX_LAUNCH_CHECK();
-            std::swap(v[0], v[1]);   // v_j becomes v_{j-1}, the new vector v_{j+1} sits in v[1]
+            if (j + 1 < m) EDX_TRY(r.step(prod, j + 1));
         }
-        for (int k = 0; k < nvec && k < m; ++k) {   // unit norm
+        Lanczos L{};
+        L.n = n;
+        L.nbv = nbv;
+        L.part = r.k.part;
+        for (int k = 0; k < nk; ++k) {   // unit norm
             double2 nn;
             EDX_TRY(host_dot(L, X + (int64_t)k * n, X + (int64_t)k * n, &nn));
             if (nn.x > 0)
@@ -798,15 +838,15 @@ int edx_build_krylov_reorth(const edx_csr *h, int precision, const void *d_v0, i
     const int64_t n = h->n;
     if (maxn > n) maxn = (int)n;
     const int cap_cols = maxn + 2;
-    DevBuf basis, x32, w, part, hv;
+    DevBuf basis, x32;
+    LanczosBufs lb;
     EDX_TRY(basis.alloc((size_t)n * cap_cols * sizeof(double2), "krylov basis"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(n * sizeof(float2), "krylov x32"));
-    EDX_TRY(w.alloc(n * sizeof(double2), "krylov w"));
     const int nbv = vec_blocks(n);
-    EDX_TRY(part.alloc(((size_t)cap_cols * GEMV_NBX + nbv + 64) * sizeof(double2), "partials"));
-    EDX_TRY(hv.alloc((size_t)cap_cols * sizeof(double2), "coefficients"));
-    Lanczos L{h, precision, n, basis.as<double2>(), n, cap_cols, x32.as<float2>(), w.as<double2>(),
-              part.as<double2>(), hv.as<double2>(), nbv};
+    EDX_TRY(lb.alloc(h, n, cap_cols, nbv));
+    Lanczos L{h, precision, n, basis.as<double2>(), n, cap_cols, x32.as<float2>(), nullptr, nullptr,
+              nullptr, nbv};
+    lb.set(L);
     hipStream_t s = edx::stream();
     EDX_HIP(hipMemcpyAsync(L.basis, d_v0, n * sizeof(double2), hipMemcpyDeviceToDevice, s));
     double2 nn;
