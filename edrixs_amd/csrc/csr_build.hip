@@ -426,7 +426,7 @@ int build_by_plan(const BuildParams &p, const PlanSpaces &sp, const TermTable &t
                   bool *done) {
     PlanStore<W> plan;
     EDX_TRY(plan_make<W>(sp, tt.ops.data(), tt.vals.data(), tt.nhop, tt.T, p.omega_on != 0,
-                         p.omega, p.negate != 0, false, plan));
+                         p.omega, p.negate != 0, PLAN_WAVES, false, plan));
     EDX_HIP(hipMemsetAsync(o.rowptr + p.M, 0, sizeof(int64_t), edx::stream()));
     EDX_HIP(hipMemsetAsync(o.flag, 0, sizeof(int), edx::stream()));
     EDX_TRY((plan_count<RK, W>(plan.p, o.rowptr, o.flag)));

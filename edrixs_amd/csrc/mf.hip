@@ -12,8 +12,8 @@
 // vectors, and the work is the term tests (integer ALU).  Two kernels:
 //   * k_plan_apply, for complete bases: 64 rows per workgroup over the terms
 //     grouped by column (termplan.hip), those of equal action merged;
-//   * k_mf, for incomplete bases, more than 4096 terms or rows of more than 255
-//     entries: one 64-lane wave per row, its lanes testing the terms in
+//   * k_mf, for incomplete bases, more than 4096 terms, rows of more than 255
+//     entries, and few terms on few rows (mf_try_plan): one 64-lane wave per row, its lanes testing the terms in
 //     parallel and accumulating val * sign * x[col] over the survivors.
 
 namespace {
@@ -146,43 +146,47 @@ __global__ __launch_bounds__(64) void k_mf(BuildParams p, const MfMask *__restri
     if (e.dvec && lane == 0) e.partials[blockIdx.x] = dot;
 }
 
-// The product over a term plan.  A workgroup of four waves owns 64 rows.  Lane
-// = row throughout: the waves find the surviving groups of their chunks and
-// list them per row in LDS; the diagonal group, whose density terms are the
-// same for every lane, is summed by one wave from scalar loads; then wave q
-// takes entries q, q + 4, ... of each row (sum of the group's terms, column
-// rank, x gather) and the four partial rows are added in wave order, so the
-// result does not depend on timing.  Bound by integer and LDS instructions (a
-// thousand terms tested, 24 columns ranked per row; the vectors take 0.03 ms):
-// H_n norb 20, 1.0M rows, 0.56 ms a product, by k_mf 4.38 ms.
-template <int RK, int CK, class W>
-__global__ __launch_bounds__(256) void k_plan_apply(Plan<W> p, int cap, const double2 *__restrict__ x,
+// The product over a term plan.  A workgroup of NW waves owns 64 rows.  Lane =
+// row throughout: the waves find the surviving groups of their chunks and list
+// them per row in LDS; each wave sums its share of the diagonal group, whose
+// density terms are the same for every lane and come by scalar loads, and takes
+// entries q, q + NW, ... of each row (sum of the group's terms, column rank, x
+// gather); the partial rows are added in wave order, so the result does not
+// depend on timing.  Bound by integer and LDS instructions (136 groups tested,
+// 24 columns ranked per row; the vectors take 0.03 ms): H_n norb 20, 1.0M rows,
+// 0.44 ms a product, by k_mf 4.38 ms.
+template <int NW, int RK, int CK, class W>
+__global__ __launch_bounds__(64 * NW) void k_plan_apply(Plan<W> p, int cap, const double2 *__restrict__ x,
                                                     SpmvEpi e) {
     if (e.run && *e.run == 0) return;
-    extern __shared__ int32_t s_bin[];                                          // nbits * nocc
-    uint16_t *s_grp = reinterpret_cast<uint16_t *>(s_bin + p.nbits * p.nocc);   // [cap][64]
-    __shared__ int s_cnt[PLAN_WAVES][PLAN_ROWS];
-    __shared__ double2 s_acc[PLAN_WAVES][PLAN_ROWS];
-    __shared__ double2 s_big[PLAN_ROWS];
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
+    int32_t *s_rank = reinterpret_cast<int32_t *>(s_mem);                   // rank_len
+    uint16_t *s_grp = reinterpret_cast<uint16_t *>(s_rank + p.rank_len);    // [cap][64]
+    __shared__ int s_cnt[NW][PLAN_ROWS];
+    __shared__ double2 s_acc[NW][PLAN_ROWS];
     const int lane = threadIdx.x & 63, wave = plan_wave();
     const int64_t r = (int64_t)blockIdx.x * PLAN_ROWS + lane;
     const bool on = r < p.M;
     const W w = on ? plan_row_word<RK, W>(p, r) : W(0);
-    plan_stage_binomials<W>(p, s_bin);
-    const int n = plan_expand<W>(p, w, on, s_cnt, [&](int i, int g) {
+    plan_stage_rank<W>(p, s_rank);
+    const int n = plan_expand<NW, W>(p, w, on, s_cnt, [&](int i, int g) {
         if (i < cap) s_grp[i * PLAN_ROWS + lane] = (uint16_t)g;
     });
-    if (p.big >= 0 && wave == PLAN_WAVES - 1) {
-        const PlanGroup<W> g = p.groups[p.big];
-        s_big[lane] = plan_sum<W>(p, g.tbeg, g.tend, w);
-    }
     __syncthreads();
     double2 acc = make_double2(0.0, 0.0);
-    for (int i = wave; i < n; i += PLAN_WAVES) {
+    if (p.big >= 0) {   // this wave's share of the diagonal's terms
+        const bool omega = wave == 0 && p.big == p.diag;
+        bool any = omega;
+        double2 v = plan_big<W>(p, wave, NW, w, any);
+        if (omega) v = cadd(v, p.omega);
+        if (any && on) acc = cmul(v, x[plan_col<CK, W>(p, w ^ p.groups[p.big].flip, s_rank)]);
+    }
+    for (int i = wave; i < n; i += NW) {
         const int gi = s_grp[i * PLAN_ROWS + lane];
+        if (gi == p.big) continue;
         const PlanGroup<W> g = p.groups[gi];
-        const double2 xv = x[plan_col<CK, W>(p, w ^ g.flip, s_bin)];
-        double2 v = gi == p.big ? s_big[lane] : plan_sum<W>(p, g.tbeg, g.tend, w);
+        const double2 xv = x[plan_col<CK, W>(p, w ^ g.flip, s_rank)];
+        double2 v = plan_sum<W>(p, g.tbeg, g.tend, w);
         if (gi == p.diag) v = cadd(v, p.omega);
         acc = cadd(acc, cmul(v, xv));
     }
@@ -191,7 +195,7 @@ __global__ __launch_bounds__(256) void k_plan_apply(Plan<W> p, int cap, const do
     if (wave != 0) return;
     double2 dot = make_double2(0, 0);
     if (on) {
-        for (int q = 1; q < PLAN_WAVES; ++q) acc = cadd(acc, s_acc[q][lane]);
+        for (int q = 1; q < NW; ++q) acc = cadd(acc, s_acc[q][lane]);
         double2 out = e.c0 ? cmul(*e.c0, acc) : acc;
         if (e.z) out = cadd(out, e.c1 ? cmul(*e.c1, e.z[r]) : e.z[r]);
         e.y[r] = out;
@@ -219,6 +223,22 @@ struct edx_mfop {
 
 namespace {
 
+// Waves per workgroup of k_plan_apply.  While the workgroups fill less than two
+// a CU the time is one workgroup's own, and sixteen waves share its terms and
+// entries: 26 us for 30 at 12,870 rows, 39.1 for 40.6 at 18,018; at 24,310 rows
+// (380 workgroups) both take 32.5, at 48,620 sixteen waves 39.7 and four 34.6,
+// at 705,432 347 and 202.
+constexpr int MF_WIDE = 16;
+
+int mf_waves(int64_t rows) {
+    return (rows + PLAN_ROWS - 1) / PLAN_ROWS <= (int64_t)edx::num_cus() * 3 / 2 ? MF_WIDE : PLAN_WAVES;
+}
+
+// Few terms on few rows keep k_mf, whose waves take a row each: 362 terms 23.5
+// us for 25.9 at 2,002 rows and 25.8 for 25.7 at 3,432; 950 terms 33 for 29 at
+// 1,512.
+constexpr int MF_TINY_ROWS = 3072, MF_TINY_TERMS = 512;
+
 int mf_blocks(const edx_mfop *op) {
     if (op->plan) return (int)std::max<int64_t>((op->p.M + PLAN_ROWS - 1) / PLAN_ROWS, 1);
     int64_t b = op->p.M;
@@ -233,9 +253,13 @@ template <int RK, int CK, class W>
 void mf_launch_plan(const edx_mfop *op, const Plan<W> &p, int nb, const double2 *x,
                     const SpmvEpi &e) {
     const int cap = std::max(op->maxrow, 1);
-    const size_t lds = (size_t)p.nbits * p.nocc * 4 + (size_t)cap * PLAN_ROWS * 2;
-    hipLaunchKernelGGL((k_plan_apply<RK, CK, W>), dim3(nb), dim3(256), lds, edx::stream(), p, cap,
-                       x, e);
+    const size_t lds = (size_t)p.rank_len * 4 + (size_t)cap * PLAN_ROWS * 2;
+    if (mf_waves(op->p.M) == MF_WIDE)
+        hipLaunchKernelGGL((k_plan_apply<MF_WIDE, RK, CK, W>), dim3(nb), dim3(64 * MF_WIDE), lds,
+                           edx::stream(), p, cap, x, e);
+    else
+        hipLaunchKernelGGL((k_plan_apply<PLAN_WAVES, RK, CK, W>), dim3(nb), dim3(64 * PLAN_WAVES), lds,
+                           edx::stream(), p, cap, x, e);
 }
 
 // Groups the operator's terms where the basis allows; the longest row sizes
@@ -243,7 +267,7 @@ void mf_launch_plan(const edx_mfop *op, const Plan<W> &p, int nb, const double2 
 template <int RK, int CK, class W>
 int mf_plan(edx_mfop *op, const PlanSpaces &sp, PlanStore<W> &store) {
     EDX_TRY(plan_make<W>(sp, op->tt.ops.data(), op->tt.vals.data(), op->tt.nhop, op->tt.T,
-                         op->p.omega_on != 0, op->p.omega, op->p.negate != 0, true, store));
+                         op->p.omega_on != 0, op->p.omega, op->p.negate != 0, mf_waves(op->p.M), true, store));
     store.p.inter = 0;
     DevBuf flag;
     EDX_TRY(flag.alloc(sizeof(int), "longest row"));
@@ -256,6 +280,7 @@ int mf_plan(edx_mfop *op, const PlanSpaces &sp, PlanStore<W> &store) {
 
 template <int RK, int CK> int mf_try_plan(edx_mfop *op, const edx_basis *fock) {
     const PlanSpaces sp{RK, CK, op->p.nv, op->p.nc, fock, fock};
+    if (op->p.M <= MF_TINY_ROWS && op->tt.T <= MF_TINY_TERMS) return EDX_OK;
     if (op->p.M == 0 || !plan_usable(sp, op->tt.ops.data(), op->tt.nhop, op->tt.T) ||
         op->p.M >= ((int64_t)1 << 31))
         return EDX_OK;

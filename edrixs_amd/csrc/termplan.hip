@@ -26,14 +26,21 @@ enum { ROW_PLAIN = 0, ROW_COREHOLE = 1, ROW_FULLCORE = 2 };
 enum { COL_PLAIN = 0, COL_COREHOLE = 1, COL_VALONLY = 2 };
 
 // the words of a plan: 32 bits where valence and core orbitals fit, else 64
-template <class W> struct PlanTest {   // four survival tests; bit: the group's in its chunk
-    W m[4], v[4];
+template <class W> struct PlanTest {   // two survival tests; bit: the group's in its chunk
+    W m[2], v[2];
     uint32_t bit, pad;
+};
+template <class W> struct PlanDens {   // a term of the big group whose sign is constant
+    W m, v;
+    double x;
 };
 template <class W> struct PlanTerm {
     W m, v, s;
-    uint32_t neg;     // c, and the operator's overall sign
+    uint32_t neg;     // bit 0: c, and the operator's overall sign; PLAN_FLIP_X, _Y
 };
+// The sign applies to the real / imaginary part; clear on a part of merged
+// terms that is +0 whatever their sign.
+constexpr uint32_t PLAN_FLIP_X = 1u << 30, PLAN_FLIP_Y = 1u << 31;
 template <class W> struct PlanGroup {
     W flip;
     int32_t tbeg, tend;   // its terms, in term order
@@ -42,8 +49,13 @@ template <class W> struct PlanGroup {
 
 constexpr int PLAN_ROWS = 64;        // rows per workgroup: lane = row
 constexpr int PLAN_WAVES = 4;        // waves share the groups (chunks) of the same rows
+constexpr int RANK_BITS = 4;         // bits per lookup of a column's rank
+constexpr int RANK_UNROLL = 24 / RANK_BITS;   // lookups without a test
+constexpr int RANK_MAX = (64 + RANK_BITS - 1) / RANK_BITS;
 constexpr int PLAN_CHUNK = 32;       // groups per chunk (bits of a survival mask)
 constexpr int PLAN_MAX_TERMS = 4096; // the term-by-term build's limit per row
+constexpr int PLAN_SMALL_ROW = 64;   // longest row of the fill's compact lists
+constexpr int FILL_U = 2;            // entries a thread of the fill has in flight
 constexpr int PLAN_BIG = 24;         // a group of more terms (the diagonal) is summed per row
 
 // A plan on the device, with what its kernels need to know of the spaces.
@@ -53,8 +65,15 @@ template <class W> struct Plan {
     const PlanTerm<W> *terms;
     const double2 *vals;             // value of each term, the sign not applied
     const PlanGroup<W> *groups;
-    int nchunk, gpc;                 // chunks (a multiple of PLAN_WAVES), groups per chunk
+    const int32_t *rank;             // rank tables (plan_rank)
+    int rank_len, nrank;             // their length, lookups per word
+    int rank_off[RANK_MAX];
+    int ngroups;
+    int nchunk, gpc;                 // chunks (a multiple of the kernel's waves), groups per chunk
     int big;                         // group summed lane = row, or -1
+    const PlanDens<W> *dens;         // its terms if all have constant signs and the same
+    int ndens;                       // zero imaginary part, else none
+    double dens_y;                   // that zero, signed
     int diag;                        // group of the diagonal when omega is added, or -1
     double2 omega;
     int64_t M;                       // rows
@@ -90,18 +109,35 @@ __device__ __forceinline__ W plan_key(const Plan<W> &p, W w) {
     return p.inter ? (W)((val << p.nc) | (w >> p.nv)) : w;
 }
 
-// Column of a word; s_bin[p * nocc + k] = C(p, k + 1) staged in LDS.
-template <int CK, class W>
-__device__ __forceinline__ int32_t plan_col(const Plan<W> &p, W w, const int32_t *s_bin) {
-    W val = CK == COL_PLAIN ? w : w & (W)((W(1) << p.nv) - 1);
+// Rank of a word of the column basis: sum of C(q_k, k + 1) over its orbitals
+// q_0 < q_1 < ...  RANK_BITS of the word and the number of orbitals below them
+// index a table (staged in LDS): six independent lookups for 24 orbitals, where a
+// walk over the orbitals takes twelve dependent steps.  Six-bit tables (7 KB
+// instead of 3) take a workgroup per CU: the fill below 1.14 for 1.05 ms.
+template <class W>
+__device__ __forceinline__ int32_t plan_rank(const Plan<W> &p, W val, const int32_t *s_rank) {
+    constexpr uint32_t mask = (1u << RANK_BITS) - 1;
     int32_t l = 0;
-    const int32_t *b = s_bin;
-    while (val) {
-        const int q = (sizeof(W) == 4 ? __ffs((unsigned)val) : __ffsll((unsigned long long)val)) - 1;
-        l += b[q * p.nocc];
-        ++b;
-        val &= val - 1;
+    uint32_t k = 0;
+#pragma unroll
+    for (int j = 0; j < RANK_UNROLL; ++j) {   // past the last orbital: a zero entry
+        const uint32_t c = (uint32_t)(val >> (RANK_BITS * j)) & mask;
+        l += s_rank[p.rank_off[j] + (int)((k << RANK_BITS) | c)];
+        k += __popc(c);
     }
+    for (int j = RANK_UNROLL; j < p.nrank; ++j) {
+        const uint32_t c = (uint32_t)(val >> (RANK_BITS * j)) & mask;
+        l += s_rank[p.rank_off[j] + (int)((k << RANK_BITS) | c)];
+        k += __popc(c);
+    }
+    return l;
+}
+
+// Column of a word.
+template <int CK, class W>
+__device__ __forceinline__ int32_t plan_col(const Plan<W> &p, W w, const int32_t *s_rank) {
+    const W val = CK == COL_PLAIN ? w : w & (W)((W(1) << p.nv) - 1);
+    const int32_t l = plan_rank<W>(p, val, s_rank);
     if (CK != COL_COREHOLE) return l;
     const W holes = (W)(((W(1) << p.nc) - 1) ^ (w >> p.nv));
     const int k = p.nc - 1 - ((sizeof(W) == 4 ? __ffs((unsigned)holes)
@@ -110,11 +146,10 @@ __device__ __forceinline__ int32_t plan_col(const Plan<W> &p, W w, const int32_t
 }
 
 template <class W>
-__device__ __forceinline__ void plan_stage_binomials(const Plan<W> &p, int32_t *s_bin) {
-    for (int i = threadIdx.x; i < p.nbits * p.nocc; i += blockDim.x) {
-        const int64_t b = binom_dev(i / p.nocc, i % p.nocc + 1);
-        s_bin[i] = b < (int64_t(1) << 31) ? (int32_t)b : 0;   // larger ones are in no rank
-    }
+__device__ __forceinline__ void plan_stage_rank(const Plan<W> &p, int32_t *s_rank) {
+    const int4 *from = reinterpret_cast<const int4 *>(p.rank);
+    int4 *to = reinterpret_cast<int4 *>(s_rank);
+    for (int i = threadIdx.x; i < p.rank_len / 4; i += blockDim.x) to[i] = from[i];
 }
 
 // Which groups of chunk c have a surviving term on word w.  Chunk, test and
@@ -127,19 +162,22 @@ __device__ __forceinline__ uint32_t plan_mask(const Plan<W> &p, int c, W w) {
 #pragma unroll 2
     for (int i = ib; i < ie; ++i) {
         const PlanTest<W> &t = p.tests[i];
-        const bool ok = ((w & t.m[0]) == t.v[0]) | ((w & t.m[1]) == t.v[1]) |
-                        ((w & t.m[2]) == t.v[2]) | ((w & t.m[3]) == t.v[3]);
+        const bool ok = ((w & t.m[0]) == t.v[0]) | ((w & t.m[1]) == t.v[1]);
         mask |= ok ? t.bit : 0u;
     }
     return mask;
 }
 
+__device__ __forceinline__ double plan_flip(double v, uint32_t sign) {
+    return __hiloint2double(__double2hiint(v) ^ (int)sign, __double2loint(v));
+}
+
 template <class W>
 __device__ __forceinline__ void plan_add_term(const PlanTerm<W> &t, double2 v, W w, double2 &acc) {
     if ((w & t.m) == t.v) {
-        if ((plan_popc<W>(w & t.s) ^ t.neg) & 1) v = make_double2(-v.x, -v.y);
-        acc.x += v.x;
-        acc.y += v.y;
+        const uint32_t flip = (uint32_t)(plan_popc<W>(w & t.s) ^ t.neg) << 31;
+        acc.x += plan_flip(v.x, flip & (t.neg << 1));
+        acc.y += plan_flip(v.y, flip & t.neg);
     }
 }
 
@@ -150,6 +188,31 @@ __device__ __forceinline__ double2 plan_sum(const Plan<W> &p, int tb, int te, W 
     double2 acc = make_double2(-0.0, -0.0);
 #pragma unroll 2
     for (int t = tb; t < te; ++t) plan_add_term<W>(p.terms[t], p.vals[t], w, acc);
+    return acc;
+}
+
+// Sum of terms first, first + step, ... of the big group; any: one survives.
+template <class W>
+__device__ __forceinline__ double2 plan_big(const Plan<W> &p, int first, int step, W w, bool &any) {
+    const PlanGroup<W> g = p.groups[p.big];
+    if (p.ndens) {
+        double acc = -0.0;
+#pragma unroll 4
+        for (int t = first; t < p.ndens; t += step) {
+            const PlanDens<W> d = p.dens[t];
+            const bool ok = (w & d.m) == d.v;
+            any |= ok;
+            acc += ok ? d.x : -0.0;
+        }
+        return make_double2(acc, p.dens_y);
+    }
+    double2 acc = make_double2(-0.0, -0.0);
+#pragma unroll 2
+    for (int t = g.tbeg + first; t < g.tend; t += step) {
+        const PlanTerm<W> &tm = p.terms[t];
+        any |= (w & tm.m) == tm.v;
+        plan_add_term<W>(tm, p.vals[t], w, acc);
+    }
     return acc;
 }
 
@@ -183,20 +246,20 @@ __global__ __launch_bounds__(256) void k_plan_count(Plan<W> p, int64_t *counts, 
 
 // Lists the row's surviving groups: entry e of row `lane` at list[e * 64 +
 // lane] by emit(e, group), groups in plan order; returns the row's count.
-// Every thread of the workgroup calls it (barriers inside).
-template <class W, class Emit>
+// Every thread of the workgroup of NW waves calls it (barriers inside).
+template <int NW, class W, class Emit>
 __device__ __forceinline__ int plan_expand(const Plan<W> &p, W w, bool on, int (*s_cnt)[PLAN_ROWS],
                                            Emit emit) {
     const int lane = threadIdx.x & 63, wave = plan_wave();
     int n = 0;
-    for (int c0 = 0; c0 < p.nchunk; c0 += PLAN_WAVES) {
+    for (int c0 = 0; c0 < p.nchunk; c0 += NW) {
         const int c = c0 + wave;
         uint32_t mask = on ? plan_mask<W>(p, c, w) : 0u;
         __syncthreads();
         s_cnt[wave][lane] = __popc(mask);
         __syncthreads();
         int e = n;
-        for (int q = 0; q < PLAN_WAVES; ++q) {
+        for (int q = 0; q < NW; ++q) {
             const int k = s_cnt[q][lane];
             if (q < wave) e += k;
             n += k;
@@ -216,22 +279,27 @@ __device__ __forceinline__ int plan_expand(const Plan<W> &p, W w, bool on, int (
 // (2) lane = row: an entry's place in its row is the number of smaller keys.
 // (3) lane = entry, in output order: sums its group's few terms, ranks its
 // column and stores, so a wave writes 64 consecutive columns and values.
-// 512 * cap bytes of LDS and 4 KB decide the workgroups per CU (cap = the longest
-// row, about 40: six); the time goes to the integer instructions of (1) and (3),
-// the 20 bytes per entry are written behind them.  Measured, count and fill:
-// H_i norb 24 (2.7M rows, 44M entries) 0.11 + 1.09 ms (0.9 TB/s written), by the
+// LDS decides the workgroups per CU and with them the speed: lists of at most 64
+// entries a row over at most 256 groups (SMALL) take 5 bytes an entry (32-bit
+// words), the places in output order lying over the keys, and leave room for
+// eight workgroups; other lists take 8.  The time goes to the integer
+// instructions of (1) and (3) and their dependent loads, the 20 bytes per entry
+// are written behind them.  Measured, count and fill: H_i norb 24 (2.7M rows,
+// 44M entries) 0.08 + 0.74 ms (1.2 TB/s written; 8-byte lists 0.80), by the
 // term-by-term kernel 16.1 + 21.4 ms; H_n norb 21 N 9 (2.1M rows, 50M entries)
-// 0.19 + 1.76 ms, before 27.9 + 36.9 ms.
-template <int RK, int CK, class W>
+// 0.11 + 1.05 ms (8-byte lists 1.48), before 27.9 + 36.9 ms.
+template <bool SMALL, int RK, int CK, class W>
 __global__ __launch_bounds__(256) void k_plan_fill(Plan<W> p, int cap,
                                                    const int64_t *__restrict__ rowptr,
                                                    int32_t *__restrict__ cols,
                                                    double2 *__restrict__ vals) {
-    extern __shared__ char s_mem[];
+    using G = typename std::conditional<SMALL, uint8_t, uint16_t>::type;
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
     W *s_key = reinterpret_cast<W *>(s_mem);                                  // [cap][64]
-    int32_t *s_bin = reinterpret_cast<int32_t *>(s_key + cap * PLAN_ROWS);   // nbits * nocc
-    uint16_t *s_grp = reinterpret_cast<uint16_t *>(s_bin + p.nbits * p.nocc);   // [cap][64]
-    uint16_t *s_flat = s_grp + cap * PLAN_ROWS;                               // [cap * 64]
+    int32_t *s_rank = reinterpret_cast<int32_t *>(s_key + cap * PLAN_ROWS);   // rank_len
+    G *s_grp = reinterpret_cast<G *>(s_rank + p.rank_len);                    // [cap][64]
+    uint16_t *s_flat = SMALL ? reinterpret_cast<uint16_t *>(s_mem)            // [cap * 64]
+                             : reinterpret_cast<uint16_t *>(s_grp + cap * PLAN_ROWS);
     __shared__ W s_w[PLAN_ROWS];
     __shared__ double2 s_big[PLAN_ROWS];
     __shared__ int s_cnt[PLAN_WAVES][PLAN_ROWS];
@@ -240,21 +308,22 @@ __global__ __launch_bounds__(256) void k_plan_fill(Plan<W> p, int cap,
     const bool on = r < p.M;
     const W w = on ? plan_row_word<RK, W>(p, r) : W(0);
     if (wave == 0) s_w[lane] = w;
-    plan_stage_binomials<W>(p, s_bin);
+    plan_stage_rank<W>(p, s_rank);
     if (p.big >= 0 && wave == PLAN_WAVES - 1) {
-        const PlanGroup<W> g = p.groups[p.big];
-        s_big[lane] = plan_sum<W>(p, g.tbeg, g.tend, w);
+        bool any = false;
+        s_big[lane] = plan_big<W>(p, 0, 1, w, any);
     }
-    const int n = plan_expand<W>(p, w, on, s_cnt, [&](int e, int g) {
+    const int n = plan_expand<PLAN_WAVES, W>(p, w, on, s_cnt, [&](int e, int g) {
         if (e < cap) {
             s_key[e * PLAN_ROWS + lane] = plan_key<CK, W>(p, w ^ p.groups[g].flip);
-            s_grp[e * PLAN_ROWS + lane] = (uint16_t)g;
+            s_grp[e * PLAN_ROWS + lane] = (G)g;
         }
     });
     __syncthreads();
     const int64_t base = rowptr[r0];
     const int off = on ? (int)(rowptr[r] - base) : 0;
-    for (int i0 = wave; i0 < n; i0 += 4 * PLAN_WAVES) {
+    // four entries a round: how many keys of the row are smaller
+    auto places = [&](int i0) {
         W key[4];
         int below[4];
 #pragma unroll
@@ -268,24 +337,54 @@ __global__ __launch_bounds__(256) void k_plan_fill(Plan<W> p, int cap,
 #pragma unroll
             for (int u = 0; u < 4; ++u) below[u] += kj < key[u];
         }
+        return (uint32_t)(below[0] | below[1] << 8 | below[2] << 16 | below[3] << 24);
+    };
+    auto put = [&](int i0, uint32_t at) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int i = i0 + u * PLAN_WAVES;
-            if (i < n) s_flat[off + below[u]] = (uint16_t)(lane | (i << 6));
+            if (i < n) s_flat[off + (int)(at >> (8 * u) & 255)] = (uint16_t)(lane | (i << 6));
         }
+    };
+    if constexpr (SMALL) {   // the keys' room is written once they are all read
+        constexpr int ROUNDS = PLAN_SMALL_ROW / (4 * PLAN_WAVES);
+        uint32_t at[ROUNDS];
+#pragma unroll
+        for (int q = 0; q < ROUNDS; ++q) {
+            const int i0 = wave + q * 4 * PLAN_WAVES;
+            at[q] = i0 < n ? places(i0) : 0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < ROUNDS; ++q) put(wave + q * 4 * PLAN_WAVES, at[q]);
+    } else {
+        for (int i0 = wave; i0 < n; i0 += 4 * PLAN_WAVES) put(i0, places(i0));
     }
     __syncthreads();
     const int64_t rend = r0 + PLAN_ROWS < p.M ? r0 + PLAN_ROWS : p.M;
     const int total = (int)(rowptr[rend] - base);
-    for (int e = threadIdx.x; e < total; e += 256) {
-        const int f = s_flat[e], row = f & 63;
-        const int gi = s_grp[(f >> 6) * PLAN_ROWS + row];
-        const W rw = s_w[row];
-        const PlanGroup<W> g = p.groups[gi];
-        double2 acc = gi == p.big ? s_big[row] : plan_sum<W>(p, g.tbeg, g.tend, rw);
-        if (gi == p.diag) acc = make_double2(acc.x + p.omega.x, acc.y + p.omega.y);
-        cols[base + e] = plan_col<CK, W>(p, rw ^ g.flip, s_bin);
-        vals[base + e] = acc;
+    for (int e0 = threadIdx.x; e0 < total; e0 += 256 * FILL_U) {
+        int gi[FILL_U], row[FILL_U];
+        W rw[FILL_U];
+        PlanGroup<W> g[FILL_U];
+#pragma unroll
+        for (int u = 0; u < FILL_U; ++u) {
+            const int e = e0 + 256 * u;
+            const int f = s_flat[e < total ? e : e0];
+            row[u] = f & 63;
+            gi[u] = s_grp[(f >> 6) * PLAN_ROWS + row[u]];
+            rw[u] = s_w[row[u]];
+            g[u] = p.groups[gi[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < FILL_U; ++u) {
+            const int e = e0 + 256 * u;
+            if (e >= total) break;
+            double2 acc = gi[u] == p.big ? s_big[row[u]] : plan_sum<W>(p, g[u].tbeg, g[u].tend, rw[u]);
+            if (gi[u] == p.diag) acc = make_double2(acc.x + p.omega.x, acc.y + p.omega.y);
+            cols[base + e] = plan_col<CK, W>(p, rw[u] ^ g[u].flip, s_rank);
+            vals[base + e] = acc;
+        }
     }
 }
 
@@ -346,11 +445,89 @@ template <class W> struct PlanStore {
     PlanStore &operator=(const PlanStore &) = delete;
 };
 
-// Groups the terms.  merge: terms that differ in their value only become one
+// The tables of plan_rank: for each RANK_BITS bits of a word, and each number of
+// orbitals below them that a word of the basis can have, the part of the rank.
+void plan_rank_tables(int nbits, int nocc, std::vector<int32_t> &tab, int *off, int *nrank) {
+    std::vector<std::vector<int64_t>> C(nbits + 1, std::vector<int64_t>(nocc + 2, 0));
+    for (int a = 0; a <= nbits; ++a) {
+        C[a][0] = 1;
+        for (int b = 1; b <= nocc + 1 && b <= a; ++b)
+            C[a][b] = std::min(C[a - 1][b - 1] + C[a - 1][b], (int64_t)1 << 31);
+    }
+    *nrank = std::max((nbits + RANK_BITS - 1) / RANK_BITS, 1);
+    const int words = 1 << RANK_BITS;
+    for (int j = 0; j < RANK_MAX; ++j) {
+        if (j >= *nrank) {   // nocc orbitals below and none here: entry 0 of the first row
+            off[j] = -nocc * words;
+            continue;
+        }
+        const int below = RANK_BITS * j;
+        const int lo = std::max(0, nocc - (nbits - below)), hi = std::min(below, nocc);
+        off[j] = (int)tab.size() - lo * words;
+        for (int k0 = lo; k0 <= hi; ++k0)
+            for (int c = 0; c < words; ++c) {
+                int64_t l = 0;
+                int k = k0;
+                for (int b = 0; b < RANK_BITS; ++b)
+                    if (c >> b & 1) {
+                        ++k;   // a larger value is in no word's rank
+                        if (below + b <= nbits && k <= nocc) l += C[below + b][k];
+                    }
+                tab.push_back(l < ((int64_t)1 << 31) ? (int32_t)l : 0);
+            }
+    }
+}
+
+// Terms of a group with the same test and parity mask have the same sign on
+// every row up to one constant, so their sum may be taken here: summed in term
+// order it is the row's own sum, or its negative, bit for bit (rounding is
+// symmetric), as long as no row has survivors of two such classes, whose terms
+// might alternate.  A part that sums to zero is +0 on every row unless all its
+// terms are zeros of one sign (neg's flip flags).  Two-body terms come in four
+// orders of their operators and two directions: eight terms become two.
+struct TermClass {
+    int lead;         // its first term
+    double2 sum;      // in the lead's sign
+    uint32_t flips;   // PLAN_FLIP_X, _Y
+};
+
+bool plan_merge_exact(const std::vector<HostTerm> &ht, const std::vector<double2> &hv,
+                      const std::vector<int> &terms, std::vector<TermClass> &out) {
+    out.clear();
+    auto same_zero = [](double a, double b) {
+        return a == 0.0 && b == 0.0 && std::signbit(a) == std::signbit(b);
+    };
+    for (int q : terms) {
+        size_t c = 0;
+        for (; c < out.size(); ++c) {
+            const HostTerm &l = ht[out[c].lead];
+            if (l.m == ht[q].m && l.v == ht[q].v && l.s == ht[q].s) break;
+            if (((l.v ^ ht[q].v) & l.m & ht[q].m) == 0) return false;   // one row may have both
+        }
+        if (c == out.size()) {
+            out.push_back(TermClass{q, hv[q], PLAN_FLIP_X | PLAN_FLIP_Y});
+            continue;
+        }
+        TermClass &k = out[c];
+        const double sg = ht[q].neg == ht[k.lead].neg ? 1.0 : -1.0;
+        const double2 v = make_double2(sg * hv[q].x, sg * hv[q].y);
+        if (!same_zero(hv[k.lead].x, v.x)) k.flips &= ~PLAN_FLIP_X;
+        if (!same_zero(hv[k.lead].y, v.y)) k.flips &= ~PLAN_FLIP_Y;
+        k.sum.x += v.x;
+        k.sum.y += v.y;
+    }
+    for (TermClass &k : out) {
+        if (k.sum.x != 0.0) k.flips |= PLAN_FLIP_X;
+        if (k.sum.y != 0.0) k.flips |= PLAN_FLIP_Y;
+    }
+    return true;
+}
+
+// Groups the terms.  waves: those of the kernels that expand it.  merge: terms that differ in their value only become one
 // (the matrix-free apply, whose sums need not keep the term order).
 template <class W>
 int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int nhop, int T,
-              bool omega_on, double2 omega, bool negate, bool merge, PlanStore<W> &out) {
+              bool omega_on, double2 omega, bool negate, int waves, bool merge, PlanStore<W> &out) {
     struct Group {
         uint64_t key;
         std::vector<int> terms;
@@ -396,7 +573,7 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
     }
     const int G = (int)groups.size();
     int nchunk = (G + PLAN_CHUNK - 1) / PLAN_CHUNK;
-    nchunk = std::max((nchunk + PLAN_WAVES - 1) / PLAN_WAVES, 1) * PLAN_WAVES;
+    nchunk = std::max((nchunk + waves - 1) / waves, 1) * waves;
     const int gpc = std::max((G + nchunk - 1) / nchunk, 1);
     std::vector<PlanTest<W>> tests;
     std::vector<int32_t> chunks(nchunk + 1, 0);
@@ -405,6 +582,7 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
     std::vector<PlanGroup<W>> dg(std::max(G, 1));
     int big = -1, nbig = PLAN_BIG;
     std::vector<std::pair<uint64_t, uint64_t>> kept;
+    std::vector<TermClass> classes;
     for (int c = 0; c < nchunk; ++c) {
         chunks[c] = (int32_t)tests.size();
         for (int g = c * gpc; g < std::min((c + 1) * gpc, G); ++g) {
@@ -412,9 +590,13 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
             PlanGroup<W> &d = dg[g];
             d.flip = 0;
             d.tbeg = (int32_t)terms.size();
-            for (int q : gr.terms) {
-                terms.push_back(PlanTerm<W>{(W)ht[q].m, (W)ht[q].v, (W)ht[q].s, ht[q].neg});
-                vals.push_back(hv[q]);
+            const bool exact = !merge && plan_merge_exact(ht, hv, gr.terms, classes);
+            const size_t count = exact ? classes.size() : gr.terms.size();
+            for (size_t i = 0; i < count; ++i) {
+                const int q = exact ? classes[i].lead : gr.terms[i];
+                const uint32_t flips = exact ? classes[i].flips : PLAN_FLIP_X | PLAN_FLIP_Y;
+                terms.push_back(PlanTerm<W>{(W)ht[q].m, (W)ht[q].v, (W)ht[q].s, ht[q].neg | flips});
+                vals.push_back(exact ? classes[i].sum : hv[q]);
                 d.flip = (W)ht[q].f;
             }
             if (sp.ck == COL_VALONLY) d.flip = (W)gr.key;
@@ -440,10 +622,10 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
                         if (!implied) kept.emplace_back(ht[q].m, ht[q].v);
                     }
             }
-            for (size_t i = 0; i < kept.size(); i += 4) {
+            for (size_t i = 0; i < kept.size(); i += 2) {
                 PlanTest<W> q{};
                 q.bit = 1u << (g - c * gpc);
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < 2; ++u) {
                     const auto &k = kept[std::min(i + u, kept.size() - 1)];
                     q.m[u] = (W)k.first;
                     q.v[u] = (W)k.second;
@@ -453,6 +635,22 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
         }
     }
     chunks[nchunk] = (int32_t)tests.size();
+    std::vector<PlanDens<W>> dens;
+    double dens_y = 0.0;
+    if (big >= 0) {
+        for (int t = dg[big].tbeg; t < dg[big].tend; ++t) {
+            const uint32_t neg = terms[t].neg;
+            double2 v = vals[t];
+            if ((neg & 1) && (neg & PLAN_FLIP_X)) v.x = -v.x;
+            if ((neg & 1) && (neg & PLAN_FLIP_Y)) v.y = -v.y;
+            if (t == dg[big].tbeg) dens_y = v.y;
+            if (terms[t].s != 0 || v.y != 0.0 || std::signbit(v.y) != std::signbit(dens_y)) {
+                dens.clear();
+                break;
+            }
+            dens.push_back(PlanDens<W>{terms[t].m, terms[t].v, v.x});
+        }
+    }
     auto up = [](size_t b) { return (b + 63) / 64 * 64; };
     // two spare records: the scalar loads of the unrolled loop stay inside
     const size_t b_tests = up((tests.size() + 2) * sizeof(PlanTest<W>));
@@ -460,10 +658,16 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
     const size_t b_terms = up((terms.size() + 2) * sizeof(PlanTerm<W>));
     const size_t b_vals = up((vals.size() + 2) * sizeof(double2));
     const size_t b_groups = up(dg.size() * sizeof(PlanGroup<W>));
-    std::vector<char> buf(b_tests + b_chunks + b_terms + b_vals + b_groups, 0);
+    Plan<W> &p = out.p;
+    std::vector<int32_t> rank;
+    plan_rank_tables(sp.right->nbits, sp.right->nocc, rank, p.rank_off, &p.nrank);
+    const size_t b_rank = up(rank.size() * sizeof(int32_t));
+    const size_t b_dens = up((dens.size() + 4) * sizeof(PlanDens<W>));
+    std::vector<char> buf(b_tests + b_chunks + b_terms + b_vals + b_groups + b_rank + b_dens, 0);
     char *h = buf.data();
     const size_t o_chunks = b_tests, o_terms = o_chunks + b_chunks, o_vals = o_terms + b_terms,
-                 o_groups = o_vals + b_vals;
+                 o_groups = o_vals + b_vals, o_rank = o_groups + b_groups,
+                 o_dens = o_rank + b_rank;
     if (!tests.empty()) memcpy(h, tests.data(), tests.size() * sizeof(PlanTest<W>));
     memcpy(h + o_chunks, chunks.data(), chunks.size() * sizeof(int32_t));
     if (!terms.empty()) {
@@ -471,19 +675,26 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
         memcpy(h + o_vals, vals.data(), vals.size() * sizeof(double2));
     }
     memcpy(h + o_groups, dg.data(), dg.size() * sizeof(PlanGroup<W>));
+    memcpy(h + o_rank, rank.data(), rank.size() * sizeof(int32_t));
+    if (!dens.empty()) memcpy(h + o_dens, dens.data(), dens.size() * sizeof(PlanDens<W>));
     out.d_buf = edx::dmalloc(buf.size(), "term plan");
     if (!out.d_buf) return EDX_ERR_NOMEM;
     EDX_HIP(edx::copy_sync(out.d_buf, h, buf.size(), hipMemcpyHostToDevice));
     char *d = (char *)out.d_buf;
-    Plan<W> &p = out.p;
     p.tests = (const PlanTest<W> *)d;
     p.chunks = (const int32_t *)(d + o_chunks);
     p.terms = (const PlanTerm<W> *)(d + o_terms);
     p.vals = (const double2 *)(d + o_vals);
     p.groups = (const PlanGroup<W> *)(d + o_groups);
+    p.rank = (const int32_t *)(d + o_rank);
+    p.rank_len = (int)rank.size();
+    p.ngroups = G;
     p.nchunk = nchunk;
     p.gpc = gpc;
     p.big = big;
+    p.dens = (const PlanDens<W> *)(d + o_dens);
+    p.ndens = (int)dens.size();
+    p.dens_y = dens_y;
     p.diag = omega_on ? 0 : -1;
     p.omega = omega;
     p.left = sp.left->d_words;
@@ -520,7 +731,7 @@ constexpr int PLAN_LDS = 144 << 10;   // of 160 KB, with room for the static arr
 // Longest row the fill's lists can hold.
 template <class W> int plan_max_row(const Plan<W> &p) {
     const int per = PLAN_ROWS * (int)(sizeof(W) + 4);
-    return std::min((PLAN_LDS - p.nbits * p.nocc * 4) / per, 255);
+    return std::min((PLAN_LDS - p.rank_len * 4) / per, 255);
 }
 
 template <int RK, class W>
@@ -531,17 +742,26 @@ int plan_count(const Plan<W> &p, int64_t *counts, int *d_maxrow) {
     return EDX_OK;
 }
 
+template <bool SMALL, int RK, int CK, class W>
+int plan_fill_launch(const Plan<W> &p, int cap, size_t entry, const int64_t *rowptr, int32_t *cols,
+                     double2 *vals) {
+    const size_t lds = (size_t)cap * PLAN_ROWS * entry + (size_t)p.rank_len * 4;
+    if (lds > (64 << 10))
+        EDX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_plan_fill<SMALL, RK, CK, W>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_plan_fill<SMALL, RK, CK, W>),
+                       dim3((unsigned)((p.M + PLAN_ROWS - 1) / PLAN_ROWS)), dim3(256), lds,
+                       edx::stream(), p, cap, rowptr, cols, vals);
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
+}
+
 template <int RK, int CK, class W>
 int plan_fill(const Plan<W> &p, int maxrow, const int64_t *rowptr, int32_t *cols, double2 *vals) {
     const int cap = std::max((maxrow + 3) / 4 * 4, 4);
-    const size_t lds = (size_t)cap * PLAN_ROWS * (sizeof(W) + 4) + (size_t)p.nbits * p.nocc * 4;
-    if (lds > (64 << 10))
-        EDX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_plan_fill<RK, CK, W>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_plan_fill<RK, CK, W>), dim3((unsigned)((p.M + PLAN_ROWS - 1) / PLAN_ROWS)),
-                       dim3(256), lds, edx::stream(), p, cap, rowptr, cols, vals);
-    EDX_LAUNCH_CHECK();
-    return EDX_OK;
+    if (cap <= PLAN_SMALL_ROW && p.ngroups <= 256)
+        return plan_fill_launch<true, RK, CK, W>(p, cap, sizeof(W) + 1, rowptr, cols, vals);
+    return plan_fill_launch<false, RK, CK, W>(p, cap, sizeof(W) + 4, rowptr, cols, vals);
 }
 
 }  // namespace

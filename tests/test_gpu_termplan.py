@@ -131,7 +131,8 @@ def test_builds_that_keep_the_term_by_term_kernel(core, case):
 
 
 @pytest.mark.parametrize("space,nv,nocc", [("i", 6, 1), ("i", 8, 4), ("i", 33, 2), ("i", 16, 8),
-                                           ("n", 7, 3), ("n", 28, 1)])
+                                           ("i", 18, 9), ("n", 7, 3), ("n", 28, 1), ("n", 13, 6),
+                                           ("n", 15, 7)])
 def test_matrix_free_apply_at_word_and_workgroup_edges(core, space, nv, nocc):
     """y += H x from the term plan against the oracle's product.  Both add the
     same products in another order (the plan also adds equal terms' values
@@ -167,3 +168,35 @@ def test_matrix_free_apply_at_word_and_workgroup_edges(core, space, nv, nocc):
         assert np.abs(y - ref).max() <= 2 * T * 2.3e-16 * T * big * np.abs(x).max()
         again = op.apply(dev[0], torch.from_numpy(y0).cuda()).cpu().numpy()
         assert np.array_equal(y, again)
+
+
+@pytest.mark.parametrize("nbits,nocc,sets,sign", [(7, 3, 40, 1.0), (10, 5, 90, -1.0),
+                                                  (12, 6, 700, 1.0), (12, 6, 700, -1.0)])
+def test_merged_terms_keep_every_bit(core, nbits, nocc, sets, sign):
+    """Terms in all orders of their operators, with equal, opposite, unrelated and
+    zero values: the entries are the oracle's sums in term order, signs of zeros
+    included.  700 sets make rows of more than 64 entries and more than 256 groups."""
+    rng = np.random.default_rng(nbits + sets)
+    u = np.zeros((nbits,) * 4, dtype=np.complex128)
+    for q in range(sets):
+        i, j, k, l = rng.integers(0, nbits, size=4)
+        if i == j or k == l:
+            continue
+        v = [0.5, -1.25, rng.normal(), 1j * rng.normal(), rng.normal() + 1j * rng.normal()][q % 5]
+        orders = [(i, j, k, l), (j, i, k, l), (i, j, l, k), (j, i, l, k)]
+        rel = [(1, -1, -1, 1), (1, 1, 1, 1), (1, -1, 1, -1), (1, 0, 0, 1), (1, 0.3, -0.7, 1)][q % 4 + (q % 7 == 0)]
+        for o4, r in zip(orders, rel):
+            u[o4] += r * v
+            u[o4[::-1]] += r * np.conj(v)
+    ht, ut = siam.emat_terms(H.random_hermitian_emat(nbits, rng, density=0.5)), siam.umat_terms(u)
+    ut["re"][::9] *= 0.0
+    ut["im"][::4] = -0.0
+    A = core.build_ham_i(core.Basis.combinations(nbits, nocc), ht, ut, omega=-0.0 + 0.5j, ham_sign=sign)
+    R = o.build_ham_i(H.fock_words(nbits, nocc), ht, ut, omega=-0.0 + 0.5j, ham_sign=sign)
+    if sets == 700:
+        assert 64 < np.diff(R.rowptr).max() <= 255
+    rp, cols, vals = A.download()
+    assert np.array_equal(rp, np.asarray(R.rowptr)) and np.array_equal(cols, np.asarray(R.cols))
+    ref = np.ascontiguousarray(R.vals).view(np.float64)
+    got = np.ascontiguousarray(vals).view(np.float64)
+    assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
