@@ -588,13 +588,13 @@ struct BMinres {
     int *iters;          // [K]
     double tol;
     int maxit;
-    const int *istep;    // nullptr: the iteration is the launch argument i; else *istep
+    int *istep;          // nullptr: the iteration is the launch argument i; else istep[0]
+                         // in k_bm_alpha, istep[1] - 1 after it (each advanced by a
+                         // kernel that does not read it, so that no launch is spent)
 };
 
-// the iteration a MINRES kernel works on
-__device__ __forceinline__ int bm_step(const BMinres &s, int i) { return s.istep ? *s.istep : i; }
-
-__global__ void k_bm_next(int *istep) { *istep += 1; }
+// the iteration a MINRES kernel after k_bm_alpha works on
+__device__ __forceinline__ int bm_step(const BMinres &s, int i) { return s.istep ? s.istep[1] - 1 : i; }
 
 __global__ void k_bm_init(BMinres s, int K, const double2 *sums) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -609,9 +609,9 @@ __global__ void k_bm_init(BMinres s, int K, const double2 *sums) {
     s.run[k] = (b0 > s.tol && 0 < s.maxit) ? 1 : 0;
 }
 
-__global__ void k_bm_divbeta(int64_t n, int K, double2 *v, BMinres s, int i) {
+__global__ void k_bm_divbeta(int64_t n, int K, double2 *v, BMinres s) {
     ELEM_SETUP
-    if (!kv || !s.run[(int64_t)bm_step(s, i) * K + k]) return;
+    if (!kv || !s.run[k]) return;
     const double d = s.beta0[k];
     for (int64_t r = rstart; r < n; r += rstride) {
         const double2 t = v[r * K + k];
@@ -619,11 +619,16 @@ __global__ void k_bm_divbeta(int64_t n, int K, double2 *v, BMinres s, int i) {
     }
 }
 
-__global__ void k_bm_alpha(BMinres s, int K, int i, const double2 *sums) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    i = bm_step(s, i);
-    if (k >= K || !s.run[i * K + k]) return;
-    s.alpha[k] = sums[k];
+// alpha from the nb partials of <v|tmp>, a workgroup per system
+__global__ __launch_bounds__(256) void k_bm_alpha(BMinres s, int K, int i, const double2 *partials,
+                                                  int nb) {
+    const int k = blockIdx.x;
+    if (s.istep) {
+        i = s.istep[0];
+        if (k == 0 && threadIdx.x == 0) s.istep[1] = i + 1;
+    }
+    const double2 sum = block_partials(partials, nb, K, k);
+    if (threadIdx.x == 0 && s.run[(int64_t)i * K + k]) s.alpha[k] = sum;
 }
 
 // vp = tmp - alpha vc - beta0 vp ; partial |vp|^2   (src/linsys.f90:87)
@@ -645,15 +650,19 @@ __global__ void k_bm_vupdate(int64_t n, int K, const double2 *tmp, const double2
     elem_reduce(acc, K, partials);
 }
 
-__global__ void k_bm_scalars(BMinres s, int K, int i, const double2 *sums) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+// The step's scalars from the nb partials of |vp|^2, a workgroup per system
+__global__ __launch_bounds__(256) void k_bm_scalars(BMinres s, int K, int i, const double2 *partials,
+                                                    int nb) {
+    const int k = blockIdx.x;
     i = bm_step(s, i);
-    if (k >= K) return;
-    if (!s.run[i * K + k]) {
-        s.run[(i + 1) * K + k] = 0;
+    if (s.istep && k == 0 && threadIdx.x == 0) s.istep[0] = i + 1;
+    const double2 sum = block_partials(partials, nb, K, k);
+    if (threadIdx.x != 0) return;
+    if (!s.run[(int64_t)i * K + k]) {
+        s.run[(int64_t)(i + 1) * K + k] = 0;
         return;
     }
-    const double beta1 = sqrt(sums[k].x);
+    const double beta1 = sqrt(sum.x);
     const double beta0 = s.beta0[k];
     const double2 alpha = s.alpha[k];
     const double2 g0 = s.gamma0[k], g1 = s.gamma1[k], sg0 = s.sigma0[k], sg1 = s.sigma1[k];
@@ -676,20 +685,28 @@ __global__ void k_bm_scalars(BMinres s, int K, int i, const double2 *sums) {
     s.eta[k] = make_double2(-(ns0.x * eta.x - ns0.y * eta.y), -(ns0.x * eta.y + ns0.y * eta.x));
     s.beta0[k] = beta1;
     s.iters[k] = i + 1;
-    s.run[(i + 1) * K + k] = (hypot(s.res[k].x, s.res[k].y) > s.tol && i + 1 < s.maxit) ? 1 : 0;
+    s.run[(int64_t)(i + 1) * K + k] = (hypot(s.res[k].x, s.res[k].y) > s.tol && i + 1 < s.maxit) ? 1 : 0;
 }
 
-// w_prev = (v_curr - rho3 w_prev - rho2 w_curr) / rho1 ; x += gamma0 eta w_prev
+// w_prev = (v_curr - rho3 w_prev - rho2 w_curr) / rho1 ; x += gamma0 eta w_prev ;
+// vp /= beta for the next iteration, if there is one
 __global__ void k_bm_wx(int64_t n, int K, const double2 *vc, double2 *wp, const double2 *wc,
-                        double2 *x, BMinres s, int i) {
+                        double2 *x, double2 *vp, BMinres s, int i) {
     ELEM_SETUP
-    if (!kv || !s.run[(int64_t)bm_step(s, i) * K + k]) return;
+    i = bm_step(s, i);
+    if (!kv || !s.run[(int64_t)i * K + k]) return;
     const double2 r3 = s.rho3[k], r2 = s.rho2[k], ir1 = s.inv_rho1[k], xc = s.xcoef[k];
+    const bool next = s.run[(int64_t)(i + 1) * K + k] != 0;
+    const double d = s.beta0[k];
     for (int64_t r = rstart; r < n; r += rstride) {
         const int64_t o = r * K + k;
         const double2 w = cmul(csub(csub(vc[o], cmul(r3, wp[o])), cmul(r2, wc[o])), ir1);
         wp[o] = w;
         x[o] = cadd(x[o], cmul(xc, w));
+        if (next) {
+            const double2 t = vp[o];
+            vp[o] = make_double2(t.x / d, t.y / d);
+        }
     }
 }
 
@@ -1674,11 +1691,12 @@ int bminres_run(const edx_csr *h, int precision, int K, const double2 *sigma, co
     hipLaunchKernelGGL(k_bm_init, dim3(kb), dim3(64), 0, s, st, K, sums);
     EDX_LAUNCH_CHECK();
     st.istep = nullptr;
-    // one iteration on edx::stream(); its step is i, or *sti.istep (then
-    // advanced) when the launches are captured
+    // One iteration on edx::stream(); its step is i, or read from sti.istep (and
+    // advanced) when the launches are captured.  Five launches: the sums carry
+    // the scalars, and the last pass divides the next vector by beta (nine took
+    // 424 us at 145,860 rows and 32 systems, 45 us of them in one-block kernels).
     auto iterate = [&](int i, int cur, int prv, const BMinres &sti) -> int {
         hipStream_t ls = edx::stream();
-        ELAUNCH(k_bm_divbeta, n, K, n, K, v[cur], sti, i);
         if (precision == EDX_C64) ELAUNCH(k_il_to_c64, n, K, n, K, v[cur], x32.as<float2>());
         BEpi e{};   // tmp = sigma_k v - H v ; partial <v|tmp>
         e.y = tmp;
@@ -1688,26 +1706,24 @@ int bminres_run(const edx_csr *h, int precision, int K, const double2 *sigma, co
         e.partials = part.as<double2>();
         int nb = 0;
         EDX_TRY(edx::bspmm(h, precision, K, v[cur], x32.as<float2>(), e, &nb));
-        hipLaunchKernelGGL(k_breduce, dim3(K), dim3(256), 0, ls, part.as<double2>(), nb, K, sums);
-        hipLaunchKernelGGL(k_bm_alpha, dim3(kb), dim3(64), 0, ls, sti, K, i, sums);
+        hipLaunchKernelGGL(k_bm_alpha, dim3(K), dim3(256), 0, ls, sti, K, i, part.as<double2>(), nb);
         ELAUNCH(k_bm_vupdate, n, K, n, K, tmp, v[cur], v[prv], sti, i, part.as<double2>());
-        hipLaunchKernelGGL(k_breduce, dim3(K), dim3(256), 0, ls, part.as<double2>(), nbe, K, sums);
-        hipLaunchKernelGGL(k_bm_scalars, dim3(kb), dim3(64), 0, ls, sti, K, i, sums);
-        ELAUNCH(k_bm_wx, n, K, n, K, v[cur], w[prv], w[cur], x, sti, i);
-        if (sti.istep) hipLaunchKernelGGL(k_bm_next, dim3(1), dim3(1), 0, ls, (int *)sti.istep);
+        hipLaunchKernelGGL(k_bm_scalars, dim3(K), dim3(256), 0, ls, sti, K, i, part.as<double2>(), nbe);
+        ELAUNCH(k_bm_wx, n, K, n, K, v[cur], w[prv], w[cur], x, v[prv], sti, i);
         EDX_LAUNCH_CHECK();
         return EDX_OK;
     };
     // iteration 0 runs eagerly (it also times the SpMM schedules on first use);
     // then an odd/even pair of iterations is captured once into a HIP graph and
     // replayed, the kernels reading the step from device memory
+    ELAUNCH(k_bm_divbeta, n, K, n, K, v[0], st);
     EDX_TRY(iterate(0, 0, 1, st));
     int i = 1, checked = 0;
     Dbuf stepb;
     hipGraphExec_t exec = nullptr;
     hipStream_t cap = nullptr;
     if (graphs_enabled() && !edx::g_prof && maxit >= 3) {
-        EDX_TRY(stepb.alloc(sizeof(int), "minres step"));
+        EDX_TRY(stepb.alloc(2 * sizeof(int), "minres step"));
         EDX_HIP(edx::copy_sync(stepb.p, &i, sizeof(int), hipMemcpyHostToDevice));
         BMinres sg = st;
         sg.istep = stepb.as<int>();

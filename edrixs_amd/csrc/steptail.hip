@@ -251,19 +251,26 @@ __device__ __forceinline__ void step_tail(const StepTail &t, const double2 *part
     }
 }
 
+// The sum of right-hand side k's partials by one workgroup of 256 threads, in
+// its wave 0.
+__device__ __forceinline__ double2 block_partials(const double2 *partials, int nb, int K, int k) {
+    __shared__ double2 s_sum[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double2 s = make_double2(0, 0);
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nb; b += 256) s = cadd(s, partials[(int64_t)b * K + k]);
+    s_sum[wave][lane] = s;   // wave q: quarter q
+    __syncthreads();
+    if (wave != 0) return s;
+    return wave_sum_tail(join_quarters(s, s_sum[1][lane], s_sum[2][lane], s_sum[3][lane]));
+}
+
 // The same for a launch without a tail: workgroup k sums nb partials of
 // right-hand side k.
 __global__ __launch_bounds__(256) void k_step_reduce(StepTail t, const double2 *partials, int nb) {
-    __shared__ double2 s_sum[4][64];
-    const int k = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double2 s = make_double2(0, 0);
-#pragma unroll 4
-    for (int b = threadIdx.x; b < nb; b += 256) s = cadd(s, partials[(int64_t)b * t.K + k]);
-    s_sum[wave][lane] = s;   // wave q: quarter q
-    __syncthreads();
-    if (wave == 0)
-        step_finish(t, k, wave_sum_tail(join_quarters(s, s_sum[1][lane], s_sum[2][lane],
-                                                      s_sum[3][lane])), lane);
+    const int k = blockIdx.x;
+    const double2 s = block_partials(partials, nb, t.K, k);
+    if (threadIdx.x < 64) step_finish(t, k, s, threadIdx.x);
 }
 
 // After a pass with tail t: nb = 0 if the pass ran it, else its partials per
