@@ -285,11 +285,24 @@ __global__ __launch_bounds__(VB) void k_gemv_ct(int64_t n, const double2 *V, int
     }
 }
 
-// h[c] = sum_b partials[c * nbx + b], a workgroup per column; with alpha, the last
-// column is v_j and *alpha = dot + its component
+// h[c] = sum_b partials[c * nbx + b] in the order of b, a workgroup per column: the
+// partials are fetched by all threads, added by one.  With alpha, the last
+// column is v_j and *alpha = dot + its component.
 __global__ __launch_bounds__(VB) void k_reduce_cols(const double2 *partials, int nbx, double2 *h,
                                                     const double2 *dot, double *alpha) {
-    const double2 s = reduce_partials(partials + (int64_t)blockIdx.x * nbx, nbx);
+    __shared__ double2 s_p[VB];
+    const double2 *p = partials + (int64_t)blockIdx.x * nbx;
+    double2 s = make_double2(0, 0);
+    for (int b0 = 0; b0 < nbx; b0 += VB) {
+        __syncthreads();
+        if (b0 + (int)threadIdx.x < nbx) s_p[threadIdx.x] = p[b0 + threadIdx.x];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int e = nbx - b0 < VB ? nbx - b0 : VB;
+#pragma unroll 8
+            for (int b = 0; b < e; ++b) s = cadd(s, s_p[b]);
+        }
+    }
     if (threadIdx.x != 0) return;
     h[blockIdx.x] = s;
     if (alpha && blockIdx.x == gridDim.x - 1) *alpha = dot->x + s.x;
@@ -300,125 +313,127 @@ __global__ __launch_bounds__(VB) void k_reduce_cols(const double2 *partials, int
 // w = H v_j - alpha v_j - beta v_{j-1}, made orthogonal to the k basis columns V
 // by two classical Gram-Schmidt passes, in three passes over V instead of four
 // (a pass reads 16 n k bytes and little else):
-//   k_cgs_tile<FIRST>  the three-term part and c = V^H w;
-//   k_cgs_tile         w -= V c and c' = V^H w, both from one copy of V in LDS;
+//   k_cgs_pass<FIRST>  the three-term part and c = V^H w;
+//   k_cgs_pass         w -= V c and c' = V^H w, V's row staying in registers;
 //   k_cgs_last         w -= V c' and |w|^2.
-// The scalars stay on the device, so the host waits once per cycle.  A step over
-// 705,432 rows and 3 to 22 columns (trlan, three states): 370 us with two
-// separate passes of two kernels, one-thread column sums (26 us each) and three
-// waits.  k_cgs_tile reads 22 columns in 35 us (7 TB/s: the basis stays in the
-// last-level cache), lane-per-row kernels with 8 or 12 sums each 52 and 64 us.
+// The scalars stay on the device, so the host waits once per cycle.  Every sum
+// is taken in the order of the plain kernels (k_dot, k_gemv_ct, k_gemv_n_sub):
+// the signs of the Ritz vectors hang on the last bits of the coefficients (an
+// off-diagonal entry at the eigensolver's threshold), so that another order
+// would turn them around in a few runs of a hundred.
+// A step over 705,432 rows and 3 to 22 columns (trlan, three states) takes 175 us,
+// with two separate passes of two kernels, one-thread column sums (26 us each)
+// and three waits 320.  k_cgs_pass reads 17 to 22 columns in 45 to 49 us (62
+// without the next row's loads in flight); more workgroups would be faster
+// (35 us) in another order of summation.
 
-constexpr int CGS_ROWS = 64;            // rows per tile
-constexpr int CGS_LD = CGS_ROWS + 1;    // lanes over columns then hit different banks
-constexpr int CGS_MAXK = 64;            // columns whose next tile fits in registers
+constexpr int CGS_MAXK = 32;   // columns a lane holds with their sums (8 registers each)
 
-// FIRST: w = t - dot v - b vprev, v and vprev columns k-1 and k-2 (tri).  Else w -=
-// V h.  Then partials[c * gridDim.x + bx] of V^H w.  A workgroup walks tiles of 64
-// rows: its waves put the columns (lane = row) into LDS, adding up V h on the way,
-// then lanes are columns and the waves (and KP-lane groups, k <= KP) share the
-// rows.  The next tile's columns are loaded into registers before the current
-// tile is worked on.
+// FIRST: w -= dot v + b vprev (dot: the sum of nd partials, also stored to *dot).
+// Else w -= V h.  Then partials[c * gridDim.x + bx] of V^H w.  A lane takes a row:
+// its k <= KP entries in registers, k running sums.
 template <int KP, bool FIRST>
-__global__ __launch_bounds__(VB) void k_cgs_tile(int64_t n, const double2 *V, int64_t ld, int k,
-                                                 const double2 *h, const double2 *t, int tri,
-                                                 const double *bprev, double2 *w, double2 *partials) {
-    extern __shared__ double2 s_V[];            // [k][CGS_LD]
-    __shared__ double2 s_p[4][CGS_ROWS], s_w[CGS_ROWS], s_h[KP];
-    constexpr int G = 64 / KP;                  // row groups per wave
-    constexpr int NL = KP / 4;                  // columns a wave loads
+__global__ __launch_bounds__(VB, 1) void k_cgs_pass(int64_t n, const double2 *V, int64_t ld, int k,
+                                                    const double2 *h, const double2 *dotp, int nd,
+                                                    double2 *dot, const double2 *vprev,
+                                                    const double *bprev, double2 *w,
+                                                    double2 *partials) {
+    __shared__ double2 s_h[KP];
+    __shared__ double2 s_sum[4][KP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = lane % KP, sub = lane / KP;
-    const double a = FIRST ? h->x : 0.0, b = FIRST && tri ? *bprev : 0.0;   // FIRST: h is the dot
-    if (!FIRST)
+    const double2 *vj = V + (int64_t)(k - 1) * ld;
+    double a = 0.0, b = 0.0;
+    if (FIRST) {
+        const double2 d = reduce_partials(dotp, nd);
+        a = d.x;
+        if (vprev) b = *bprev;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *dot = d;
+    } else {
         for (int c = threadIdx.x; c < k; c += VB) s_h[c] = h[c];
-    __syncthreads();
-    double2 acc = make_double2(0, 0);
-    double2 v[NL], wr = make_double2(0, 0);
-    const double2 *win = FIRST ? t : w;
-    auto load = [&](int64_t r0) {
-        const int64_t r = r0 + lane;
-        const bool on = r < n;
-        wr = on ? win[r] : make_double2(0, 0);
+        __syncthreads();
+    }
+    double2 acc[KP];
 #pragma unroll
-        for (int i = 0; i < NL; ++i)
-            v[i] = on && wave + 4 * i < k ? V[(int64_t)(wave + 4 * i) * ld + r] : make_double2(0, 0);
+    for (int c = 0; c < KP; ++c) acc[c] = make_double2(0, 0);
+    constexpr bool AHEAD = KP <= 24;   // the next row's columns fit in registers too
+    const int64_t stride = (int64_t)gridDim.x * VB;
+    int64_t r = blockIdx.x * (int64_t)VB + threadIdx.x;
+    double2 vn[AHEAD ? KP : 1], xn = make_double2(0, 0);
+    auto ahead = [&](int64_t q) {
+        if constexpr (AHEAD) {
+            const int64_t o = q < n ? q : n - 1;
+            xn = w[o];
+#pragma unroll
+            for (int c = 0; c < KP; ++c) vn[c] = V[(int64_t)(c < k ? c : k - 1) * ld + o];
+        }
     };
-    const int64_t stride = (int64_t)gridDim.x * CGS_ROWS;
-    int64_t r0 = (int64_t)blockIdx.x * CGS_ROWS;
-    load(r0);
-    for (; r0 < n; r0 += stride) {
-        double2 p = make_double2(0, 0);
+    if (r < n) ahead(r);
+    for (; r < n; r += stride) {
+        double2 v[KP], x;
+        if constexpr (AHEAD) {
+            x = xn;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int c = wave + 4 * i;
-            if (c < k) {
-                s_V[c * CGS_LD + lane] = v[i];
-                if (!FIRST) p = cadd(p, cmul(v[i], s_h[c]));
-            }
+            for (int c = 0; c < KP; ++c) v[c] = vn[c];
+            ahead(r + stride);
+        } else {
+            x = w[r];
+#pragma unroll
+            for (int c = 0; c < KP; ++c) v[c] = V[(int64_t)(c < k ? c : k - 1) * ld + r];
         }
-        if (!FIRST) s_p[wave][lane] = p;
-        double2 x = wr;
-        load(r0 + stride);
-        __syncthreads();
-        if (wave == 0) {
-            if (FIRST) {
-                x = csub(x, cscale(s_V[(k - 1) * CGS_LD + lane], a));
-                if (tri) x = csub(x, cscale(s_V[(k - 2) * CGS_LD + lane], b));
-            } else {
-                x = csub(x, cadd(cadd(s_p[0][lane], s_p[1][lane]), cadd(s_p[2][lane], s_p[3][lane])));
-            }
-            s_w[lane] = x;
-            if (r0 + lane < n) w[r0 + lane] = x;
+        if (FIRST) {
+            x = csub(x, cscale(vj[r], a));
+            if (vprev) x = csub(x, cscale(vprev[r], b));
+        } else {
+            double2 s = make_double2(0, 0);
+#pragma unroll
+            for (int c = 0; c < KP; ++c)
+                if (c < k) s = cadd(s, cmul(v[c], s_h[c]));
+            x = csub(x, s);
         }
-        __syncthreads();
-        if (col < k)
-            for (int i = sub; i < CGS_ROWS / 4; i += G) {
-                const int row = wave * (CGS_ROWS / 4) + i;
-                acc = cadd(acc, cconjmul(s_V[col * CGS_LD + row], s_w[row]));
-            }
-        __syncthreads();
+        w[r] = x;
+#pragma unroll
+        for (int c = 0; c < KP; ++c) acc[c] = cadd(acc[c], cconjmul(v[c], x));
     }
-    // the row groups' sums, in order (4 G <= 32 of a column's 65 places)
-    if (col < k) s_V[(wave * G + sub) * k + col] = acc;
+#pragma unroll
+    for (int c = 0; c < KP; ++c) {
+        double2 q = acc[c];
+        for (int off = 32; off > 0; off >>= 1) {
+            q.x += __shfl_xor(q.x, off, 64);
+            q.y += __shfl_xor(q.y, off, 64);
+        }
+        if (lane == 0) s_sum[wave][c] = q;
+    }
     __syncthreads();
-    for (int c = threadIdx.x; c < k; c += VB) {
-        double2 q = s_V[c];
-        for (int i = 1; i < 4 * G; ++i) q = cadd(q, s_V[i * k + c]);
-        partials[(int64_t)c * gridDim.x + blockIdx.x] = q;
-    }
-}
-
-template <int KP, bool FIRST>
-int cgs_tile_launch(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double2 *h,
-                    const double2 *t, int tri, const double *bprev, double2 *w, double2 *partials) {
-    const size_t lds = (size_t)k * CGS_LD * sizeof(double2);
-    if (lds > (56 << 10))
-        EDX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_cgs_tile<KP, FIRST>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_cgs_tile<KP, FIRST>), dim3(nb), dim3(VB), lds, edx::stream(), n, V, ld, k, h, t,
-                       tri, bprev, w, partials);
-    EDX_LAUNCH_CHECK();
-    return EDX_OK;
+    for (int c = threadIdx.x; c < k; c += VB)   // block_sum_256's order
+        partials[(int64_t)c * gridDim.x + blockIdx.x] =
+            cadd(cadd(s_sum[0][c], s_sum[1][c]), cadd(s_sum[2][c], s_sum[3][c]));
 }
 
 // k <= CGS_MAXK columns
 template <bool FIRST>
-int cgs_tile(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double2 *h, const double2 *t,
-             int tri, const double *bprev, double2 *w, double2 *partials) {
-    if (k <= 8) return cgs_tile_launch<8, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
-    if (k <= 16) return cgs_tile_launch<16, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
-    if (k <= 32) return cgs_tile_launch<32, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
-    return cgs_tile_launch<64, FIRST>(nb, n, V, ld, k, h, t, tri, bprev, w, partials);
+int cgs_pass(int nb, int64_t n, const double2 *V, int64_t ld, int k, const double2 *h,
+             const double2 *dotp, int nd, double2 *dot, const double2 *vprev, const double *bprev,
+             double2 *w, double2 *partials) {
+    hipStream_t s = edx::stream();
+#define CGS_PASS(KP)                                                                             \
+    hipLaunchKernelGGL((k_cgs_pass<KP, FIRST>), dim3(nb), dim3(VB), 0, s, n, V, ld, k, h, dotp, \
+                       nd, dot, vprev, bprev, w, partials)
+    if (k <= 8) CGS_PASS(8);
+    else if (k <= 16) CGS_PASS(16);
+    else if (k <= 24) CGS_PASS(24);
+    else CGS_PASS(CGS_MAXK);
+#undef CGS_PASS
+    EDX_LAUNCH_CHECK();
+    return EDX_OK;
 }
 
-// w = t - dot vj - bprev vprev (more columns than a tile takes)
-__global__ __launch_bounds__(VB) void k_cgs_three(int64_t n, const double2 *t, const double2 *vj,
+// w -= dot vj + bprev vprev (more columns than k_cgs_pass takes)
+__global__ __launch_bounds__(VB) void k_cgs_three(int64_t n, double2 *w, const double2 *vj,
                                                   const double2 *dot, const double2 *vprev,
-                                                  const double *bprev, double2 *w) {
+                                                  const double *bprev) {
     const double a = dot->x, b = vprev ? *bprev : 0.0;
     for (int64_t r = blockIdx.x * (int64_t)VB + threadIdx.x; r < n; r += (int64_t)gridDim.x * VB) {
-        double2 x = csub(t[r], cscale(vj[r], a));
+        double2 x = csub(w[r], cscale(vj[r], a));
         if (vprev) x = csub(x, cscale(vprev[r], b));
         w[r] = x;
     }
@@ -449,7 +464,7 @@ __global__ __launch_bounds__(VB) void k_cgs_last(int64_t n, const double2 *V, in
         for (int c = 0; c < k; ++c) s = cadd(s, cmul(V[(int64_t)c * ld + r], c < 1024 ? hs[c] : h[c]));
         const double2 x = csub(w[r], s);
         w[r] = x;
-        nrm.x += x.x * x.x + x.y * x.y;
+        nrm = cadd(nrm, cconjmul(x, x));
     }
     nrm = block_sum_256(nrm);
     if (threadIdx.x == 0) partials[blockIdx.x] = nrm;
@@ -460,11 +475,13 @@ __global__ __launch_bounds__(VB) void k_cgs_beta(const double2 *partials, int nb
     if (threadIdx.x == 0) *beta = sqrt(fabs(s.x));
 }
 
-// the next basis column w / beta; zero where the space is exhausted
-__global__ void k_cgs_next(int64_t n, const double2 *w, const double *beta, double2 *out) {
-    const double b = *beta;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
+// *beta = |w| from the nd partials of k_cgs_last, out = w / *beta; 0 past an invariant
+// subspace
+__global__ __launch_bounds__(VB) void k_cgs_next(int64_t n, const double2 *w, const double2 *partials,
+                                                 int nd, double *beta, double2 *out) {
+    const double b = sqrt(fabs(reduce_partials(partials, nd).x));
+    if (blockIdx.x == 0 && threadIdx.x == 0) *beta = b;
+    for (int64_t i = blockIdx.x * (int64_t)VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
         out[i] = b < 1e-10 ? make_double2(0, 0) : make_double2(w[i].x / b, w[i].y / b);
 }
 
@@ -512,12 +529,37 @@ int combine_launch(int nb, int64_t n, const double2 *V, int64_t ld, int k, const
     return EDX_OK;
 }
 
-// x += *c y
-__global__ __launch_bounds__(VB) void k_axpy_coef(int64_t n, double2 *x, const double2 *y,
-                                                  const double *c) {
-    const double a = *c;
-    for (int64_t i = blockIdx.x * (int64_t)VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
-        x[i] = cadd(x[i], cscale(y[i], a));
+// A step of the two-pass recurrence after its product w = H v (k_dot's partials
+// dotp): w -= alpha v + *bprev vprev, *alpha = Re <v|w>, norm partials.
+__global__ __launch_bounds__(VB) void k_two_pass_first(int64_t n, double2 *w, const double2 *v,
+                                                       const double2 *dotp, int nd, double *alpha,
+                                                       const double2 *vprev, const double *bprev,
+                                                       double2 *partials) {
+    const double a = reduce_partials(dotp, nd).x, b = vprev ? *bprev : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *alpha = a;
+    double2 s = make_double2(0, 0);
+    for (int64_t i = blockIdx.x * (int64_t)VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
+        double2 x = csub(w[i], cscale(v[i], a));
+        if (vprev) x = csub(x, cscale(vprev[i], b));
+        w[i] = x;
+        s = cadd(s, cconjmul(x, x));
+    }
+    s = block_sum_256(s);
+    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
+// The same step run again with its alpha a and betas: X -= c v, and the next
+// vector (w - a v - b vprev) / beta over vprev.
+__global__ __launch_bounds__(VB) void k_two_pass_again(int64_t n, const double2 *w, const double2 *v,
+                                                       double a, double2 *vprev, int tri, double b,
+                                                       double beta, double2 *X, double c) {
+    for (int64_t i = blockIdx.x * (int64_t)VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
+        const double2 vi = v[i];
+        X[i] = csub(X[i], cscale(vi, c));
+        double2 x = csub(w[i], cscale(vi, a));
+        if (tri) x = csub(x, cscale(vprev[i], b));
+        vprev[i] = make_double2(x.x / beta, x.y / beta);
+    }
 }
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {

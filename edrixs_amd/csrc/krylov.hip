@@ -290,7 +290,6 @@ int minres_run(const edx_csr *a, int precision, const double2 *b, double2 *x, do
 // ------------------------------------------------------------- Lanczos
 
 constexpr int GEMV_NBX = 256;   // row workgroups per column group of the projections
-constexpr int CGS_NBX = 512;    // workgroups of k_cgs_tile
 
 struct Lanczos {
     const edx_csr *h;
@@ -305,8 +304,7 @@ struct Lanczos {
     double2 *hvec;
     int nbv;
     // of the reorthogonalized steps (lanczos_step)
-    double2 *t = nullptr;       // H v
-    double2 *spart = nullptr;   // the product's dot partials
+    double2 *spart = nullptr;   // dot partials of v_j and the product
     double2 *dot = nullptr;
     double *al = nullptr;       // alpha_j, beta_j of the run's steps, cap_cols each
     double *be = nullptr;
@@ -314,18 +312,16 @@ struct Lanczos {
 
 // Device memory of reorthogonalized steps over cap_cols basis columns.
 struct LanczosBufs {
-    DevBuf w, t, part, hv, spart, sc;
+    DevBuf w, part, hv, spart, sc;
     int alloc(const edx_csr *h, int64_t n, int cap_cols, int nbv) {
         EDX_TRY(w.alloc(n * sizeof(double2), "lanczos w"));
-        EDX_TRY(t.alloc(n * sizeof(double2), "lanczos H v"));
-        EDX_TRY(part.alloc(((size_t)cap_cols * CGS_NBX + nbv + 64) * sizeof(double2), "partials"));
+        EDX_TRY(part.alloc(((size_t)cap_cols * GEMV_NBX + nbv + 64) * sizeof(double2), "partials"));
         EDX_TRY(hv.alloc((size_t)cap_cols * sizeof(double2), "coefficients"));
-        EDX_TRY(spart.alloc((size_t)edx::spmv_partials_len(h) * sizeof(double2), "product partials"));
+        EDX_TRY(spart.alloc((size_t)nbv * sizeof(double2), "dot partials"));
         return sc.alloc(sizeof(double2) + (size_t)cap_cols * 2 * sizeof(double), "lanczos scalars");
     }
     void set(Lanczos &L) const {
         L.w = w.as<double2>();
-        L.t = t.as<double2>();
         L.part = part.as<double2>();
         L.hvec = hv.as<double2>();
         L.spart = spart.as<double2>();
@@ -374,34 +370,32 @@ int lanczos_step(Lanczos &L, int first, int j, bool tri) {
     const int k = first + j + 1, nbx = std::min(L.nbv, GEMV_NBX);
     const double2 *vj = L.basis + (int64_t)(first + j) * L.ld;
     SpmvEpi e{};
-    e.y = L.t;
-    e.dvec = vj;
-    e.partials = L.spart;
-    int nb = 0;
-    EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, &nb, nullptr));
-    hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(VB), 0, s, L.spart, nb, L.dot, nullptr);
+    e.y = L.w;
+    EDX_TRY(apply(L.h, L.precision, vj, L.x32, e, nullptr, nullptr));
+    hipLaunchKernelGGL(k_dot, dim3(L.nbv), dim3(VB), 0, s, n, vj, L.w, L.spart, nullptr);
     const double2 *vprev = tri ? vj - L.ld : nullptr;
     const double *bprev = tri ? L.be + j - 1 : nullptr;
-    const bool tile = k <= CGS_MAXK;
-    int nbc = tile ? (int)std::min<int64_t>((n + CGS_ROWS - 1) / CGS_ROWS, CGS_NBX) : nbx;
-    if (tile) {
-        EDX_TRY(cgs_tile<true>(nbc, n, L.basis, L.ld, k, L.dot, L.t, tri, bprev, L.w, L.part));
+    const bool pass = k <= CGS_MAXK;
+    if (pass) {
+        EDX_TRY(cgs_pass<true>(nbx, n, L.basis, L.ld, k, nullptr, L.spart, L.nbv, L.dot, vprev, bprev,
+                               L.w, L.part));
     } else {   // the two passes as four kernels
-        hipLaunchKernelGGL(k_cgs_three, dim3(L.nbv), dim3(VB), 0, s, n, L.t, vj, L.dot, vprev, bprev, L.w);
+        hipLaunchKernelGGL(k_reduce_to, dim3(1), dim3(VB), 0, s, L.spart, L.nbv, L.dot, nullptr);
+        hipLaunchKernelGGL(k_cgs_three, dim3(L.nbv), dim3(VB), 0, s, n, L.w, vj, L.dot, vprev, bprev);
         hipLaunchKernelGGL(k_gemv_ct, dim3(nbx, (k + 7) / 8), dim3(VB), 0, s, n, L.basis, L.ld, k, L.w,
                            L.part);
     }
-    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbc, L.hvec, L.dot, L.al + j);
-    if (tile) {
-        EDX_TRY(cgs_tile<false>(nbc, n, L.basis, L.ld, k, L.hvec, nullptr, 0, nullptr, L.w, L.part));
+    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbx, L.hvec, L.dot, L.al + j);
+    if (pass) {
+        EDX_TRY(cgs_pass<false>(nbx, n, L.basis, L.ld, k, L.hvec, nullptr, 0, nullptr, nullptr, nullptr,
+                                L.w, L.part));
     } else {
         hipLaunchKernelGGL(k_gemv_n_sub, dim3(L.nbv), dim3(VB), 0, s, n, L.basis, L.ld, k, L.hvec, L.w);
         hipLaunchKernelGGL(k_gemv_ct, dim3(nbx, (k + 7) / 8), dim3(VB), 0, s, n, L.basis, L.ld, k, L.w,
                            L.part);
     }
-    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbc, L.hvec, nullptr, nullptr);
+    hipLaunchKernelGGL(k_reduce_cols, dim3(k), dim3(VB), 0, s, L.part, nbx, L.hvec, nullptr, nullptr);
     hipLaunchKernelGGL(k_cgs_last, dim3(L.nbv), dim3(VB), 0, s, n, L.basis, L.ld, k, L.hvec, L.w, L.part);
-    hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(VB), 0, s, L.part, L.nbv, L.be + j);
     EDX_LAUNCH_CHECK();
     return EDX_OK;
 }
@@ -409,6 +403,8 @@ int lanczos_step(Lanczos &L, int first, int j, bool tri) {
 // The same with alpha_j and beta_{j+1} appended to the host's lists.
 int lanczos_one(Lanczos &L, int first, int j, std::vector<double> &al, std::vector<double> &be) {
     EDX_TRY(lanczos_step(L, first, j, j > 0));
+    hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(VB), 0, edx::stream(), L.part, L.nbv, L.be + j);
+    EDX_LAUNCH_CHECK();
     double ab[2];
     EDX_HIP(hipMemcpyAsync(ab, L.al + j, sizeof(double), hipMemcpyDeviceToHost, edx::stream()));
     EDX_HIP(edx::copy_sync(ab + 1, L.be + j, sizeof(double), hipMemcpyDeviceToHost));
@@ -501,11 +497,12 @@ int trl_run(Lanczos &L, int first, int nev, int m, int max_cycles, double tol,
             // three-term part inside a tridiagonal stretch; after a restart the
             // arrow couplings go with the Gram-Schmidt passes
             EDX_TRY(lanczos_step(L, first, j, j > k));
-            if (j + 1 < m) {
-                hipLaunchKernelGGL(k_cgs_next, dim3(L.nbv), dim3(VB), 0, s, n, L.w, L.be + j,
-                                   L.basis + (int64_t)(first + j + 1) * L.ld);
-                EDX_LAUNCH_CHECK();
-            }
+            if (j + 1 < m)
+                hipLaunchKernelGGL(k_cgs_next, dim3(L.nbv), dim3(VB), 0, s, n, L.w, L.part, L.nbv,
+                                   L.be + j, L.basis + (int64_t)(first + j + 1) * L.ld);
+            else
+                hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(VB), 0, s, L.part, L.nbv, L.be + j);
+            EDX_LAUNCH_CHECK();
         }
         std::vector<double> al(m - k), be(m - k);
         EDX_HIP(hipMemcpyAsync(al.data(), L.al + k, (m - k) * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -730,42 +727,75 @@ int lanczos_rerun_impl(const edx_csr *h, int precision, int nev, int maxiter, do
     if (nvec > nev) nvec = nev;
     if (maxiter > n) maxiter = (int)n;
     const int nbv = vec_blocks(n);
-    const int64_t plen = edx::spmv_partials_len(h);
-    DevBuf buf, x32, coef;
-    EDX_TRY(buf.alloc(krylov_scratch_bytes(n, plen, maxiter), "lanczos scratch"));
+    DevBuf vb, x32, part, sc;
+    EDX_TRY(vb.alloc((size_t)n * 3 * sizeof(double2), "lanczos vectors"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(n * sizeof(float2), "lanczos x32"));
-    KrylovRun r(n, krylov_scratch_carve(buf.as<char>(), n, plen, maxiter), maxiter);
+    EDX_TRY(part.alloc((2 * (size_t)nbv + 64) * sizeof(double2), "partials"));
+    EDX_TRY(sc.alloc(2 * (size_t)maxiter * sizeof(double), "lanczos scalars"));
+    double2 *pdot = part.as<double2>(), *pnorm = pdot + nbv + 32;
+    double *dal = sc.as<double>(), *dbe = dal + maxiter;
+    Lanczos L{};
+    L.n = n;
+    L.nbv = nbv;
+    L.part = pdot;
     hipStream_t s = edx::stream();
+    double2 *buf[3] = {vb.as<double2>(), vb.as<double2>() + n, vb.as<double2>() + 2 * n};
     double2 *X = (double2 *)d_evecs;
-    auto prod = [&](const double2 *x, const SpmvEpi &e, int *nb, const int *run) {
-        return apply(h, precision, x, x32.as<float2>(), e, nb, run);
-    };
     // v_1: the seeded start vector, normalised
-    auto start = [&]() -> int {
-        hipLaunchKernelGGL(k_random_real, dim3(nbv), dim3(VB), 0, s, n, seed, r.v[0]);
+    auto start = [&](double2 *v) -> int {
+        hipLaunchKernelGGL(k_random_real, dim3(nbv), dim3(VB), 0, s, n, seed, v);
         EDX_LAUNCH_CHECK();
-        return r.begin();
+        double2 nn;
+        EDX_TRY(host_dot(L, v, v, &nn));
+        EDX_CHECK(nn.x > 0, EDX_ERR_NUMERIC, "zero start vector");
+        hipLaunchKernelGGL(k_scale_real, dim3(nbv), dim3(VB), 0, s, n, v, 1.0 / sqrt(nn.x));
+        EDX_LAUNCH_CHECK();
+        return EDX_OK;
+    };
+    auto product = [&](const double2 *v, double2 *w) -> int {
+        SpmvEpi e{};
+        e.y = w;
+        return apply(h, precision, v, x32.as<float2>(), e, nullptr, nullptr);
     };
     std::vector<double> al(maxiter), be(maxiter), ritz;
     int m = 0;
-    EDX_TRY(start());
-    for (int done = 0;;) {   // pass 1, from one test to the next
-        int next = (done / 10 + 1) * 10;
-        while (next < nev) next += 10;
-        next = std::min(next, maxiter);
-        for (int i = done + 1; i <= next; ++i) EDX_TRY(r.step(prod, i));
-        double norm = 0.0;
-        EDX_TRY(r.read(next, al.data(), be.data(), &m, &norm));
-        EDX_CHECK(norm > 0, EDX_ERR_NUMERIC, "zero start vector");
-        done = next;
-        const double beta = be[m - 1];
-        std::vector<double> wv(m), zl(m);
-        EDX_CHECK(edx::tridiag_ql(m, al.data(), be.data(), wv.data(), nullptr, zl.data()) == 0,
-                  EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
-        int nconv = 0;
-        for (int k = 0; k < std::min(nev, m); ++k)
-            if (fabs(beta * zl[k]) < tol) ++nconv;
-        if (nconv >= std::min(nev, m) || m < next || beta < 1e-10 || m == maxiter) break;
+    EDX_TRY(start(buf[1]));
+    {   // pass 1, from one test to the next; a breakdown is seen at the test
+        double2 *v[3] = {buf[0], buf[1], buf[2]};   // v[0] = v_{j-1}, v[1] = v_j, v[2] = w
+        for (int done = 0;;) {
+            int next = (done / 10 + 1) * 10;
+            while (next < nev) next += 10;
+            next = std::min(next, maxiter);
+            for (int j = done; j < next; ++j) {
+                EDX_TRY(product(v[1], v[2]));
+                hipLaunchKernelGGL(k_dot, dim3(nbv), dim3(VB), 0, s, n, v[1], v[2], pdot, nullptr);
+                hipLaunchKernelGGL(k_two_pass_first, dim3(nbv), dim3(VB), 0, s, n, v[2], v[1], pdot, nbv,
+                                   dal + j, j > 0 ? v[0] : nullptr, dbe + (j > 0 ? j - 1 : 0), pnorm);
+                // v_{j+1} = w / beta over v_{j-1}, which the next step no longer needs
+                hipLaunchKernelGGL(k_cgs_next, dim3(nbv), dim3(VB), 0, s, n, v[2], pnorm, nbv, dbe + j,
+                                   v[0]);
+                EDX_LAUNCH_CHECK();
+                std::swap(v[0], v[1]);
+            }
+            EDX_HIP(hipMemcpyAsync(al.data(), dal, next * sizeof(double), hipMemcpyDeviceToHost, s));
+            EDX_HIP(edx::copy_sync(be.data(), dbe, next * sizeof(double), hipMemcpyDeviceToHost));
+            m = next;
+            for (int j = done; j < next; ++j)
+                if (be[j] < 1e-10) {
+                    m = j + 1;
+                    break;
+                }
+            done = next;
+            const double beta = be[m - 1];
+            const bool last = beta < 1e-10 || m == maxiter;
+            std::vector<double> wv(m), zl(m);
+            EDX_CHECK(edx::tridiag_ql(m, al.data(), be.data(), wv.data(), nullptr, zl.data()) == 0,
+                      EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
+            int nconv = 0;
+            for (int k = 0; k < std::min(nev, m); ++k)
+                if (fabs(beta * zl[k]) < tol) ++nconv;
+            if (nconv >= std::min(nev, m) || last) break;
+        }
     }
     ritz.assign(m, 0.0);
     std::vector<double> S((size_t)m * m);   // row k: eigenvector k of the tridiagonal matrix
@@ -773,26 +803,22 @@ int lanczos_rerun_impl(const edx_csr *h, int precision, int nev, int maxiter, do
               EDX_ERR_NUMERIC, "tridiagonal eigensolver did not converge");
     for (int k = 0; k < nev; ++k) evals[k] = k < m ? ritz[k] : 0.0;
     if (nvec > 0) {   // pass 2
-        const int nk = std::min(nvec, m);
-        std::vector<double> c((size_t)nk * m);   // x_k += y_{j,k} v_j, v_j = u_j / beta_{j-1}
-        for (int k = 0; k < nk; ++k)
-            for (int j = 0; j < m; ++j)
-                c[(size_t)k * m + j] = S[(size_t)k * m + j] / (j ? be[j - 1] : 1.0);
-        EDX_TRY(coef.alloc(c.size() * sizeof(double), "ritz coefficients"));
-        EDX_HIP(edx::copy_sync(coef.p, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice));
         EDX_HIP(hipMemsetAsync(X, 0, (size_t)n * nvec * sizeof(double2), s));
-        EDX_TRY(start());
+        EDX_TRY(start(buf[1]));
+        const int nk = std::min(nvec, m);
+        double2 *v[3] = {buf[0], buf[1], buf[2]};   // v[0] = v_{j-1}, v[1] = v_j, v[2] = w
         for (int j = 0; j < m; ++j) {
-            for (int k = 0; k < nk; ++k)
-                hipLaunchKernelGGL(k_axpy_coef, dim3(nbv), dim3(VB), 0, s, n, X + (int64_t)k * n,
-                                   r.v[r.curr], coef.as<double>() + (size_t)k * m + j);
+            for (int k = j + 1 < m ? 1 : 0; k < nk; ++k)   // x_k += y_{j,k} v_j
+                hipLaunchKernelGGL(k_axpby_sub, dim3(nbv), dim3(VB), 0, s, n, X + (int64_t)k * n, v[1],
+                                   -S[(size_t)k * m + j], nullptr, 0.0);
             EDX_LAUNCH_CHECK();
-            if (j + 1 < m) EDX_TRY(r.step(prod, j + 1));
+            if (j + 1 == m) break;
+            EDX_TRY(product(v[1], v[2]));
+            hipLaunchKernelGGL(k_two_pass_again, dim3(nbv), dim3(VB), 0, s, n, v[2], v[1], al[j], v[0],
+                               j > 0, j > 0 ? be[j - 1] : 0.0, be[j], X, -S[j]);
+            EDX_LAUNCH_CHECK();
+            std::swap(v[0], v[1]);   // v_j becomes v_{j-1}, the new vector v_{j+1} sits in v[1]
         }
-        Lanczos L{};
-        L.n = n;
-        L.nbv = nbv;
-        L.part = r.k.part;
         for (int k = 0; k < nk; ++k) {   // unit norm
             double2 nn;
             EDX_TRY(host_dot(L, X + (int64_t)k * n, X + (int64_t)k * n, &nn));
