@@ -217,21 +217,21 @@ int tune_bspmm(const edx_csr *a, int precision, int K, BSched *sched) {
     // the pipelined RHS-parallel schedules for every K: a block compacted below
     // 8 vectors keeps them (lanes past K of each 16-lane group idle)
     for (int bpc : {4, 5, 8})   // workgroups per CU
-        if (bsched_blocks(a, BSched{2, bpc}) <= bspmm_blocks(a->m))
+        if (bsched_blocks(a, BSched{2, bpc}) <= bspmm_partials(a->m))
             cand.push_back(BSched{2, bpc});
     if (packed_spmm_ok(a, precision))   // the same over the packed words, table in LDS
         for (int bpc : {4, 5, 8})
-            if (bsched_blocks(a, BSched{4, bpc}) <= bspmm_blocks(a->m))
+            if (bsched_blocks(a, BSched{4, bpc}) <= bspmm_partials(a->m))
                 cand.push_back(BSched{4, bpc});
     if (fac_spmm_ok(a, precision, K))   // slot-factored, workgroups per CU
         for (int bpc : {4, 5, 6, 8})
-            if (bsched_blocks(a, BSched{3, bpc}) <= bspmm_blocks(a->m))
+            if (bsched_blocks(a, BSched{3, bpc}) <= bspmm_partials(a->m))
                 cand.push_back(BSched{3, bpc});
     const size_t nk = (size_t)a->n * K;
     double2 *X = (double2 *)dmalloc(nk * sizeof(double2), "tune X");
     float2 *X32 = precision == EDX_C64 ? (float2 *)dmalloc(nk * sizeof(float2), "tune X32") : nullptr;
     double2 *Y = (double2 *)dmalloc((size_t)a->m * K * sizeof(double2), "tune Y");
-    double2 *part = (double2 *)dmalloc((size_t)bspmm_blocks(a->m) * K * sizeof(double2), "tune partials");
+    double2 *part = (double2 *)dmalloc((size_t)bspmm_partials(a->m) * K * sizeof(double2), "tune partials");
     hipEvent_t ev[2] = {nullptr, nullptr};
     int rc = EDX_OK;
     BSched best = *sched;

@@ -388,8 +388,12 @@ int bspmm_blocks(int64_t m) {
     int64_t cap = (int64_t)edx::num_cus() * 8;
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
-    return (int)((blocks + 7) / 8 * 8);   // the XCD-contiguous schedules need a multiple of 8
+    return (int)blocks;
 }
+
+// Dot partials per right-hand side that callers provide: the XCD-contiguous
+// schedules launch a multiple of 8 workgroups.
+int bspmm_partials(int64_t m) { return (bspmm_blocks(m) + 7) / 8 * 8; }
 
 int pick_lanes(const edx_csr *a) {
     if (a->spmm_lanes) return a->spmm_lanes;
@@ -898,7 +902,7 @@ void forced_bsched(int K, BSched *sched) {
 
 // Workgroups (and dot partials per right-hand side) of a schedule's launch.
 // The pipelined and factored schedules need a multiple of 8 and at most
-// bspmm_blocks(m), the partials every caller provides; a matrix with fewer rows
+// bspmm_partials(m), which every caller provides; a matrix with fewer rows
 // than their grid would take gets a smaller one.
 int bsched_blocks(const edx_csr *a, BSched sched) {
     if (sched.rl == 3) return fac_spmm_blocks(a, sched.p);
@@ -922,18 +926,18 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
         if (!fac_spmm_ok(a, precision, K))
             return set_error(EDX_ERR_ARG, "the factored multi-RHS product needs the slot-factored "
                              "form, the indexed precision and 2 <= K <= 4");
-        if (bsched_blocks(a, sched) > nb)
+        if (bsched_blocks(a, sched) > bspmm_partials(a->m))
             return set_error(EDX_ERR_ARG, "factored SpMM needs %d workgroups, %d available",
-                             bsched_blocks(a, sched), nb);
+                             bsched_blocks(a, sched), bspmm_partials(a->m));
         return fac_spmm_launch(a, K, X64, e, sched.p);
     }
     if (sched.rl == 4) {   // packed words, value table in LDS, sched.p workgroups per CU
         if (!packed_spmm_ok(a, precision))
             return set_error(EDX_ERR_ARG, "multi-RHS schedule 4 needs the packed indexed form");
         const int nbp = bsched_blocks(a, sched);
-        if (nbp > nb)
+        if (nbp > bspmm_partials(a->m))
             return set_error(EDX_ERR_ARG, "pipelined SpMM needs %d workgroups, %d available", nbp,
-                             nb);
+                             bspmm_partials(a->m));
         dim3 grid((unsigned)nbp, (unsigned)((K + 15) / 16));
         hipLaunchKernelGGL((k_spmm_rlp<PkPtr, double2, double, true, true>), grid, dim3(256),
                            (size_t)a->nvtab * sizeof(double2), stream(), a->m, K, a->d_off_rowptr,
@@ -941,9 +945,9 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
                            (int)a->nvtab);
     } else if (sched.rl == 2) {   // pipelined RHS-parallel, sched.p workgroups per CU
         const int nbp = bsched_blocks(a, sched);
-        if (nbp > nb)
+        if (nbp > bspmm_partials(a->m))
             return set_error(EDX_ERR_ARG, "pipelined SpMM needs %d workgroups, %d available", nbp,
-                             nb);
+                             bspmm_partials(a->m));
         dim3 grid((unsigned)nbp, (unsigned)((K + 15) / 16));
         if (precision == EDX_C128)
             hipLaunchKernelGGL((k_spmm_rlp<const double2 *, double2, double, false>), grid,
@@ -1043,10 +1047,13 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
 
 // The schedule the mean row length and K suggest (used below TUNE_MIN_ROWS
 // rows, where products are too short to time).
-BSched bspmm_rule(const edx_csr *a, int precision, int K) {
-    // a few vectors over the slot-factored form: an H_v entry is read once for
-    // its six rows (K = 3 over 68,640 rows: 24 us, row-split 43 us)
-    if (fac_spmm_ok(a, precision, K)) return BSched{3, 4};
+BSched bspmm_rule(const edx_csr *a, int precision, int K, const BEpi &e) {
+    // A few vectors over the slot-factored form: an H_v entry is read once for
+    // its six rows (K = 3 over 68,640 rows: 24 us, row-split 43 us).  Solves that
+    // stop at a tolerance (shifts in the epilogue or the tail) keep the row-split
+    // sums: where they stop, and so their solutions to 1e-9, hangs on the last bits.
+    const bool solve = e.c2 || e.tail.nshift;
+    if (!solve && fac_spmm_ok(a, precision, K)) return BSched{3, 4};
     if (K >= 8) {
         const int kp = K < RL_MAXK ? K : RL_MAXK;
         return BSched{1, kp <= 16 ? 1 : (kp <= 32 ? 2 : (kp <= 64 ? 4 : 8))};
@@ -1078,7 +1085,7 @@ int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const floa
     }
     if (nblocks_out) *nblocks_out = bspmm_blocks(a->m);
     if (a->m == 0 || K == 0) return EDX_OK;
-    BSched sched = bspmm_rule(a, precision, K);
+    BSched sched = bspmm_rule(a, precision, K, e_in);
     if (a->m >= TUNE_MIN_ROWS) EDX_TRY(tune_bspmm(a, precision, K, &sched));
     forced_bsched(K, &sched);
     if (sched.rl == 3 && !fac_spmm_ok(a, precision, K))
@@ -1443,7 +1450,7 @@ int kb_start(edx_krylov_batch *q, const double2 *V0cm, int cap) {
     EDX_TRY(q->vb.alloc((size_t)2 * n * K * sizeof(double2), "batched krylov vectors"));
     if (q->precision == EDX_C64)
         EDX_TRY(q->x32.alloc((size_t)n * K * sizeof(float2), "batched x32"));
-    const int nbs = bspmm_blocks(n), nbe = elem_grid_x(n);
+    const int nbs = bspmm_partials(n), nbe = elem_grid_x(n);
     EDX_TRY(q->part.alloc(std::max<size_t>((size_t)std::max(nbs, nbe) * K + 64,
                                            (size_t)edx::spmv_partials_len(q->h)) * sizeof(double2),
                           "partials"));
@@ -1648,7 +1655,7 @@ int bminres_run(const edx_csr *h, int precision, int K, const double2 *sigma, co
     const size_t nk = (size_t)n * K;
     EDX_TRY(vb.alloc(6 * nk * sizeof(double2), "batched minres vectors"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(nk * sizeof(float2), "batched x32"));
-    const int nbs = bspmm_blocks(n), nbe = elem_grid_x(n);
+    const int nbs = bspmm_partials(n), nbe = elem_grid_x(n);
     EDX_TRY(part.alloc((size_t)std::max(nbs, nbe) * K * sizeof(double2) + 64, "partials"));
     const int nvec_scalars = 14;
     EDX_TRY(sc.alloc((size_t)K * (nvec_scalars * sizeof(double2) + sizeof(double)), "minres scalars"));

@@ -499,7 +499,7 @@ int shifted_fom_batch_run(const edx_csr *h, int precision, int R, const double2 
     Dbuf vb, x32, part, sc, flags, shb, ctlb, qb, wb, slb, nrm, cntb;
     EDX_TRY(vb.alloc(2 * nr * sizeof(double2), "batched fom lanczos vectors"));
     if (precision == EDX_C64) EDX_TRY(x32.alloc(nr * sizeof(float2), "batched fom x32"));
-    const int nbs = bspmm_blocks(n), nbe = elem_grid_x(n);
+    const int nbs = bspmm_partials(n), nbe = elem_grid_x(n);
     EDX_TRY(part.alloc(std::max<size_t>((size_t)std::max(nbs, nbe) * R + 64,
                                         (size_t)edx::spmv_partials_len(h)) * sizeof(double2),
                        "partials"));
