@@ -80,8 +80,8 @@ __device__ __forceinline__ double2 shfl16(double2 v, int src) {
 
 // Pipelined RHS-parallel schedule: 16-lane groups own rows and lane l owns
 // right-hand side blockIdx.y * 16 + l, as in k_spmm_rl, on a capped grid whose
-// workgroups of one XCD (blockIdx.x % 8) walk one contiguous eighth of the
-// rows.  Lane l holds the column and value numbers of nonzeros l and l + 16 of
+// workgroups of one XCD (blockIdx.x % 8) walk one contiguous eighth of each
+// part of the rows (bspmm_part).  Lane l holds the column and value numbers of nonzeros l and l + 16 of
 // its group's row (one coalesced load per row instead of a broadcast per
 // nonzero), hands them to the group by shuffles while each lane gathers its own
 // right-hand side, and loads those of the group's next row first.  Nonzeros
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void k_spmm_rlp(int64_t m, int K, const int64_
                                                   const double2 *__restrict__ diag,
                                                   const XT *__restrict__ X,
                                                   const double2 *__restrict__ X64, BEpi e,
-                                                  int ntab = 0) {
+                                                  int64_t part, int ntab = 0) {
     using PV = PipeVal<VP>;
     using H = typename PV::type;
     __shared__ double2 red[16 * 16];
@@ -111,97 +111,99 @@ __global__ __launch_bounds__(256) void k_spmm_rlp(int64_t m, int K, const int64_
     const int k = blockIdx.y * 16 + l;
     const bool kv = k < K;
     const int64_t per_x = gridDim.x / 8, xcd = blockIdx.x % 8, w = blockIdx.x / 8;
-    const int64_t rows_x = (m + 7) / 8;
-    const int64_t rbeg = xcd * rows_x, rend = min(m, rbeg + rows_x);
     const int64_t stride = per_x * 16;
     double2 dot = make_double2(0, 0);
-    int64_t r = rbeg + w * 16 + grp;
-    int64_t b = 0, end = 0;
-    if (r < rend) {
-        b = rowptr[r];
-        end = rowptr[r + 1];
-    }
-    int ca, cb;
-    H ha, hb;
-    PV::fetch(cols, vals, b + l, b + l < end, ca, ha);
-    PV::fetch(cols, vals, b + 16 + l, b + 16 + l < end, cb, hb);
-    while (__any(r < rend)) {
-        const int64_t rn = r + stride;
-        int64_t bn = 0, endn = 0;
-        if (rn < rend) {
-            bn = rowptr[rn];
-            endn = rowptr[rn + 1];
-        }
-        int can, cbn;
-        H han, hbn;
-        PV::fetch(cols, vals, bn + l, bn + l < endn, can, han);
-        PV::fetch(cols, vals, bn + 16 + l, bn + 16 + l < endn, cbn, hbn);
+    for (int64_t c0 = 0; c0 < m; c0 += part) {
+        const int64_t cend = min(m, c0 + part), rows_x = (cend - c0 + 7) / 8;
+        const int64_t rbeg = c0 + xcd * rows_x, rend = min(cend, rbeg + rows_x);
+        int64_t r = rbeg + w * 16 + grp;
+        int64_t b = 0, end = 0;
         if (r < rend) {
-            ACC sr = 0, si = 0;
-            const int cnt = (int)(end - b);
-            const int nf = cnt < 32 ? cnt : 32;
-            // four nonzeros at a time: their columns and values by shuffles,
-            // then four gathers in flight before the sums (in nonzero order)
-            int t = 0;
-            for (; t + 4 <= nf; t += 4) {
-                int c[4];
-                decltype(value(ha)) a[4];
-                XT xv[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int tt = t + u, src = tt & 15;
-                    c[u] = __shfl(tt < 16 ? ca : cb, src, 16);
-                    a[u] = value(shfl16(tt < 16 ? ha : hb, src));
-                }
-                if (kv) {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) xv[u] = X[(int64_t)c[u] * K + k];
+            b = rowptr[r];
+            end = rowptr[r + 1];
+        }
+        int ca, cb;
+        H ha, hb;
+        PV::fetch(cols, vals, b + l, b + l < end, ca, ha);
+        PV::fetch(cols, vals, b + 16 + l, b + 16 + l < end, cb, hb);
+        while (__any(r < rend)) {
+            const int64_t rn = r + stride;
+            int64_t bn = 0, endn = 0;
+            if (rn < rend) {
+                bn = rowptr[rn];
+                endn = rowptr[rn + 1];
+            }
+            int can, cbn;
+            H han, hbn;
+            PV::fetch(cols, vals, bn + l, bn + l < endn, can, han);
+            PV::fetch(cols, vals, bn + 16 + l, bn + 16 + l < endn, cbn, hbn);
+            if (r < rend) {
+                ACC sr = 0, si = 0;
+                const int cnt = (int)(end - b);
+                const int nf = cnt < 32 ? cnt : 32;
+                // four nonzeros at a time: their columns and values by shuffles,
+                // then four gathers in flight before the sums (in nonzero order)
+                int t = 0;
+                for (; t + 4 <= nf; t += 4) {
+                    int c[4];
+                    decltype(value(ha)) a[4];
+                    XT xv[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        sr += (ACC)a[u].x * (ACC)xv[u].x - (ACC)a[u].y * (ACC)xv[u].y;
-                        si += (ACC)a[u].x * (ACC)xv[u].y + (ACC)a[u].y * (ACC)xv[u].x;
+                        const int tt = t + u, src = tt & 15;
+                        c[u] = __shfl(tt < 16 ? ca : cb, src, 16);
+                        a[u] = value(shfl16(tt < 16 ? ha : hb, src));
+                    }
+                    if (kv) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) xv[u] = X[(int64_t)c[u] * K + k];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            sr += (ACC)a[u].x * (ACC)xv[u].x - (ACC)a[u].y * (ACC)xv[u].y;
+                            si += (ACC)a[u].x * (ACC)xv[u].y + (ACC)a[u].y * (ACC)xv[u].x;
+                        }
                     }
                 }
-            }
-            for (; t < nf; ++t) {
-                const int src = t & 15;
-                const int c = __shfl(t < 16 ? ca : cb, src, 16);
-                const auto a = value(shfl16(t < 16 ? ha : hb, src));
+                for (; t < nf; ++t) {
+                    const int src = t & 15;
+                    const int c = __shfl(t < 16 ? ca : cb, src, 16);
+                    const auto a = value(shfl16(t < 16 ? ha : hb, src));
+                    if (kv) {
+                        const XT xv = X[(int64_t)c * K + k];
+                        sr += (ACC)a.x * (ACC)xv.x - (ACC)a.y * (ACC)xv.y;
+                        si += (ACC)a.x * (ACC)xv.y + (ACC)a.y * (ACC)xv.x;
+                    }
+                }
+                for (int64_t j = b + 32; j < end; ++j) {
+                    int c;
+                    H h;
+                    PV::fetch(cols, vals, j, true, c, h);
+                    const auto a = value(h);
+                    if (kv) {
+                        const XT xv = X[(int64_t)c * K + k];
+                        sr += (ACC)a.x * (ACC)xv.x - (ACC)a.y * (ACC)xv.y;
+                        si += (ACC)a.x * (ACC)xv.y + (ACC)a.y * (ACC)xv.x;
+                    }
+                }
                 if (kv) {
-                    const XT xv = X[(int64_t)c * K + k];
-                    sr += (ACC)a.x * (ACC)xv.x - (ACC)a.y * (ACC)xv.y;
-                    si += (ACC)a.x * (ACC)xv.y + (ACC)a.y * (ACC)xv.x;
+                    // single-use operands and the output non-temporal, so the
+                    // reused lines of X stay in L2 (2 % faster, K=16 over H_i)
+                    const int64_t o = r * K + k;
+                    double2 hx = make_double2((double)sr, (double)si);
+                    if (SPLIT) hx = cadd(hx, cmul(nt_load2(diag + r), X64[o]));
+                    const double2 out = epilogue_nt(e, k, o, hx, X64);
+                    nt_store2(e.y + o, out);
+                    if (e.dvec) dot = cadd(dot, cconjmul(nt_load2(e.dvec + o), out));
                 }
             }
-            for (int64_t j = b + 32; j < end; ++j) {
-                int c;
-                H h;
-                PV::fetch(cols, vals, j, true, c, h);
-                const auto a = value(h);
-                if (kv) {
-                    const XT xv = X[(int64_t)c * K + k];
-                    sr += (ACC)a.x * (ACC)xv.x - (ACC)a.y * (ACC)xv.y;
-                    si += (ACC)a.x * (ACC)xv.y + (ACC)a.y * (ACC)xv.x;
-                }
-            }
-            if (kv) {
-                // single-use operands and the output non-temporal, so the
-                // reused lines of X stay in L2 (2 % faster, K=16 over H_i)
-                const int64_t o = r * K + k;
-                double2 hx = make_double2((double)sr, (double)si);
-                if (SPLIT) hx = cadd(hx, cmul(nt_load2(diag + r), X64[o]));
-                const double2 out = epilogue_nt(e, k, o, hx, X64);
-                nt_store2(e.y + o, out);
-                if (e.dvec) dot = cadd(dot, cconjmul(nt_load2(e.dvec + o), out));
-            }
+            r = rn;
+            b = bn;
+            end = endn;
+            ca = can;
+            cb = cbn;
+            ha = han;
+            hb = hbn;
         }
-        r = rn;
-        b = bn;
-        end = endn;
-        ca = can;
-        cb = cbn;
-        ha = han;
-        hb = hbn;
     }
     if (e.dvec) {
         red[grp * 16 + l] = dot;
@@ -919,9 +921,22 @@ int bsched_passes(int K, BSched sched) {
     return sched.rl ? (K + 15) / 16 : (K + BKT - 1) / BKT;
 }
 
+// Whether the capped grids walk a matrix in parts of a few passes, all XCDs in
+// the same part, instead of an eighth of it each.  Partners a moved electron
+// away then meet in the last-level cache, which eight far windows overflow once
+// the block of vectors is larger than it (256 MB): K = 3 over 15.0M core-hole
+// rows (719 MB) 2.31 ms for 2.40, K = 16 over 2.7M rows (692 MB) 1.16 for 1.19.
+// Solves keep the one order at every size (bspmm_rule).
+bool bspmm_part(const edx_csr *a, int K, const BEpi &e) {
+    return !e.c2 && !e.tail.nshift && a->m * K * 16 > ((int64_t)256 << 20);
+}
+
 int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, const float2 *X32,
                  const BEpi &e, BSched sched) {
     const int nb = bspmm_blocks(a->m);
+    // k_spmm_rlp's: eight passes of 16 rows a workgroup
+    const int64_t part = bspmm_part(a, K, e) ? (int64_t)bsched_blocks(a, sched) * 16 * 8
+                                             : std::max<int64_t>(a->m, 1);
     if (sched.rl == 3) {   // slot-factored, sched.p workgroups per CU
         if (!fac_spmm_ok(a, precision, K))
             return set_error(EDX_ERR_ARG, "the factored multi-RHS product needs the slot-factored "
@@ -941,7 +956,7 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
         dim3 grid((unsigned)nbp, (unsigned)((K + 15) / 16));
         hipLaunchKernelGGL((k_spmm_rlp<PkPtr, double2, double, true, true>), grid, dim3(256),
                            (size_t)a->nvtab * sizeof(double2), stream(), a->m, K, a->d_off_rowptr,
-                           nullptr, PkPtr{a->d_off_pk, a->d_vtab}, a->d_diag, X64, X64, e,
+                           nullptr, PkPtr{a->d_off_pk, a->d_vtab}, a->d_diag, X64, X64, e, part,
                            (int)a->nvtab);
     } else if (sched.rl == 2) {   // pipelined RHS-parallel, sched.p workgroups per CU
         const int nbp = bsched_blocks(a, sched);
@@ -952,19 +967,19 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
         if (precision == EDX_C128)
             hipLaunchKernelGGL((k_spmm_rlp<const double2 *, double2, double, false>), grid,
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,
-                               (const double2 *)a->d_vals, nullptr, X64, X64, e);
+                               (const double2 *)a->d_vals, nullptr, X64, X64, e, part);
         else if (precision == EDX_C64)
             hipLaunchKernelGGL((k_spmm_rlp<const float2 *, float2, float, false>), grid, dim3(256),
                                0, stream(), a->m, K, a->d_rowptr, a->d_cols,
-                               (const float2 *)a->d_vals32, nullptr, X32, X64, e);
+                               (const float2 *)a->d_vals32, nullptr, X32, X64, e, part);
         else if (precision == EDX_C128I)
             hipLaunchKernelGGL((k_spmm_rlp<IdxPtr, double2, double, true>), grid, dim3(256), 0,
                                stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,
-                               IdxPtr{a->d_off_idx, a->d_vtab}, a->d_diag, X64, X64, e);
+                               IdxPtr{a->d_off_idx, a->d_vtab}, a->d_diag, X64, X64, e, part);
         else
             hipLaunchKernelGGL((k_spmm_rlp<const float2 *, double2, double, true>), grid,
                                dim3(256), 0, stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,
-                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e);
+                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e, part);
     } else if (sched.rl) {
         const int npl = sched.p;
         dim3 grid((unsigned)nb, (unsigned)((K + 16 * npl - 1) / (16 * npl)));

@@ -367,10 +367,12 @@ __global__ __launch_bounds__(256, WPE) void k_spmv_fac(FacArgs f, const double2 
 // k_spmv_fac computes its row for all K right-hand sides, so an H_v entry
 // gathers NC K 16-byte values contiguous over the valence row's lanes and an
 // R entry K contiguous values.  A capped grid (a multiple of 8 workgroups)
-// walks XCD-contiguous eighths of the valence rows, 4 (64 / NC) valence rows
-// per workgroup per pass; dot partials per workgroup and right-hand side.
+// walks the valence rows part after part (bspmm_part), XCD-contiguous eighths
+// of each, 4 (64 / NC) valence rows per workgroup per pass; dot partials per
+// workgroup and right-hand side.
 template <int NC, int K, bool TAIL>
-__global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__restrict__ X, BEpi e) {
+__global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__restrict__ X, BEpi e,
+                                                  int64_t part) {
     extern __shared__ double2 s_tab[];
     __shared__ double2 red[4][K];
     const uint64_t *s_typ = fac_stage_lds(f, s_tab);
@@ -378,12 +380,12 @@ __global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__re
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int vl = lane / NC, s = lane - vl * NC;
     const int64_t per_x = gridDim.x / 8, xcd = blockIdx.x % 8, wg = blockIdx.x / 8;
-    const int64_t vrows_x = (f.mv + 7) / 8;
-    const int64_t vbeg = xcd * vrows_x, vend = min(f.mv, vbeg + vrows_x);
     double2 dot[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) dot[k] = make_double2(0, 0);
-    if (vl < VPW) {
+    for (int64_t c0 = 0; vl < VPW && c0 < f.mv; c0 += part) {
+        const int64_t cend = min(f.mv, c0 + part), vrows_x = (cend - c0 + 7) / 8;
+        const int64_t vbeg = c0 + xcd * vrows_x, vend = min(cend, vbeg + vrows_x);
         for (int64_t v = vbeg + (wg * 4 + wave) * VPW + vl; v < vend; v += per_x * 4 * VPW) {
             const int64_t r = v * NC + s;
             double sr[K], si[K];
@@ -564,15 +566,17 @@ int fac_spmm_launch(const edx_csr *a, int K, const double2 *X, const BEpi &e, in
     const int nb = fac_spmm_blocks(a, bpc);
     const FacArgs f = fac_args(a);
     const size_t lds = fac_lds_bytes(a);
+    const int64_t mv = a->m / a->nc_slots, pass = fac_rows_per_block(a->nc_slots) * nb;
+    const int64_t part = bspmm_part(a, K, e) ? 4 * pass : std::max<int64_t>(mv, 1);
     if (a->m == 0) return EDX_OK;
 #define EDX_FAC_CASE(KK)                                                                          \
     case KK:                                                                                      \
         if (e.tail.count)                                                                         \
             hipLaunchKernelGGL((k_spmm_fac<6, KK, true>), dim3(nb), dim3(256), lds, stream(), f, X, \
-                               e);                                                                \
+                               e, part);                                                                \
         else                                                                                      \
             hipLaunchKernelGGL((k_spmm_fac<6, KK, false>), dim3(nb), dim3(256), lds, stream(), f, X, \
-                               e);                                                                \
+                               e, part);                                                                \
         break;
     switch (K) {
         EDX_FAC_CASE(2)
