@@ -5,7 +5,7 @@
 // over its own request's matrix, started and finished at different times.
 // Launched one by one, each of their products is a few microseconds of work
 // behind a launch; here every step of every live member is ONE SpMV launch,
-// one vector launch and three tiny reductions, whatever the number of members.
+// one vector launch and two tiny reductions, whatever the number of members.
 //
 // Each member is a build_krylov_mp recurrence (src/lanczos.f90:266-298) on one
 // vector.  Its rows map to a contiguous range of the SpMV grid (32 rows per
@@ -31,8 +31,13 @@ constexpr int G_VEC = 1024;              // vector elements per vector block
 constexpr int64_t G_PIPE_MIN_ROWS = 65536;   // members this large take the pipelined SpMV
 constexpr int GP_G = 4, GP_U = 8;            // its lanes per row and prefetched nonzeros per lane
 
+// As in the batched recurrence (BKrylov), the stored vector is u_i = s_i v_i, the
+// residual of the step before, and no pass divides it: the product is
+// y = c0 H u_i + c1 u_{i-1}, alpha_i = c0 <u_i|y>, u_{i+1} = y - c0 alpha_i u_i.
+// (Seven members over up to 1.0M rows: a step 280 us, with the division 300.)
 struct GState {
-    double2 c1;      // -beta of the last step (addend scale of the next product)
+    double2 c1;      // -beta_i / s_{i-1}
+    double c0, s;    // 1 / s_i, s_i (beta_i; 1 at the start)
     double norm;     // <v0|v0>
     int run;         // recurrence still going
     int steps;       // steps done; parity selects the current vector
@@ -87,14 +92,14 @@ __device__ __forceinline__ IdxPtr g_vals<IdxPtr>(const GMember &M) {
     return IdxPtr{M.idx, M.tab};
 }
 
-// A large member's product y = H x + c1 y in the pipelined schedule of
+// A large member's product y = c0 H x + c1 y in the pipelined schedule of
 // k_spmv_pipe: the member's nblk workgroups (a multiple of 8, starting at a
 // multiple of 8) split its rows into XCD-contiguous eighths and walk them
 // grid-stride; each lane loads its next row's GP_U column/value numbers and
 // epilogue operands before it gathers x for the current row.  Returns this
 // thread's share of <x|y>.
 template <class VP, bool SPLIT>
-__device__ double2 g_spmv_pipe(const GMember &M, VP vals, const double2 *s_tab, double2 c1,
+__device__ double2 g_spmv_pipe(const GMember &M, VP vals, const double2 *s_tab, double c0, double2 c1,
                                const double2 *__restrict__ x, double2 *y, int64_t l) {
     using PV = PipeVal<VP>;
     using Hd = typename PV::type;
@@ -179,7 +184,7 @@ __device__ double2 g_spmv_pipe(const GMember &M, VP vals, const double2 *s_tab, 
         if (r < rend && lig == 0) {
             double2 ax = make_double2(sr, si);
             if constexpr (SPLIT) ax = cadd(ax, cmul(pd, px));
-            const double2 out = cadd(ax, cmul(c1, py));
+            const double2 out = cadd(cscale(ax, c0), cmul(c1, py));
             y[r] = out;
             dot = cadd(dot, cconjmul(px, out));
         }
@@ -198,11 +203,11 @@ __device__ double2 g_spmv_pipe(const GMember &M, VP vals, const double2 *s_tab, 
     return dot;
 }
 
-// A factored member's product y = H x + c1 y over its 64 / NC valence rows per
+// A factored member's product y = c0 H x + c1 y over its 64 / NC valence rows per
 // wave (the product of k_spmv_fac): block l of the member takes valence rows
 // 4 (64 / NC) l ... + 4 (64 / NC) - 1.  Returns this thread's share of <x|y>.
 template <int NC>
-__device__ double2 g_spmv_fac(const GMember &M, const double2 *s_tab, const uint64_t *s_typ, double2 c1,
+__device__ double2 g_spmv_fac(const GMember &M, const double2 *s_tab, const uint64_t *s_typ, double c0, double2 c1,
                               const double2 *__restrict__ x, double2 *y, int64_t l) {
     constexpr int VPW = 64 / NC;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -214,7 +219,7 @@ __device__ double2 g_spmv_fac(const GMember &M, const double2 *s_tab, const uint
         const int64_t r = v * NC + s;
         const double2 dg = M.diag[r], xr = x[r], yr = y[r];
         const double2 ax = cadd(fac_offdiag_sum<NC, 8>(M.fa, x, s_tab, s_typ, v, s, r), cmul(dg, xr));
-        const double2 out = cadd(ax, cmul(c1, yr));
+        const double2 out = cadd(cscale(ax, c0), cmul(c1, yr));
         y[r] = out;
         dot = cconjmul(xr, out);
     }
@@ -237,7 +242,7 @@ __global__ __launch_bounds__(256) void k_gspmv(const GMember *mem, int nmem, dou
         if (M.fac == 6) {   // the member's value table and block types in LDS, then the factored product
             extern __shared__ double2 s_tab[];
             const uint64_t *s_typ = fac_stage_lds(M.fa, s_tab);
-            double2 dot = g_spmv_fac<6>(M, s_tab, s_typ, st.c1, x, y, bid - M.blk0);
+            double2 dot = g_spmv_fac<6>(M, s_tab, s_typ, st.c0, st.c1, x, y, bid - M.blk0);
             dot = block_sum_256(dot);
             if (threadIdx.x == 0) partials[bid] = dot;
             return;
@@ -256,11 +261,11 @@ __global__ __launch_bounds__(256) void k_gspmv(const GMember *mem, int nmem, dou
         double2 dot;
         if constexpr (std::is_same<VP, IdxPtr>::value) {
             if (M.pk)
-                dot = g_spmv_pipe<PkPtr, SPLIT>(M, PkPtr{M.pk, M.tab}, s_tab, st.c1, x, y, l);
+                dot = g_spmv_pipe<PkPtr, SPLIT>(M, PkPtr{M.pk, M.tab}, s_tab, st.c0, st.c1, x, y, l);
             else
-                dot = g_spmv_pipe<VP, SPLIT>(M, g_vals<VP>(M), s_tab, st.c1, x, y, l);
+                dot = g_spmv_pipe<VP, SPLIT>(M, g_vals<VP>(M), s_tab, st.c0, st.c1, x, y, l);
         } else {
-            dot = g_spmv_pipe<VP, SPLIT>(M, g_vals<VP>(M), s_tab, st.c1, x, y, l);
+            dot = g_spmv_pipe<VP, SPLIT>(M, g_vals<VP>(M), s_tab, st.c0, st.c1, x, y, l);
         }
         dot = block_sum_256(dot);
         if (threadIdx.x == 0) partials[bid] = dot;
@@ -286,7 +291,7 @@ __global__ __launch_bounds__(256) void k_gspmv(const GMember *mem, int nmem, dou
         if (lig == 0) {
             double2 ax = make_double2(sr, si);
             if constexpr (SPLIT) ax = cadd(ax, cmul(M.diag[r], x[r]));
-            const double2 out = cadd(ax, cmul(st.c1, y[r]));
+            const double2 out = cadd(cscale(ax, st.c0), cmul(st.c1, y[r]));
             y[r] = out;
             dot = cconjmul(x[r], out);
         }
@@ -295,17 +300,17 @@ __global__ __launch_bounds__(256) void k_gspmv(const GMember *mem, int nmem, dou
     if (threadIdx.x == 0) partials[bid] = dot;
 }
 
-// alpha_i = Re <x|y> over the member's SpMV blocks (src/lanczos.f90:277-281)
+// alpha_i = c0 Re <x|y> over the member's SpMV blocks (src/lanczos.f90:277-281)
 __global__ __launch_bounds__(256) void k_galpha(const GMember *mem, const double2 *partials) {
     const GMember M = mem[blockIdx.x];
     if (!M.st->run) return;
     double2 s = make_double2(0, 0);
     for (int64_t b = threadIdx.x; b < M.nblk; b += 256) s = cadd(s, partials[M.blk0 + b]);
     s = block_sum_256(s);
-    if (threadIdx.x == 0) M.alpha[M.st->steps] = s.x;
+    if (threadIdx.x == 0) M.alpha[M.st->steps] = s.x * M.st->c0;
 }
 
-// y -= alpha x; partial |y|^2 per vector block
+// y -= c0 alpha x; partial |y|^2 per vector block
 __global__ __launch_bounds__(256) void k_gaxpy(const GMember *mem, int nmem, double2 *vpartials) {
     const int64_t bid = blockIdx.x;
     const GMember M = mem[g_find(mem, nmem, bid, true)];
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(256) void k_gaxpy(const GMember *mem, int nmem, dou
     }
     const double2 *x = (st.steps & 1) ? M.v1 : M.v0;
     double2 *y = (st.steps & 1) ? M.v0 : M.v1;
-    const double al = M.alpha[st.steps];
+    const double al = M.alpha[st.steps] * st.c0;
     const int64_t base = (bid - M.vblk0) * G_VEC;
     double2 s = make_double2(0, 0);
     for (int t = threadIdx.x; t < G_VEC; t += 256) {
@@ -343,25 +348,12 @@ __global__ __launch_bounds__(256) void k_gbeta(const GMember *mem, const double2
         GState st = *M.st;
         const double b = sqrt(s.x);
         M.beta[st.steps] = b;
-        st.c1 = make_double2(-b, -0.0);
+        st.c1 = make_double2(-b / st.s, -0.0);
+        st.s = b;
+        st.c0 = b > 0.0 ? 1.0 / b : 0.0;
         st.steps += 1;
         st.run = (fabs(b) >= 1e-10 && st.steps < cap) ? 1 : 0;
         *M.st = st;
-    }
-}
-
-// the new current vector /= beta (members still running)
-__global__ __launch_bounds__(256) void k_gdiv(const GMember *mem, int nmem) {
-    const int64_t bid = blockIdx.x;
-    const GMember M = mem[g_find(mem, nmem, bid, true)];
-    const GState st = *M.st;
-    if (!st.run) return;
-    double2 *v = (st.steps & 1) ? M.v1 : M.v0;
-    const double b = M.beta[st.steps - 1];
-    const int64_t base = (bid - M.vblk0) * G_VEC;
-    for (int t = threadIdx.x; t < G_VEC; t += 256) {
-        const int64_t i = base + t;
-        if (i < M.m) v[i] = make_double2(v[i].x / b, v[i].y / b);
     }
 }
 
@@ -373,6 +365,7 @@ __global__ __launch_bounds__(256) void k_ginit(const double2 *partials, int nb, 
     if (threadIdx.x == 0) {
         GState g;
         g.c1 = make_double2(-0.0, -0.0);
+        g.c0 = g.s = 1.0;
         g.norm = s.x;
         g.run = s.x > 0.0 ? 1 : 0;
         g.steps = 0;
@@ -463,7 +456,6 @@ int group_step(edx_group *g, hipStream_t s) {
     hipLaunchKernelGGL(k_gaxpy, dim3((unsigned)g->nvblk), dim3(256), 0, s, g->d_mem, nmem,
                        g->vpartials);
     hipLaunchKernelGGL(k_gbeta, dim3(nmem), dim3(256), 0, s, g->d_mem, g->vpartials, g->cap);
-    hipLaunchKernelGGL(k_gdiv, dim3((unsigned)g->nvblk), dim3(256), 0, s, g->d_mem, nmem);
     EDX_LAUNCH_CHECK();
     return EDX_OK;
 }
