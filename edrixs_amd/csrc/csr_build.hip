@@ -14,7 +14,7 @@
 //   * k_plan_count / k_plan_fill (termplan.hip), for complete bases: 64 rows per
 //     workgroup over the terms grouped by column;
 //   * k_build, for incomplete bases (columns found by search), more than 4096
-//     terms, or rows longer than the plan kernels' LDS lists (255 entries, about 185
+//     terms, few terms on few rows (BUILD_TINY_ROWS), or rows longer than the plan kernels' LDS lists (255 entries, about 185
 //     with words of more than 32 bits): one 64-lane wavefront per row.  Lanes
 //     evaluate 64 terms at a time; survivors are compacted with a ballot into an
 //     LDS list that stays in term order; the list is bitonic-sorted on the key
@@ -477,6 +477,10 @@ int build_by_term(BuildParams p, TermTable &tt, BuildOut &o) {
     return EDX_OK;
 }
 
+// Few terms on few rows: grouping the terms costs more than it saves (362
+// terms: 495 rows 161 us, over the plan 165; 924 rows 172 and 161).
+constexpr int BUILD_TINY_ROWS = 512, BUILD_TINY_TERMS = 512;
+
 template <int RK, int CK>
 int build_csr(BuildParams p, const edx_basis *left, const edx_basis *right, TermTable &tt,
               int64_t ncols, int precision, edx_csr **out) {
@@ -493,7 +497,8 @@ int build_csr(BuildParams p, const edx_basis *left, const edx_basis *right, Term
     if (!o.rowptr || !o.flag) return EDX_ERR_NOMEM;
     const PlanSpaces sp{RK, CK, p.nv, p.nc, left, right};
     bool done = false;
-    if (p.M > 0 && plan_usable(sp, tt.ops.data(), tt.nhop, tt.T)) {
+    const bool tiny = p.M <= BUILD_TINY_ROWS && tt.T <= BUILD_TINY_TERMS;
+    if (p.M > 0 && !tiny && plan_usable(sp, tt.ops.data(), tt.nhop, tt.T)) {
         if (plan_bits(sp) <= 32) EDX_TRY((build_by_plan<RK, CK, uint32_t>(p, sp, tt, o, &done)));
         else EDX_TRY((build_by_plan<RK, CK, uint64_t>(p, sp, tt, o, &done)));
     }

@@ -52,7 +52,8 @@ def _terms(n, seed, nnz_u, density=0.5):
 
 
 @pytest.mark.parametrize("nbits,nocc", [(1, 0), (1, 1), (5, 5), (6, 1), (8, 4), (12, 6), (31, 2),
-                                        (32, 2), (33, 2), (40, 1), (62, 1)])
+                                        (32, 2), (33, 2), (40, 1), (62, 1),
+                                        (11, 5), (15, 12), (31, 3), (32, 3), (33, 3)])
 def test_plain_builds_at_word_and_workgroup_edges(core, nbits, nocc):
     ht, ut = _terms(min(nbits, 14), nbits, 60)
     if nbits > 14:       # spread the orbitals over the whole word
