@@ -34,7 +34,7 @@ constexpr int GP_G = 4, GP_U = 8;            // its lanes per row and prefetched
 // As in the batched recurrence (BKrylov), the stored vector is u_i = s_i v_i, the
 // residual of the step before, and no pass divides it: the product is
 // y = c0 H u_i + c1 u_{i-1}, alpha_i = c0 <u_i|y>, u_{i+1} = y - c0 alpha_i u_i.
-// (Seven members over up to 1.0M rows: a step 280 us, with the division 300.)
+// (Seven members over up to 1.0M rows: 282 us of kernels a step, with the division 301.)
 struct GState {
     double2 c1;      // -beta_i / s_{i-1}
     double c0, s;    // 1 / s_i, s_i (beta_i; 1 at the start)

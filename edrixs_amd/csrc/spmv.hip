@@ -418,11 +418,12 @@ __global__ void k_to_c64_vec(int64_t n, const double2 *in, float2 *out, const in
         out[i] = make_float2((float)in[i].x, (float)in[i].y);
 }
 
-// Per-block dot partials of a launch with more than FOLD_MIN blocks are folded
-// to FOLD_N sums (block j adds the j-th contiguous chunk in a fixed order) so
-// the one-block scalar kernels that consume them stay short.  (Below that the two
-// launches cost more than they save: 16 partials a thread are one or two trips
-// to memory.)
+// Per-block dot partials of a launch with more than FOLD_N blocks are folded to
+// FOLD_N sums (block j adds the j-th contiguous chunk in a fixed order) so the
+// one-block scalar kernels that consume them stay short.  Krylov recurrences fold
+// above FOLD_MIN only: below it the two launches cost more than they save (16
+// partials a thread are one or two trips to memory).  Solves that stop at a
+// tolerance keep their order of summation.
 constexpr int FOLD_N = 256;
 constexpr int FOLD_MIN = 4096;
 
@@ -648,13 +649,13 @@ bool xcd_map_enabled() {
 }
 
 // After a launch of nb workgroups with dot partials: 0 left to sum if the launch
-// ran its tail, else at most FOLD_MIN.
+// ran its tail, else at most FOLD_MIN (solves: FOLD_N).
 int finish_partials(const SpmvEpi &e, int nb, int *nblocks_out) {
     if (nblocks_out) *nblocks_out = nb;
     if (!e.dvec) return EDX_OK;
     if (e.tail.count) {
         if (nblocks_out) *nblocks_out = 0;
-    } else if (nb > FOLD_MIN) {
+    } else if (nb > (e.tail.K && !e.tail.nshift ? FOLD_MIN : FOLD_N)) {
         hipLaunchKernelGGL(k_fold_partials, dim3(FOLD_N), dim3(256), 0, stream(), e.partials, nb,
                            e.run);
         hipLaunchKernelGGL(k_move_folded, dim3(1), dim3(FOLD_N), 0, stream(), e.partials, nb, e.run);
