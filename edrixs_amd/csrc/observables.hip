@@ -48,14 +48,21 @@ __global__ __launch_bounds__(256) void k_denmat_pairs(BasisView b, int norb, con
 // The fraction without its divisions.  With D_n = 1, D_{n+1} = 0 and
 //     D_j = (z - a_{j+1}) D_{j+1} - b_{j+1}^2 D_{j+2}        (j = n-1 .. 0)
 // (the determinants of the trailing blocks of z - T) the fraction is D_1 / D_0.
-// Each computed D_j is the exact one of coefficients perturbed by a few eps, as
-// each quotient of the nested form is, so the two are equally accurate; but a
-// step is two dependent multiply-adds where the nested form waits for a complex
+// A step is two dependent multiply-adds where the nested form waits for a complex
 // quotient, and that serial chain is all there is: 300 poles on 2000 points
-// took 62 us nested.  D and its predecessor are rescaled by a power of
-// two every CF_BLOCK steps; k_cf_nested serves coefficients outside the range
-// in which that many steps cannot overflow or underflow.  The coefficients are
-// staged in LDS, one grid point per lane.
+// took 62 us nested (the whole call 154 us, now 42).  The phases of D_1 and D_0 gather a rounding a step, so
+// far from the poles, where the fraction is almost real, the imaginary part of
+// their quotient is a difference of nearly equal products (300 poles, 40 eV from
+// the middle of a 30 eV band, broadening 0.1 eV: off by 6e-14 of itself, nested
+// 4e-16).  It is taken there from P_j = Im(D_{j+1} conj(D_j)),
+//     P_j = b_{j+1}^2 P_{j+1} - gamma |D_{j+1}|^2,
+// a sum of terms of one sign, as P_0 / |D_0|^2 (4e-16 too).  Where the imaginary
+// part is at least half the real one the quotient loses nothing and is the closer of
+// the two (broadening 0.5 eV inside the band: 3.4e-16, nested 3.6e-16, P 5.1e-16).
+// D, its predecessor and P are rescaled by powers of two every CF_BLOCK steps;
+// k_cf_nested serves coefficients outside the range in which that many steps
+// cannot overflow or underflow.  The coefficients are staged in LDS, one grid
+// point per lane.
 constexpr int CF_BLOCK = 8;
 constexpr int CF_STAGE = 512;
 constexpr int CF_MAX_EXP = 50;   // largest coefficient in 2^-50 .. 2^50
@@ -70,6 +77,7 @@ __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ 
     const bool on = w < nw;
     const double zx = on ? omega[w] + e_gs : 0.0, zy = on ? gamma[w] : 1.0;
     double2 d = make_double2(1.0, 0.0), q = make_double2(0.0, 0.0);   // D_{j+1}, D_{j+2}
+    double p = 0.0;                                                   // P_{j+1}
     for (int top = neff; top > 0; top -= CF_STAGE) {
         const int n = top < CF_STAGE ? top : CF_STAGE;
         __syncthreads();
@@ -84,6 +92,7 @@ __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ 
             const double x = zx - s_a[i], b2 = s_b2[i];
             const double2 t = make_double2(x * d.x - (zy * d.y + b2 * q.x),
                                            x * d.y + (zy * d.x - b2 * q.y));
+            p = b2 * p - zy * (d.x * d.x + d.y * d.y);
             q = d;
             d = t;
         };
@@ -95,12 +104,14 @@ __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ 
             const double sc = ldexp(1.0, -ilogb(big));
             d = cscale(d, sc);
             q = cscale(q, sc);
+            p *= sc * sc;
         }
         for (; i < n; ++i) step(i);
     }
     if (!on) return;
     const double2 t = cdiv(q, d);
-    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * t.y * norm * weight;
+    const double im = fabs(t.y) >= 0.5 * fabs(t.x) ? t.y : p / (d.x * d.x + d.y * d.y);
+    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * im * norm * weight;
 }
 
 // The nested fraction, for coefficients of any size.

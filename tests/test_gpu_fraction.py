@@ -41,3 +41,28 @@ def test_breakdown_and_zero_couplings():
     s = core.cf_spectrum(a, b, 1.0, 0.0, om, 0.3)
     t = core.cf_spectrum(a[:2], b[:2], 1.0, 0.0, om, 0.3)
     np.testing.assert_allclose(s, t, rtol=1e-14)
+
+
+@pytest.mark.parametrize("neff", [1, 8, 60, 300, 1000, 4000])
+@pytest.mark.parametrize("gamma", [1.0, 0.1, 1e-3, 1e-8])
+def test_fraction_keeps_its_digits_far_from_the_poles(neff, gamma):
+    """Grid points far from the band, where the imaginary part is a small fraction of
+    the real one, point by point.  With |z - a| >= 4 b each quotient of neighbours
+    D_j / D_{j+1} = z - a - b^2 D_{j+2} / D_{j+1} carries a rounding of at most 5 eps
+    (the error of the one before comes in with weight b^2 / |w|^2 < 1/12), so does
+    P_j / |D_{j+1}|^2 = -gamma + b^2 P_{j+1} / |D_{j+1}|^2 with at most 6, and the final
+    quotient and prefactors add 2 * 5 + 6: 22 eps, whatever the number of poles."""
+    from edrixs_amd import core
+    rng = np.random.default_rng(neff)
+    a, b = rng.uniform(-4.0, 4.0, neff), rng.uniform(4.0, 8.0, neff)
+    om = np.concatenate([np.linspace(-400.0, -36.0, 70), np.linspace(36.0, 120.0, 70),
+                         np.geomspace(1e3, 1e8, 30)])
+    got = core.cf_spectrum(a, b, 0.7, 0.0, om, gamma, weight=0.6)
+    al, bl = a.astype(np.longdouble), b.astype(np.longdouble)
+    z = om.astype(np.longdouble) + 1j * np.longdouble(gamma)
+    t = np.zeros(len(om), dtype=np.clongdouble)
+    for j in range(neff - 1, 0, -1):
+        t = bl[j - 1] ** 2 / (z - al[j] - t)
+    ref = -np.imag(1 / (z - al[0] - t)) * np.longdouble(0.7) * np.longdouble(0.6) / np.longdouble(np.pi)
+    assert np.all(got > 0)
+    assert np.max(np.abs(got - ref) / ref) <= 22 * np.finfo(float).eps
