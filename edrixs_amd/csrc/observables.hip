@@ -50,22 +50,25 @@ __global__ __launch_bounds__(256) void k_denmat_pairs(BasisView b, int norb, con
 // (the determinants of the trailing blocks of z - T) the fraction is D_1 / D_0.
 // A step is two dependent multiply-adds where the nested form waits for a complex
 // quotient, and that serial chain is all there is: 300 poles on 2000 points
-// took 62 us nested (the whole call 154 us, now 42).  The phases of D_1 and D_0 gather a rounding a step, so
-// far from the poles, where the fraction is almost real, the imaginary part of
-// their quotient is a difference of nearly equal products (300 poles, 40 eV from
-// the middle of a 30 eV band, broadening 0.1 eV: off by 6e-14 of itself, nested
-// 4e-16).  It is taken there from P_j = Im(D_{j+1} conj(D_j)),
+// took 62 us nested (the whole call 154 us, now 42).  The phases of D_1 and D_0
+// gather a rounding a step, so far from the poles, where the fraction is almost
+// real, the imaginary part of their quotient is a difference of nearly equal
+// products (300 poles, 45 to 85 eV from the middle of a band 60 eV wide, broadening
+// 0.1 eV: off by 6e-14 of itself, nested 4e-16).  It is taken there from
+// P_j = Im(D_{j+1} conj(D_j)),
 //     P_j = b_{j+1}^2 P_{j+1} - gamma |D_{j+1}|^2,
 // a sum of terms of one sign, as P_0 / |D_0|^2 (4e-16 too).  Where the imaginary
 // part is at least half the real one the quotient loses nothing and is the closer of
 // the two (broadening 0.5 eV inside the band: 3.4e-16, nested 3.6e-16, P 5.1e-16).
-// D, its predecessor and P are rescaled by powers of two every CF_BLOCK steps;
-// k_cf_nested serves coefficients outside the range in which that many steps
-// cannot overflow or underflow.  The coefficients are staged in LDS, one grid
-// point per lane.
+// D, its predecessor and P are rescaled by powers of two every CF_BLOCK steps.
+// Between two rescalings nothing overflows while |a|, b, |omega|, |gamma| and |e_gs|
+// are below 2^CF_MAX_EXP (|D| grows by at most 2^53 a step), and nothing that
+// counts underflows while |gamma| is above 2^-CF_MAX_EXP: Im(D_{j+2} / D_{j+1}) has
+// the sign that makes |D_j| >= |gamma| |D_{j+1}|, whatever a and b.  k_cf_nested serves
+// other coefficients.  They are staged in LDS, one grid point per lane.
 constexpr int CF_BLOCK = 8;
 constexpr int CF_STAGE = 512;
-constexpr int CF_MAX_EXP = 50;   // largest coefficient in 2^-50 .. 2^50
+constexpr int CF_MAX_EXP = 50;
 
 __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ alpha,
                                            const double *__restrict__ beta, double norm, double e_gs,
@@ -114,6 +117,15 @@ __global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ 
     out[w] = spec[w] + -1.0 / 3.14159265358979323846 * im * norm * weight;
 }
 
+// a / b with the squares of b in range (the same bits as cdiv where they are anyway)
+__device__ __forceinline__ double2 cdiv_scaled(double2 a, double2 b) {
+    const double m = fmax(fabs(b.x), fabs(b.y));
+    if (!(m > 0.0 && m < __builtin_inf())) return cdiv(a, b);
+    const int e = ilogb(m);
+    const double s = ldexp(1.0, e > -1000 ? -e : 1000);
+    return cdiv(cscale(a, s), cscale(b, s));
+}
+
 // The nested fraction, for coefficients of any size.
 __global__ void k_cf_nested(int neff, const double *alpha, const double *beta, double norm,
                             double e_gs, double weight, int nw, const double *omega,
@@ -124,18 +136,18 @@ __global__ void k_cf_nested(int neff, const double *alpha, const double *beta, d
     double2 t = make_double2(0, 0);
     for (int j = neff - 1; j >= 1; --j) {
         const double b2 = beta[j - 1] * beta[j - 1];
-        t = cdiv(make_double2(b2, 0.0), csub(make_double2(z.x - alpha[j], z.y), t));
+        t = cdiv_scaled(make_double2(b2, 0.0), csub(make_double2(z.x - alpha[j], z.y), t));
     }
-    t = cdiv(make_double2(1.0, 0.0), csub(make_double2(z.x - alpha[0], z.y), t));
+    t = cdiv_scaled(make_double2(1.0, 0.0), csub(make_double2(z.x - alpha[0], z.y), t));
     out[w] = spec[w] + -1.0 / 3.14159265358979323846 * t.y * norm * weight;
 }
 
-// Whether the division-free recurrence stays in range: the largest of the
-// coefficients |a|, |b|, |omega|, |gamma|, |e_gs| neither huge nor tiny.
+// Whether the division-free recurrence stays in range: every coefficient finite and
+// below 2^CF_MAX_EXP, every |gamma| above 2^-CF_MAX_EXP.
 bool cf_in_range(int neff, const double *alpha, const double *beta, double e_gs, int nw,
                  const double *omega, const double *gamma) {
     double big = fabs(e_gs);
-    bool finite = true;
+    bool finite = e_gs - e_gs == 0.0;
     auto scan = [&](const double *x, int n) {
         double m = 0.0;
         for (int i = 0; i < n; ++i) {
@@ -148,7 +160,9 @@ bool cf_in_range(int neff, const double *alpha, const double *beta, double e_gs,
     scan(beta, neff - 1);
     scan(omega, nw);
     scan(gamma, nw);
-    return finite && big < ldexp(1.0, CF_MAX_EXP) && big > ldexp(1.0, -CF_MAX_EXP);
+    double least = fabs(gamma[0]);
+    for (int i = 1; i < nw; ++i) least = std::min(least, fabs(gamma[i]));
+    return finite && big < ldexp(1.0, CF_MAX_EXP) && least > ldexp(1.0, -CF_MAX_EXP);
 }
 
 // Page-locked staging of a thread's small transfers, allocated at its first

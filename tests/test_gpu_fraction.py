@@ -66,3 +66,23 @@ def test_fraction_keeps_its_digits_far_from_the_poles(neff, gamma):
     ref = -np.imag(1 / (z - al[0] - t)) * np.longdouble(0.7) * np.longdouble(0.6) / np.longdouble(np.pi)
     assert np.all(got > 0)
     assert np.max(np.abs(got - ref) / ref) <= 22 * np.finfo(float).eps
+
+
+@pytest.mark.parametrize("tiny", [1e-14, 1e-16, 1e-30, 1e-39, 1e-60, 1e-120])
+@pytest.mark.parametrize("neff", [2, 8, 9, 24])
+def test_fraction_on_a_pole_with_tiny_broadening_and_couplings(tiny, neff):
+    """Poles all at one place, seen from there with broadening and couplings far below
+    it, beside ordinary points: every step shrinks the determinants by the
+    broadening.  On the pole the fraction is i times b^2 / (gamma + b^2 / (gamma + ...)),
+    positive throughout, so each step adds at most 4 eps."""
+    from edrixs_amd import core
+    a, b = np.full(neff, 10.0), np.full(neff, tiny) * np.linspace(0.5, 2.0, neff)
+    om, g = np.array([10.0, 10.0, 12.0]), np.array([tiny, 3 * tiny, 0.5])
+    got = core.cf_spectrum(a, b, 1.0, 0.0, om, g)
+    al, bl = a.astype(np.longdouble), b.astype(np.longdouble)
+    z = om.astype(np.longdouble) + 1j * g.astype(np.longdouble)
+    t = np.zeros(3, dtype=np.clongdouble)
+    for j in range(neff - 1, 0, -1):
+        t = bl[j - 1] ** 2 / (z - al[j] - t)
+    ref = -np.imag(1 / (z - al[0] - t)) / np.longdouble(np.pi)
+    assert np.max(np.abs(got - ref) / ref) <= (4 * neff + 8) * np.finfo(float).eps
