@@ -61,61 +61,15 @@ __global__ __launch_bounds__(256) void k_denmat_pairs(BasisView b, int norb, con
 // part is at least half the real one the quotient loses nothing and is the closer of
 // the two (broadening 0.5 eV inside the band: 3.4e-16, nested 3.6e-16, P 5.1e-16).
 // D, its predecessor and P are rescaled by powers of two every CF_BLOCK steps.
-// Between two rescalings nothing overflows while |a|, b, |omega|, |gamma| and |e_gs|
-// are below 2^CF_MAX_EXP (|D| grows by at most 2^53 a step), and nothing that
-// counts underflows while |gamma| is above 2^-CF_MAX_EXP: Im(D_{j+2} / D_{j+1}) has
-// the sign that makes |D_j| >= |gamma| |D_{j+1}|, whatever a and b.  k_cf_nested serves
-// other coefficients.  They are staged in LDS, one grid point per lane.
+// Between two rescalings nothing overflows while |a|, b, |gamma| and |e_gs| are below
+// CF_MAX and |z| below twice that (|D| grows by at most 2^53 a step), and nothing that
+// counts underflows while |gamma| is above 1 / CF_MAX: Im(D_{j+2} / D_{j+1}) has the
+// sign that makes |D_j| >= |gamma| |D_{j+1}|, whatever a and b.  Grid points outside
+// that take the nested form, all of them (nested) if a coefficient is outside.  The
+// coefficients are staged in LDS, one grid point per lane.
 constexpr int CF_BLOCK = 8;
 constexpr int CF_STAGE = 512;
-constexpr int CF_MAX_EXP = 50;
-
-__global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ alpha,
-                                           const double *__restrict__ beta, double norm, double e_gs,
-                                           double weight, int nw, const double *__restrict__ omega,
-                                           const double *__restrict__ gamma, const double *spec,
-                                           double *out) {
-    __shared__ double s_a[CF_STAGE], s_b2[CF_STAGE];
-    const int w = blockIdx.x * 64 + threadIdx.x;
-    const bool on = w < nw;
-    const double zx = on ? omega[w] + e_gs : 0.0, zy = on ? gamma[w] : 1.0;
-    double2 d = make_double2(1.0, 0.0), q = make_double2(0.0, 0.0);   // D_{j+1}, D_{j+2}
-    double p = 0.0;                                                   // P_{j+1}
-    for (int top = neff; top > 0; top -= CF_STAGE) {
-        const int n = top < CF_STAGE ? top : CF_STAGE;
-        __syncthreads();
-        for (int i = threadIdx.x; i < n; i += 64) {
-            const int j = top - 1 - i;      // a_{j+1} and the b that follows it
-            const double b = j + 1 < neff ? beta[j] : 0.0;
-            s_a[i] = alpha[j];
-            s_b2[i] = b * b;
-        }
-        __syncthreads();
-        auto step = [&](int i) {
-            const double x = zx - s_a[i], b2 = s_b2[i];
-            const double2 t = make_double2(x * d.x - (zy * d.y + b2 * q.x),
-                                           x * d.y + (zy * d.x - b2 * q.y));
-            p = b2 * p - zy * (d.x * d.x + d.y * d.y);
-            q = d;
-            d = t;
-        };
-        int i = 0;
-        for (; i + CF_BLOCK <= n; i += CF_BLOCK) {
-#pragma unroll
-            for (int u = 0; u < CF_BLOCK; ++u) step(i + u);
-            const double big = fmax(fmax(fabs(d.x), fabs(d.y)), fmax(fabs(q.x), fabs(q.y)));
-            const double sc = ldexp(1.0, -ilogb(big));
-            d = cscale(d, sc);
-            q = cscale(q, sc);
-            p *= sc * sc;
-        }
-        for (; i < n; ++i) step(i);
-    }
-    if (!on) return;
-    const double2 t = cdiv(q, d);
-    const double im = fabs(t.y) >= 0.5 * fabs(t.x) ? t.y : p / (d.x * d.x + d.y * d.y);
-    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * im * norm * weight;
-}
+constexpr double CF_MAX = 1125899906842624.0;   // 2^50
 
 // a / b with the squares of b in range (the same bits as cdiv where they are anyway)
 __device__ __forceinline__ double2 cdiv_scaled(double2 a, double2 b) {
@@ -126,43 +80,78 @@ __device__ __forceinline__ double2 cdiv_scaled(double2 a, double2 b) {
     return cdiv(cscale(a, s), cscale(b, s));
 }
 
-// The nested fraction, for coefficients of any size.
-__global__ void k_cf_nested(int neff, const double *alpha, const double *beta, double norm,
-                            double e_gs, double weight, int nw, const double *omega,
-                            const double *gamma, const double *spec, double *out) {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nw) return;
-    const double2 z = make_double2(omega[w] + e_gs, gamma[w]);
-    double2 t = make_double2(0, 0);
-    for (int j = neff - 1; j >= 1; --j) {
-        const double b2 = beta[j - 1] * beta[j - 1];
-        t = cdiv_scaled(make_double2(b2, 0.0), csub(make_double2(z.x - alpha[j], z.y), t));
+__global__ __launch_bounds__(64) void k_cf(int neff, const double *__restrict__ alpha,
+                                           const double *__restrict__ beta, double norm, double e_gs,
+                                           double weight, int nw, const double *__restrict__ omega,
+                                           const double *__restrict__ gamma, const double *spec,
+                                           double *out, int nested) {
+    __shared__ double s_a[CF_STAGE], s_b2[CF_STAGE];
+    const int w = blockIdx.x * 64 + threadIdx.x;
+    const bool on = w < nw;
+    const double zx = on ? omega[w] + e_gs : 0.0, zy = on ? gamma[w] : 1.0;
+    // a_{j+1} and the b^2 that follows it, j = neff-1 .. 0, a stage of n at a time
+    auto sweep = [&](auto take) {
+        for (int top = neff; top > 0; top -= CF_STAGE) {
+            const int n = top < CF_STAGE ? top : CF_STAGE;
+            __syncthreads();
+            for (int i = threadIdx.x; i < n; i += 64) {
+                const int j = top - 1 - i;
+                const double b = j + 1 < neff ? beta[j] : 0.0;
+                s_a[i] = alpha[j];
+                s_b2[i] = b * b;
+            }
+            __syncthreads();
+            take(n);
+        }
+    };
+    double im = 0.0;
+    if (!nested) {
+        double2 d = make_double2(1.0, 0.0), q = make_double2(0.0, 0.0);   // D_{j+1}, D_{j+2}
+        double p = 0.0;                                                   // P_{j+1}
+        auto step = [&](int i) {
+            const double x = zx - s_a[i], b2 = s_b2[i];
+            const double2 t = make_double2(x * d.x - (zy * d.y + b2 * q.x),
+                                           x * d.y + (zy * d.x - b2 * q.y));
+            p = b2 * p - zy * (d.x * d.x + d.y * d.y);
+            q = d;
+            d = t;
+        };
+        sweep([&](int n) {
+            int i = 0;
+            for (; i + CF_BLOCK <= n; i += CF_BLOCK) {
+#pragma unroll
+                for (int u = 0; u < CF_BLOCK; ++u) step(i + u);
+                const double big = fmax(fmax(fabs(d.x), fabs(d.y)), fmax(fabs(q.x), fabs(q.y)));
+                const double sc = ldexp(1.0, -ilogb(big));
+                d = cscale(d, sc);
+                q = cscale(q, sc);
+                p *= sc * sc;
+            }
+            for (; i < n; ++i) step(i);
+        });
+        const double2 t = cdiv(q, d);
+        im = fabs(t.y) >= 0.5 * fabs(t.x) ? t.y : p / (d.x * d.x + d.y * d.y);
     }
-    t = cdiv_scaled(make_double2(1.0, 0.0), csub(make_double2(z.x - alpha[0], z.y), t));
-    out[w] = spec[w] + -1.0 / 3.14159265358979323846 * t.y * norm * weight;
+    const bool out_of_range = nested || !(fabs(zx) < 2.0 * CF_MAX && fabs(zy) < CF_MAX &&
+                                          fabs(zy) > 1.0 / CF_MAX);
+    if (__any(on && out_of_range)) {
+        double2 t = make_double2(1.0, 0.0);
+        sweep([&](int n) {
+            for (int i = 0; i < n; ++i)
+                t = csub(make_double2(zx - s_a[i], zy), cdiv_scaled(make_double2(s_b2[i], 0.0), t));
+        });
+        if (out_of_range) im = cdiv_scaled(make_double2(1.0, 0.0), t).y;
+    }
+    if (on) out[w] = spec[w] + -1.0 / 3.14159265358979323846 * im * norm * weight;
 }
 
-// Whether the division-free recurrence stays in range: every coefficient finite and
-// below 2^CF_MAX_EXP, every |gamma| above 2^-CF_MAX_EXP.
-bool cf_in_range(int neff, const double *alpha, const double *beta, double e_gs, int nw,
-                 const double *omega, const double *gamma) {
-    double big = fabs(e_gs);
-    bool finite = e_gs - e_gs == 0.0;
-    auto scan = [&](const double *x, int n) {
-        double m = 0.0;
-        for (int i = 0; i < n; ++i) {
-            m = std::max(m, fabs(x[i]));
-            finite = finite && x[i] - x[i] == 0.0;
-        }
-        big = std::max(big, m);
-    };
-    scan(alpha, neff);
-    scan(beta, neff - 1);
-    scan(omega, nw);
-    scan(gamma, nw);
-    double least = fabs(gamma[0]);
-    for (int i = 1; i < nw; ++i) least = std::min(least, fabs(gamma[i]));
-    return finite && big < ldexp(1.0, CF_MAX_EXP) && least > ldexp(1.0, -CF_MAX_EXP);
+// Whether the division-free recurrence serves these coefficients (k_cf looks at the
+// grid points).
+bool cf_in_range(int neff, const double *alpha, const double *beta, double e_gs) {
+    bool in = fabs(e_gs) < CF_MAX;
+    for (int i = 0; i < neff; ++i) in = in && fabs(alpha[i]) < CF_MAX;
+    for (int i = 0; i + 1 < neff; ++i) in = in && fabs(beta[i]) < CF_MAX;
+    return in;
 }
 
 // Page-locked staging of a thread's small transfers, allocated at its first
@@ -241,42 +230,42 @@ int edx_cf_spectrum(int neff, const double *alpha, const double *beta, double no
     // kernel writes its result there.  Where the workgroups together read at most
     // CF_DIRECT bytes of coefficients it reads the inputs there too: one launch
     // and one wait (a transfer each way costs another 10 us; 300 poles on 2000
-    // points read 150 KB, 3 us over the bus).  Larger inputs are copied first.
+    // points read 150 KB, 3 us over the bus).  Larger inputs are copied first, those
+    // larger than the staging memory from where they are (100 poles on a million
+    // points: another copy on the host took 1.5 of 3.9 ms).
     constexpr size_t CF_DIRECT = 256 << 10;
     const int nb = (nw + 63) / 64;
     const size_t count = 2 * (size_t)neff + 4 * (size_t)nw, bytes = sizeof(double) * count;
-    std::vector<double> pageable;
-    double *host = (double *)g_stage.get(bytes);
-    const bool pinned = host != nullptr;
-    const bool direct = pinned && (size_t)nb * neff * 16 <= CF_DIRECT;
-    if (!pinned) {
-        pageable.resize(count);
-        host = pageable.data();
-    }
     const size_t o_om = 2 * (size_t)neff, o_sp = o_om + 2 * (size_t)nw, o_out = o_sp + nw;
-    memcpy(host, alpha, neff * sizeof(double));
-    memcpy(host + neff, beta, neff * sizeof(double));
-    memcpy(host + o_om, omega, nw * sizeof(double));
-    memcpy(host + o_om + nw, gamma, nw * sizeof(double));
-    memcpy(host + o_sp, spec, nw * sizeof(double));
+    double *host = (double *)g_stage.get(bytes);
+    const bool direct = host && (size_t)nb * neff * 16 <= CF_DIRECT;
     DevBuf buf;
     double *d = host;
     hipStream_t s = edx::stream();
     if (!direct) {
         EDX_TRY(buf.alloc(bytes, "cf buffers"));
         d = buf.as<double>();
-        EDX_HIP(hipMemcpyAsync(d, host, o_out * sizeof(double), hipMemcpyHostToDevice, s));
     }
-    double *out = pinned ? host + o_out : d + o_out;
-    if (cf_in_range(neff, alpha, beta, e_gs, nw, omega, gamma))
-        hipLaunchKernelGGL(k_cf, dim3(nb), dim3(64), 0, s, neff, d, d + neff, norm, e_gs, weight, nw,
-                           d + o_om, d + o_om + nw, d + o_sp, out);
-    else
-        hipLaunchKernelGGL(k_cf_nested, dim3(nb), dim3(64), 0, s, neff, d, d + neff, norm, e_gs, weight,
-                           nw, d + o_om, d + o_om + nw, d + o_sp, out);
+    const struct {
+        size_t at;
+        const double *from;
+        int n;
+    } in[] = {{0, alpha, neff}, {(size_t)neff, beta, neff}, {o_om, omega, nw},
+              {o_om + nw, gamma, nw}, {o_sp, spec, nw}};
+    for (const auto &q : in) {
+        if (host) memcpy(host + q.at, q.from, q.n * sizeof(double));
+        else EDX_HIP(hipMemcpyAsync(d + q.at, q.from, q.n * sizeof(double), hipMemcpyHostToDevice, s));
+    }
+    if (host && !direct) EDX_HIP(hipMemcpyAsync(d, host, o_out * sizeof(double), hipMemcpyHostToDevice, s));
+    double *out = host ? host + o_out : d + o_out;
+    hipLaunchKernelGGL(k_cf, dim3(nb), dim3(64), 0, s, neff, d, d + neff, norm, e_gs, weight, nw,
+                       d + o_om, d + o_om + nw, d + o_sp, out, !cf_in_range(neff, alpha, beta, e_gs));
     EDX_LAUNCH_CHECK();
-    if (pinned) EDX_HIP(hipStreamSynchronize(s));
-    else EDX_HIP(edx::copy_sync(host + o_out, out, nw * sizeof(double), hipMemcpyDeviceToHost));
+    if (!host) {
+        EDX_HIP(edx::copy_sync(spec, out, nw * sizeof(double), hipMemcpyDeviceToHost));
+        return EDX_OK;
+    }
+    EDX_HIP(hipStreamSynchronize(s));
     memcpy(spec, host + o_out, nw * sizeof(double));
     return EDX_OK;
 }

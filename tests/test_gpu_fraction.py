@@ -86,3 +86,25 @@ def test_fraction_on_a_pole_with_tiny_broadening_and_couplings(tiny, neff):
         t = bl[j - 1] ** 2 / (z - al[j] - t)
     ref = -np.imag(1 / (z - al[0] - t)) / np.longdouble(np.pi)
     assert np.max(np.abs(got - ref) / ref) <= (4 * neff + 8) * np.finfo(float).eps
+
+
+@pytest.mark.parametrize("nw", [32765, 32770, 100001])
+def test_fraction_on_grids_beyond_the_staging_memory(nw):
+    """Around and beyond 1 MB of inputs, with points in and out of the recurrence's range
+    side by side; a quotient of three poles in the band adds at most
+    8 eps (|z - a| + 2 b) / gamma^2 to a spectrum of order 1 / gamma, as above."""
+    from edrixs_amd import core
+    a, b = np.array([1.0, -2.0, 0.5]), np.array([0.8, 1.5])
+    om, g = np.linspace(-6.0, 6.0, nw), np.full(nw, 0.3)
+    g[::1000] = 1e-17
+    om[::1000] = 1e3
+    start = np.linspace(0.0, 1.0, nw)
+    got = core.cf_spectrum(a, np.append(b, 7.0), 1.0, 0.25, om, g, out=start.copy())
+    z = (om + 0.25).astype(np.longdouble) + 1j * g.astype(np.longdouble)
+    t = b[1] ** 2 / (z - a[2])
+    t = b[0] ** 2 / (z - a[1] - t)
+    ref = -np.imag(1 / (z - a[0] - t)) / np.longdouble(np.pi)
+    eps = np.finfo(float).eps
+    assert np.abs(got - (start + ref)).max() <= 8 * eps * (9.0 + 3.0) / 0.3 ** 2 / np.pi + 2 * eps
+    far = core.cf_spectrum(a, np.append(b, 7.0), 1.0, 0.25, om, g)[::1000]
+    assert np.max(np.abs(far - ref[::1000]) / ref[::1000]) <= 32 * eps
