@@ -14,9 +14,10 @@
 //   * k_plan_count / k_plan_fill (termplan.hip), for complete bases: 64 rows per
 //     workgroup over the terms grouped by column;
 //   * k_build, for incomplete bases (columns found by search), more than 4096
-//     terms, few terms on few rows (BUILD_TINY_ROWS), or rows longer than the plan kernels' LDS lists (255 entries, about 185
-//     with words of more than 32 bits): one 64-lane wavefront per row.  Lanes
-//     evaluate 64 terms at a time; survivors are compacted with a ballot into an
+//     terms, too few rows for their terms (build_max_groups), long rows
+//     (BUILD_MEAN_ROW, and any row longer than the plan kernels' LDS lists: 255
+//     entries, about 185 with words of more than 32 bits): one 64-lane wavefront
+//     per row.  Lanes evaluate 64 terms at a time; survivors are compacted with a ballot into an
 //     LDS list that stays in term order; the list is bitonic-sorted on the key
 //     (column << 32 | term << 1 | sign), which orders by column and, within a
 //     column, by term; a head lane per column then sums its run sequentially,
@@ -422,11 +423,10 @@ int build_alloc(BuildOut &o, int64_t M, int *flag) {
 
 // The plan kernels' build; *done stays false where a row is too long for them.
 template <int RK, int CK, class W>
-int build_by_plan(const BuildParams &p, const PlanSpaces &sp, const TermTable &tt, BuildOut &o,
+int build_by_plan(const BuildParams &p, const PlanSpaces &sp, const PlanTerms &pt, BuildOut &o,
                   bool *done) {
     PlanStore<W> plan;
-    EDX_TRY(plan_make<W>(sp, tt.ops.data(), tt.vals.data(), tt.nhop, tt.T, p.omega_on != 0,
-                         p.omega, p.negate != 0, PLAN_WAVES, false, plan));
+    EDX_TRY(plan_make<W>(sp, pt, p.omega_on != 0, p.omega, PLAN_WAVES, true, plan));
     EDX_HIP(hipMemsetAsync(o.rowptr + p.M, 0, sizeof(int64_t), edx::stream()));
     EDX_HIP(hipMemsetAsync(o.flag, 0, sizeof(int), edx::stream()));
     EDX_TRY((plan_count<RK, W>(plan.p, o.rowptr, o.flag)));
@@ -477,9 +477,25 @@ int build_by_term(BuildParams p, TermTable &tt, BuildOut &o) {
     return EDX_OK;
 }
 
-// Few terms on few rows: grouping the terms costs more than it saves (362
-// terms: 495 rows 161 us, over the plan 165; 924 rows 172 and 161).
-constexpr int BUILD_TINY_ROWS = 512, BUILD_TINY_TERMS = 512;
+// The most groups that T terms on M rows may have for the plan to be the faster build;
+// negative: it is the slower one however they group.  A call's time beyond what the two
+// have in common, in us: a plan takes 0.055 a term (most of it on the host), 0.15 a group
+// and 10; the term-by-term kernel 22 and, a row, 5e-4 and 1.9e-5 a term.  Measured (whole
+// calls, term by term and over the plan): an impurity's 370 terms in 46 groups 136 and
+// 139 us on 792 rows, 144 and 142 on 1,716, 199 and 154 on 8,008; its core-hole operator,
+// 965 in 129, 187 and 198 on 1,260, 218 and 209 on 2,772, 391 and 218 on 10,296; random
+// terms, 1000 in 500, 206 and 300 on 3,432, 262 and 301 on 6,435, 380 and 322 on 12,870;
+// 30 in 30, 111 and 91 on 70 rows.
+double build_max_groups(int64_t M, int T) {
+    const double g = (12.0 + M * (5e-4 + 1.9e-5 * T) - 0.055 * T) / 0.15;
+    return 16.0 * g < T ? -1.0 : g;   // an impurity operator's terms group eight to one
+}
+
+// Rows of more entries on the mean (plan_mean_row) are the term-by-term kernel's: the
+// plan's lists leave room for fewer workgroups and every entry is compared with its row's
+// others.  Random terms on 12,870 rows: 59 entries 380 and 322 us (over the plan), 85
+// entries 1387 and 1588; on 3,432 rows 68 entries 466 and 498.
+constexpr double BUILD_MEAN_ROW = 64.0;
 
 template <int RK, int CK>
 int build_csr(BuildParams p, const edx_basis *left, const edx_basis *right, TermTable &tt,
@@ -497,10 +513,14 @@ int build_csr(BuildParams p, const edx_basis *left, const edx_basis *right, Term
     if (!o.rowptr || !o.flag) return EDX_ERR_NOMEM;
     const PlanSpaces sp{RK, CK, p.nv, p.nc, left, right};
     bool done = false;
-    const bool tiny = p.M <= BUILD_TINY_ROWS && tt.T <= BUILD_TINY_TERMS;
-    if (p.M > 0 && !tiny && plan_usable(sp, tt.ops.data(), tt.nhop, tt.T)) {
-        if (plan_bits(sp) <= 32) EDX_TRY((build_by_plan<RK, CK, uint32_t>(p, sp, tt, o, &done)));
-        else EDX_TRY((build_by_plan<RK, CK, uint64_t>(p, sp, tt, o, &done)));
+    const double most = build_max_groups(p.M, tt.T);
+    PlanTerms pt;
+    if (p.M > 0 && most >= 0.0 && plan_usable(sp, tt.ops.data(), tt.nhop, tt.T) &&
+        plan_group(sp, tt.ops.data(), tt.vals.data(), tt.nhop, tt.T, p.omega_on != 0, p.negate != 0,
+                   false, most, pt) &&
+        plan_mean_row(sp, pt) <= BUILD_MEAN_ROW) {
+        if (plan_bits(sp) <= 32) EDX_TRY((build_by_plan<RK, CK, uint32_t>(p, sp, pt, o, &done)));
+        else EDX_TRY((build_by_plan<RK, CK, uint64_t>(p, sp, pt, o, &done)));
     }
     if (!done) EDX_TRY((build_by_term<RK, CK>(p, tt, o)));
     edx_csr *a = new edx_csr{};

@@ -13,8 +13,9 @@
 //   * k_plan_apply, for complete bases: 64 rows per workgroup over the terms
 //     grouped by column (termplan.hip), those of equal action merged;
 //   * k_mf, for incomplete bases, more than 4096 terms, rows of more than 255
-//     entries, and few terms on few rows (mf_try_plan): one 64-lane wave per row, its lanes testing the terms in
-//     parallel and accumulating val * sign * x[col] over the survivors.
+//     entries, and too few rows for their terms (mf_max_groups): one 64-lane wave per
+//     row, its lanes testing the terms in parallel and accumulating
+//     val * sign * x[col] over the survivors.
 
 namespace {
 
@@ -234,10 +235,18 @@ int mf_waves(int64_t rows) {
     return (rows + PLAN_ROWS - 1) / PLAN_ROWS <= (int64_t)edx::num_cus() * 3 / 2 ? MF_WIDE : PLAN_WAVES;
 }
 
-// Few terms on few rows keep k_mf, whose waves take a row each: 362 terms 23.5
-// us for 25.9 at 2,002 rows and 25.8 for 25.7 at 3,432; 950 terms 33 for 29 at
-// 1,512.
-constexpr int MF_TINY_ROWS = 3072, MF_TINY_TERMS = 512;
+// The most groups that T terms on M rows may have for the plan to be the faster product;
+// negative: it is the slower one however they group.  A product's time beyond a launch, in
+// us: the plan takes 0.05 a group and 3 (its waves test all groups, whatever the rows, while
+// the workgroups fill the chip less than twice); k_mf, whose waves take a row each, 0.004 a
+// term and, a row, 5e-4 and 2.2e-6 a term.  Measured (k_mf, plan): 370 terms in 46
+// groups 21.8 and 22.5 us on 1,716 rows, 27.1 and 23.0 on 8,008; 965 in 129, 24.2 and 25.5 on
+// 1,320, 31.6 and 26.1 on 2,772; random terms, 1000 in 500, 37.7 and 46.0 on 6,435, 58.1 and
+// 47.6 on 12,870.
+double mf_max_groups(int64_t M, int T) {
+    const double g = (M * (5e-4 + 2.2e-6 * T) + 0.004 * T - 3.0) / 0.05;
+    return 16.0 * g < T ? -1.0 : g;
+}
 
 int mf_blocks(const edx_mfop *op) {
     if (op->plan) return (int)std::max<int64_t>((op->p.M + PLAN_ROWS - 1) / PLAN_ROWS, 1);
@@ -265,9 +274,8 @@ void mf_launch_plan(const edx_mfop *op, const Plan<W> &p, int nb, const double2 
 // Groups the operator's terms where the basis allows; the longest row sizes
 // the kernel's lists.
 template <int RK, int CK, class W>
-int mf_plan(edx_mfop *op, const PlanSpaces &sp, PlanStore<W> &store) {
-    EDX_TRY(plan_make<W>(sp, op->tt.ops.data(), op->tt.vals.data(), op->tt.nhop, op->tt.T,
-                         op->p.omega_on != 0, op->p.omega, op->p.negate != 0, mf_waves(op->p.M), true, store));
+int mf_plan(edx_mfop *op, const PlanSpaces &sp, const PlanTerms &pt, PlanStore<W> &store) {
+    EDX_TRY(plan_make<W>(sp, pt, op->p.omega_on != 0, op->p.omega, mf_waves(op->p.M), false, store));
     store.p.inter = 0;
     DevBuf flag;
     EDX_TRY(flag.alloc(sizeof(int), "longest row"));
@@ -280,12 +288,15 @@ int mf_plan(edx_mfop *op, const PlanSpaces &sp, PlanStore<W> &store) {
 
 template <int RK, int CK> int mf_try_plan(edx_mfop *op, const edx_basis *fock) {
     const PlanSpaces sp{RK, CK, op->p.nv, op->p.nc, fock, fock};
-    if (op->p.M <= MF_TINY_ROWS && op->tt.T <= MF_TINY_TERMS) return EDX_OK;
-    if (op->p.M == 0 || !plan_usable(sp, op->tt.ops.data(), op->tt.nhop, op->tt.T) ||
-        op->p.M >= ((int64_t)1 << 31))
+    const double most = mf_max_groups(op->p.M, op->tt.T);
+    PlanTerms pt;
+    if (op->p.M == 0 || op->p.M >= ((int64_t)1 << 31) || most < 0.0 ||
+        !plan_usable(sp, op->tt.ops.data(), op->tt.nhop, op->tt.T) ||
+        !plan_group(sp, op->tt.ops.data(), op->tt.vals.data(), op->tt.nhop, op->tt.T,
+                    op->p.omega_on != 0, op->p.negate != 0, true, most, pt))
         return EDX_OK;
-    return plan_bits(sp) <= 32 ? mf_plan<RK, CK, uint32_t>(op, sp, op->plan32)
-                               : mf_plan<RK, CK, uint64_t>(op, sp, op->plan64);
+    return plan_bits(sp) <= 32 ? mf_plan<RK, CK, uint32_t>(op, sp, pt, op->plan32)
+                               : mf_plan<RK, CK, uint64_t>(op, sp, pt, op->plan64);
 }
 
 int mf_launch(const edx_mfop *op, const double2 *x, const SpmvEpi &e, int *nblocks_out) {

@@ -523,29 +523,38 @@ bool plan_merge_exact(const std::vector<HostTerm> &ht, const std::vector<double2
     return true;
 }
 
-// Groups the terms.  waves: those of the kernels that expand it.  merge: terms that differ in their value only become one
-// (the matrix-free apply, whose sums need not keep the term order).
-template <class W>
-int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int nhop, int T,
-              bool omega_on, double2 omega, bool negate, int waves, bool merge, PlanStore<W> &out) {
+// The terms that reach the column space, grouped by where they lead.
+struct PlanTerms {
     struct Group {
         uint64_t key;
-        std::vector<int> terms;
+        int head, tail;   // its terms, chained by next in term order
     };
     std::vector<HostTerm> ht;
     std::vector<double2> hv;
+    std::vector<int> next;
     std::vector<Group> groups;
+};
+
+// Groups the terms; false as soon as there are more than max_groups.  merge: terms
+// that differ in their value only become one (the matrix-free apply, whose sums
+// need not keep the term order).
+bool plan_group(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int nhop, int T,
+                bool omega_on, bool negate, bool merge, double max_groups, PlanTerms &out) {
+    auto &ht = out.ht;
+    auto &hv = out.hv;
+    auto &next = out.next;
+    auto &groups = out.groups;
     ht.reserve(T);
     hv.reserve(T);
-    int hsize = 64;
-    while (hsize < 4 * (T + 1)) hsize *= 2;
-    std::vector<int> table(hsize, -1);
+    next.reserve(T);
+    int bits = 6;
+    while ((1 << bits) < 2 * (T + 1)) ++bits;
+    std::vector<int> table((size_t)1 << bits, -1);
     auto group_of = [&](uint64_t key) {
-        uint64_t h = key * 0x9e3779b97f4a7c15ull;
-        for (int i = (int)(h >> 40) & (hsize - 1);; i = (i + 1) & (hsize - 1)) {
+        for (int i = (int)(key * 0x9e3779b97f4a7c15ull >> (64 - bits));; i = (i + 1) & ((1 << bits) - 1)) {
             if (table[i] < 0) {
                 table[i] = (int)groups.size();
-                groups.push_back(Group{key, {}});
+                groups.push_back(PlanTerms::Group{key, -1, -1});
             }
             if (groups[table[i]].key == key) return table[i];
         }
@@ -554,10 +563,11 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
     for (int t = 0; t < T; ++t) {
         HostTerm h;
         if (!plan_term(sp, ops[t], t < nhop, negate, h)) continue;
-        Group &g = groups[group_of(h.group)];
+        PlanTerms::Group &g = groups[group_of(h.group)];
+        if ((double)groups.size() > max_groups) return false;
         if (merge) {
             bool found = false;
-            for (int q : g.terms)
+            for (int q = g.head; q >= 0; q = next[q])
                 if (ht[q].m == h.m && ht[q].v == h.v && ht[q].s == h.s) {
                     const double sg = ht[q].neg == h.neg ? 1.0 : -1.0;
                     hv[q].x += sg * tv[t].x;
@@ -567,10 +577,53 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
                 }
             if (found) continue;
         }
-        g.terms.push_back((int)ht.size());
+        const int q = (int)ht.size();
+        (g.head < 0 ? g.head : next[g.tail]) = q;
+        g.tail = q;
         ht.push_back(h);
         hv.push_back(tv[t]);
+        next.push_back(-1);
     }
+    return true;
+}
+
+// Entries of a mean row, from below: the largest share of rows that one term of
+// each group survives on.
+double plan_mean_row(const PlanSpaces &sp, const PlanTerms &pt) {
+    const int n = sp.left->nbits, N = sp.left->nocc;
+    auto falling = [](int x, int k) {   // x (x-1) ... (x-k+1), 0 if it runs out
+        double r = 1.0;
+        for (int i = 0; i < k; ++i) r *= std::max(x - i, 0);
+        return r;
+    };
+    const uint64_t val = sp.rk == ROW_PLAIN ? ~0ull : (1ull << sp.nv) - 1;
+    double rows = 0.0;
+    for (const PlanTerms::Group &g : pt.groups) {
+        double best = 0.0;
+        for (int q = g.head; q >= 0; q = pt.next[q]) {
+            const HostTerm &h = pt.ht[q];
+            const int full = __builtin_popcountll(h.v & val), empty = __builtin_popcountll(h.m & val) - full;
+            double share = falling(N, full) * falling(n - N, empty) / std::max(falling(n, full + empty), 1.0);
+            const int cfull = __builtin_popcountll(h.v & ~val), cempty = __builtin_popcountll(h.m & ~val) - cfull;
+            if (sp.rk == ROW_COREHOLE)
+                share *= cempty == 0 ? (double)(sp.nc - cfull) / sp.nc : (cempty == 1 ? 1.0 / sp.nc : 0.0);
+            if (sp.rk == ROW_FULLCORE && cempty) share = 0.0;
+            best = std::max(best, share);
+        }
+        rows += best;
+    }
+    return rows;
+}
+
+// The plan of grouped terms.  waves: those of the kernels that expand it.
+// exact_sums: a group's terms are summed in term order, bit for bit.
+template <class W>
+int plan_make(const PlanSpaces &sp, const PlanTerms &pt, bool omega_on, double2 omega, int waves,
+              bool exact_sums, PlanStore<W> &out) {
+    const auto &ht = pt.ht;
+    const auto &hv = pt.hv;
+    const auto &next = pt.next;
+    const auto &groups = pt.groups;
     const int G = (int)groups.size();
     int nchunk = (G + PLAN_CHUNK - 1) / PLAN_CHUNK;
     nchunk = std::max((nchunk + waves - 1) / waves, 1) * waves;
@@ -583,17 +636,23 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
     int big = -1, nbig = PLAN_BIG;
     std::vector<std::pair<uint64_t, uint64_t>> kept;
     std::vector<TermClass> classes;
+    std::vector<int> members;
+    terms.reserve(ht.size());
+    vals.reserve(ht.size());
+    tests.reserve(ht.size());
     for (int c = 0; c < nchunk; ++c) {
         chunks[c] = (int32_t)tests.size();
         for (int g = c * gpc; g < std::min((c + 1) * gpc, G); ++g) {
-            const Group &gr = groups[g];
+            const PlanTerms::Group &gr = groups[g];
+            members.clear();
+            for (int q = gr.head; q >= 0; q = next[q]) members.push_back(q);
             PlanGroup<W> &d = dg[g];
             d.flip = 0;
             d.tbeg = (int32_t)terms.size();
-            const bool exact = !merge && plan_merge_exact(ht, hv, gr.terms, classes);
-            const size_t count = exact ? classes.size() : gr.terms.size();
+            const bool exact = exact_sums && plan_merge_exact(ht, hv, members, classes);
+            const size_t count = exact ? classes.size() : members.size();
             for (size_t i = 0; i < count; ++i) {
-                const int q = exact ? classes[i].lead : gr.terms[i];
+                const int q = exact ? classes[i].lead : members[i];
                 const uint32_t flips = exact ? classes[i].flips : PLAN_FLIP_X | PLAN_FLIP_Y;
                 terms.push_back(PlanTerm<W>{(W)ht[q].m, (W)ht[q].v, (W)ht[q].s, ht[q].neg | flips});
                 vals.push_back(exact ? classes[i].sum : hv[q]);
@@ -611,7 +670,7 @@ int plan_make(const PlanSpaces &sp, const uint32_t *ops, const double2 *tv, int 
                 kept.emplace_back(0, 0);
             } else {
                 for (int bits = 1; bits <= 4; ++bits)
-                    for (int q : gr.terms) {
+                    for (int q : members) {
                         if (__builtin_popcountll(ht[q].m) != bits) continue;
                         bool implied = false;
                         for (auto &k : kept)

@@ -201,3 +201,113 @@ def test_merged_terms_keep_every_bit(core, nbits, nocc, sets, sign):
     ref = np.ascontiguousarray(R.vals).view(np.float64)
     got = np.ascontiguousarray(vals).view(np.float64)
     assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
+
+
+def _few_terms(n, seed, most=56):
+    """At most `most` terms over n orbitals spread from the first to the last: hoppings, densities,
+    two-body terms and their conjugates."""
+    rng = np.random.default_rng(seed)
+    k = min(n, 9)
+    orb = np.unique(np.linspace(0, n - 1, k).round().astype(int))
+    hop = [[i + 1, j + 1, *rng.normal(size=2)] for i in orb for j in orb if rng.random() < 0.3]
+    coul = []
+    for _ in range(most):
+        i, j, p, q = rng.choice(orb, size=4)
+        if i == j or p == q:
+            continue
+        re, im = rng.normal(size=2)
+        coul += [[i + 1, j + 1, p + 1, q + 1, re, im], [q + 1, p + 1, j + 1, i + 1, re, -im]]
+    hop = hop[:most // 2]
+    return hop, coul[:most - len(hop)]
+
+
+def test_calls_of_few_terms_take_the_plan_on_any_number_of_rows():
+    """The sizes below count on it: the rule's constants are read from the source."""
+    import os
+    import re
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src = open(os.path.join(root, "edrixs_amd", "csrc", "csr_build.hip")).read()
+    a, t, g = (float(x) for x in re.search(
+        r"const double g = \(([\d.]+) \+ M \* \([^)]*\) - ([\d.]+) \* T\) / ([\d.]+);", src).groups())
+    assert (a - t * 56) / g >= 56          # 56 terms in 56 groups, no rows
+
+
+@pytest.mark.parametrize("nbits,nocc", [(1, 0), (1, 1), (5, 5), (6, 1), (8, 4), (11, 5), (15, 12),
+                                        (31, 2), (32, 2), (33, 2), (40, 1), (62, 1), (62, 2)])
+def test_few_terms_at_word_and_workgroup_edges(core, nbits, nocc):
+    ht, ut = _few_terms(nbits, nbits + nocc)
+    b, fock = core.Basis.combinations(nbits, nocc), H.fock_words(nbits, nocc)
+    for omega, sign in ((0j, 1.0), (-0.75 + 0.25j, -1.0)):
+        _same(core.build_ham_i(b, ht, ut, omega=omega, ham_sign=sign),
+              o.build_ham_i(fock, ht, ut, omega=omega, ham_sign=sign))
+
+
+@pytest.mark.parametrize("nv,nc,nocc", [(1, 1, 0), (7, 6, 3), (10, 2, 5), (26, 6, 2), (27, 6, 1), (40, 6, 1)])
+def test_few_corehole_terms_in_both_layouts(core, nv, nc, nocc):
+    ht, ut = _few_terms(nv + nc, nv)
+    tr = _few_terms(nv + nc, nv + 1)[0]
+    fi, fn = H.fock_words(nv, nocc), H.fock_words(nv, nocc + 1)
+    bi, bn = core.Basis.combinations(nv, nocc), core.Basis.combinations(nv, nocc + 1)
+    perm = core.corehole_permutation(len(fn), nc)
+    for lay, p in (("reference", None), ("interleaved", perm)):
+        for omega, sign in ((0j, 1.0), (1.5 + 0.5j, -1.0)):
+            _same(core.build_ham_n(bn, nv, nc, ht, ut, omega=omega, ham_sign=sign, layout=lay),
+                  o.build_ham_n(fn, nv, nc, ht, ut, omega=omega, ham_sign=sign), p, p)
+        _same(core.build_transop_i(bn, bi, nv, nc, tr, layout=lay),
+              o.build_transop_i(fn, fi, nv, nc, tr), p, None)
+        _same(core.build_transop_f(bi, bn, nv, nc, tr, layout=lay),
+              o.build_transop_f(fi, fn, nv, nc, tr), None, p)
+
+
+def test_few_terms_on_incomplete_bases(core):
+    """Words left out, at the end, at the front and inside: columns are found by search."""
+    ht, ut = _few_terms(12, 3)
+    fock = H.fock_words(12, 6)
+    for part in (fock[:-1], fock[1:], fock[::3], np.delete(fock, 400)):
+        part = part.copy()
+        _same(core.build_ham_i(core.Basis.from_words(part, 12), ht, ut), o.build_ham_i(part, ht, ut))
+
+
+def test_a_few_long_rows_among_short_ones(core):
+    """Terms on 14 of 20 orbitals: rows with all six electrons there are longer than the
+    plan's lists. By the largest share of rows that a term of each group survives on, the mean
+    row has 61 entries, so the plan's count is what finds them."""
+    ht, ut = _terms(14, 3, 4000, density=1.0)
+    ut = ut[:4090 - len(ht)]
+    fock = H.fock_words(20, 6)
+    R = o.build_ham_i(fock, ht, ut)
+    assert np.diff(R.rowptr).max() > 255
+    _same(core.build_ham_i(core.Basis.combinations(20, 6), ht, ut), R)
+
+
+@pytest.mark.parametrize("space,nv,nocc", [("i", 33, 4), ("i", 40, 3), ("i", 24, 4), ("n", 26, 2), ("n", 36, 2)])
+def test_matrix_free_apply_of_few_terms_on_many_rows(core, space, nv, nocc):
+    """Hoppings and densities of one sign, so no sum cancels: row by row within
+    (entries + terms on the diagonal + 4) eps of sum |value| |x|, in 32- and 64-bit
+    words, by four and by sixteen waves."""
+    import torch
+    nc = 6 if space == "n" else 0
+    rng = np.random.default_rng(nv)
+    k = nv + nc
+    orb = np.unique(np.linspace(0, k - 1, 7).round().astype(int))
+    ht = [[i + 1, j + 1, *rng.normal(size=2)] for i in orb for j in orb if i < j]
+    ht += [[j, i, re, -im] for i, j, re, im in ht]
+    ut = [[i + 1, j + 1, j + 1, i + 1, -rng.uniform(0.5, 2.0), 0.0] for i in orb for j in orb if i < j][:14]
+    N = nocc + (space == "n")
+    fock, b = H.fock_words(nv, N), core.Basis.combinations(nv, N)
+    if space == "i":
+        op, R = core.mf_ham_i(b, ht, ut), o.build_ham_i(fock, ht, ut)
+    else:
+        op, R = core.mf_ham_n(b, nv, nc, ht, ut), o.build_ham_n(fock, nv, nc, ht, ut)
+    # 56 terms in at most 43 groups: the rule's line
+    assert R.m * (5e-4 + 2.2e-6 * 56) + 0.004 * 56 - 3.0 > 0.05 * 43
+    x = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
+    y0 = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
+    y = op.apply(torch.from_numpy(x).cuda(), torch.from_numpy(y0).cuda()).cpu().numpy()
+    rp, c, v = (np.asarray(q) for q in (R.rowptr, R.cols, R.vals))
+    size = np.zeros(R.m)
+    rows = np.repeat(np.arange(R.m), np.diff(rp))
+    np.add.at(size, rows, 2.0 * np.abs(v) * np.abs(x[c]))
+    size += np.abs(y0)
+    eps = np.finfo(float).eps
+    assert np.all(np.abs(y - o.matvec(R, x, y0)) <= (np.diff(rp) + 14 + 4) * eps * size)
