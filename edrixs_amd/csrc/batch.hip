@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256) void k_spmm_il(int64_t m, int K, const int64_t
 // one XCD (blockIdx.x % 8) sweep one contiguous eighth of the rows, so rows
 // that gather the same X lines share that XCD's L2; otherwise consecutive
 // 16-row groups go to consecutive workgroups, i.e. to all eight XCDs.
-template <int NPL, class VP, class XT, class ACC, bool SPLIT, bool TAIL>
+template <int NPL, class VP, class XT, class ACC, bool SPLIT>
 __global__ __launch_bounds__(256) void k_spmm_rl(int64_t m, int K, const int64_t *__restrict__ rowptr,
                                                  const int32_t *__restrict__ cols, VP vals,
                                                  const double2 *__restrict__ diag,
@@ -378,9 +378,8 @@ __global__ __launch_bounds__(256) void k_spmm_rl(int64_t m, int K, const int64_t
             if (k >= K) continue;
             double2 s = make_double2(0, 0);
             for (int g = 0; g < 16; ++g) s = cadd(s, red[(g * NPL + q) * 16 + ll]);
-            part_put<TAIL>(e.partials + (int64_t)blockIdx.x * K + k, s);
+            e.partials[(int64_t)blockIdx.x * K + k] = s;
         }
-        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -421,8 +420,10 @@ int elem_grid_x(int64_t n) {
     return (int)g;
 }
 
-// Workgroups per 16 right-hand sides of a step's vector update: see
-// step_vec_blocks.
+// Workgroups per 16 right-hand sides of a step's vector update: up to 2^17 rows no more
+// than CUs, whose partials are sooner summed.  Us a step against eight a CU: one vector,
+// 24,310 rows 23.2, 23.8, 48,620 28.6, 30.2, 92,378 37.1, 37.4; sixteen, 48,620 48.7, 50.0,
+// 68,640 73.2, 74.6; 145,860 rows 90.3 both.
 int step_elem_grid_x(int64_t n) {
     const int g = elem_grid_x(n);
     return n <= (1 << 17) ? std::min(g, edx::num_cus()) : g;
@@ -914,13 +915,6 @@ int bsched_blocks(const edx_csr *a, BSched sched) {
     return bspmm_blocks(a->m);
 }
 
-// Passes (blockIdx.y) of a schedule's launch.
-int bsched_passes(int K, BSched sched) {
-    if (sched.rl == 3) return 1;
-    if (sched.rl == 1) return (K + 16 * sched.p - 1) / (16 * sched.p);
-    return sched.rl ? (K + 15) / 16 : (K + BKT - 1) / BKT;
-}
-
 // Whether the capped grids walk a matrix in parts of a few passes, all XCDs in
 // the same part, instead of an eighth of it each.  Partners a moved electron
 // away then meet in the last-level cache, which eight far windows overflow once
@@ -984,30 +978,24 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
         const int npl = sched.p;
         dim3 grid((unsigned)nb, (unsigned)((K + 16 * npl - 1) / (16 * npl)));
         const int xmap = nb % 8 == 0 && xcd_map_enabled();
-#define EDX_RLT(NP, TL)                                                                            \
+#define EDX_RL(NP)                                                                                 \
+    case NP:                                                                                       \
         if (precision == EDX_C128)                                                                 \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const double2 *, double2, double, false, TL>), grid,      \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const double2 *, double2, double, false>), grid,      \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const double2 *)a->d_vals, nullptr, X64, X64, e, xmap);           \
         else if (precision == EDX_C64)                                                             \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, float2, float, false, TL>), grid,         \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, float2, float, false>), grid,         \
                                dim3(256), 0, stream(), a->m, K, a->d_rowptr, a->d_cols,            \
                                (const float2 *)a->d_vals32, nullptr, X32, X64, e, xmap);          \
         else if (precision == EDX_C128I)                                                           \
-            hipLaunchKernelGGL((k_spmm_rl<NP, IdxPtr, double2, double, true, TL>), grid, dim3(256), 0,  \
+            hipLaunchKernelGGL((k_spmm_rl<NP, IdxPtr, double2, double, true>), grid, dim3(256), 0,  \
                                stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,                  \
                                IdxPtr{a->d_off_idx, a->d_vtab}, a->d_diag, X64, X64, e, xmap);     \
         else                                                                                       \
-            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, double2, double, true, TL>), grid,        \
+            hipLaunchKernelGGL((k_spmm_rl<NP, const float2 *, double2, double, true>), grid,        \
                                dim3(256), 0, stream(), a->m, K, a->d_off_rowptr, a->d_off_cols,    \
-                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e, xmap);
-#define EDX_RL(NP)                                                                                 \
-    case NP:                                                                                       \
-        if (e.tail.count) {                                                                        \
-            EDX_RLT(NP, true)                                                                      \
-        } else {                                                                                   \
-            EDX_RLT(NP, false)                                                                     \
-        }                                                                                          \
+                               (const float2 *)a->d_off_vals32, a->d_diag, X64, X64, e, xmap);     \
         break;
         switch (npl) {
             EDX_RL(1)
@@ -1016,7 +1004,6 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
             EDX_RL(8)
             default: return set_error(EDX_ERR_ARG, "bad RHS tile %d", 16 * npl);
         }
-#undef EDX_RLT
 #undef EDX_RL
     } else {
         const int G = sched.p;
@@ -1108,9 +1095,7 @@ int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const floa
                          "form, the indexed precision and 2 <= K <= 4");
     if (sched.rl == 4 && !packed_spmm_ok(a, precision))
         return set_error(EDX_ERR_ARG, "multi-RHS schedule 4 needs the packed indexed form");
-    if (sched.rl == 2 || sched.rl == 4 ||
-        !tail_fits(bsched_blocks(a, sched), bsched_passes(K, sched), K))
-        e.tail.count = nullptr;
+    if (sched.rl || !product_tail(bsched_blocks(a, sched), K)) e.tail.count = nullptr;
     if (nblocks_out) *nblocks_out = e.tail.count ? 0 : bsched_blocks(a, sched);
     // the packed words read 4 bytes of index per nonzero instead of 6
     const double bytes = sched.rl == 3 ? fac_bytes_k(a, K, e.z != nullptr, e.dvec != nullptr)
@@ -1383,7 +1368,7 @@ int baxpy_norm_step(int64_t n, int K, double2 *y, const double2 *x, const double
     const ELaunch el = elaunch(n, K);
     const dim3 grid(nbx, el.grid.y);
     t.op = TAIL_BETA;
-    if (tail_fits(nbx, el.grid.y, K)) {
+    if (update_tail(nbx, K, n)) {
         hipLaunchKernelGGL(k_baxpy_norm<true>, grid, el.block, 0, edx::stream(), n, K, y, x, a,
                            partials, t);
         EDX_LAUNCH_CHECK();

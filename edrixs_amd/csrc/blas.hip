@@ -18,13 +18,6 @@ int vec_blocks(int64_t n) {
     return (int)g;
 }
 
-// Workgroups of a step's vector update: a vector of up to 2^17 rows takes few
-// enough for the update to end with the step's scalar work.
-int step_vec_blocks(int64_t n) {
-    const int g = vec_blocks(n);
-    return n <= (1 << 17) ? std::min(g, edx::num_cus()) : g;
-}
-
 // sum of partials[0, nb) by one block; returns the total in thread 0
 __device__ double2 reduce_partials(const double2 *partials, int nb) {
     __shared__ double sx[VB], sy[VB];
@@ -94,7 +87,7 @@ int axpy_norm_step(int64_t n, double2 *y, const double2 *x, const double *a, dou
                    const int *run, StepTail t, int nb) {
     hipStream_t s = edx::stream();
     t.op = TAIL_BETA;
-    if (tail_fits(nb, 1, 1)) {
+    if (update_tail(nb, 1, n)) {
         hipLaunchKernelGGL(k_axpy_norm<true>, dim3(nb), dim3(VB), 0, s, n, y, x, a, partials, run, t);
         EDX_LAUNCH_CHECK();
         return EDX_OK;

@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256, WPE) void k_spmv_fac(FacArgs f, const double2 
 // walks the valence rows part after part (bspmm_part), XCD-contiguous eighths
 // of each, 4 (64 / NC) valence rows per workgroup per pass; dot partials per
 // workgroup and right-hand side.
-template <int NC, int K, bool TAIL>
+template <int NC, int K>
 __global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__restrict__ X, BEpi e,
                                                   int64_t part) {
     extern __shared__ double2 s_tab[];
@@ -489,10 +489,9 @@ __global__ __launch_bounds__(256) void k_spmm_fac(FacArgs f, const double2 *__re
         __syncthreads();
         if (threadIdx.x < K) {
             const int k = threadIdx.x;
-            part_put<TAIL>(e.partials + (int64_t)blockIdx.x * K + k,
-                           cadd(cadd(red[0][k], red[1][k]), cadd(red[2][k], red[3][k])));
+            e.partials[(int64_t)blockIdx.x * K + k] =
+                cadd(cadd(red[0][k], red[1][k]), cadd(red[2][k], red[3][k]));
         }
-        step_tail<TAIL>(e.tail, e.partials);
     }
 }
 
@@ -569,22 +568,18 @@ int fac_spmm_launch(const edx_csr *a, int K, const double2 *X, const BEpi &e, in
     const int64_t mv = a->m / a->nc_slots, pass = fac_rows_per_block(a->nc_slots) * nb;
     const int64_t part = bspmm_part(a, K, e) ? 4 * pass : std::max<int64_t>(mv, 1);
     if (a->m == 0) return EDX_OK;
-#define EDX_FAC_CASE(KK)                                                                          \
-    case KK:                                                                                      \
-        if (e.tail.count)                                                                         \
-            hipLaunchKernelGGL((k_spmm_fac<6, KK, true>), dim3(nb), dim3(256), lds, stream(), f, X, \
-                               e, part);                                                                \
-        else                                                                                      \
-            hipLaunchKernelGGL((k_spmm_fac<6, KK, false>), dim3(nb), dim3(256), lds, stream(), f, X, \
-                               e, part);                                                                \
-        break;
     switch (K) {
-        EDX_FAC_CASE(2)
-        EDX_FAC_CASE(3)
-        EDX_FAC_CASE(4)
+        case 2:
+            hipLaunchKernelGGL((k_spmm_fac<6, 2>), dim3(nb), dim3(256), lds, stream(), f, X, e, part);
+            break;
+        case 3:
+            hipLaunchKernelGGL((k_spmm_fac<6, 3>), dim3(nb), dim3(256), lds, stream(), f, X, e, part);
+            break;
+        case 4:
+            hipLaunchKernelGGL((k_spmm_fac<6, 4>), dim3(nb), dim3(256), lds, stream(), f, X, e, part);
+            break;
         default: return set_error(EDX_ERR_ARG, "factored multi-RHS product for K = %d not built", K);
     }
-#undef EDX_FAC_CASE
     EDX_LAUNCH_CHECK();
     return EDX_OK;
 }

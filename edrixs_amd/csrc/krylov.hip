@@ -111,7 +111,7 @@ struct KrylovRun {
     int curr = 0, prev = 1;
     StepTail t{};
     KrylovRun(int64_t n_, const KrylovScratch &k_, int maxn_)
-        : n(n_), k(k_), maxn(maxn_), nbv(step_vec_blocks(n_)), v{k_.v, k_.v + n_} {
+        : n(n_), k(k_), maxn(maxn_), nbv(vec_blocks(n_)), v{k_.v, k_.v + n_} {
         t.K = 1;
         t.st = krylov_state(k.S, k.ab, k.ab + maxn + 1, k.run);
     }

@@ -698,7 +698,7 @@ int spmv_launch(const edx_csr *a, int precision, const void *x, const SpmvEpi &e
     if (nblocks_out) *nblocks_out = nb;
     if (a->m == 0) return EDX_OK;
     SpmvEpi e = e_in;
-    if (pipe || !tail_fits(nb, 1, 1)) e.tail.count = nullptr;
+    if (pipe || !product_tail(nb, 1)) e.tail.count = nullptr;
     e.xmap = nb % 8 == 0 && xcd_map_enabled();
     e.lds_tab = precision == EDX_C128I && pipe && a->nvtab <= LDS_TAB_MAX && lds_tab_enabled()
                     ? (int)a->nvtab

@@ -80,11 +80,23 @@ struct StepTail {
     const double *sqn;   // [K] norms of the right-hand sides
 };
 
-// Whether a launch of nbx workgroups (partials per right-hand side) times ny
-// ends with a tail: few enough arrivals, and few enough partials that a wave's
-// sum of one right-hand side takes a few loads.
-bool tail_fits(int64_t nbx, int ny, int K) {
-    return nbx * ny <= 1024 && nbx * (K == 1 ? 1 : 2) <= 1024;
+// Whether a product's launch of nbx workgroups, each with a partial for K right-hand
+// sides, ends with a tail.  The four waves of the last one sum a right-hand side each, so
+// a fifth waits; a single one they share.  Measured, us a step with the tail and without:
+// one vector, 462 to 24,310 rows 13.5 to 15.4, 14.2 to 16.9; two vectors, 174
+// partials 17.4, 18.3, 297 18.5, 18.5, 403 19.3, 18.4; four, 108 18.9, 19.6, 174 19.7,
+// 19.7, 215 19.8, 19.5; eight, 29 20.0, 19.9, 403 26.9, 22.8.
+bool product_tail(int64_t nbx, int K) {
+    return K == 1 ? nbx <= 1024 : K <= 4 && nbx * K <= 640;
+}
+
+// The same for the update of K interleaved vectors over n rows, whose workgroups have up
+// to sixteen waves.  Measured the same way, without tails of the product: twelve vectors,
+// 75 partials 25.3, 25.8, 101 24.0, 23.8; four, 161 23.6, 24.1, 256 (18,018 rows) 26.5,
+// 26.4; two, 256 22.3, 23.3, but over 38,610 rows 30.8, 30.6; 24 vectors, 8 partials
+// 25.9, 25.6, 256 (48,620 rows) 76.5, 67.0.
+bool update_tail(int64_t nbx, int K, int64_t n) {
+    return K == 1 ? nbx <= 1024 : K <= 16 && nbx * K <= 900 && n <= 32768;
 }
 
 // TAIL: the kernel is the instance for launches with a tail.  (The others stay

@@ -40,3 +40,12 @@ def test_recurrences_match_the_oracle_and_repeat(nbits, nocc, K, precision):
         assert abs(nr[k] - rn) <= 1e-13 * rn
         a1, b1, _ = core.build_krylov(A, Vd[k].contiguous(), steps, precision)
         assert np.abs(a1 - ra).max() <= tol and np.abs(b1 - rb).max() <= tol
+
+
+@pytest.mark.parametrize("nbits,nocc", [(10, 5), (13, 6), (14, 7), (15, 7), (16, 8)])
+@pytest.mark.parametrize("K", [3, 4, 8, 12, 16])
+def test_blocks_around_the_widths_of_the_tails(nbits, nocc, K):
+    """Four vectors at 640 partials, twelve and sixteen at 900, and more, of the product and
+    of the update."""
+    test_recurrences_match_the_oracle_and_repeat(nbits, nocc, K, "c128")
+
