@@ -1047,15 +1047,19 @@ int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, con
     return EDX_OK;
 }
 
+constexpr int64_t FAC_MIN_ROWS = 28000;
+
 // The schedule the mean row length and K suggest (used below TUNE_MIN_ROWS
 // rows, where products are too short to time).
 BSched bspmm_rule(const edx_csr *a, int precision, int K, const BEpi &e) {
-    // A few vectors over the slot-factored form: an H_v entry is read once for
-    // its six rows (K = 3 over 68,640 rows: 24 us, row-split 43 us).  Solves that
+    // A few vectors over the slot-factored form: an H_v entry is read once for its six
+    // rows, by waves that walk long rows while few of them fill the chip.  Us a step of
+    // three vectors, factored and row-split: 2,772 rows 26.4, 19.6, 18,018 27.6, 24.3, 38,610
+    // 29.2, 35.2, 68,640 32.9, 57.6 (two: 18,018 25.2, 22.4, 38,610 26.5, 30.6).  Solves that
     // stop at a tolerance (shifts in the epilogue or the tail) keep the row-split
     // sums: where they stop, and so their solutions to 1e-9, hangs on the last bits.
     const bool solve = e.c2 || e.tail.nshift;
-    if (!solve && fac_spmm_ok(a, precision, K)) return BSched{3, 4};
+    if (!solve && a->m >= FAC_MIN_ROWS && fac_spmm_ok(a, precision, K)) return BSched{3, 4};
     if (K >= 8) {
         const int kp = K < RL_MAXK ? K : RL_MAXK;
         return BSched{1, kp <= 16 ? 1 : (kp <= 32 ? 2 : (kp <= 64 ? 4 : 8))};

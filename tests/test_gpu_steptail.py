@@ -49,3 +49,24 @@ def test_blocks_around_the_widths_of_the_tails(nbits, nocc, K):
     of the update."""
     test_recurrences_match_the_oracle_and_repeat(nbits, nocc, K, "c128")
 
+
+@pytest.mark.parametrize("nbath,N", [(1, 5), (4, 7), (5, 8)])
+@pytest.mark.parametrize("K", [2, 3, 4])
+def test_small_blocks_over_corehole_matrices(nbath, N, K):
+    """2,772, 20,592 and 38,610 rows: below and above those the factored product takes."""
+    import torch
+    from edrixs_amd import core, siam
+    m = siam.SiamModel(nbath=nbath, nocc=N - 1, seed=2)
+    fn, bn = H.fock_words(m.norb, N), core.Basis.combinations(m.norb, N)
+    A = core.build_ham_n(bn, m.norb, m.ncore, m.hop_n, m.coul_n, layout="interleaved").prepare("c128i")
+    R = o.build_ham_n(fn, m.norb, m.ncore, m.hop_n, m.coul_n)
+    perm = core.corehole_permutation(len(fn), m.ncore)
+    rng = np.random.default_rng(nbath + K)
+    V = rng.normal(size=(K, R.m)) + 1j * rng.normal(size=(K, R.m))
+    al, be, nr = core.build_krylov_batch(A, torch.from_numpy(V[:, perm].copy()).cuda(), 6, "c128i")
+    scale = np.abs(R.vals).sum() / R.m
+    for k in range(K):
+        ra, rb, rn = o.build_krylov(R, V[k], 6)
+        tol = 1e4 * 2.3e-16 * scale
+        assert np.abs(al[k] - ra).max() <= tol and np.abs(be[k] - rb).max() <= tol
+        assert abs(nr[k] - rn) <= 1e-13 * rn
