@@ -463,9 +463,17 @@ __global__ __launch_bounds__(VB) void k_cgs_last(int64_t n, const double2 *V, in
     if (threadIdx.x == 0) partials[blockIdx.x] = nrm;
 }
 
-__global__ __launch_bounds__(VB) void k_cgs_beta(const double2 *partials, int nb, double *beta) {
+// *beta = |w|; with ab, *alpha and it there
+__global__ __launch_bounds__(VB) void k_cgs_beta(const double2 *partials, int nb, double *beta,
+                                                 const double *alpha, double *ab) {
     const double2 s = reduce_partials(partials, nb);
-    if (threadIdx.x == 0) *beta = sqrt(fabs(s.x));
+    if (threadIdx.x != 0) return;
+    const double b = sqrt(fabs(s.x));
+    *beta = b;
+    if (ab) {
+        ab[0] = *alpha;
+        ab[1] = b;
+    }
 }
 
 // *beta = |w| from the nd partials of k_cgs_last, out = w / *beta; 0 past an invariant
