@@ -61,19 +61,19 @@ struct KrylovScratch {
     double2 *v;        // 2 n
     double2 *part;     // max(partials_len, vec_blocks(n))
     KrylovDev *S;
-    double *ab;        // 2 maxn + 2, right behind S (read back with it)
+    double *ab;        // 2 maxn + 2, KRYLOV_HEAD behind S (read back with it)
     int *run;          // maxn + 2
     unsigned *count;   // arrival counters of the step tails
 };
 
-constexpr size_t KRYLOV_HEAD = (sizeof(KrylovDev) + 15) / 16 * 16;
+constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
-inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
+constexpr size_t KRYLOV_HEAD = align256(sizeof(KrylovDev));
 
 size_t krylov_scratch_bytes(int64_t n, int64_t partials_len, int maxn) {
     const int64_t np = std::max<int64_t>(partials_len, vec_blocks(n));
     return align256(2 * (size_t)n * sizeof(double2)) + align256((size_t)np * sizeof(double2)) +
-           align256(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double)) +
+           KRYLOV_HEAD + align256((2 * (size_t)maxn + 2) * sizeof(double)) +
            align256(((size_t)maxn + 2) * sizeof(int)) + align256(TAIL_BYTES);
 }
 
@@ -86,7 +86,7 @@ KrylovScratch krylov_scratch_carve(char *base, int64_t n, int64_t partials_len, 
     base += align256((size_t)np * sizeof(double2));
     k.S = (KrylovDev *)base;
     k.ab = (double *)(base + KRYLOV_HEAD);
-    base += align256(KRYLOV_HEAD + (2 * (size_t)maxn + 2) * sizeof(double));
+    base += KRYLOV_HEAD + align256((2 * (size_t)maxn + 2) * sizeof(double));
     k.run = (int *)base;
     base += align256(((size_t)maxn + 2) * sizeof(int));
     k.count = (unsigned *)base;
@@ -917,7 +917,8 @@ int edx_lanczos_refine(const edx_csr *h, int precision, int nev, int maxiter, do
 
 namespace {
 
-constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(64) << 20;
+// 64 MB for the run, and the arrival counters of its step tails
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t(64) << 20) + align256(TAIL_BYTES);
 __device__ __align__(256) char scratch[NOALLOC_SCRATCH_BYTES];
 
 std::mutex g_scratch_mu;

@@ -53,3 +53,37 @@ def test_noalloc_krylov_equals_allocating_entry_point():
     # more than the static array holds: a clear error, nothing run
     with pytest.raises(Exception, match="bytes of scratch"):
         _krylov(core, "edx_build_krylov_noalloc", Hn, "c128", v0, 1 << 23)
+
+
+def test_noalloc_krylov_up_to_the_size_of_its_scratch():
+    """64 MB of vectors, partials, state, history and flags run; 256 bytes more are refused.
+    The bytes a run needs are read from the message of a refused one; the step tails'
+    counters in it (33 of 128 bytes) come on top of the 64 MB."""
+    import re
+    import torch
+    from edrixs_amd import core
+    from tests import helpers as H
+    hop = [[i, i % 6 + 1, 0.5, 0.0] for i in range(1, 7)] + [[i % 6 + 1, i, 0.5, 0.0] for i in range(1, 7)]
+    A = core.build_ham_i(core.Basis.combinations(6, 3), hop, None)
+    v0 = torch.ones(A.n, dtype=torch.complex128, device="cuda")
+    counters = 33 * 128 + 128
+
+    def need(maxn):
+        with pytest.raises(Exception, match="bytes of scratch") as err:
+            _krylov(core, "edx_build_krylov_noalloc", A, "c128", v0, maxn)
+        return int(re.search(r"needs (\d+) bytes", str(err.value)).group(1)) - counters
+    lo, hi = 1, 1 << 22
+    assert need(hi) > 64 << 20
+    fixed = need(hi) - (-(-(2 * hi + 2) * 8 // 256) * 256 + -(-(hi + 2) * 4 // 256) * 256)
+    def size(maxn):
+        return fixed + -(-(2 * maxn + 2) * 8 // 256) * 256 + -(-(maxn + 2) * 4 // 256) * 256
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if size(mid) <= 64 << 20 else (lo, mid)
+    assert size(lo) <= 64 << 20 < size(lo + 1)
+    assert need(lo + 1) == size(lo + 1)
+    a, b, nrm = _krylov(core, "edx_build_krylov_noalloc", A, "c128", v0, lo)
+    a2, b2, nrm2 = _krylov(core, "edx_build_krylov", A, "c128", v0, 64)
+    k = len(a2)
+    assert len(a) >= k > 0 and nrm == nrm2
+    assert np.array_equal(a[:k], a2) and np.array_equal(b[:k], b2)
