@@ -204,7 +204,7 @@ __device__ __forceinline__ double2 plan_big(const Plan<W> &p, int first, int ste
             any |= ok;
             acc += ok ? d.x : -0.0;
         }
-        return make_double2(acc, p.dens_y);
+        return make_double2(acc, any ? p.dens_y : -0.0);   // -0.0 + omega is omega bit for bit
     }
     double2 acc = make_double2(-0.0, -0.0);
 #pragma unroll 2

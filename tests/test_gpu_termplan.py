@@ -311,3 +311,22 @@ def test_matrix_free_apply_of_few_terms_on_many_rows(core, space, nv, nocc):
     size += np.abs(y0)
     eps = np.finfo(float).eps
     assert np.all(np.abs(y - o.matvec(R, x, y0)) <= (np.diff(rp) + 14 + 4) * eps * size)
+
+
+@pytest.mark.parametrize("im", [0.0, -0.0])
+@pytest.mark.parametrize("order", [0, 1])
+def test_rows_with_omega_alone_on_the_diagonal_keep_its_bits(core, im, order):
+    """More than 24 density terms, none of which survives on rows without a pair of
+    electrons among the first nine orbitals: there the entry is omega itself, signs of
+    zeros included."""
+    nbits, nocc = 16, 4
+    pairs = [(i, j) for i in range(1, 10) for j in range(i + 1, 10)][:30]
+    coul = [[i, j, j, i, 0.5, im] if order else [i, j, i, j, 0.5, im] for i, j in pairs]
+    omega = complex(0.25, -0.0)
+    A = core.build_ham_i(core.Basis.combinations(nbits, nocc), None, coul, omega=omega, ham_sign=-1.0)
+    R = o.build_ham_i(H.fock_words(nbits, nocc), None, coul, omega=omega, ham_sign=-1.0)
+    rp, cols, vals = A.download()
+    ref, got = (np.ascontiguousarray(v).view(np.float64) for v in (R.vals, vals))
+    assert np.array_equal(rp, np.asarray(R.rowptr)) and np.array_equal(cols, np.asarray(R.cols))
+    assert np.sum(np.asarray(R.vals) == omega) > 20
+    assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
