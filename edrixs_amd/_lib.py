@@ -46,6 +46,8 @@ _SIGS = {
     "edx_last_error": (ctypes.c_char_p, []),
     "edx_init": (_I, [_I]),
     "edx_mem_in_use": (_I, [ctypes.POINTER(_I64)]),
+    "edx_mem_reserved": (_I, [ctypes.POINTER(_I64), ctypes.POINTER(_I64)]),
+    "edx_mem_trim": (_I, []),
     "edx_set_stream": (_I, [_P]),
     "edx_basis_combinations": (_I, [_I, _I, _PP]),
     "edx_basis_from_words": (_I, [_P, _I64, _I, _PP]),

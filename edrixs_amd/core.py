@@ -65,6 +65,17 @@ def device():
     return torch().device("cuda", 0)
 
 
+def _zeros(shape, dev):
+    """complex128 zeros; where torch finds no room, the library's kept blocks
+    go back to the driver first."""
+    T = torch()
+    try:
+        return T.zeros(shape, dtype=T.complex128, device=dev)
+    except T.cuda.OutOfMemoryError:
+        mem_trim()
+        return T.zeros(shape, dtype=T.complex128, device=dev)
+
+
 def as_terms2(t):
     if t is None or len(t) == 0:
         return np.zeros(0, dtype=T2)
@@ -209,7 +220,7 @@ class CSRMatrix:
         return y
 
     def matvec(self, x, precision="c128"):
-        y = torch().zeros(self.m, dtype=torch().complex128, device=x.device)
+        y = _zeros(self.m, x.device)
         return self.spmv(x, y, precision)
 
     def spmm(self, X, Y, precision="c128"):
@@ -298,10 +309,9 @@ def build_transop_f(basis_f, basis_n, num_val_orbs, num_core_orbs, trans, precis
 def lanczos_eigs(H, nev, maxiter=500, tol=1e-10, seed=1, deflate=True, nvec=None,
                  precision="c128"):
     """Lowest nev eigenvalues (numpy) and nvec eigenvectors (device tensor, nvec x n)."""
-    T = torch()
     nvec = nev if nvec is None else nvec
     ev = np.zeros(nev)
-    vecs = T.zeros((max(nvec, 1), H.n), dtype=T.complex128, device=device())
+    vecs = _zeros((max(nvec, 1), H.n), device())
     it = ctypes.c_int()
     _lib.call("edx_lanczos_eigs", H._h, _prec(precision), nev, maxiter, float(tol),
               int(seed), int(bool(deflate)), nvec, _ptr(ev), _dptr(vecs), ctypes.byref(it))
@@ -314,10 +324,9 @@ def lanczos_ground(H, nev=1, maxiter=500, tol=1e-10, seed=1, nvec=None, precisio
     reorthogonalization, Ritz vectors from a second run of the recurrence.
     One copy of a degenerate level.  Returns (evals, evecs (nvec x n device
     tensor), steps)."""
-    T = torch()
     nvec = nev if nvec is None else nvec
     ev = np.zeros(nev)
-    vecs = T.zeros((max(nvec, 1), H.n), dtype=T.complex128, device=device())
+    vecs = _zeros((max(nvec, 1), H.n), device())
     it = ctypes.c_int()
     _lib.call("edx_lanczos_ground", H._h, _prec(precision), nev, maxiter, float(tol), int(seed),
               nvec, _ptr(ev), _dptr(vecs), ctypes.byref(it))
@@ -330,11 +339,10 @@ def trlan_eigs(H, nev, ncv=None, maxiter=500, tol=1e-10, seed=1, deflate=True, n
     ``diag_ham_arpack`` src/arpack.f90:2-112).  ncv: basis size (at least
     2 nev + 16 is used); maxiter: restarts.  Returns (evals,
     evecs (nvec x n device tensor), products with H, converged values)."""
-    T = torch()
     nvec = nev if nvec is None else nvec
     ncv = nev + 2 if ncv is None else ncv
     ev = np.zeros(nev)
-    vecs = T.zeros((max(nvec, 1), H.n), dtype=T.complex128, device=device())
+    vecs = _zeros((max(nvec, 1), H.n), device())
     it, nc = ctypes.c_int(), ctypes.c_int()
     _lib.call("edx_trlan_eigs", H._h, _prec(precision), nev, ncv, maxiter, float(tol), int(seed),
               int(bool(deflate)), nvec, _ptr(ev), _dptr(vecs), ctypes.byref(it), ctypes.byref(nc))
@@ -343,11 +351,10 @@ def trlan_eigs(H, nev, ncv=None, maxiter=500, tol=1e-10, seed=1, deflate=True, n
 
 def lanczos_refine(H, start, nev, maxiter=200, tol=1e-10, nvec=None, precision="c128"):
     """Lanczos started from the sum of the rows of ``start`` (k x n device tensor)."""
-    T = torch()
     nvec = nev if nvec is None else nvec
     st = start.contiguous()
     ev = np.zeros(nev)
-    vecs = T.zeros((max(nvec, 1), H.n), dtype=T.complex128, device=device())
+    vecs = _zeros((max(nvec, 1), H.n), device())
     it = ctypes.c_int()
     _lib.call("edx_lanczos_refine", H._h, _prec(precision), nev, maxiter, float(tol),
               st.shape[0], _dptr(st), nvec, _ptr(ev), _dptr(vecs), ctypes.byref(it))
@@ -358,11 +365,10 @@ def block_lanczos_eigs(H, nev, maxblocks=60, tol=1e-10, seed=1, nvec=None, preci
     """Lowest nev eigenpairs by block Lanczos (blocks of 8, reorthogonalization
     on the FP64 matrix cores).  Returns (evals, evecs (nvec x n device tensor),
     block steps, residual estimates)."""
-    T = torch()
     nvec = nev if nvec is None else nvec
     ev = np.zeros(nev)
     res = np.zeros(nev)
-    vecs = T.zeros((max(nvec, 1), H.n), dtype=T.complex128, device=device())
+    vecs = _zeros((max(nvec, 1), H.n), device())
     nb = ctypes.c_int()
     _lib.call("edx_block_lanczos_eigs", H._h, _prec(precision), nev, maxblocks, float(tol),
               int(seed), nvec, _ptr(ev), _dptr(vecs), ctypes.byref(nb), _ptr(res))
@@ -512,7 +518,7 @@ class MatrixFreeOp:
         return y
 
     def matvec(self, x):
-        y = torch().zeros(self.m, dtype=torch().complex128, device=x.device)
+        y = _zeros(self.m, x.device)
         return self.apply(x, y)
 
     def build_krylov(self, v0, maxn):
@@ -704,12 +710,11 @@ def shifted_fom(H, b, sigma, projections=(None,), tol=1e-8, maxit=2000, precisio
     ``projections`` lists CSR operators P (``None`` = identity); returns
     ``(outs, iters, res)`` where ``outs[p]`` is a (K, rows(P)) complex128 device
     tensor holding P x_k, and ``res`` the relative residual of each iterate."""
-    T = torch()
     _check_vec(b, H.n)
     sig = np.ascontiguousarray(np.atleast_1d(np.asarray(sigma, dtype=np.complex128)))
     K = len(sig)
     projs = list(projections)
-    outs = [T.zeros((K, P.m if P is not None else H.n), dtype=T.complex128, device=b.device)
+    outs = [_zeros((K, P.m if P is not None else H.n), b.device)
             for P in projs]
     hp = (ctypes.c_void_p * len(projs))(*[P._h if P is not None else None for P in projs])
     op = (ctypes.c_void_p * len(projs))(*[o.data_ptr() for o in outs])
@@ -733,7 +738,7 @@ def shifted_fom_batch(H, B, sigma, projections, tol=1e-8, maxit=2000, precision=
     assert len(projections) == R
     sig = np.ascontiguousarray(np.atleast_1d(np.asarray(sigma, dtype=np.complex128)))
     K = len(sig)
-    outs = [T.zeros((K, P.m if P is not None else H.n), dtype=T.complex128, device=B.device)
+    outs = [_zeros((K, P.m if P is not None else H.n), B.device)
             for P in projections]
     hp = (ctypes.c_void_p * R)(*[P._h if P is not None else None for P in projections])
     op = (ctypes.c_void_p * R)(*[o.data_ptr() for o in outs])
@@ -752,7 +757,6 @@ def shifted_fom_rhs(H, B, sigma, projections, tol=1e-8, maxit=2000, precision="c
     rows, or a block within SPLIT_BLOCK_BYTES), else one recurrence per row
     (a larger interleaved block of a few rows overflows the last-level cache
     and its row-wise product loses to the single-vector ones)."""
-    T = torch()
     B = B.contiguous()
     R = B.shape[0]
     fac_block = 2 <= R <= 4 and _prec(precision) == EDX_C128I and H.factored() is not None
@@ -803,6 +807,19 @@ def mem_in_use():
     v = ctypes.c_int64()
     _lib.call("edx_mem_in_use", ctypes.byref(v))
     return v.value
+
+
+def mem_reserved():
+    """(live, idle): device bytes the library holds in blocks in use, and in
+    freed blocks it keeps for its next allocations."""
+    live, idle = ctypes.c_int64(), ctypes.c_int64()
+    _lib.call("edx_mem_reserved", ctypes.byref(live), ctypes.byref(idle))
+    return live.value, idle.value
+
+
+def mem_trim():
+    """Give the library's kept device blocks back to the driver."""
+    _lib.call("edx_mem_trim")
 
 
 def set_stream(stream=None):

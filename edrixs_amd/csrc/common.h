@@ -21,6 +21,9 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 void *dmalloc(size_t bytes, const char *what);
 void dfree(void *p);
 int64_t mem_in_use();
+// Bytes held from the device: by blocks in use, and by freed ones kept for reuse.
+void mem_reserved(int64_t *live, int64_t *idle);
+void mem_trim();   // gives the kept blocks back
 
 // The stream all library work of the calling thread is queued on: by default
 // the legacy default stream, so it is ordered with torch's default stream; a

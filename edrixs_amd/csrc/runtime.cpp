@@ -41,10 +41,11 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line) {
 // 1 GB: 1.6 ms of kernels, 25 ms a call through hipMalloc / hipFree, 2 ms
 // reusing the blocks).  A block is only kept once the device has finished all
 // work (hipFree waits for the same), so any thread on any stream may have it
-// next.  What is kept is bounded (1/16 of the device's memory, the blocks
-// unused longest go first) and given back when an allocation fails, when little
-// device memory is left for others, and, but for 64 MB, when the last library
-// object is freed.
+// next.  Kept blocks are memory that other users of the device do not get, so
+// they are bounded, on each device, by 1/16 of its memory and by a quarter of
+// what would be free without them, looked at again for every 64 MB freed; the
+// blocks unused longest go first.  All are given back when an allocation here
+// fails and by mem_trim, and all but 64 MB when the last library object is freed.
 namespace {
 
 struct Live {
@@ -53,15 +54,19 @@ struct Live {
 };
 struct Idle {
     void *p;
-    int dev;
     uint64_t freed;      // order of the frees
+};
+struct DevPool {
+    std::multimap<size_t, Idle> idle;   // by allocated size
+    size_t idle_bytes = 0;
+    size_t unlooked = 0;                // bytes freed since the device's memory was looked at
+    size_t limit = 0;                   // bound of idle_bytes found then
 };
 struct Pool {
     std::mutex mu;
     std::unordered_map<void *, Live> live;
-    std::multimap<size_t, Idle> idle;   // by allocated size
-    size_t idle_bytes = 0;
-    int64_t in_use = 0;
+    std::map<int, DevPool> devs;
+    int64_t in_use = 0, live_bytes = 0;   // asked for, allocated
     uint64_t frees = 0;
 };
 Pool &pool() {
@@ -70,36 +75,41 @@ Pool &pool() {
 }
 
 constexpr size_t POOL_SMALL = 64ull << 20;   // kept even when nothing is live
-constexpr size_t POOL_BIG = 256ull << 20;    // blocks this large heed the free memory
 
 size_t pool_cap(size_t bytes) {
     const size_t g = bytes <= (1u << 20) ? 512 : 2u << 20;
     return (bytes + g - 1) / g * g;
 }
 
-// Releases idle blocks, oldest first, until at most keep bytes stay (mu held).
-void pool_trim(Pool &q, size_t keep) {
-    while (q.idle_bytes > keep && !q.idle.empty()) {
-        auto old = q.idle.begin();
-        for (auto it = q.idle.begin(); it != q.idle.end(); ++it)
+// Releases a device's idle blocks, oldest first, until at most keep bytes stay (mu held).
+void pool_trim(DevPool &d, size_t keep) {
+    while (d.idle_bytes > keep && !d.idle.empty()) {
+        auto old = d.idle.begin();
+        for (auto it = d.idle.begin(); it != d.idle.end(); ++it)
             if (it->second.freed < old->second.freed) old = it;
         (void)hipFree(old->second.p);
-        q.idle_bytes -= old->first;
-        q.idle.erase(old);
+        d.idle_bytes -= old->first;
+        d.idle.erase(old);
     }
 }
 
-size_t pool_limit(int dev) {
-    static std::mutex mu;
-    static std::unordered_map<int, size_t> total;
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = total.find(dev);
-    if (it == total.end()) {
+void pool_trim_all(Pool &q, size_t keep) {
+    for (auto &d : q.devs) pool_trim(d.second, keep);
+}
+
+// The bound of the current device's idle bytes (mu held).
+size_t pool_limit(DevPool &d, size_t freed) {
+    d.unlooked += freed;
+    if (!d.limit || d.unlooked >= POOL_SMALL) {
         size_t fr = 0, tot = 0;
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess) (void)hipGetLastError();
-        it = total.emplace(dev, tot).first;
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
+            (void)hipGetLastError();
+            fr = tot = 0;
+        }
+        d.limit = std::max(std::min(tot / 16, (fr + d.idle_bytes) / 4), (size_t)1);
+        d.unlooked = 0;
     }
-    return it->second / 16;
+    return d.limit;
 }
 
 }  // namespace
@@ -110,17 +120,22 @@ void *dmalloc(size_t bytes, const char *what) {
     int dev = 0;
     (void)hipGetDevice(&dev);
     Pool &q = pool();
+    auto take = [&](void *p, size_t size) {
+        q.live[p] = Live{bytes, size, dev};
+        q.in_use += (int64_t)bytes;
+        q.live_bytes += (int64_t)size;
+        return p;
+    };
     {
         std::lock_guard<std::mutex> lk(q.mu);
-        for (auto it = q.idle.lower_bound(cap); it != q.idle.end() && it->first <= cap + cap / 8; ++it)
-            if (it->second.dev == dev) {
-                void *p = it->second.p;
-                q.live[p] = Live{bytes, it->first, dev};
-                q.in_use += (int64_t)bytes;
-                q.idle_bytes -= it->first;
-                q.idle.erase(it);
-                return p;
-            }
+        DevPool &d = q.devs[dev];
+        auto it = d.idle.lower_bound(cap);
+        if (it != d.idle.end() && it->first <= cap + cap / 8) {
+            void *p = take(it->second.p, it->first);
+            d.idle_bytes -= it->first;
+            d.idle.erase(it);
+            return p;
+        }
     }
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, cap);
@@ -128,7 +143,7 @@ void *dmalloc(size_t bytes, const char *what) {
         (void)hipGetLastError();
         {
             std::lock_guard<std::mutex> lk(q.mu);
-            pool_trim(q, 0);
+            pool_trim_all(q, 0);
         }
         e = hipMalloc(&p, cap);
     }
@@ -139,9 +154,7 @@ void *dmalloc(size_t bytes, const char *what) {
         return nullptr;
     }
     std::lock_guard<std::mutex> lk(q.mu);
-    q.live[p] = Live{bytes, cap, dev};
-    q.in_use += (int64_t)bytes;
-    return p;
+    return take(p, cap);
 }
 
 void dfree(void *p) {
@@ -154,32 +167,44 @@ void dfree(void *p) {
         if (it != q.live.end()) {
             l = it->second;
             q.in_use -= (int64_t)l.bytes;
+            q.live_bytes -= (int64_t)l.cap;
             q.live.erase(it);
         }
     }
     int dev = 0;
-    bool keep = l.dev >= 0 && hipGetDevice(&dev) == hipSuccess && dev == l.dev &&
-                hipDeviceSynchronize() == hipSuccess;
-    if (keep && l.cap >= POOL_BIG) {
-        size_t fr = 0, tot = 0;
-        keep = hipMemGetInfo(&fr, &tot) == hipSuccess && fr >= tot / 8;
-    }
+    const bool keep = l.dev >= 0 && hipGetDevice(&dev) == hipSuccess && dev == l.dev &&
+                      hipDeviceSynchronize() == hipSuccess;
     if (!keep) {
         (void)hipGetLastError();
         (void)hipFree(p);
         return;
     }
-    const size_t limit = pool_limit(dev);
     std::lock_guard<std::mutex> lk(q.mu);
-    q.idle.emplace(l.cap, Idle{p, dev, ++q.frees});
-    q.idle_bytes += l.cap;
-    pool_trim(q, q.in_use > 0 ? limit : std::min(limit, POOL_SMALL));
+    DevPool &d = q.devs[dev];
+    d.idle.emplace(l.cap, Idle{p, ++q.frees});
+    d.idle_bytes += l.cap;
+    pool_trim(d, pool_limit(d, l.cap));
+    if (q.in_use == 0) pool_trim_all(q, POOL_SMALL);
 }
 
 int64_t mem_in_use() {
     Pool &q = pool();
     std::lock_guard<std::mutex> lk(q.mu);
     return q.in_use;
+}
+
+void mem_reserved(int64_t *live, int64_t *idle) {
+    Pool &q = pool();
+    std::lock_guard<std::mutex> lk(q.mu);
+    *live = q.live_bytes;
+    *idle = 0;
+    for (auto &d : q.devs) *idle += (int64_t)d.second.idle_bytes;
+}
+
+void mem_trim() {
+    Pool &q = pool();
+    std::lock_guard<std::mutex> lk(q.mu);
+    pool_trim_all(q, 0);
 }
 
 int current_device() { return g_device; }
@@ -223,6 +248,17 @@ int edx_init(int device) {
 int edx_mem_in_use(int64_t *bytes) {
     EDX_CHECK(bytes, EDX_ERR_ARG, "null output");
     *bytes = edx::mem_in_use();
+    return EDX_OK;
+}
+
+int edx_mem_reserved(int64_t *live, int64_t *idle) {
+    EDX_CHECK(live && idle, EDX_ERR_ARG, "null output");
+    edx::mem_reserved(live, idle);
+    return EDX_OK;
+}
+
+int edx_mem_trim(void) {
+    edx::mem_trim();
     return EDX_OK;
 }
 

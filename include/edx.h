@@ -64,6 +64,12 @@ const char *edx_last_error(void);
 int edx_init(int device);
 /* Device-memory bytes currently held by library objects. */
 int edx_mem_in_use(int64_t *bytes);
+/* Device-memory bytes held from the driver: by the blocks in use (their sizes
+ * are rounded up), and by freed blocks kept for the next allocation.  No
+ * reference counterpart. */
+int edx_mem_reserved(int64_t *live, int64_t *idle);
+/* Give the kept blocks back, for a caller whose own allocation failed. */
+int edx_mem_trim(void);
 /* The stream this thread's library work is queued on: a hipStream_t, or NULL
  * for the legacy default stream (the initial choice of every thread).  All
  * launches and host-device copies of the thread's later calls go to it, and a
