@@ -4,18 +4,19 @@ Each request is an impurity model of its own size and parameters.  Requests
 arrive over time; a request is admitted as soon as the HBM it will hold fits
 in the budget next to what the device holds now, and leaves as soon as its
 spectra have converged, freeing its memory for the next one.  What the device
-holds is measured, not estimated: the library's own allocations
-(``edx_mem_in_use``) plus torch's.  What a new request will hold is estimated
-from its dimensions, scaled by what earlier requests of the same size class
-were measured to take (the bytes the device gained over their setup).  Every Krylov
-recurrence of every running request (the three XAS dipole components, the
-RIXS final states of each (incident energy, polarization)) is a member of
-the :class:`core.KrylovGroup` of its request's size class (norb): a step of
-all of them is one SpMV launch over all their rows, so requests that arrive
-while others run share the device instead of queueing behind them.  Each
-round gives every size class about ``slice_s`` of device time (its step
-count is set from its measured step time), so small requests are not held to
-the pace of the largest ones.
+holds is measured, not estimated: the library's own blocks, those it keeps for
+reuse included (``edx_mem_reserved``), plus torch's; kept blocks are given back
+when they stand between a request and the budget.  What a new request will hold
+is estimated from its dimensions, scaled by what earlier requests of the same
+size class were measured to take (the bytes the device gained over their setup).
+Every Krylov recurrence of every running request (the three XAS dipole
+components, the RIXS final states of each (incident energy, polarization)) is a
+member of the :class:`core.KrylovGroup` of its request's size class (norb): a
+step of all of them is one SpMV launch over all their rows, so requests that
+arrive while others run share the device instead of queueing behind them.  Each
+round gives every size class about ``slice_s`` of device time (its step count is
+set from its measured step time), so small requests are not held to the pace of
+the largest ones.
 
 Per-request work that is not a Krylov step -- CSR builds, the ground state
 (Lanczos), the edge estimate and the RIXS multi-shift solve -- runs on a
@@ -119,6 +120,7 @@ class Engine:
         self.used = 0.0         # bytes the running requests were measured to take
         self.scale = {}         # norb -> measured / estimated bytes of past setups
         self.device_bytes = self._device_bytes
+        self.idle_bytes = self._idle_bytes
 
     def group_for(self, norb):
         if norb not in self.groups:
@@ -147,9 +149,25 @@ class Engine:
 
     @staticmethod
     def _device_bytes():
-        """Device memory in use now: the library's allocations plus torch's."""
+        """Device memory in use now: the library's blocks in use plus torch's."""
         import torch
-        return float(core.mem_in_use()) + float(torch.cuda.memory_allocated())
+        return float(core.mem_reserved()[0]) + float(torch.cuda.memory_allocated())
+
+    @staticmethod
+    def _idle_bytes():
+        """Device memory the library keeps in freed blocks."""
+        return float(core.mem_reserved()[1])
+
+    def next_request(self, queue, running, now):
+        """pick() by what the device holds now.  Kept blocks count; where they
+        are all that is in the way, or what is held exceeds the budget, they
+        go back first."""
+        live, idle = self.device_bytes(), self.idle_bytes()
+        req = self.pick(queue, running, now, live + idle)
+        if idle > 0 and (live + idle > self.budget or (req is None and queue)):
+            core.mem_trim()
+            req = self.pick(queue, running, now, self.device_bytes() + self.idle_bytes())
+        return req
 
     def pick(self, queue, running, now, in_use):
         """The queued request to admit now, or None.  The oldest request that
@@ -331,8 +349,8 @@ class Engine:
                     inflight = None
                 # admission against the HBM budget by the bytes the device
                 # holds now, one setup at a time
-                if inflight is None and queue:
-                    req = self.pick(queue, len(active), now(), self.device_bytes())
+                if inflight is None:
+                    req = self.next_request(queue, len(active), now())
                     if req is not None:
                         queue.remove(req)
                         req.admitted = now()
