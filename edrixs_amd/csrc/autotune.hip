@@ -198,9 +198,11 @@ done:
     return rc;
 }
 
+// A block of one vector (a solve's: others take the single-vector product) is
+// keyed as -1, apart from the single-vector choice, whose codes mean lanes.
 int tune_bspmm(const edx_csr *a, int precision, int K, BSched *sched) {
     if (a->m < TUNE_MIN_ROWS || tuning_off()) return EDX_OK;
-    const TuneKey key = tune_key(a, precision, K);
+    const TuneKey key = tune_key(a, precision, K == 1 ? -1 : K);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();

@@ -102,3 +102,47 @@ def test_tuning_key_separates_storage_forms():
     A2.prepare("c128i")
     B2.prepare("c128i")
     assert A2.spmv_lanes("c128i") == ga and B2.spmv_lanes("c128i") == gb
+
+
+ONE_SYSTEM = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np, torch
+from edrixs_amd import core, siam
+m = siam.SiamModel(nbath=8, seed=7)
+bn = core.Basis.combinations(m.norb, m.nocc + 1)
+H = core.build_ham_n(bn, m.norb, m.ncore, m.hop_n, m.coul_n, layout="interleaved")
+H.prepare("c128i")
+i = np.arange(H.n)
+b = torch.from_numpy(np.cos(0.37 * i) + 1j * np.sin(0.11 * i)).cuda()
+for _ in range(2):
+    core.build_krylov(H, b, 3, precision="c128i")          # the single-vector choice
+    # a shift far above the spectrum: a few iterations
+    x, it, res = core.minres_shifted_batch(H, [5000.0 + 1.0j], b[None].contiguous(), 1e-10, 300, "c128i")
+assert it[0] < 300, (it, res)
+r = (5000.0 + 1.0j) * x[0] - H.matvec(x[0].contiguous()) - b
+assert float(r.norm() / b.norm()) < 1e-8, float(r.norm() / b.norm())
+print("lanes", H.spmv_lanes("c128i"))
+"""
+
+
+@pytest.mark.parametrize("lanes", [0, 64, 144, 145])
+def test_one_system_beside_the_single_vector_choice(tmp_path, lanes):
+    """A batch of one solve and a single recurrence on the same large matrix: two choices,
+    whichever is made or read from the file first."""
+    cache = tmp_path / "tune.txt"
+    first = _run(cache)
+    key = "%s %d %d %d 3 1 3 " % (first["device"], first["m"], first["n"], first["nnz"])
+    cache = tmp_path / "one.txt"
+    if lanes:
+        cache.write_text(key + "%d\n" % lanes)
+    env = dict(os.environ, EDX_TUNE_CACHE=str(cache))
+    for _ in range(2):
+        out = subprocess.run([sys.executable, "-c", ONE_SYSTEM, ROOT], env=env, capture_output=True,
+                             text=True, timeout=300)
+        assert out.returncode == 0, out.stderr[-2000:]
+        if lanes:
+            assert out.stdout.strip().endswith("lanes %d" % lanes)
+    lines = [ln for ln in cache.read_text().splitlines() if ln.startswith(key[:-6])]
+    ks = [int(ln.split()[5]) for ln in lines]
+    assert sorted(ks) == [-1, 1], lines
