@@ -198,11 +198,13 @@ done:
     return rc;
 }
 
-// A block of one vector (a solve's: others take the single-vector product) is
-// keyed as -1, apart from the single-vector choice, whose codes mean lanes.
-int tune_bspmm(const edx_csr *a, int precision, int K, BSched *sched) {
+// whole: a solve's product over a block so large that other products walk it in
+// parts (bspmm_part): timed as it runs, and keyed as -K.  So is a block of one
+// vector (a solve's: others take the single-vector product), apart from the
+// single-vector choice, whose codes mean lanes.
+int tune_bspmm(const edx_csr *a, int precision, int K, bool whole, BSched *sched) {
     if (a->m < TUNE_MIN_ROWS || tuning_off()) return EDX_OK;
-    const TuneKey key = tune_key(a, precision, K == 1 ? -1 : K);
+    const TuneKey key = tune_key(a, precision, whole || K == 1 ? -K : K);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();
@@ -258,6 +260,7 @@ int tune_bspmm(const edx_csr *a, int precision, int K, BSched *sched) {
         e.z = Y;
         e.dvec = X;
         e.partials = part;
+        e.tail.nshift = whole;
         if ((rc = bspmm_launch(a, precision, K, X, X32, e, c)) != EDX_OK) goto done;
         (void)hipEventRecord(ev[0], stream());
         for (int r = 0; r < TUNE_REPS; ++r)

@@ -885,7 +885,7 @@ inline bool packed_spmm_ok(const edx_csr *a, int precision) {
     return precision == EDX_C128I && a->d_off_pk && a->nvtab <= LDS_TAB_MAX;
 }
 int tune_spmv(edx_csr *a, int precision);
-int tune_bspmm(const edx_csr *a, int precision, int K, BSched *sched);
+int tune_bspmm(const edx_csr *a, int precision, int K, bool whole, BSched *sched);
 int bsched_blocks(const edx_csr *a, BSched sched);
 
 // One launch of the multi-RHS product with an explicit schedule: row-split
@@ -915,15 +915,18 @@ int bsched_blocks(const edx_csr *a, BSched sched) {
     return bspmm_blocks(a->m);
 }
 
+bool bspmm_large(const edx_csr *a, int K) { return a->m * K * 16 > ((int64_t)256 << 20); }
+
+// A product of a solve, by its shifts in the epilogue or the tail.
+bool bspmm_solve(const BEpi &e) { return e.c2 || e.tail.nshift; }
+
 // Whether the capped grids walk a matrix in parts of a few passes, all XCDs in
 // the same part, instead of an eighth of it each.  Partners a moved electron
 // away then meet in the last-level cache, which eight far windows overflow once
 // the block of vectors is larger than it (256 MB): K = 3 over 15.0M core-hole
 // rows (719 MB) 2.31 ms for 2.40, K = 16 over 2.7M rows (692 MB) 1.16 for 1.19.
 // Solves keep the one order at every size (bspmm_rule).
-bool bspmm_part(const edx_csr *a, int K, const BEpi &e) {
-    return !e.c2 && !e.tail.nshift && a->m * K * 16 > ((int64_t)256 << 20);
-}
+bool bspmm_part(const edx_csr *a, int K, const BEpi &e) { return !bspmm_solve(e) && bspmm_large(a, K); }
 
 int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, const float2 *X32,
                  const BEpi &e, BSched sched) {
@@ -1058,8 +1061,7 @@ BSched bspmm_rule(const edx_csr *a, int precision, int K, const BEpi &e) {
     // 29.2, 35.2, 68,640 32.9, 57.6 (two: 18,018 25.2, 22.4, 38,610 26.5, 30.6).  Solves that
     // stop at a tolerance (shifts in the epilogue or the tail) keep the row-split
     // sums: where they stop, and so their solutions to 1e-9, hangs on the last bits.
-    const bool solve = e.c2 || e.tail.nshift;
-    if (!solve && a->m >= FAC_MIN_ROWS && fac_spmm_ok(a, precision, K)) return BSched{3, 4};
+    if (!bspmm_solve(e) && a->m >= FAC_MIN_ROWS && fac_spmm_ok(a, precision, K)) return BSched{3, 4};
     if (K >= 8) {
         const int kp = K < RL_MAXK ? K : RL_MAXK;
         return BSched{1, kp <= 16 ? 1 : (kp <= 32 ? 2 : (kp <= 64 ? 4 : 8))};
@@ -1092,7 +1094,8 @@ int bspmm(const edx_csr *a, int precision, int K, const double2 *X64, const floa
     if (nblocks_out) *nblocks_out = bspmm_blocks(a->m);
     if (a->m == 0 || K == 0) return EDX_OK;
     BSched sched = bspmm_rule(a, precision, K, e_in);
-    if (a->m >= TUNE_MIN_ROWS) EDX_TRY(tune_bspmm(a, precision, K, &sched));
+    if (a->m >= TUNE_MIN_ROWS)
+        EDX_TRY(tune_bspmm(a, precision, K, bspmm_solve(e) && bspmm_large(a, K), &sched));
     forced_bsched(K, &sched);
     if (sched.rl == 3 && !fac_spmm_ok(a, precision, K))
         return set_error(EDX_ERR_ARG, "the factored multi-RHS product needs the slot-factored "

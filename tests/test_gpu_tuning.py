@@ -146,3 +146,33 @@ def test_one_system_beside_the_single_vector_choice(tmp_path, lanes):
     lines = [ln for ln in cache.read_text().splitlines() if ln.startswith(key[:-6])]
     ks = [int(ln.split()[5]) for ln in lines]
     assert sorted(ks) == [-1, 1], lines
+
+
+LARGE_BLOCK = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np, torch
+from edrixs_amd import core, siam
+m = siam.SiamModel(nbath=8, seed=7)
+bn = core.Basis.combinations(m.norb, m.nocc + 1)
+H = core.build_ham_n(bn, m.norb, m.ncore, m.hop_n, m.coul_n, layout="interleaved")
+H.prepare("c128i")
+K = 64
+assert H.n * K * 16 > 256 << 20
+B = torch.randn(K, H.n, dtype=torch.complex128, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+a, b, _ = core.build_krylov_batch(H, B, 2, "c128i")
+x, it, res = core.minres_shifted_batch(H, np.linspace(4000.0, 6000.0, K) + 1.0j, B, 1e-10, 300, "c128i")
+assert it.max() < 300
+r = (6000.0 + 1.0j) * x[-1] - H.matvec(x[-1].contiguous()) - B[-1]
+assert float(r.norm() / B[-1].norm()) < 1e-8
+"""
+
+
+def test_solves_over_large_blocks_tune_the_walk_they_run(tmp_path):
+    cache = tmp_path / "tune.txt"
+    env = dict(os.environ, EDX_TUNE_CACHE=str(cache))
+    out = subprocess.run([sys.executable, "-c", LARGE_BLOCK, ROOT], env=env, capture_output=True,
+                         text=True, timeout=300)
+    assert out.returncode == 0, out.stderr[-2000:]
+    ks = [int(ln.split()[5]) for ln in cache.read_text().splitlines()]
+    assert 64 in ks and -64 in ks, ks
