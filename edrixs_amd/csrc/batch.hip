@@ -923,9 +923,12 @@ bool bspmm_solve(const BEpi &e) { return e.c2 || e.tail.nshift; }
 // Whether the capped grids walk a matrix in parts of a few passes, all XCDs in
 // the same part, instead of an eighth of it each.  Partners a moved electron
 // away then meet in the last-level cache, which eight far windows overflow once
-// the block of vectors is larger than it (256 MB): K = 3 over 15.0M core-hole
-// rows (719 MB) 2.31 ms for 2.40, K = 16 over 2.7M rows (692 MB) 1.16 for 1.19.
-// Solves keep the one order at every size (bspmm_rule).
+// the block of vectors is larger than it (256 MB).  Us a step whole and in parts:
+// core-hole rows (parts of 4 passes) K = 3, 177 MB 662, 660, 371 MB 1474, 1456, 685 MB
+// 2821, 2740; K = 2, 247 MB 954, 948, 457 MB 1818, 1775.  H_i (8 passes) K = 16, 172 MB
+// 371, 366, 330 MB 774, 761, 660 MB 1608, 1577; K = 8, 165 MB 551, 553, 330 MB 1180,
+// 1169.  Other lengths: K = 3, 685 MB 2 passes 2733, 8 2752, 16 2764; K = 16, 660 MB 2
+// passes 1595, 4 1583, 16 1575.  Solves keep the one order at every size (bspmm_rule).
 bool bspmm_part(const edx_csr *a, int K, const BEpi &e) { return !bspmm_solve(e) && bspmm_large(a, K); }
 
 int bspmm_launch(const edx_csr *a, int precision, int K, const double2 *X64, const float2 *X32,

@@ -18,7 +18,8 @@ int vec_blocks(int64_t n) {
     return (int)g;
 }
 
-// sum of partials[0, nb) by one block; returns the total in thread 0
+// sum of partials[0, nb) by one block; every thread gets the total.  A kernel that
+// calls it twice needs a barrier between the calls.
 __device__ double2 reduce_partials(const double2 *partials, int nb) {
     __shared__ double sx[VB], sy[VB];
     double2 s = make_double2(0, 0);

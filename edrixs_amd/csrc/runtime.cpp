@@ -43,9 +43,10 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line) {
 // work (hipFree waits for the same), so any thread on any stream may have it
 // next.  Kept blocks are memory that other users of the device do not get, so
 // they are bounded, on each device, by 1/16 of its memory and by a quarter of
-// what would be free without them, looked at again for every 64 MB freed; the
-// blocks unused longest go first.  All are given back when an allocation here
-// fails and by mem_trim, and all but 64 MB when the last library object is freed.
+// what would be free without them, looked at again for every eighth of that
+// freed (64 MB at least; a look costs a build of 1 GB 1 % of its time).  The blocks
+// unused longest go first.  All are given back when an allocation here fails and
+// by mem_trim, and all but 64 MB when the last library object is freed.
 namespace {
 
 struct Live {
@@ -100,7 +101,7 @@ void pool_trim_all(Pool &q, size_t keep) {
 // The bound of the current device's idle bytes (mu held).
 size_t pool_limit(DevPool &d, size_t freed) {
     d.unlooked += freed;
-    if (!d.limit || d.unlooked >= POOL_SMALL) {
+    if (!d.limit || d.unlooked >= std::max(POOL_SMALL, d.limit / 8)) {
         size_t fr = 0, tot = 0;
         if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
             (void)hipGetLastError();
