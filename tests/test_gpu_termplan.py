@@ -221,15 +221,49 @@ def _few_terms(n, seed, most=56):
     return hop, coul[:most - len(hop)]
 
 
-def test_calls_of_few_terms_take_the_plan_on_any_number_of_rows():
-    """The sizes below count on it: the rule's constants are read from the source."""
+def _rule(source, pattern):
+    """The numbers of a rule of the library, read from its source: a test that means one
+    route fails when the line moves past its sizes."""
     import os
     import re
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    src = open(os.path.join(root, "edrixs_amd", "csrc", "csr_build.hip")).read()
-    a, t, g = (float(x) for x in re.search(
-        r"const double g = \(([\d.]+) \+ M \* \([^)]*\) - ([\d.]+) \* T\) / ([\d.]+);", src).groups())
-    assert (a - t * 56) / g >= 56          # 56 terms in 56 groups, no rows
+    src = open(os.path.join(root, "edrixs_amd", "csrc", source)).read()
+    return [float(x) for x in re.search(pattern, src).groups()]
+
+
+def _build_max_groups(M, T):
+    a, r, t, u, g = _rule("csr_build.hip", r"const double g = \(([\d.e-]+) \+ M \* \(([\d.e-]+) \+ ([\d.e-]+) \* T\)"
+                                           r" - ([\d.e-]+) \* T\) / ([\d.e-]+);")
+    most = (a + M * (r + t * T) - u * T) / g
+    return most if 16 * most >= T else -1
+
+
+def _mf_max_groups(M, T):
+    r, t, u, a, g = _rule("mf.hip", r"const double g = \(M \* \(([\d.e-]+) \+ ([\d.e-]+) \* T\) \+ ([\d.e-]+) \* T"
+                                    r" - ([\d.e-]+)\) / ([\d.e-]+);")
+    most = (M * (r + t * T) + u * T - a) / g
+    return most if 16 * most >= T else -1
+
+
+def _groups_and_mean_row(n, N, ht, ut):
+    """Groups of the terms, and the rule's measure of a mean row: the largest share of the
+    C(n, N) rows that a term of each group survives on."""
+    from math import comb
+    share = {}
+    for t in list(ht) + list(ut):
+        ops = [int(t[f]) - 1 for f in ("ind1", "ind2", "ind3", "ind4") if f in t.dtype.names]
+        out, into = ops[:len(ops) // 2], ops[len(ops) // 2:]
+        if len(set(out)) < len(out) or len(set(into)) < len(into):
+            continue
+        full, empty = len(out), len(set(into) - set(out))
+        key = sum(1 << q for q in set(out) ^ set(into))
+        share[key] = max(share.get(key, 0.0), comb(n - full - empty, N - full) / comb(n, N))
+    return len(share), sum(share.values())
+
+
+def test_calls_of_few_terms_take_the_plan_on_any_number_of_rows():
+    """The sizes below count on it."""
+    assert _build_max_groups(0, 56) >= 56          # 56 terms in 56 groups, no rows
 
 
 @pytest.mark.parametrize("nbits,nocc", [(1, 0), (1, 1), (5, 5), (6, 1), (8, 4), (11, 5), (15, 12),
@@ -277,6 +311,9 @@ def test_a_few_long_rows_among_short_ones(core):
     fock = H.fock_words(20, 6)
     R = o.build_ham_i(fock, ht, ut)
     assert np.diff(R.rowptr).max() > 255
+    groups, mean = _groups_and_mean_row(20, 6, ht, ut)
+    assert _build_max_groups(R.m, len(ht) + len(ut)) >= groups
+    assert mean <= _rule("csr_build.hip", r"BUILD_MEAN_ROW = ([\d.]+);")[0]
     _same(core.build_ham_i(core.Basis.combinations(20, 6), ht, ut), R)
 
 
@@ -299,8 +336,7 @@ def test_matrix_free_apply_of_few_terms_on_many_rows(core, space, nv, nocc):
         op, R = core.mf_ham_i(b, ht, ut), o.build_ham_i(fock, ht, ut)
     else:
         op, R = core.mf_ham_n(b, nv, nc, ht, ut), o.build_ham_n(fock, nv, nc, ht, ut)
-    # 56 terms in at most 43 groups: the rule's line
-    assert R.m * (5e-4 + 2.2e-6 * 56) + 0.004 * 56 - 3.0 > 0.05 * 43
+    assert _mf_max_groups(R.m, len(ht) + len(ut)) >= 43      # 42 hoppings and the diagonal
     x = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
     y0 = rng.normal(size=R.m) + 1j * rng.normal(size=R.m)
     y = op.apply(torch.from_numpy(x).cuda(), torch.from_numpy(y0).cuda()).cpu().numpy()
@@ -329,4 +365,38 @@ def test_rows_with_omega_alone_on_the_diagonal_keep_its_bits(core, im, order):
     ref, got = (np.ascontiguousarray(v).view(np.float64) for v in (R.vals, vals))
     assert np.array_equal(rp, np.asarray(R.rowptr)) and np.array_equal(cols, np.asarray(R.cols))
     assert np.sum(np.asarray(R.vals) == omega) > 20
+    assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
+
+
+@pytest.mark.parametrize("nbits,nocc,sets,density,sign", [(16, 8, 300, 0.5, 1.0), (16, 8, 300, 0.5, -1.0),
+                                                          (14, 7, 40, 0.1, -1.0), (14, 7, 40, 0.1, 1.0)])
+def test_merged_terms_keep_every_bit_over_the_plan(core, nbits, nocc, sets, density, sign):
+    """Terms in all orders of their operators, as above, on enough rows for the plan: with
+    rows of more than 64 entries and more than 256 groups, and with short ones."""
+    rng = np.random.default_rng(nbits + sets)
+    u = np.zeros((nbits,) * 4, dtype=np.complex128)
+    for q in range(sets):
+        i, j, k, l = rng.integers(0, nbits, size=4)
+        if i == j or k == l:
+            continue
+        v = [0.5, -1.25, rng.normal(), 1j * rng.normal(), rng.normal() + 1j * rng.normal()][q % 5]
+        rel = [(1, -1, -1, 1), (1, 1, 1, 1), (1, -1, 1, -1), (1, 0, 0, 1), (1, 0.3, -0.7, 1)][q % 4 + (q % 7 == 0)]
+        for o4, r in zip([(i, j, k, l), (j, i, k, l), (i, j, l, k), (j, i, l, k)], rel):
+            u[o4] += r * v
+            u[o4[::-1]] += r * np.conj(v)
+    ht = siam.emat_terms(H.random_hermitian_emat(nbits, rng, density=density))
+    ut = siam.umat_terms(u)
+    ut["re"][::9] *= 0.0
+    ut["im"][::4] = -0.0
+    R = o.build_ham_i(H.fock_words(nbits, nocc), ht, ut, omega=-0.0 + 0.5j, ham_sign=sign)
+    groups, mean = _groups_and_mean_row(nbits, nocc, ht, ut)
+    assert _build_max_groups(R.m, len(ht) + len(ut)) >= groups + 1
+    assert mean <= _rule("csr_build.hip", r"BUILD_MEAN_ROW = ([\d.]+);")[0]
+    if sets == 300:
+        assert 64 < np.diff(R.rowptr).max() <= 255 and groups > 256
+    A = core.build_ham_i(core.Basis.combinations(nbits, nocc), ht, ut, omega=-0.0 + 0.5j, ham_sign=sign)
+    rp, cols, vals = A.download()
+    assert np.array_equal(rp, np.asarray(R.rowptr)) and np.array_equal(cols, np.asarray(R.cols))
+    ref = np.ascontiguousarray(R.vals).view(np.float64)
+    got = np.ascontiguousarray(vals).view(np.float64)
     assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
