@@ -152,10 +152,10 @@ __global__ __launch_bounds__(64) void k_mf(BuildParams p, const MfMask *__restri
 // them per row in LDS; each wave sums its share of the diagonal group, whose
 // density terms are the same for every lane and come by scalar loads, and takes
 // entries q, q + NW, ... of each row (sum of the group's terms, column rank, x
-// gather); the partial rows are added in wave order, so the result does not
-// depend on timing.  Bound by integer and LDS instructions (136 groups tested,
+// gather); the partial rows are added as a tree, so the result does not depend on
+// timing.  Bound by integer and LDS instructions (136 groups tested,
 // 24 columns ranked per row; the vectors take 0.03 ms): H_n norb 20, 1.0M rows,
-// 0.44 ms a product, by k_mf 4.38 ms.
+// 0.35 ms a product, by k_mf 4.38 ms.
 template <int NW, int RK, int CK, class W>
 __global__ __launch_bounds__(64 * NW) void k_plan_apply(Plan<W> p, int cap, const double2 *__restrict__ x,
                                                     SpmvEpi e) {
@@ -174,13 +174,14 @@ __global__ __launch_bounds__(64 * NW) void k_plan_apply(Plan<W> p, int cap, cons
         if (i < cap) s_grp[i * PLAN_ROWS + lane] = (uint16_t)g;
     });
     __syncthreads();
-    double2 acc = make_double2(0.0, 0.0);
-    if (p.big >= 0) {   // this wave's share of the diagonal's terms
+    // this wave's share of the diagonal's terms; added after the others, which are smaller
+    double2 diag = make_double2(0.0, 0.0), acc = make_double2(0.0, 0.0);
+    if (p.big >= 0) {
         const bool omega = wave == 0 && p.big == p.diag;
         bool any = omega;
-        double2 v = plan_big<W>(p, wave, NW, w, any);
+        double2 v = plan_big<4, W>(p, wave, NW, w, any);
         if (omega) v = cadd(v, p.omega);
-        if (any && on) acc = cmul(v, x[plan_col<CK, W>(p, w ^ p.groups[p.big].flip, s_rank)]);
+        if (any && on) diag = cmul(v, x[plan_col<CK, W>(p, w ^ p.groups[p.big].flip, s_rank)]);
     }
     for (int i = wave; i < n; i += NW) {
         const int gi = s_grp[i * PLAN_ROWS + lane];
@@ -191,12 +192,20 @@ __global__ __launch_bounds__(64 * NW) void k_plan_apply(Plan<W> p, int cap, cons
         if (gi == p.diag) v = cadd(v, p.omega);
         acc = cadd(acc, cmul(v, xv));
     }
+    acc = cadd(acc, diag);
     s_acc[wave][lane] = acc;
     __syncthreads();
     if (wave != 0) return;
     double2 dot = make_double2(0, 0);
     if (on) {
-        for (int q = 1; q < NW; ++q) acc = cadd(acc, s_acc[q][lane]);
+        double2 part[NW];
+#pragma unroll
+        for (int q = 0; q < NW; ++q) part[q] = s_acc[q][lane];
+#pragma unroll
+        for (int h = NW / 2; h > 0; h /= 2)
+#pragma unroll
+            for (int q = 0; q < h; ++q) part[q] = cadd(part[q], part[q + h]);
+        acc = part[0];
         double2 out = e.c0 ? cmul(*e.c0, acc) : acc;
         if (e.z) out = cadd(out, e.c1 ? cmul(*e.c1, e.z[r]) : e.z[r]);
         e.y[r] = out;
@@ -237,12 +246,13 @@ int mf_waves(int64_t rows) {
 
 // The most groups that T terms on M rows may have for the plan to be the faster product;
 // negative: it is the slower one however they group.  A product's time beyond a launch, in
-// us: the plan takes 0.05 a group and 3 (its waves test all groups, whatever the rows, while
-// the workgroups fill the chip less than twice); k_mf, whose waves take a row each, 0.004 a
-// term and, a row, 5e-4 and 2.2e-6 a term.  Measured (k_mf, plan): 370 terms in 46
-// groups 21.8 and 22.5 us on 1,716 rows, 27.1 and 23.0 on 8,008; 965 in 129, 24.2 and 25.5 on
-// 1,320, 31.6 and 26.1 on 2,772; random terms, 1000 in 500, 37.7 and 46.0 on 6,435, 58.1 and
-// 47.6 on 12,870.
+// us: the plan takes 0.05 a group and 3 (its waves test all groups, whatever the rows,
+// while the workgroups fill the chip less than twice); k_mf, whose waves take a row each,
+// 0.004 a term and, a row, 5e-4 and 2.2e-6 a term.  Measured (k_mf, plan): 370 terms in
+// 46 groups 21.0 and 21.9 us on 2,002 rows, 23.4 and 22.2 on 3,432, 27.1 and 22.5 on 8,008; 965
+// in 129, 24.2 and 24.5 on 1,320, 31.6 and 25.0 on 2,772, 53.2 and 25.7 on 10,296; 2,500 in
+// 160, 27.7 and 37.6 on 120; random terms, 1000 in 500, 37.7 and 46.0 on 6,435, 58.1 and 47.6
+// on 12,870.
 double mf_max_groups(int64_t M, int T) {
     const double g = (M * (5e-4 + 2.2e-6 * T) + 0.004 * T - 3.0) / 0.05;
     return 16.0 * g < T ? -1.0 : g;

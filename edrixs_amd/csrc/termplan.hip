@@ -191,20 +191,37 @@ __device__ __forceinline__ double2 plan_sum(const Plan<W> &p, int tb, int te, W 
     return acc;
 }
 
-// Sum of terms first, first + step, ... of the big group; any: one survives.
-template <class W>
+// Sum of terms first, first + step, ... of the big group; any: one survives.  SUMS: running
+// sums of the density terms; 1 keeps the term order, 4 round less (the rounding of a
+// hundred terms of one sign added one by one is the largest of a row's).
+template <int SUMS, class W>
 __device__ __forceinline__ double2 plan_big(const Plan<W> &p, int first, int step, W w, bool &any) {
     const PlanGroup<W> g = p.groups[p.big];
     if (p.ndens) {
-        double acc = -0.0;
-#pragma unroll 4
-        for (int t = first; t < p.ndens; t += step) {
+        double acc[SUMS];
+#pragma unroll
+        for (int u = 0; u < SUMS; ++u) acc[u] = -0.0;
+        auto take = [&](int t, double &a) {
             const PlanDens<W> d = p.dens[t];
             const bool ok = (w & d.m) == d.v;
             any |= ok;
-            acc += ok ? d.x : -0.0;
+            a += ok ? d.x : -0.0;
+        };
+        int t = first;
+        if constexpr (SUMS == 1) {
+#pragma unroll 4
+            for (; t < p.ndens; t += step) take(t, acc[0]);
+        } else {
+            for (; t + (SUMS - 1) * step < p.ndens; t += SUMS * step)
+#pragma unroll
+                for (int u = 0; u < SUMS; ++u) take(t + u * step, acc[u]);
+            for (; t < p.ndens; t += step) take(t, acc[0]);
+#pragma unroll
+            for (int h = SUMS / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int u = 0; u < h; ++u) acc[u] += acc[u + h];
         }
-        return make_double2(acc, any ? p.dens_y : -0.0);   // -0.0 + omega is omega bit for bit
+        return make_double2(acc[0], any ? p.dens_y : -0.0);   // -0.0 + omega is omega bit for bit
     }
     double2 acc = make_double2(-0.0, -0.0);
 #pragma unroll 2
@@ -311,7 +328,7 @@ __global__ __launch_bounds__(256) void k_plan_fill(Plan<W> p, int cap,
     plan_stage_rank<W>(p, s_rank);
     if (p.big >= 0 && wave == PLAN_WAVES - 1) {
         bool any = false;
-        s_big[lane] = plan_big<W>(p, 0, 1, w, any);
+        s_big[lane] = plan_big<1, W>(p, 0, 1, w, any);
     }
     const int n = plan_expand<PLAN_WAVES, W>(p, w, on, s_cnt, [&](int e, int g) {
         if (e < cap) {
@@ -702,8 +719,9 @@ int plan_make(const PlanSpaces &sp, const PlanTerms &pt, bool omega_on, double2 
             double2 v = vals[t];
             if ((neg & 1) && (neg & PLAN_FLIP_X)) v.x = -v.x;
             if ((neg & 1) && (neg & PLAN_FLIP_Y)) v.y = -v.y;
-            if (t == dg[big].tbeg) dens_y = v.y;
-            if (terms[t].s != 0 || v.y != 0.0 || std::signbit(v.y) != std::signbit(dens_y)) {
+            if (t == dg[big].tbeg) dens_y = exact_sums ? v.y : 0.0;
+            if (terms[t].s != 0 || v.y != 0.0 ||
+                (exact_sums && std::signbit(v.y) != std::signbit(dens_y))) {
                 dens.clear();
                 break;
             }
